@@ -501,7 +501,10 @@ void build_storage(spkhip_handle* h) {
     h->fvec[f] = voff;
     voff += L;
   }
-  h->arena_elems = off;
+  // the trailing update's vector loads may start at a front's last element
+  // and read up to three past it (into accumulator rows that are not stored
+  // or a staged tail that is zeroed)
+  h->arena_elems = off + 4;
   h->vec_elems = voff;
 }
 
@@ -753,10 +756,15 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
         auto& out = dest == 1 ? g2desc : dest == 2 ? carry : gdesc;
         const int big = h->fW[f] > 256 ? 1 : 0;
         const double kk = k1 - k0;
+        constexpr i32 kT = spk::kTile;
+        auto push = [&](i32 pr0, i32 nr, i32 pj0, i32 nc, i32 ntr, i32 mirror) {
+          out.push_back(spk::GemmDesc{f, k0, k1, pr0, nr, pj0, nc, Lc.wg, ntr, big, mirror,
+                                      h->fL[f], h->foff[f]});
+        };
         if (!lub) {
           // symmetric (SPD) fronts stay symmetric: of A22 -= L21 U12 only
           // the tiles on or below the diagonal are computed, one descriptor
-          // per 128-column tile column with rows from that column's start;
+          // per tile column with rows from that column's start;
           // the entries below the column's own square also write their
           // transposes. A rectangle above the diagonal is the transpose of
           // one below it in the same launch (the plan's rectangles pair up
@@ -769,18 +777,18 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
             // descriptor whose every entry lies past its columns and so
             // also writes its transpose; the columns from r0 on follow as
             // tile columns of their own
-            const i32 jl = std::min(r0, j1), ntr = (r1 - r0 + 127) / 128,
-                      ntc = (jl - j0 + 127) / 128;
-            out.push_back(spk::GemmDesc{f, k0, k1, r0, r1 - r0, j0, jl - j0, Lc.wg, ntr, big, 1});
+            const i32 jl = std::min(r0, j1), ntr = (r1 - r0 + kT - 1) / kT,
+                      ntc = (jl - j0 + kT - 1) / kT;
+            push(r0, r1 - r0, j0, jl - j0, ntr, 1);
             Lc.wg += ntr * ntc;
             const double m = r1 - r0, nn = jl - j0;
             Lc.flops += 2.0 * m * nn * kk;
             Lc.elems += 2.0 * m * nn + (m + nn) * kk + m * nn;  // + the transposes
             j0 = jl;
           }
-          for (i32 cj = j0; cj < j1; cj += 128) {
-            const i32 ce = std::min(cj + 128, j1), ntr = (r1 - cj + 127) / 128;
-            out.push_back(spk::GemmDesc{f, k0, k1, cj, r1 - cj, cj, ce - cj, Lc.wg, ntr, big, 1});
+          for (i32 cj = j0; cj < j1; cj += kT) {
+            const i32 ce = std::min(cj + kT, j1), ntr = (r1 - cj + kT - 1) / kT;
+            push(cj, r1 - cj, cj, ce - cj, ntr, 1);
             Lc.wg += ntr;
             const double m = r1 - cj, nn = ce - cj;
             Lc.flops += 2.0 * m * nn * kk;
@@ -788,8 +796,8 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
           }
           return;
         }
-        const i32 ntr = (r1 - r0 + 127) / 128, ntc = (j1 - j0 + 127) / 128;
-        out.push_back(spk::GemmDesc{f, k0, k1, r0, r1 - r0, j0, j1 - j0, Lc.wg, ntr, big, 0});
+        const i32 ntr = (r1 - r0 + kT - 1) / kT, ntc = (j1 - j0 + kT - 1) / kT;
+        push(r0, r1 - r0, j0, j1 - j0, ntr, 0);
         Lc.wg += ntr * ntc;
         const double m = r1 - r0, nn = j1 - j0;
         Lc.flops += 2.0 * m * nn * kk;

@@ -86,7 +86,7 @@ struct BlkDesc {
 
 // Per-launch descriptor of the trailing-update kernel: one rectangle of one
 // front, F[r0:r0+nr, j0:j0+nc] -= F[r0:r0+nr, k0:k1] F[k0:k1, j0:j0+nc],
-// in 128 x 128 tiles.
+// in 64 x 64 tiles (kTile).
 struct GemmDesc {
   int32_t front;
   int32_t k0, k1;    // inner dimension: front columns / rows [k0, k1)
@@ -98,6 +98,8 @@ struct GemmDesc {
   int32_t mirror;    // symmetric front: entries whose row lies past their
                      // tile's last column also write their transposes
                      // (no tile above the diagonal is computed)
+  int32_t L;         // the front's rows
+  int64_t foff;      // the front's offset in the arena
 };
 
 // The large-front assembly's items, resolved on the host so that its kernels

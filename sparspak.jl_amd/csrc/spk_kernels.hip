@@ -1630,37 +1630,70 @@ blk_offdiag_kernel(DevSym s, const BlkDesc* __restrict__ desc, int ndesc,
   }
 }
 
-// The trailing update on the matrix cores: 128 x 128 tiles, each of the
-// four waves owns a 64 x 64 quadrant as 4 x 4 MFMA 16x16x4 tiles. The
-// operands are passed as (U^T, L^T) so that the accumulator holds the tile
-// transposed: lane l keeps row l % 16 of four columns, and each group of 16
-// lanes writes 16 contiguous rows of the column-major front.
+// The trailing update on the matrix cores: 64 x 64 tiles, each of the four
+// waves owns a 32 x 32 quadrant as 2 x 2 MFMA tiles. The operands are passed
+// as (U^T, L^T) so that the accumulator holds the tile transposed: lane l
+// keeps row l % 16 of four consecutive columns, and each group of 16 lanes
+// writes 16 contiguous rows of the column-major front.
+//
+// What bounds it, and why 64 x 64: most launches hold few tiles or a short
+// inner dimension (K = 60 .. 480), so the fixed cost of a workgroup (first
+// loads, the read-modify-write of its tile) and the last, nearly empty wave
+// of workgroups weigh as much as the products. Against 128 x 128 tiles with
+// 64 x 64 per wave (two workgroups per CU), four workgroups per CU of a
+// quarter of the size measured, in us for fp64 / fp32 / split-bf16 (R the
+// order of the updated square, before -> now):
+//   12 fronts, R 1500, K 178: 318 -> 237 / 180 -> 120 / 102 -> 85
+//   40 fronts, R  800, K 120: 238 -> 158 / 127 ->  85 /  92 -> 71
+//   1 front,   R 2000, K 480: 103 ->  83 /  64 ->  47 /  41 -> 30
+//   1 front,   R 1200, K 480:  94 ->  45 /  60 ->  25 /  39 -> 21
+//   1 front,   R  500, K 200:  46 ->  14 /  29 ->   9 /  21 -> 10
+//   1 front,   R 4000, K 480: 340 -> 342 / 193 -> 166 /  95 -> 104
+// (only the last, in split-bf16, reads its panels often enough for the
+// larger tile to win). Loads are unconditional vectors of 16 bytes from
+// clamped addresses: rows past the rectangle only reach accumulator rows
+// that are not stored, the inner dimension's tail is zeroed as it is staged.
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-
-// The 16-bit trailing update of one 128 x 128 tile on the gfx950 bf16
-// matrix cores (v_mfma_f32_16x16x32_bf16), K-chunks of 32, double-buffered
-// in LDS as rows of kB16 halves: A(i, k) = L21 rows at As[i kB16 + k],
-// B(k, j) = U12 columns at Bs[j kB16 + k]. Global reads are four-float
-// vectors (rows of an L21 column, k of a U12 column); each thread converts
-// them and stores four bf16 per row or column (8 bytes); each lane reads its
-// MFMA operand (eight consecutive k) with one 16-byte LDS read. Split mode:
-// x = hi + lo, both bf16, products lo_b hi_a + hi_b lo_a + hi_b hi_a.
-constexpr int kB16 = 40;                       // halves per LDS row (80 bytes)
-constexpr int kB16Part = 128 * kB16;           // one operand array, halves
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
-// p[0 .. 3], element e read only when e < nvalid (0 otherwise)
-__device__ inline f4u load4(const float* p, int nvalid) {
-  if (nvalid >= 4) return *reinterpret_cast<const f4u*>(p);
-  f4u v = {0.f, 0.f, 0.f, 0.f};
-  if (nvalid > 0) v.x = p[0];
-  if (nvalid > 1) v.y = p[1];
-  if (nvalid > 2) v.z = p[2];
-  return v;
+constexpr int kTile = 64;  // rows and columns of a trailing-update tile
+
+// 16-byte vectors of the front's elements: as loaded (element alignment)
+// and as staged in LDS (16-byte alignment).
+template <typename T>
+struct Vec16;
+template <>
+struct Vec16<double> {
+  static constexpr int n = 2;
+  typedef double load __attribute__((ext_vector_type(2), aligned(8)));
+  typedef double lds __attribute__((ext_vector_type(2)));
+};
+template <>
+struct Vec16<float> {
+  static constexpr int n = 4;
+  typedef f4u load;
+  typedef float lds __attribute__((ext_vector_type(4)));
+};
+
+// Tile of workgroup bid among n: workgroups go to the eight XCDs in turn, so
+// each XCD takes runs of up to kXcdRun consecutive tiles (which share the
+// panels of one front in its L2) out of every 8 kXcdRun; the last n mod
+// (8 run) tiles keep their order. Measured on 200 fronts of R 300, K 90:
+// 131 -> 99 us (fp64), 77 -> 47 us (split-bf16); on one large front the
+// same within 2 %. Runs are short so that fronts of unlike depth in one
+// launch still spread over all XCDs.
+constexpr int kXcdRun = 32;
+__device__ inline int xcd_tile(int bid, int n) {
+  const int run = min(kXcdRun, n / 8);
+  if (run < 2) return bid;
+  const int round = 8 * run;
+  if (bid >= n / round * round) return bid;
+  const int x = bid % 8, g = bid / 8;
+  return (g / run) * round + x * run + g % run;
 }
 
 // four floats to bf16 (round to nearest even), two per v_cvt_pk_bf16_f32
@@ -1672,314 +1705,344 @@ __device__ inline uint2 pack_bf16(float a, float b, float c, float d) {
 // the part of x below its bf16 rounding (exact: x and its rounding are floats
 // within a factor of two of each other)
 __device__ inline float bf_lo(float x) { return x - (float)(__bf16)x; }
+__device__ inline uint2 pack_f16(float a, float b, float c, float d) {
+  const f16x4 p = {(_Float16)a, (_Float16)b, (_Float16)c, (_Float16)d};
+  return __builtin_bit_cast(uint2, p);
+}
 
-__device__ void gemm_bf16_chunks(const float* __restrict__ F, int L, int k0, int bw, int r0,
-                                 int rend, int j0, int cend, bool split,
-                                 unsigned char* lds_raw, f32x4 (&acc)[4][4]) {
+// One tile's products with 16-bit operands on the gfx950 matrix cores
+// (v_mfma_f32_16x16x32_bf16 / _f16), K-chunks of 32, double-buffered in LDS
+// as rows of kB16 halves: A(i, k) = L21 rows at part 0, [i kB16 + k],
+// B(k, j) = U12 columns at part 1, [j kB16 + k]; each lane reads its operand
+// (eight consecutive k) with one 16-byte LDS read. lowp 1: bf16; lowp 3:
+// split bf16, x = hi + lo (lo at parts 2 and 3), products lo_b hi_a +
+// hi_b lo_a + hi_b hi_a; lowp 2: fp16 under diagonal scaling: A(i, k) times
+// and B(k, j) divided by 2^e_k, the power of two nearest below |U(k, k)|
+// (the product is unchanged; both stay in fp16 range when A is diagonally
+// scaled). Waves 0-1 stage A (rows 4 ag .. 4 ag + 3, k = 4 q + u), waves
+// 2-3 B (columns bc + 16 u, k = 4 q .. 4 q + 3); the 32 lanes of a half-wave
+// store rows 4 apart, which at 80 bytes per row start 16 banks apart.
+constexpr int kB16 = 40;                  // halves per LDS row (80 bytes)
+constexpr int kB16Part = kTile * kB16;    // one operand array, halves
+template <int lowp>
+__device__ __attribute__((always_inline)) inline void gemm16_tile(
+    const float* __restrict__ F, int L, int k0, int bw, int r0, int rend, int j0, int cend,
+    unsigned char* lds_raw, f32x4 (&acc)[2][2]) {
   constexpr int KC = 32;
   unsigned short* base = reinterpret_cast<unsigned short*>(lds_raw);
-  // buffer b: [A hi, B hi, A lo, B lo], each kB16Part halves
   auto part = [&](int buf, int which) { return base + (buf * 4 + which) * kB16Part; };
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int wr = (wave % 2) * 64, wc = (wave / 2) * 64;
+  const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
+  const int wr = (wave % 2) * 32, wc = (wave / 2) * 32;
   const int l16 = lane % 16, lk = lane / 16;
-  // A: rows 4 ag .. 4 ag + 3 of the tile, k = 4 aq + u; B: columns
-  // bc + 32 u, k = 4 bq .. 4 bq + 3. The 32 lanes of a half-wave store rows
-  // 4 apart (A: ag = tid / 8; B: bc = 4 ((tid / 8) % 4) + ...), which at 80
-  // bytes per LDS row start 16 banks apart: their 8-byte stores hit 64
-  // distinct banks (rows 1 apart would collide every fourth row, rows 16
-  // apart every row)
-  const int ag = tid / 8, aq = tid % 8;
-  const int bq = tid % 8, bc = 4 * ((tid / 8) % 4) + (tid / 32) % 4 + 16 * (tid / 128);
-  const int arow = r0 + 4 * ag;
-  const int anv = rend - arow;  // valid rows of this thread's A groups
-  f4u ra[4], rb[4];
-  auto gload = [&](int kc) {
+  const bool isA = wave < 2;
+  const int t7 = tid % 128, q = t7 % 8, ag = t7 / 8;
+  const int bc = 4 * ((t7 / 8) % 4) + t7 / 32;
+  // A: p[u] = row 4 ag of column k0 + 4 q + u; B: p[u] = k0 + 4 q of column
+  // j0 + bc + 16 u
+  const float* pA = F + min(r0 + 4 * ag, rend - 1) + (int64_t)k0 * L;
+  const float* pB[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int k = kc + 4 * aq + u;
-      ra[u] = load4(F + arow + (int64_t)(k0 + k) * L, k < bw ? anv : 0);
-      const int c = j0 + bc + 32 * u;
-      const int kb = kc + 4 * bq;
-      rb[u] = load4(F + (k0 + kb) + (int64_t)c * L, c < cend ? bw - kb : 0);
-    }
+  for (int u = 0; u < 4; ++u) pB[u] = F + k0 + (int64_t)min(j0 + bc + 16 * u, cend - 1) * L;
+  f4u rg[4];
+  float sc[4];
+  // 2^e (A) or 2^-e (B) of the diagonal entry of front column k0 + k (1 when
+  // the entry is zero, subnormal or not finite)
+  auto pow2 = [&](int k) {
+    const float dg = F[(int64_t)(k0 + min(k, bw - 1)) * (L + 1)];
+    const unsigned be = (__float_as_uint(dg) >> 23) & 0xffu;
+    if (be == 0u || be >= 254u) return 1.0f;
+    return __uint_as_float((isA ? be : 254u - be) << 23);
   };
-  auto lstore = [&](int buf) {
-    unsigned short* Ah = part(buf, 0);
-    unsigned short* Bh = part(buf, 1);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      *reinterpret_cast<uint2*>(Ah + (4 * ag + e) * kB16 + 4 * aq) =
-          pack_bf16(ra[0][e], ra[1][e], ra[2][e], ra[3][e]);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      *reinterpret_cast<uint2*>(Bh + (bc + 32 * u) * kB16 + 4 * bq) =
-          pack_bf16(rb[u][0], rb[u][1], rb[u][2], rb[u][3]);
-    if (split) {
-      unsigned short* Al = part(buf, 2);
-      unsigned short* Bl = part(buf, 3);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        *reinterpret_cast<uint2*>(Al + (4 * ag + e) * kB16 + 4 * aq) =
-            pack_bf16(bf_lo(ra[0][e]), bf_lo(ra[1][e]), bf_lo(ra[2][e]), bf_lo(ra[3][e]));
+  auto gload = [&](int kc) {
+    const int kq = kc + 4 * q;
+    if (isA) {
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        *reinterpret_cast<uint2*>(Bl + (bc + 32 * u) * kB16 + 4 * bq) =
-            pack_bf16(bf_lo(rb[u][0]), bf_lo(rb[u][1]), bf_lo(rb[u][2]), bf_lo(rb[u][3]));
+        rg[u] = *reinterpret_cast<const f4u*>(pA + (int64_t)min(kq + u, bw - 1) * L);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) rg[u] = *reinterpret_cast<const f4u*>(pB[u] + min(kq, bw - 1));
+    }
+    if (lowp == 2)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sc[u] = pow2(kq + u);
+  };
+  auto lstore = [&](int buf, int kc) {
+    const int kq = kc + 4 * q;
+    // rg[u][e]: row e of k = kq + u (A), column u of k = kq + e (B)
+    const bool tail = kc + KC > bw;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (lowp == 2) rg[u][e] *= isA ? sc[u] : sc[e];
+        if (tail && kq + (isA ? u : e) >= bw) rg[u][e] = 0.0f;
+      }
+    if (isA) {
+      unsigned short* P = part(buf, 0) + 4 * ag * kB16 + 4 * q;
+      unsigned short* Q = part(buf, 2) + 4 * ag * kB16 + 4 * q;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x0 = rg[0][e], x1 = rg[1][e], x2 = rg[2][e], x3 = rg[3][e];
+        *reinterpret_cast<uint2*>(P + e * kB16) =
+            lowp == 2 ? pack_f16(x0, x1, x2, x3) : pack_bf16(x0, x1, x2, x3);
+        if (lowp == 3)
+          *reinterpret_cast<uint2*>(Q + e * kB16) =
+              pack_bf16(bf_lo(x0), bf_lo(x1), bf_lo(x2), bf_lo(x3));
+      }
+    } else {
+      unsigned short* P = part(buf, 1) + bc * kB16 + 4 * q;
+      unsigned short* Q = part(buf, 3) + bc * kB16 + 4 * q;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float x0 = rg[u][0], x1 = rg[u][1], x2 = rg[u][2], x3 = rg[u][3];
+        *reinterpret_cast<uint2*>(P + 16 * u * kB16) =
+            lowp == 2 ? pack_f16(x0, x1, x2, x3) : pack_bf16(x0, x1, x2, x3);
+        if (lowp == 3)
+          *reinterpret_cast<uint2*>(Q + 16 * u * kB16) =
+              pack_bf16(bf_lo(x0), bf_lo(x1), bf_lo(x2), bf_lo(x3));
+      }
     }
   };
   const int nch = (bw + KC - 1) / KC;
   gload(0);
-  lstore(0);
+  lstore(0, 0);
+  if (nch > 1) gload(KC);
   __syncthreads();
   for (int ch = 0; ch < nch; ++ch) {
     const int cur = ch & 1;
-    if (ch + 1 < nch) gload((ch + 1) * KC);
-    bf16x8 ah[4], bh[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      ah[t] = *reinterpret_cast<const bf16x8*>(part(cur, 0) + (wr + t * 16 + l16) * kB16 + 8 * lk);
-      bh[t] = *reinterpret_cast<const bf16x8*>(part(cur, 1) + (wc + t * 16 + l16) * kB16 + 8 * lk);
+    // the next chunk goes to the other buffer (every wave left it at the
+    // last barrier) and the one after is requested before the products
+    if (ch + 1 < nch) {
+      lstore(cur ^ 1, (ch + 1) * KC);
+      if (ch + 2 < nch) gload((ch + 2) * KC);
     }
-    if (split) {
-      bf16x8 al[4], bl[4];
+    auto frag = [&](int which, int row) {
+      return *reinterpret_cast<const bf16x8*>(part(cur, which) + row * kB16 + 8 * lk);
+    };
+    bf16x8 ah[2], bh[2];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        al[t] = *reinterpret_cast<const bf16x8*>(part(cur, 2) + (wr + t * 16 + l16) * kB16 + 8 * lk);
-        bl[t] = *reinterpret_cast<const bf16x8*>(part(cur, 3) + (wc + t * 16 + l16) * kB16 + 8 * lk);
+    for (int t = 0; t < 2; ++t) {
+      ah[t] = frag(0, wr + t * 16 + l16);
+      bh[t] = frag(1, wc + t * 16 + l16);
+    }
+    if (lowp == 3) {
+      bf16x8 al[2], bl[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        al[t] = frag(2, wr + t * 16 + l16);
+        bl[t] = frag(3, wc + t * 16 + l16);
       }
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+      for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < 2; ++c) {
           acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[c], ah[a], acc[a][c], 0, 0, 0);
           acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[c], al[a], acc[a][c], 0, 0, 0);
           acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[c], ah[a], acc[a][c], 0, 0, 0);
         }
+    } else if (lowp == 2) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(f16x8, bh[c]), __builtin_bit_cast(f16x8, ah[a]), acc[a][c], 0, 0,
+              0);
     } else {
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+      for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < 2; ++c)
           acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[c], ah[a], acc[a][c], 0, 0, 0);
     }
-    if (ch + 1 < nch) lstore(cur ^ 1);
     __syncthreads();
   }
 }
 
-// With lowp set, a float update of a front wider than 256 columns takes its
-// L21 / U12 operands in 16 bits and accumulates in float: lowp 1 rounds them
-// to bf16 for v_mfma_f32_16x16x16bf16_1k, lowp 2 scales column k of L21 up
-// and row k of U12 down by the power of two of |U(k, k)| and rounds to fp16
-// for v_mfma_f32_16x16x16f16 (operand k = 4 (l / 16) .. + 3 per lane, the
-// accumulator layout of the f32 form); refinement in double recovers the
-// accuracy.
-// double-buffered: As[buf][i * KP + k] = L(r0 + i, k0 + k),
-//                  Bs[buf][j * KP + k] = U(k0 + k, j0 + j)
-// (the split-bf16 form stages four bf16 arrays, hi and lo of A and B, in
-// the same bytes: 2 buffers x 4 x 128 rows of 20 halves)
+// The same tile in the front's own type (v_mfma_f64_16x16x4f64 /
+// v_mfma_f32_16x16x4f32), K-chunks of 16, double-buffered in LDS:
+// A(i, k) at As[k kLdA + i] (rows 16 elements past the tile apart, so that
+// the four k of an operand read fall in different banks), B(k, j) at
+// Bs[j ldB + k]. Column j of an accumulator tile is taken from U column
+// mcol(j), chosen so that both types leave four consecutive columns
+// 4 lk .. 4 lk + 3 in a lane (the f64 form puts row 4 v + lk in element v).
+constexpr int kGK = 16;            // inner dimension per chunk
+constexpr int kLdA = kTile + 16;
 template <typename T>
-constexpr int kGemmLds = (std::is_same<T, float>::value && 2 * 4 * kB16Part * 2 >
-                                                              2 * 2 * 128 * 17 * (int)sizeof(T))
-                             ? 2 * 4 * kB16Part * 2
-                             : 2 * 2 * 128 * 17 * (int)sizeof(T);
+constexpr int kGemmTLds = 2 * (kGK * kLdA + kTile * (kGK + Vec16<T>::n)) * (int)sizeof(T);
+template <typename T>
+__device__ __attribute__((always_inline)) inline void gemmT_tile(
+    const T* __restrict__ F, int L, int k0, int bw, int r0, int rend, int j0, int cend,
+    unsigned char* lds_raw, typename Mfma16<T>::v4 (&acc)[2][2]) {
+  constexpr int VE = Vec16<T>::n, ldB = kGK + VE;
+  constexpr int U = kTile * kGK / VE / kWG;  // vectors per thread and operand
+  typedef typename Vec16<T>::load V;
+  typedef typename Vec16<T>::lds VL;
+  T (*As)[kGK * kLdA] = reinterpret_cast<T (*)[kGK * kLdA]>(lds_raw);
+  T (*Bs)[kTile * ldB] =
+      reinterpret_cast<T (*)[kTile * ldB]>(lds_raw + 2 * kGK * kLdA * sizeof(T));
+  const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
+  const int wr = (wave % 2) * 32, wc = (wave / 2) * 32;
+  const int l16 = lane % 16, lk = lane / 16;
+  const int mcol = std::is_same<T, double>::value ? 4 * (l16 % 4) + l16 / 4 : l16;
+  // vector v of a chunk: A rows VE (v % (64 / VE)) .. of k = v / (64 / VE);
+  // B k = VE (v % (16 / VE)) .. of column v / (16 / VE)
+  constexpr int RV = kTile / VE, KV = kGK / VE;
+  const T* pA[U];
+  const T* pB[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int v = tid + u * kWG;
+    pA[u] = F + min(r0 + VE * (v % RV), rend - 1) + (int64_t)k0 * L;
+    pB[u] = F + k0 + (int64_t)min(j0 + v / KV, cend - 1) * L;
+  }
+  V ra[U], rb[U];
+  auto gload = [&](int kc) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int v = tid + u * kWG;
+      ra[u] = *reinterpret_cast<const V*>(pA[u] + (int64_t)min(kc + v / RV, bw - 1) * L);
+      rb[u] = *reinterpret_cast<const V*>(pB[u] + min(kc + VE * (v % KV), bw - 1));
+    }
+  };
+  auto lstore = [&](int buf, int kc) {
+    if (kc + kGK > bw) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int v = tid + u * kWG;
+        const bool in = kc + v / RV < bw;
+#pragma unroll
+        for (int e = 0; e < VE; ++e) {
+          if (!in) ra[u][e] = T(0);
+          if (kc + VE * (v % KV) + e >= bw) rb[u][e] = T(0);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int v = tid + u * kWG;
+      *reinterpret_cast<VL*>(&As[buf][(v / RV) * kLdA + VE * (v % RV)]) = ra[u];
+      *reinterpret_cast<VL*>(&Bs[buf][(v / KV) * ldB + VE * (v % KV)]) = rb[u];
+    }
+  };
+  const int nch = (bw + kGK - 1) / kGK;
+  gload(0);
+  lstore(0, 0);
+  if (nch > 1) gload(kGK);
+  __syncthreads();
+  for (int ch = 0; ch < nch; ++ch) {
+    const int cur = ch & 1;
+    if (ch + 1 < nch) {  // as in gemm16_tile
+      lstore(cur ^ 1, (ch + 1) * kGK);
+      if (ch + 2 < nch) gload((ch + 2) * kGK);
+    }
+#pragma unroll
+    for (int ks = 0; ks < kGK / 4; ++ks) {
+      const int kk = ks * 4 + lk;
+      T av[2], bv[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        av[t] = As[cur][kk * kLdA + wr + t * 16 + l16];
+        bv[t] = Bs[cur][(wc + t * 16 + mcol) * ldB + kk];
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[a][c] = Mfma16<T>::op(bv[c], av[a], acc[a][c]);
+    }
+    __syncthreads();
+  }
+}
 
-// Workgroup bid of a trailing-update launch over desc[0, ndesc); lds_raw:
-// kGemmLds<T> bytes.
+// LDS bytes of blk_gemm_body.
+template <typename T>
+constexpr int kGemmLds = (std::is_same<T, float>::value && 2 * 4 * kB16Part * 2 > kGemmTLds<T>)
+                             ? 2 * 4 * kB16Part * 2
+                             : kGemmTLds<T>;
+
+// Tile t of a trailing-update launch over desc[0, ndesc); lds_raw:
+// kGemmLds<T> bytes. With lowp set, a float update of a front wider than 256
+// columns takes its L21 / U12 operands in 16 bits and accumulates in float
+// (gemm16_tile); refinement in double recovers the accuracy.
 template <typename T>
 __device__ __attribute__((always_inline)) void blk_gemm_body(
     const DevSym& s, const GemmDesc* __restrict__ desc, int ndesc, T* __restrict__ arena,
-    int lowp, int bid, unsigned char* lds_raw) {
-  constexpr int TM = 128, KC = 16, KP = KC + 1, PER = TM * KC / kWG;  // 8 loads each
+    int lowp, int t, unsigned char* lds_raw) {
   typedef typename Mfma16<T>::v4 v4;
-  T (*As)[TM * KP] = reinterpret_cast<T (*)[TM * KP]>(lds_raw);
-  T (*Bs)[TM * KP] = reinterpret_cast<T (*)[TM * KP]>(lds_raw + 2 * TM * KP * sizeof(T));
-  const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
-  const int di = find_blk(desc, ndesc, bid);
+  const int lane = threadIdx.x % 64, wave = wave_id();
+  const int di = find_blk(desc, ndesc, t);
   const GemmDesc d = desc[di];
-  const int b = bid - d.wg_begin;
-  const int L = s.fL[d.front];
-  T* F = arena + s.foff[d.front];
+  const int b = t - d.wg_begin;
+  const int L = d.L;
+  T* F = arena + d.foff;
   const int bw = d.k1 - d.k0;
   const int rend = d.r0 + d.nr, cend = d.j0 + d.nc;
-  const int r0 = d.r0 + (b % d.ntr) * TM, j0 = d.j0 + (b / d.ntr) * TM;
+  const int r0 = d.r0 + (b % d.ntr) * kTile, j0 = d.j0 + (b / d.ntr) * kTile;
   // symmetric fronts: an entry whose row lies past the tile's last column
   // also stands for its transpose, which no tile computes (a tile column's
   // own square, its first tile, is computed whole)
-  const int mend = d.mirror ? min(j0 + TM, cend) : (1 << 30);
-  const int wr = (wave % 2) * 64, wc = (wave / 2) * 64;
+  const int mend = d.mirror ? min(j0 + kTile, cend) : (1 << 30);
+  const int wr = (wave % 2) * 32, wc = (wave / 2) * 32;
   const int l16 = lane % 16, lk = lane / 16;
-  // this thread's share of a chunk: A element (ai, ak + 2 t), B element
-  // (bk, bj + 16 t) for t < 8
-  const int ai = tid % TM, ak = tid / TM;       // ak in {0, 1}
-  const int bk = tid % KC, bj = tid / KC;       // bj in 0..15
-  const bool arow = r0 + ai < rend;
-  const T* Ap = F + (r0 + ai) + (int64_t)d.k0 * L;
-  const T* Bp = F + d.k0 + bk;
-  T ra[PER], rb[PER];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int kk = ak + 2 * t;
-      ra[t] = (arow && k0 + kk < bw) ? Ap[(int64_t)(k0 + kk) * L] : T(0);
-      const int c = j0 + bj + 16 * t;
-      rb[t] = (k0 + bk < bw && c < cend) ? Bp[k0 + (int64_t)c * L] : T(0);
-    }
-  };
-  auto lstore = [&](int buf) {
-#pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      As[buf][ai * KP + ak + 2 * t] = ra[t];
-      Bs[buf][(bj + 16 * t) * KP + bk] = rb[t];
-    }
-  };
   // the products are summed from zero and subtracted from A22 once at the
   // end: starting the accumulators from A22 instead loses accuracy when
   // |A22| >> |L21 U12| (measured 8x larger backward error on the 3D
   // convection-diffusion operator)
-  v4 acc[4][4];
+  v4 acc[2][2];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[a][c] = v4{T(0), T(0), T(0), T(0)};
-  const int nch = (bw + KC - 1) / KC;
-  bool done = false;
+    for (int c = 0; c < 2; ++c) acc[a][c] = v4{T(0), T(0), T(0), T(0)};
   if constexpr (std::is_same<T, float>::value) {
-    if (lowp == 2 && d.big) {
-      // fp16 operands under diagonal scaling: A(i, k) times and B(k, j)
-      // divided by 2^e_k, 2^e_k the power of two nearest below |U(k, k)|
-      // (the product is unchanged; both stay in fp16 range when A is
-      // diagonally scaled); rows of KB = 20 halves as in the bf16 form
-      constexpr int KB = 20;
-      _Float16* Ah = reinterpret_cast<_Float16*>(&As[0][0]);
-      _Float16* Bh = reinterpret_cast<_Float16*>(&Bs[0][0]);
-      const int akw = __builtin_amdgcn_readfirstlane(ak);
-      float sa[PER], sb = 1.0f;
-      // 2^e and 2^-e of the diagonal entry of front column k (1 when the
-      // entry is zero, subnormal or not finite)
-      auto pow2 = [&](int k, bool inv) {
-        const float dg = F[(int64_t)k * (L + 1)];
-        const unsigned be = (__float_as_uint(dg) >> 23) & 0xffu;
-        if (be == 0u || be >= 254u) return 1.0f;
-        return __uint_as_float((inv ? 254u - be : be) << 23);
-      };
-      auto scales = [&](int k0) {
+    if (lowp == 1 && d.big)
+      gemm16_tile<1>(F, L, d.k0, bw, r0, rend, j0, cend, lds_raw, acc);
+    else if (lowp == 2 && d.big)
+      gemm16_tile<2>(F, L, d.k0, bw, r0, rend, j0, cend, lds_raw, acc);
+    else if (lowp == 3 && d.big)
+      gemm16_tile<3>(F, L, d.k0, bw, r0, rend, j0, cend, lds_raw, acc);
+    else
+      gemmT_tile<T>(F, L, d.k0, bw, r0, rend, j0, cend, lds_raw, acc);
+  } else {
+    gemmT_tile<T>(F, L, d.k0, bw, r0, rend, j0, cend, lds_raw, acc);
+  }
+  // A22 -= the products: all 16 reads of a lane are issued before its writes
+  // (one memory round trip)
+  T cv[2][2][4];
 #pragma unroll
-        for (int t = 0; t < PER; ++t) {
-          const int kk = akw + 2 * t;
-          sa[t] = (k0 + kk < bw) ? pow2(d.k0 + k0 + kk, false) : 1.0f;
+  for (int a = 0; a < 2; ++a) {
+    const int r = min(r0 + wr + a * 16 + l16, rend - 1);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        cv[a][c][v] = F[r + (int64_t)min(j0 + wc + c * 16 + 4 * lk + v, cend - 1) * L];
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int r = r0 + wr + a * 16 + l16;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int col = j0 + wc + c * 16 + 4 * lk + v;
+        if (r < rend && col < cend) {
+          const T nv = cv[a][c][v] - acc[a][c][v];
+          F[r + (int64_t)col * L] = nv;
+          if (r >= mend) F[col + (int64_t)r * L] = nv;
         }
-        sb = (k0 + bk < bw) ? pow2(d.k0 + k0 + bk, true) : 1.0f;
-      };
-      auto hstore = [&](int buf) {
-#pragma unroll
-        for (int t = 0; t < PER; ++t) {
-          Ah[buf * TM * KB + ai * KB + ak + 2 * t] = (_Float16)(ra[t] * sa[t]);
-          Bh[buf * TM * KB + (bj + 16 * t) * KB + bk] = (_Float16)(rb[t] * sb);
-        }
-      };
-      gload(0);
-      scales(0);
-      hstore(0);
-      __syncthreads();
-      for (int ch = 0; ch < nch; ++ch) {
-        const int cur = ch & 1;
-        if (ch + 1 < nch) {
-          gload((ch + 1) * KC);
-          scales((ch + 1) * KC);
-        }
-        f16x4 av[4], bv[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          av[t] = *reinterpret_cast<const f16x4*>(Ah + cur * TM * KB + (wr + t * 16 + l16) * KB + 4 * lk);
-          bv[t] = *reinterpret_cast<const f16x4*>(Bh + cur * TM * KB + (wc + t * 16 + l16) * KB + 4 * lk);
-        }
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x16f16(bv[c], av[a], acc[a][c], 0, 0, 0);
-        if (ch + 1 < nch) hstore(cur ^ 1);
-        __syncthreads();
       }
-      done = true;
-    }
-    if ((lowp == 1 || lowp == 3) && d.big) {
-      gemm_bf16_chunks(F, L, d.k0, bw, r0, rend, j0, cend, lowp == 3, lds_raw, acc);
-      done = true;
-    }
-  }
-  if (!done) {
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  for (int ch = 0; ch < nch; ++ch) {
-    const int cur = ch & 1;
-    if (ch + 1 < nch) gload((ch + 1) * KC);
-#pragma unroll
-    for (int ks = 0; ks < KC / 4; ++ks) {
-      const int kk = ks * 4 + lk;
-      T av[4], bv[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        av[t] = As[cur][(wr + t * 16 + l16) * KP + kk];
-        bv[t] = Bs[cur][(wc + t * 16 + l16) * KP + kk];
-      }
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[a][c] = Mfma16<T>::op(bv[c], av[a], acc[a][c]);
-    }
-    if (ch + 1 < nch) lstore(cur ^ 1);
-    __syncthreads();
-  }
-  }
-  // A22 -= the products, AG x 16 entries at a time: all reads of a group
-  // are issued before its writes (one memory round trip per group instead
-  // of one per entry; all 64 floats at once, doubles in two groups of 32 to
-  // stay within the register budget of two workgroups per CU)
-  constexpr int AG = std::is_same<T, float>::value ? 4 : 2;
-#pragma unroll
-  for (int a0 = 0; a0 < 4; a0 += AG) {
-    T cv[AG][4][4];
-#pragma unroll
-    for (int ag = 0; ag < AG; ++ag) {
-      const int r = r0 + wr + (a0 + ag) * 16 + l16;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int col = j0 + wc + c * 16 + Mfma16<T>::row(lk, v);
-          cv[ag][c][v] = (r < rend && col < cend) ? F[r + (int64_t)col * L] : T(0);
-        }
-    }
-#pragma unroll
-    for (int ag = 0; ag < AG; ++ag) {
-      const int r = r0 + wr + (a0 + ag) * 16 + l16;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int col = j0 + wc + c * 16 + Mfma16<T>::row(lk, v);
-          if (r < rend && col < cend) {
-            const T nv = cv[ag][c][v] - acc[a0 + ag][c][v];
-            F[r + (int64_t)col * L] = nv;
-            if (r >= mend) F[col + (int64_t)r * L] = nv;
-          }
-        }
-    }
   }
 }
 
 template <typename T>
-__global__ void __launch_bounds__(kWG, 2)
+__global__ void __launch_bounds__(kWG, 4)
 blk_gemm_kernel(DevSym s, const GemmDesc* __restrict__ desc, int ndesc,
                 T* __restrict__ arena, int lowp) {
   const int64_t vs = blockIdx.y;  // value set
   arena += vs * s.vs_arena;
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[kGemmLds<T>];
-  blk_gemm_body<T>(s, desc, ndesc, arena, lowp, blockIdx.x, lds_raw);
+  blk_gemm_body<T>(s, desc, ndesc, arena, lowp, xcd_tile(blockIdx.x, gridDim.x), lds_raw);
 }
 
 // The diagonal regions of one block step (workgroups b < ndiag, with the
@@ -2001,7 +2064,8 @@ blk_diag_border_kernel(DevSym s, const BlkDesc* __restrict__ ddesc, int ndiag,
   if ((int)blockIdx.x < ndiag)
     blk_diag_slab_body<T>(s, ddesc[blockIdx.x], arena, ipvt, first_fail, lds);
   else
-    blk_gemm_body<T>(s, gdesc, ngemm, arena, lowp, (int)blockIdx.x - ndiag, lds);
+    blk_gemm_body<T>(s, gdesc, ngemm, arena, lowp,
+                     xcd_tile((int)blockIdx.x - ndiag, (int)gridDim.x - ndiag), lds);
 }
 
 // ---------------------------------------------------------------------------
