@@ -217,6 +217,9 @@ struct spkhip_handle {
   DevBuf<double> d_lnz64, d_unz64, d_arena64, d_vec64, d_rhs64;
   DevBuf<float> d_lnz32, d_unz32, d_arena32, d_vec32, d_rhs32, d_tmp32;
   DevBuf<i64> d_ipvt;
+  // per column of a factor block: the row (within the block) its position
+  // takes after the interchanges | the position its row takes << 8
+  DevBuf<i32> d_rperm;
   DevBuf<unsigned long long> d_fail;
   i64 first_fail = 0;
   // solve / refine work
@@ -738,7 +741,6 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
         const i32 nqmax = (h->kind == SPKHIP_KIND_LU) ? kNqLU : kNqSPD;
         const i32 strip = (i32)(h->xsuper[B.p0 + B.np] - 1 - h->fc0[f] - B.c0) * nqmax;
         G.offd.lds = std::max(G.offd.lds, 64 * spk::kRLD + strip);
-        if (bw <= 64) G.offd.lds = std::max(G.offd.lds, 2 * 64 * spk::kRW);  // tile + region
         G.offd.flops += 2.0 * (double)bw * bw * t;
         G.offd.elems += 4.0 * (double)bw * t;
       }
@@ -1127,6 +1129,7 @@ void run_factor(spkhip_handle* h) {
   DevBuf<T>& arena = Bufs<T>::arena(h);
   arena.ensure(per_sets(h, h->ds.vs_arena));
   h->d_ipvt.ensure((size_t)h->n * h->nvs);
+  h->d_rperm.ensure((size_t)h->n * h->nvs);
   h->d_fail.ensure(1);
   hipLaunchKernelGGL(spk::fill_kernel<unsigned long long>, dim3(1), dim3(kWG), 0, st,
                      h->d_fail.p, (int64_t)1, ~0ull);
@@ -1192,7 +1195,7 @@ void run_factor(spkhip_handle* h) {
           hipLaunchKernelGGL((spk::blk_diag_border_kernel<T>), dim3(G.diag.wg + G.bin.wg, h->nvs),
                              dim3(kWG), 0, st, h->ds, h->d_bdesc.p + G.diag.off, G.diag.wg,
                              h->d_gdesc.p + G.bin.off, G.bin.cnt, arena.p, h->d_ipvt.p,
-                             h->d_fail.p, h->lowp);
+                             h->d_rperm.p, h->d_fail.p, h->lowp);
           hipck(hipGetLastError());
         } else {
           h->cur_grid = G.diag.wg;
@@ -1200,21 +1203,27 @@ void run_factor(spkhip_handle* h) {
           if (slab && !G.wide)
             hipLaunchKernelGGL((spk::blk_diag_slab_kernel<T>), dim3(G.diag.wg, h->nvs), dim3(kWG), 0, st,
                                h->ds, h->d_bdesc.p + G.diag.off, arena.p, h->d_ipvt.p,
-                               h->d_fail.p);
+                               h->d_rperm.p, h->d_fail.p);
           else if (lu)
             hipLaunchKernelGGL((spk::blk_diag_kernel<T, kNqLU>), dim3(G.diag.wg, h->nvs), dim3(kWG),
                                (size_t)G.diag.lds * sizeof(T), st, h->ds,
-                               h->d_bdesc.p + G.diag.off, arena.p, h->d_ipvt.p, h->d_fail.p);
+                               h->d_bdesc.p + G.diag.off, arena.p, h->d_ipvt.p, h->d_rperm.p,
+                               h->d_fail.p);
           else
             hipLaunchKernelGGL((spk::blk_diag_kernel<T, kNqSPD>), dim3(G.diag.wg, h->nvs), dim3(kWG),
                                (size_t)G.diag.lds * sizeof(T), st, h->ds,
-                               h->d_bdesc.p + G.diag.off, arena.p, h->d_ipvt.p, h->d_fail.p);
+                               h->d_bdesc.p + G.diag.off, arena.p, h->d_ipvt.p, h->d_rperm.p,
+                               h->d_fail.p);
           hipck(hipGetLastError());
         }
         if (G.offd.cnt > 0) {
           h->cur_grid = G.offd.wg;
           Prof pr(h, SPKHIP_K_OFFDIAG, G.offd.flops, G.offd.elems * sizeof(T));
-          if (lu)
+          if (!G.wide)
+            hipLaunchKernelGGL(spk::blk_offdiag64_kernel<T>, dim3(G.offd.wg, h->nvs), dim3(kWG),
+                               0, st, h->d_bdesc.p + G.offd.off, G.offd.cnt, arena.p,
+                               h->d_rperm.p, h->ds.vs_arena, h->ds.n);
+          else if (lu)
             hipLaunchKernelGGL((spk::blk_offdiag_kernel<T, kNqLU>), dim3(G.offd.wg, h->nvs), dim3(kWG),
                                (size_t)G.offd.lds * sizeof(T), st, h->ds,
                                h->d_bdesc.p + G.offd.off, G.offd.cnt, arena.p, h->d_ipvt.p);
@@ -1597,11 +1606,12 @@ void factor_run(spkhip_handle* h) {
   Bufs<T>::unz(h).ensure(per_sets(h, h->ds.vs_unz));
   Bufs<T>::arena(h).ensure(per_sets(h, h->ds.vs_arena));
   h->d_ipvt.ensure((size_t)h->n * h->nvs);
+  h->d_rperm.ensure((size_t)h->n * h->nvs);
   h->d_fail.ensure(1);
   const std::vector<const void*> key = {
       (const void*)(intptr_t)sizeof(T), (const void*)(intptr_t)h->lowp,
       (const void*)(intptr_t)h->sym_gen, Bufs<T>::lnz(h).p, Bufs<T>::unz(h).p,
-      Bufs<T>::arena(h).p, h->d_ipvt.p, h->d_fail.p, h->d_nzval.p, h->d_amap.p,
+      Bufs<T>::arena(h).p, h->d_ipvt.p, h->d_rperm.p, h->d_fail.p, h->d_nzval.p, h->d_amap.p,
       (const void*)(intptr_t)h->nvs};
   if (!use_graph) {
     factor_launches<T>(h);

@@ -689,9 +689,6 @@ __device__ inline int wave_min(int v) {
 // columns wide); a compile-time stride turns every column offset into an
 // immediate LDS offset.
 constexpr int kRLD = 129;
-// Row stride of a block's diagonal region (at most 64 columns) held row by
-// row in LDS: lanes storing consecutive rows fall in different banks.
-constexpr int kRW = 65;
 // Most columns of one piece (the SPD limit 90, rounded up).
 constexpr int kMaxNq = 96;
 
@@ -1029,16 +1026,20 @@ struct Mfma16<float> {
 template <typename T, int NQ>
 __global__ void __launch_bounds__(kWG)
 blk_diag_kernel(DevSym s, const BlkDesc* __restrict__ desc, T* __restrict__ arena,
-                int64_t* __restrict__ ipvt, unsigned long long* __restrict__ first_fail) {
+                int64_t* __restrict__ ipvt, int32_t* __restrict__ rperm,
+                unsigned long long* __restrict__ first_fail) {
   const int64_t vs = blockIdx.y;  // value set
   arena += vs * s.vs_arena;
   ipvt += vs * s.n;
+  rperm += vs * s.n;
   constexpr int LD = kRLD;
   extern __shared__ unsigned char smem_raw[];
   __shared__ int piv[NQ];
   __shared__ int perm[NQ];
   __shared__ T dinv[NQ];
   __shared__ int s_zero;
+  // the row each position takes, and the position each row takes
+  __shared__ unsigned char ssrc[128], spos[128];
   T* R = reinterpret_cast<T*>(smem_raw);
   const int tid = threadIdx.x, wave = wave_id();
   const BlkDesc d = desc[blockIdx.x];
@@ -1065,7 +1066,12 @@ blk_diag_kernel(DevSym s, const BlkDesc* __restrict__ desc, T* __restrict__ aren
       nopiv_getrf<T, LD>(D, nq, piv, dinv, &s_zero);
     }
     __syncthreads();
-    if (tid < nq) ipvt[pc0 + tid] = piv[tid] + 1;
+    if (tid < nq) {
+      ipvt[pc0 + tid] = piv[tid] + 1;
+      const int src = (s.pivot && nq <= 64) ? perm[tid] : tid;
+      ssrc[o + tid] = (unsigned char)(o + src);
+      spos[o + src] = (unsigned char)(o + tid);
+    }
     if (tid == 0 && s_zero) atomicMin(first_fail, (unsigned long long)(d.piece + pi + 1));
     if (tid >= 128) {
       // U12 of the region (rows already interchanged): unit-lower solve,
@@ -1118,6 +1124,7 @@ blk_diag_kernel(DevSym s, const BlkDesc* __restrict__ desc, T* __restrict__ aren
     }
     __syncthreads();
   }
+  if (tid < bw) rperm[fc0 + c0 + tid] = ssrc[tid] | spos[tid] << 8;
   store_tile<T, 1, LD>(Fr, L, bw, bw, R);
 }
 
@@ -1161,7 +1168,8 @@ constexpr int kSlabLds = 3 * 64 * 64 * (int)sizeof(T);
 template <typename T>
 __device__ __attribute__((always_inline)) void blk_diag_slab_body(
     const DevSym& s, const BlkDesc& d, T* __restrict__ arena, int64_t* __restrict__ ipvt,
-    unsigned long long* __restrict__ first_fail, unsigned char* lds) {
+    int32_t* __restrict__ rperm, unsigned long long* __restrict__ first_fail,
+    unsigned char* lds) {
   constexpr int SW = 16;                  // columns per wave
   // step k: the multiplier of each row; finished column c, rows in lane
   // order; entries set aside while a piece's sum forms
@@ -1172,6 +1180,7 @@ __device__ __attribute__((always_inline)) void blk_diag_slab_body(
   __shared__ int spo[kMaxBlkPieces + 1];  // piece offsets in the region; spo[np] = bw
   __shared__ int scp[64];                 // piece of each region column
   __shared__ int spos[64];                // final position of each row
+  __shared__ int ssrc[64];                // the row each position takes
   __shared__ int spiv[64];                // step k: pivot position, 1-based in its piece
   __shared__ int sdone;                   // steps published
   const int lane = threadIdx.x % 64, w = wave_id();
@@ -1345,11 +1354,15 @@ __device__ __attribute__((always_inline)) void blk_diag_slab_body(
   if (kend > cb)
     __hip_atomic_store(&sdone, kend, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
   // the wave of the last column has seen every interchange
-  if (w == (bw - 1) / SW) spos[lane] = pos;
+  if (w == (bw - 1) / SW) {
+    spos[lane] = pos;
+    ssrc[pos] = lane;
+  }
   __syncthreads();
   const int fpos = spos[lane];
   if ((int)threadIdx.x < bw) {
     ipvt[fc0 + c0 + threadIdx.x] = spiv[threadIdx.x];
+    rperm[fc0 + c0 + threadIdx.x] = ssrc[threadIdx.x] | fpos << 8;
     // a zero pivot: the first piece that met one
     if (!((smeta[threadIdx.x] >> 16) & 1))
       atomicMin(first_fail, (unsigned long long)(d.piece + scp[threadIdx.x] + 1));
@@ -1367,149 +1380,196 @@ __device__ __attribute__((always_inline)) void blk_diag_slab_body(
 template <typename T>
 __global__ void __launch_bounds__(kWG)
 blk_diag_slab_kernel(DevSym s, const BlkDesc* __restrict__ desc, T* __restrict__ arena,
-                     int64_t* __restrict__ ipvt, unsigned long long* __restrict__ first_fail) {
+                     int64_t* __restrict__ ipvt, int32_t* __restrict__ rperm,
+                     unsigned long long* __restrict__ first_fail) {
   const int64_t vs = blockIdx.y;  // value set
   arena += vs * s.vs_arena;
   ipvt += vs * s.n;
+  rperm += vs * s.n;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kSlabLds<T>];
-  blk_diag_slab_body<T>(s, desc[blockIdx.x], arena, ipvt, first_fail, lds);
+  blk_diag_slab_body<T>(s, desc[blockIdx.x], arena, ipvt, rperm, first_fail, lds);
 }
 
-// Off-diagonal parts of a block of at most 64 columns. The tile, the
-// block's whole diagonal region and (columns) the block's interchanges are
-// read in one batch of loads, with the front and the piece widths (pw) taken
-// from the descriptor; the pieces then follow each other in LDS with the
-// operations, in the order, of the general path below (same results bit for
-// bit). Dynamic LDS: 2 * 64 * kRW elements.
+// Element of the operand entry (m, k) of 16 x 16 sub-block sb in LDS: the
+// sixteen m of a lane group and the four k = 4 (l / 16) + st of a step fall
+// in different banks, in float and in double, also as they are staged.
+__device__ inline int op16(int sb, int m, int k) {
+  return sb * 256 + m * 16 + ((((k & 3) << 2) | (k >> 2)) ^ m);
+}
+
+// Off-diagonal parts of blocks of at most 64 columns on the matrix cores:
+// workgroups b < d.nl take 64 rows below the block (X = A U^-1), the others
+// 64 columns right of it (X = L^-1 P A), sixteen per wave. The block is
+// solved in sub-blocks of 16 columns (rows), each in four steps of four:
+// lane l holds entries 4 (l / 16) .. + 3 of its row (column) l % 16, which is
+// an accumulator tile and, as it stands, the next product's operand, so X
+// never leaves the registers. The earlier sub-blocks' contribution is summed
+// from zero and subtracted once; inside a sub-block, step j solves the four
+// entries held by lanes l / 16 = j by substitution in those lanes and
+// subtracts their products from the entries right of them (four MFMAs whose
+// other operand lanes are zero). This is substitution throughout: an
+// explicit inverse per 16 columns costs the same and lost accuracy on small
+// pivots (factor error 1.4e-12 of the largest entry against 1.6e-13, also
+// with one correction step). U is the region's whole upper triangle, and the
+// interchanges of every piece are applied to A's rows and to the earlier
+// pieces' L rows first (rperm: row | position << 8 per column, from the
+// diagonal kernel), which does the reference's operations on the same
+// values.
+// Latency-bound (2 .. 400 workgroups per launch): 11 .. 15 us per launch
+// (events), against 20 .. 28 us for substitution by one wave, one row per
+// lane, with the other three waves idle; the whole class 15.5 -> 8.5 ms in
+// double and 11.6 -> 6.9 ms in split-bf16 at 64^3, 20.1 -> 9.5 ms on
+// elasticity 40^3 (SPD, split-bf16).
 template <typename T>
-__device__ __attribute__((always_inline)) inline void
-offdiag64_body(const BlkDesc& d, const int32_t* __restrict__ pw, int b, T* __restrict__ arena,
-               const int64_t* __restrict__ ipvt, T* __restrict__ S, int* __restrict__ spiv) {
+__global__ void __launch_bounds__(kWG)
+blk_offdiag64_kernel(const BlkDesc* __restrict__ desc, int ndesc, T* __restrict__ arena,
+                     const int32_t* __restrict__ rperm, int64_t vs_arena, int64_t vs_n) {
+  const int64_t vs = blockIdx.y;  // value set
+  arena += vs * vs_arena;
+  rperm += vs * vs_n;
+  typedef typename Mfma16<T>::v4 v4;
+  // operand sub-blocks (s, q), q <= s, at s (s + 1) / 2 + q
+  __shared__ __attribute__((aligned(16))) T S[10 * 256];
+  __shared__ T srinv[64];
+  __shared__ int ssrc[64];
   const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
-  const int L = d.L;
-  const int c0 = d.c0, bw = d.c1 - d.c0;
+  const int l16 = lane % 16, lk = lane / 16;
+  const int mi = std::is_same<T, double>::value ? 4 * (l16 % 4) + l16 / 4 : l16;
+  const int di = find_blk(desc, ndesc, blockIdx.x);
+  const BlkDesc& d = desc[di];
+  const int b = blockIdx.x - d.wg_begin;
+  const int L = d.L, c0 = d.c0, bw = d.c1 - d.c0, nl = d.nl;
+  const int ns = (bw + 15) / 16;
   T* F = arena + d.foff;
   const T* Fd = F + c0 + (int64_t)c0 * L;  // the diagonal region
-  if (b < d.nl) {
-    // rows [r0, r0 + nr): X(i, k) at X[i + 64 k]; U(k, j) of the region at
-    // R[k kRW + j]
-    const int r0 = d.c1 + b * 64, nr = min(64, L - r0);
-    T* X = S;
-    T* R = S + 64 * kRW;
-    T* Fx = F + r0 + (int64_t)c0 * L;
-    T xv[16], rv[16];
+  const bool below = b < nl;
+  const int g0 = d.c1 + (below ? b : b - nl) * 64 + 16 * wave + l16;  // row or column
+  const int g = min(g0, L - 1);
+  int rp = lane | lane << 8;
+  if (!below && lane < bw) rp = rperm[d.fc0 + c0 + lane];
+  T rv[16];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int c = wave + 4 * u;
-      xv[u] = (lane < nr && c < bw) ? Fx[lane + (int64_t)c * L] : T(0);
-      rv[u] = (lane < bw && c < bw) ? Fd[lane + (int64_t)c * L] : T(0);
-    }
+  for (int u = 0; u < 16; ++u) {
+    const int c = wave + 4 * u;
+    rv[u] = (lane < bw && c < bw) ? Fd[lane + (int64_t)c * L] : T(0);
+  }
+  v4 X[4];
+  if (below) {
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int c = wave + 4 * u;
-      X[lane + c * 64] = xv[u];
-      R[lane * kRW + c] = rv[u];
-    }
-    __syncthreads();
-    int o = 0;
-    for (int pi = 0; pi < d.np; ++pi) {
-      const int nq = pw[pi];
-      if (o > 0) {  // earlier pieces of the block: X_q -= X_<q U_<q,q
-        for (int cb = wave * 8; cb < nq; cb += 32) {
-          T acc[8];
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-          for (int jj = 0; jj < 8; ++jj) acc[jj] = T(0);
-          const int cs = min(cb, nq - 8 >= 0 ? nq - 8 : 0);  // shifted start
-          const T* xr = X + lane;
-          const T* ur = R + o + cs;
-          for (int k = 0; k < o; ++k) {
-            const T xk = xr[k * 64];
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) acc[jj] += xk * ur[k * kRW + jj];
-          }
-#pragma unroll
-          for (int jj = 0; jj < 8; ++jj) {
-            const int j = cs + jj;
-            if (j >= cb && j < nq) X[lane + (o + j) * 64] -= acc[jj];
-          }
-        }
-        __syncthreads();
+      for (int v = 0; v < 4; ++v) {
+        const int c = 16 * q + 4 * lk + v;
+        X[q][v] = c < bw ? F[g + (int64_t)(c0 + c) * L] : T(0);
       }
-      if (wave == 0)  // X_q U_qq^-1, one row per lane
-        blk_trsv<T, 64, kRW, 1, false>(X + lane + o * 64, R + o * kRW + o, nullptr, nq);
-      __syncthreads();
-      o += nq;
-    }
-    store_tile<T, 1, 64>(Fx, L, nr, bw, X);
+    T dv = T(1);  // U's diagonal (1 past the block)
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (wave + 4 * u == lane && lane < bw) dv = rv[u];
+    if (lane % 4 == wave) srinv[lane] = T(1) / dv;
   } else {
-    // columns [j0, j0 + nc): A(r, c) at A[r + c kRW]; L(r, k) of the region
-    // at R[r + k kRW]
-    const int j0 = d.c1 + (b - d.nl) * 64, nc = min(64, L - j0);
-    T* A = S;
-    T* R = S + 64 * kRW;
-    T* Fa = F + c0 + (int64_t)j0 * L;
-    const int pv = (tid < bw) ? (int)ipvt[d.fc0 + c0 + tid] - 1 : 0;
-    T av[16], rv[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int c = wave + 4 * u;
-      av[u] = (lane < bw && c < nc) ? Fa[lane + (int64_t)c * L] : T(0);
-      rv[u] = (lane < bw && c < bw) ? Fd[lane + (int64_t)c * L] : T(0);
+    // the first row of the lane's piece, and where each row comes from
+    int ps = 0;
+    for (int q = 0, o = 0; q < d.np; ++q) {
+      if (lane >= o) ps = o;
+      o += d.pw[q];
     }
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int c = wave + 4 * u;
-      A[lane + c * kRW] = av[u];
-      R[lane + c * kRW] = rv[u];
+    if (wave == 0) {
+      ssrc[lane] = rp & 0xff;
+      srinv[lane] = T(1);
     }
-    if (tid < bw) spiv[tid] = pv;  // piece-local positions
     __syncthreads();
-    int o = 0;
-    for (int pi = 0; pi < d.np; ++pi) {
-      const int nq = pw[pi];
-      if (o > 0) {  // earlier pieces: A_q -= L_q,<q A_<q (rows not yet swapped)
-        T* ac = A + lane * kRW;
-        for (int ib = wave * 8; ib < nq; ib += 32) {
-          const int is = min(ib, nq - 8 >= 0 ? nq - 8 : 0);
-          T acc[8];
+    const T* Fa = F + c0 + (int64_t)g * L;
 #pragma unroll
-          for (int ii = 0; ii < 8; ++ii) acc[ii] = T(0);
-          for (int k = 0; k < o; ++k) {
-            const T a = ac[k];
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int ii = 0; ii < 8; ++ii) acc[ii] += R[o + is + ii + k * kRW] * a;
-          }
-#pragma unroll
-          for (int ii = 0; ii < 8; ++ii) {
-            const int i = is + ii;
-            if (i >= ib && i < nq) ac[o + i] -= acc[ii];
-          }
-        }
-        __syncthreads();
+      for (int v = 0; v < 4; ++v) {
+        const int r = 16 * q + 4 * lk + v;
+        X[q][v] = r < bw ? Fa[ssrc[r]] : T(0);
       }
-      if (wave == 0) {  // interchanges, then L_qq^-1, one column per lane
-        T* a = A + lane * kRW + o;
-        for (int k = 0; k < nq; ++k) {
-          const int kp = spiv[o + k];
-          if (kp != k) {
-            const T t = a[k];
-            a[k] = a[kp];
-            a[kp] = t;
-          }
-        }
-        blk_trsv<T, 1, kRW, 1, true>(a, R + o + o * kRW, nullptr, nq);
-      }
-      __syncthreads();
-      o += nq;
+    rp = (rp >> 8 & 0xff) | ps << 8;
+  }
+  // the region's strict triangle, sub-block by sub-block (zero elsewhere)
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int c = wave + 4 * u;
+    if (below) {  // U(k, m): k = lane, m = c
+      if (lane / 16 <= c / 16)
+        S[op16((c / 16) * (c / 16 + 1) / 2 + lane / 16, c % 16, lane % 16)] =
+            lane < c ? rv[u] : T(0);
+    } else {  // L(m, k): k = c, m = the lane's row, moved in earlier pieces' columns
+      const int m = c < (rp >> 8) ? (rp & 0xff) : lane;
+      if (m / 16 >= c / 16)
+        S[op16((m / 16) * (m / 16 + 1) / 2 + c / 16, m % 16, c % 16)] = m > c ? rv[u] : T(0);
     }
-    store_tile<T, 1, kRW>(Fa, L, bw, nc, A);
+  }
+  __syncthreads();
+  // acc + sub-block sb times the tile x
+  auto mul = [&](int sb, const v4& x, v4 acc) {
+#pragma unroll
+    for (int st = 0; st < 4; ++st) acc = Mfma16<T>::op(S[op16(sb, mi, 4 * lk + st)], x[st], acc);
+    return acc;
+  };
+  const v4 zero = v4{T(0), T(0), T(0), T(0)};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (q < ns) {
+      const int sd = q * (q + 1) / 2 + q;
+      // the lane's own four-column triangle and reciprocals
+      T m01 = S[op16(sd, 4 * lk + 1, 4 * lk)], m02 = S[op16(sd, 4 * lk + 2, 4 * lk)];
+      T m03 = S[op16(sd, 4 * lk + 3, 4 * lk)], m12 = S[op16(sd, 4 * lk + 2, 4 * lk + 1)];
+      T m13 = S[op16(sd, 4 * lk + 3, 4 * lk + 1)], m23 = S[op16(sd, 4 * lk + 3, 4 * lk + 2)];
+      T r0 = srinv[16 * q + 4 * lk], r1 = srinv[16 * q + 4 * lk + 1];
+      T r2 = srinv[16 * q + 4 * lk + 2], r3 = srinv[16 * q + 4 * lk + 3];
+      v4 t = X[q];
+      if (q > 0) {
+        v4 acc = zero;
+#pragma unroll
+        for (int p = 0; p < q; ++p) acc = mul(q * (q + 1) / 2 + p, X[p], acc);
+        t = t - acc;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const T x0 = t[0] * r0;
+        const T x1 = (t[1] - x0 * m01) * r1;
+        const T x2 = ((t[2] - x0 * m02) - x1 * m12) * r2;
+        const T x3 = (((t[3] - x0 * m03) - x1 * m13) - x2 * m23) * r3;
+        const bool mine = lk == j;
+        const v4 xj = mine ? v4{x0, x1, x2, x3} : zero;
+        if (mine) X[q] = xj;
+        if (j < 3) {
+          const v4 acc = mul(sd, xj, zero);
+          if (lk > j) t = t - acc;
+        }
+      }
+    }
+  }
+  if (g0 < L) {
+    if (below) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int c = 16 * q + 4 * lk + v;
+          if (c < bw) F[g + (int64_t)(c0 + c) * L] = X[q][v];
+        }
+    } else {
+      T* Fa = F + c0 + (int64_t)g * L;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int r = 16 * q + 4 * lk + v;
+          if (r < bw) Fa[r] = X[q][v];
+        }
+    }
   }
 }
 
-// Off-diagonal parts of one block after blk_diag_kernel (see the section
-// comment); NQ bounds the piece width. Workgroups b < d.nl take 64 rows
-// below the block, the others 64 columns right of it. Dynamic LDS:
-// 64 * kRLD + 128 * NQ elements.
+// Off-diagonal parts of one block in steps that hold a block of more than 64
+// columns, by substitution (see the section comment); NQ bounds the piece
+// width. Workgroups b < d.nl take 64 rows below the block, the others 64
+// columns right of it. Dynamic LDS: 64 * kRLD + 128 * NQ elements.
 template <typename T, int NQ>
 __global__ void __launch_bounds__(kWG)
 blk_offdiag_kernel(DevSym s, const BlkDesc* __restrict__ desc, int ndesc,
@@ -1524,10 +1584,6 @@ blk_offdiag_kernel(DevSym s, const BlkDesc* __restrict__ desc, int ndesc,
   const int di = find_blk(desc, ndesc, blockIdx.x);
   const BlkDesc d = desc[di];
   const int b = blockIdx.x - d.wg_begin;
-  if (d.c1 - d.c0 <= 64) {
-    offdiag64_body<T>(d, desc[di].pw, b, arena, ipvt, S, spiv);
-    return;
-  }
   const int f = d.front;
   const int L = s.fL[f];
   const int64_t fc0 = s.fc0[f];
@@ -2054,15 +2110,16 @@ template <typename T>
 __global__ void __launch_bounds__(kWG)
 blk_diag_border_kernel(DevSym s, const BlkDesc* __restrict__ ddesc, int ndiag,
                        const GemmDesc* __restrict__ gdesc, int ngemm, T* __restrict__ arena,
-                       int64_t* __restrict__ ipvt, unsigned long long* __restrict__ first_fail,
-                       int lowp) {
+                       int64_t* __restrict__ ipvt, int32_t* __restrict__ rperm,
+                       unsigned long long* __restrict__ first_fail, int lowp) {
   const int64_t vs = blockIdx.y;  // value set
   arena += vs * s.vs_arena;
   ipvt += vs * s.n;
+  rperm += vs * s.n;
   constexpr int kL = kSlabLds<T> > kGemmLds<T> ? kSlabLds<T> : kGemmLds<T>;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kL];
   if ((int)blockIdx.x < ndiag)
-    blk_diag_slab_body<T>(s, ddesc[blockIdx.x], arena, ipvt, first_fail, lds);
+    blk_diag_slab_body<T>(s, ddesc[blockIdx.x], arena, ipvt, rperm, first_fail, lds);
   else
     blk_gemm_body<T>(s, gdesc, ngemm, arena, lowp,
                      xcd_tile((int)blockIdx.x - ndiag, (int)gridDim.x - ndiag), lds);
