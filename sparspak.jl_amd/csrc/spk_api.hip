@@ -98,6 +98,7 @@ struct LevelPlan {
     Launch gemm2;
     bool w1 = false;
     bool wide = false;  // a block of more than 64 columns: the LDS diagonal form
+    int slab = 0;       // LDS elements of the register diagonal form
     // the previous step's update within its block group, launched with this
     // step's diagonal regions (blk_diag_border_kernel)
     Launch bin;
@@ -709,6 +710,9 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
         G.diag.wg += 1;
         const i32 bw = B.c1 - B.c0;
         G.diag.lds = std::max(G.diag.lds, bw * spk::kRLD);
+        if (bw <= 64)
+          G.slab = std::max(G.slab, spk::slab_elems(bw, bdesc.back().pw[0],
+                                                    fold[fi].second > fold[fi].first));
         if (bw > 64) G.wide = true;
         for (i32 p = B.p0; p < B.p0 + B.np; ++p) {
           const double q = (double)(h->xsuper[p + 1] - h->xsuper[p]);
@@ -1100,6 +1104,12 @@ void set_lds_attrs() {
                             kSmallLmax * kSmallLmax * (int)sizeof(T)));
   hipck(hipFuncSetAttribute((const void*)spk::small_front_kernel<T, 64>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+  hipck(hipFuncSetAttribute((const void*)spk::blk_diag_slab_kernel<T>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            spk::slab_elems(64, 1, true) * (int)sizeof(T)));
+  hipck(hipFuncSetAttribute((const void*)spk::blk_diag_border_kernel<T>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            spk::slab_elems(64, 1, true) * (int)sizeof(T)));
   hipck(hipFuncSetAttribute((const void*)spk::blk_diag_kernel<T, kNqLU>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
   hipck(hipFuncSetAttribute((const void*)spk::blk_diag_kernel<T, kNqSPD>,
@@ -1192,8 +1202,10 @@ void run_factor(spkhip_handle* h) {
           h->cur_grid = G.diag.wg + G.bin.wg;
           Prof pr(h, SPKHIP_K_DIAG_BORDER, G.diag.flops + G.bin.flops,
                   (G.diag.elems + G.bin.elems) * sizeof(T));
+          const size_t lds =
+              std::max<size_t>((size_t)G.slab * sizeof(T), (size_t)spk::kGemmLds<T>);
           hipLaunchKernelGGL((spk::blk_diag_border_kernel<T>), dim3(G.diag.wg + G.bin.wg, h->nvs),
-                             dim3(kWG), 0, st, h->ds, h->d_bdesc.p + G.diag.off, G.diag.wg,
+                             dim3(kWG), lds, st, h->ds, h->d_bdesc.p + G.diag.off, G.diag.wg,
                              h->d_gdesc.p + G.bin.off, G.bin.cnt, arena.p, h->d_ipvt.p,
                              h->d_rperm.p, h->d_fail.p, h->lowp);
           hipck(hipGetLastError());
@@ -1201,8 +1213,8 @@ void run_factor(spkhip_handle* h) {
           h->cur_grid = G.diag.wg;
           Prof pr(h, SPKHIP_K_DIAG, G.diag.flops, G.diag.elems * sizeof(T));
           if (slab && !G.wide)
-            hipLaunchKernelGGL((spk::blk_diag_slab_kernel<T>), dim3(G.diag.wg, h->nvs), dim3(kWG), 0, st,
-                               h->ds, h->d_bdesc.p + G.diag.off, arena.p, h->d_ipvt.p,
+            hipLaunchKernelGGL((spk::blk_diag_slab_kernel<T>), dim3(G.diag.wg, h->nvs), dim3(kWG),
+                               (size_t)G.slab * sizeof(T), st, h->ds, h->d_bdesc.p + G.diag.off, arena.p, h->d_ipvt.p,
                                h->d_rperm.p, h->d_fail.p);
           else if (lu)
             hipLaunchKernelGGL((spk::blk_diag_kernel<T, kNqLU>), dim3(G.diag.wg, h->nvs), dim3(kWG),

@@ -1128,9 +1128,102 @@ blk_diag_kernel(DevSym s, const BlkDesc* __restrict__ desc, T* __restrict__ aren
   store_tile<T, 1, LD>(Fr, L, bw, bw, R);
 }
 
+// v, computed where it stands for every lane (keeps the compiler from
+// turning a select of it into a branch around its computation).
+__device__ inline double pin(double v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+__device__ inline float pin(float v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// 1 / v in every lane and the maximum of key over the 64 lanes (all lanes
+// active): the two dependent chains, a division (about eleven operations)
+// and four DPP maxima, are independent of each other, so each operation of
+// one fills the other's latency; the scheduling barriers keep the compiler
+// from placing one chain after the other (both one after the other: 250
+// cycles).
+#define SPK_SB __builtin_amdgcn_sched_barrier(0)
+template <int CTRL>
+__device__ inline unsigned dpp_umax(unsigned v) {
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false));
+}
+__device__ inline unsigned row_umax(unsigned v) {  // v: the rows' own maxima
+  const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)v, 0);
+  const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)v, 16);
+  const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)v, 32);
+  const unsigned d = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
+  return max(max(a, b), max(c, d));
+}
+__device__ inline double recip_and_max(double v, unsigned key, unsigned& mx) {
+  bool f0, f1;
+  const double d0 = __builtin_amdgcn_div_scale(1.0, v, false, &f0);
+  unsigned m = dpp_umax<0xB1>(key);  // lanes ^1
+  SPK_SB;
+  const double r0 = __builtin_amdgcn_rcp(d0);
+  const double n0 = __builtin_amdgcn_div_scale(1.0, v, true, &f1);
+  SPK_SB;
+  m = dpp_umax<0x4E>(m);  // lanes ^2
+  SPK_SB;
+  const double e0 = __builtin_fma(-d0, r0, 1.0);
+  SPK_SB;
+  m = dpp_umax<0x141>(m);  // mirror inside 8
+  SPK_SB;
+  const double r1 = __builtin_fma(r0, e0, r0);
+  SPK_SB;
+  m = dpp_umax<0x140>(m);  // mirror inside 16
+  SPK_SB;
+  const double e1 = __builtin_fma(-d0, r1, 1.0);
+  SPK_SB;
+  mx = row_umax(m);
+  const double r2 = __builtin_fma(r1, e1, r1);
+  const double q = n0 * r2;
+  const double e2 = __builtin_fma(-d0, q, n0);
+  return __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(e2, r2, q, f1), v, 1.0);
+}
+__device__ inline float recip_and_max(float v, unsigned key, unsigned& mx) {
+  bool f0, f1;
+  const float d0 = __builtin_amdgcn_div_scalef(1.0f, v, false, &f0);
+  unsigned m = dpp_umax<0xB1>(key);
+  SPK_SB;
+  const float r0 = __builtin_amdgcn_rcpf(d0);
+  const float n0 = __builtin_amdgcn_div_scalef(1.0f, v, true, &f1);
+  SPK_SB;
+  m = dpp_umax<0x4E>(m);
+  SPK_SB;
+  const float e0 = __builtin_fmaf(-d0, r0, 1.0f);
+  SPK_SB;
+  m = dpp_umax<0x141>(m);
+  SPK_SB;
+  const float r1 = __builtin_fmaf(e0, r0, r0);
+  SPK_SB;
+  m = dpp_umax<0x140>(m);
+  SPK_SB;
+  const float q0 = n0 * r1;
+  SPK_SB;
+  mx = row_umax(m);
+  const float e1 = __builtin_fmaf(-d0, q0, n0);
+  const float q1 = __builtin_fmaf(e1, r1, q0);
+  const float e2 = __builtin_fmaf(-d0, q1, n0);
+  return __builtin_amdgcn_div_fixupf(__builtin_amdgcn_div_fmasf(e2, r1, q1, f1), v, 1.0f);
+}
+
+// The leading 32 bits of |v|, plus one, for a candidate that is a number;
+// 0 otherwise. For floats all of |v|: the order of the keys is the order of
+// the magnitudes, up to ties in the low half of a double.
+__device__ inline unsigned pivot_key(double v, bool cand) {
+  const unsigned hi = (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffffu;
+  return cand && v == v ? hi + 1u : 0u;
+}
+__device__ inline unsigned pivot_key(float v, bool cand) {
+  return cand && v == v ? (__float_as_uint(v) & 0x7fffffffu) + 1u : 0u;
+}
+
 // Diagonal region of one block of at most 64 columns per workgroup, held
-// in registers: wave w keeps columns [16 w, 16 w + 16) of the region, one
-// row per lane. The region is factored right-looking, one column at a time,
+// in registers in panels of eight columns: wave w keeps panels w and w + 4,
+// one row per lane. The region is factored right-looking, one column at a time,
 // with the reference's pivoting confined to each piece's rows (LU; an SPD
 // front takes the row at position k, no interchanges)
 // (SpkLUFactor.jl:230-240, GenericBlasLapackFragments.jl:56-100). Step k,
@@ -1149,231 +1242,321 @@ blk_diag_kernel(DevSym s, const BlkDesc* __restrict__ desc, T* __restrict__ aren
 // as the reference's update of one supernode by another does (the sum is
 // kept in the entry itself, the entry's value aside until the piece's last
 // column). Rows never move while factoring: each lane tracks the position
-// its row holds. The wave owning column k publishes the step (multipliers,
-// pivot lane, pivot position) through LDS; the other waves apply published
-// steps to their columns as they come, without barriers (a wave only ever
-// waits for steps of columns left of its own, which the waves to its left
-// publish without waiting on it). At the end each row is stored at its
-// final position in the columns of its piece and right of it, and at its
-// own row in the columns of earlier pieces, which the reference never
-// interchanges.
+// its row holds (positions of a piece stay inside the piece, so the rows
+// below step k are those of a position past k, at any later time too). The
+// wave owning column k updates the rest of its panel only, publishes the
+// step (multipliers, pivot lane, pivot position) through LDS and goes on;
+// the waves apply published steps to their other panels as they come,
+// without barriers (a wave only ever waits for steps of columns left of its
+// own, which are published without waiting on it). At the end each row is
+// stored at its final position in the columns of its piece and right of it,
+// and at its own row in the columns of earlier pieces, which the reference
+// never interchanges.
 // When d.fk1 > d.fk0 the region first takes the product of the previous
 // block (columns [fk0, fk1)) with its own columns, summed from zero over
-// those columns in order and subtracted once (the trailing update's form),
-// so that the rest of that block's update can run beside this kernel.
-// lds: kSlabLds<T> bytes (the three 64 x 64 arrays below).
+// those columns and subtracted once (the trailing update's form), so that
+// the rest of that block's update can run beside this kernel; the product is
+// formed by MFMA from LDS in steps of 32 columns.
+// What bounds it: the chain pivot search -> reciprocal -> next column, once
+// per column, on one wave (latency and issue: a readlane pair with its FMA
+// costs 26 cycles, a DPP maximum 12, a taken branch 30). So the chain's wave
+// touches eight columns only (alternating panels: sixteen columns in one
+// wave cost 1 500 cycles per column), the search compares the leading 32
+// bits of the magnitudes (only when they tie does the full search decide),
+// and every lane forms its own entry's reciprocal beside the search. One
+// 60-column block alone, two pieces: 42.8 -> 32.1 us in double and 38.3 ->
+// 29.6 us in float, with a folded block 47.2 -> 36.1 and 41.6 -> 32.5 us
+// (of these 4 us are the folded product, 2.6 us the launch). The LDS, 97 KB
+// before, is 36 KB in double: other kernels' workgroups leave room for it
+// (diagonal regions waited for the second stream's updates to drain: 175 us
+// on average per launch in double at 64^3).
+// lds: slab_elems(bw, first piece's width, folded) elements: the finished
+// columns (bw x bw), the entries set aside (those of the later pieces), or
+// the folded panels.
 constexpr int kMaxBlkPieces = 8;  // most pieces in one block
-template <typename T>
-constexpr int kSlabLds = 3 * 64 * 64 * (int)sizeof(T);
+constexpr int kFoldK = 32;        // folded columns per step
+__host__ __device__ constexpr int slab_elems(int bw, int w0, bool fold) {
+  const int own = bw * bw + (bw - w0) * (bw - w0);
+  return fold && own < 2 * kFoldK * 64 ? 2 * kFoldK * 64 : own;
+}
 template <typename T>
 __device__ __attribute__((always_inline)) void blk_diag_slab_body(
     const DevSym& s, const BlkDesc& d, T* __restrict__ arena, int64_t* __restrict__ ipvt,
     int32_t* __restrict__ rperm, unsigned long long* __restrict__ first_fail,
     unsigned char* lds) {
-  constexpr int SW = 16;                  // columns per wave
-  // step k: the multiplier of each row; finished column c, rows in lane
-  // order; entries set aside while a piece's sum forms
-  T (*sl)[64] = reinterpret_cast<T (*)[64]>(lds);
-  T (*sout)[64] = reinterpret_cast<T (*)[64]>(lds + 64 * 64 * sizeof(T));
-  T (*ssv)[64] = reinterpret_cast<T (*)[64]>(lds + 2 * 64 * 64 * sizeof(T));
-  __shared__ int smeta[64];               // step k: pivot lane | position << 8 | nonzero << 16
+  constexpr int PW = 8;                   // columns per panel
+  // step k, once published (before: -1): pivot lane | position << 8 |
+  // nonzero << 16
+  __shared__ int smeta[64];
   __shared__ int spo[kMaxBlkPieces + 1];  // piece offsets in the region; spo[np] = bw
-  __shared__ int scp[64];                 // piece of each region column
-  __shared__ int spos[64];                // final position of each row
-  __shared__ int ssrc[64];                // the row each position takes
-  __shared__ int spiv[64];                // step k: pivot position, 1-based in its piece
-  __shared__ int sdone;                   // steps published
+  __shared__ unsigned char scp[64];       // piece of each region column
+  __shared__ unsigned char spos[64];      // final position of each row
+  __shared__ unsigned char ssrc[64];      // the row each position takes
   const int lane = threadIdx.x % 64, w = wave_id();
   const int L = d.L;
   const int64_t fc0 = d.fc0;
   const int c0 = d.c0, bw = d.c1 - d.c0, np = d.np;
   const T* const Fb = arena + d.foff;
   T* R = arena + d.foff + c0 + (int64_t)c0 * L;
-  const int cb = SW * w;
-  // the front and the piece widths come from the descriptor, so the region,
-  // the previous block's panels and the widths are read in one batch
-  // a[i] holds column c + i, c = cb while the earlier waves' steps are
-  // applied, then the column of the current step: the slab shifts left by
-  // one column after each of this wave's steps, so that the pivot column is
-  // always a[0] and the loop body indexes registers statically
-  T a[SW];
+  // finished column k, rows in lane order, at sl[k bw + row]: multipliers of
+  // the rows below the pivot, the others' values; and the entries set aside,
+  // (row, column) from (n0, n0), n0 the first piece's width
+  const int n0 = d.pw[0], nv = bw - n0;
+  T* sl = reinterpret_cast<T*>(lds);
+  T* ssv = sl + bw * bw;
+  // this wave's panels: columns ca + i and cb + i. The front and the piece
+  // widths come from the descriptor, so the region, the previous block's
+  // panels and the widths are read in one batch
+  const int ca = PW * w, cb = PW * w + 32;
+  T a[PW], b[PW];
 #pragma unroll
-  for (int i = 0; i < SW; ++i)
-    a[i] = (lane < bw && cb + i < bw) ? R[lane + (int64_t)(cb + i) * L] : T(0);
+  for (int i = 0; i < PW; ++i) {
+    a[i] = (lane < bw && ca + i < bw) ? R[lane + (int64_t)(ca + i) * L] : T(0);
+    b[i] = (lane < bw && cb + i < bw) ? R[lane + (int64_t)(cb + i) * L] : T(0);
+  }
   const int fkw = d.fk1 - d.fk0;
+  // L(c0 + r, fk0 + k) at Lp[64 k + (r ^ 16 (k % 4))], U(fk0 + k, c0 + c) at
+  // Up[32 c + (k ^ usw(c))]: stores and operand reads without bank conflicts
+  T* Lp = sl;
+  T* Up = sl + kFoldK * 64;
+  const int fk = lane % kFoldK, fc = 2 * w + lane / kFoldK;
+  auto usw = [](int c) {
+    return std::is_same<T, double>::value ? 2 * (c & 15) : 4 * ((c >> 1) & 7);
+  };
+  // both steps' panels (a block has at most 64 columns) from clamped
+  // addresses, in flight with the region; what lies outside is zeroed below
+  T pl[2][8], pu[2][8];
   if (fkw > 0) {
-    // L(c0 + r, fk0 + k) at sout[k][r], U(fk0 + k, c0 + c) at sl[k][c]
-    for (int idx = threadIdx.x; idx < 64 * fkw; idx += kWG) {
-      const int r = idx % 64, k = idx / 64;
-      sout[k][r] = (r < bw) ? Fb[c0 + r + (int64_t)(d.fk0 + k) * L] : T(0);
-      sl[k][r] = (r < bw) ? Fb[d.fk0 + k + (int64_t)(c0 + r) * L] : T(0);
-    }
+    const T* lrow = Fb + c0 + min(lane, bw - 1) + (int64_t)d.fk0 * L;
+    const T* ucol = Fb + d.fk0 + (int64_t)c0 * L;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int k = kFoldK * h + w + 4 * u, c = fc + 8 * u;
+        pl[h][u] = lrow[(int64_t)min(k, fkw - 1) * L];
+        pu[h][u] = ucol[min(kFoldK * h + fk, fkw - 1) + (int64_t)min(c, bw - 1) * L];
+      }
   }
   if ((int)threadIdx.x <= np) {
     int o = 0;  // spo[np] = bw: the pieces fill the block
     for (int q = 0; q < (int)threadIdx.x; ++q) o += d.pw[q];
     spo[threadIdx.x] = o;
   }
-  if (threadIdx.x == 0) sdone = 0;
+  if (threadIdx.x < 64) smeta[threadIdx.x] = -1;
   __syncthreads();
   if (threadIdx.x < 64) {
     int p = 0;
     while (p + 1 < np && (int)threadIdx.x >= spo[p + 1]) ++p;
-    scp[threadIdx.x] = p;
+    scp[threadIdx.x] = (unsigned char)p;
+  }
+  if (fkw > 0) {
+    typedef typename Mfma16<T>::v4 v4;
+    const int l16 = lane % 16, lk = lane / 16;
+    // operand column l16 of the wave's sixteen: panel w, then panel w + 4
+    const int mc = std::is_same<T, double>::value ? 4 * (l16 % 4) + l16 / 4 : l16;
+    const int mcol = mc < PW ? ca + mc : cb + mc - PW;
+    v4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = v4{T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k0 = kFoldK * h;
+      if (k0 < fkw) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int k = w + 4 * u, c = fc + 8 * u;
+          Lp[64 * k + (lane ^ (16 * (k & 3)))] = (lane < bw && k0 + k < fkw) ? pl[h][u] : T(0);
+          Up[kFoldK * c + (fk ^ usw(c))] = (c < bw && k0 + fk < fkw) ? pu[h][u] : T(0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < kFoldK / 4; ++ks) {
+          const int k = 4 * ks + lk;
+          const T uv = Up[kFoldK * mcol + (k ^ usw(mcol))];
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            acc[t] = Mfma16<T>::op(uv, Lp[64 * k + ((16 * t + l16) ^ (16 * lk))], acc[t]);
+        }
+        __syncthreads();
+      }
+    }
+    // lane l of tile t holds row 16 t + l % 16, columns 4 (l / 16) .. + 3:
+    // through LDS to one row per lane
+    T* Tw = sl + w * 2 * PW * 64;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) Tw[(4 * lk + v) * 64 + 16 * t + l16] = acc[t][v];
+    wave_lds_sync();
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      a[i] = a[i] - Tw[i * 64 + lane];
+      b[i] = b[i] - Tw[(PW + i) * 64 + lane];
+    }
   }
   __syncthreads();
-  // this lane's row: its piece pr (np for the rows past the region)
-  const int pr = lane < bw ? scp[lane] : np;
-  const int rlo = pr < np ? spo[pr] : 0;
-  int pos = lane;
-  if (fkw > 0) {
-    T acc[SW];
-#pragma unroll
-    for (int i = 0; i < SW; ++i) acc[i] = T(0);
-    for (int k = 0; k < fkw; ++k) {
-      const T lv = sout[k][lane];
-#pragma unroll
-      for (int i = 0; i < SW; ++i) acc[i] += lv * sl[k][cb + i];
-    }
-#pragma unroll
-    for (int i = 0; i < SW; ++i)
-      if (lane < bw && cb + i < bw) a[i] = a[i] - acc[i];
-    __syncthreads();
-  }
-  // first step of piece pk (current column c): the later pieces' entries
-  // right of the piece are set aside and the piece's products summed from
-  // zero in their place; last step: the entries take the sum off. Only this
-  // wave's own columns [cb, cb + SW): past them a[] holds placeholders, and
-  // the set-aside slots there belong to the wave owning those columns, which
-  // may still be restoring an earlier piece from them. Called under
-  // wave-uniform branches that hold a compiler barrier, so that they stay
-  // branches instead of selects executed at every step.
-  const int cown = cb + SW;
-  auto piece_begin = [&](int pk, int c) {
+  int pos = lane < bw ? lane : -1;
+  // First step of a piece ending at cn, for the panel x of columns c, c + 1,
+  // .. < cend: the later pieces' entries right of the piece are set aside and
+  // the piece's products summed from zero in their place; last step: the
+  // entries take the sum off. Called under wave-uniform branches that hold a
+  // compiler barrier, so that they stay branches instead of selects executed
+  // at every step.
+  auto piece_begin = [&](T (&x)[PW], int cn, int c, int cend) {
     __asm__ volatile("" ::: "memory");
-    const int cn = __builtin_amdgcn_readfirstlane(spo[pk + 1]);
-    const bool later = pr > pk && pr < np;
+    if (pos >= cn) {
 #pragma unroll
-    for (int i = 0; i < SW; ++i)
-      if (c + i >= cn && c + i < cown) {
-        ssv[c + i][lane] = a[i];
-        if (later) a[i] = T(0);
-      }
-  };
-  auto piece_end = [&](int pk, int c) {
-    __asm__ volatile("" ::: "memory");
-    const int cn = __builtin_amdgcn_readfirstlane(spo[pk + 1]);
-    const bool later = pr > pk && pr < np;
-#pragma unroll
-    for (int i = 0; i < SW; ++i)
-      if (c + i >= cn && c + i < cown && later) a[i] = ssv[c + i][lane] + a[i];
-  };
-  // the piece of the current step, [plo, phi): advanced at its boundaries
-  int pk = 0;
-  int plo = 0;
-  int phi = __builtin_amdgcn_readfirstlane(spo[1]);
-  // steps of the columns left of this wave's slab, as they are published
-  const int nprev = min(cb, bw);
-  for (int k = 0; k < nprev; ++k) {
-    if (k == phi) {
-      ++pk;
-      plo = phi;
-      phi = __builtin_amdgcn_readfirstlane(spo[pk + 1]);
+      for (int i = 0; i < PW; ++i)
+        if (c + i >= cn && c + i < cend) {
+          ssv[(c + i - n0) * nv + lane - n0] = x[i];
+          x[i] = T(0);
+        }
     }
-    for (int it = 0; it < (1 << 24) &&
-         __hip_atomic_load(&sdone, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <= k;
-         ++it)
-      __builtin_amdgcn_s_sleep(1);
-    const int meta = __builtin_amdgcn_readfirstlane(smeta[k]);
+  };
+  auto piece_end = [&](T (&x)[PW], int cn, int c, int cend) {
+    __asm__ volatile("" ::: "memory");
+    if (pos >= cn) {
+#pragma unroll
+      for (int i = 0; i < PW; ++i)
+        if (c + i >= cn && c + i < cend) x[i] = ssv[(c + i - n0) * nv + lane - n0] + x[i];
+    }
+  };
+  // A panel's next step k and the piece [plo, phi) holding it
+  struct At {
+    int k, pk, plo, phi;
+  };
+  auto next_piece = [&](At& t) {
+    t.pk += 1;
+    t.plo = t.phi;
+    t.phi = __builtin_amdgcn_readfirstlane(spo[t.pk + 1]);
+  };
+  auto published = [&](int k) {
+    return __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(&smeta[k], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+  };
+  int seen = 0;  // steps whose interchanges are in pos
+  // published step t.k (its word meta) applied to the panel x of columns c ..
+  auto apply = [&](T (&x)[PW], At& t, int c, int meta) {
+    const int k = t.k;
+    if (k == t.phi) next_piece(t);
+    const T lv = sl[k * bw + min(lane, bw - 1)];
     const int bl = meta & 0xff;
     const int kp = (meta >> 8) & 0xff;
-    const bool nz = (meta >> 16) & 1;
-    if (nz && kp != k) {
-      if (pos == k)
-        pos = kp;
-      else if (lane == bl)
-        pos = k;
+    if (k == seen) {
+      if ((meta >> 16) & 1) {
+        pos = pos == k ? kp : pos;
+        pos = lane == bl ? k : pos;
+      }
+      ++seen;
     }
-    const bool below = (pr == pk && pos > k) || (pr > pk && pr < np);
+    if (k == t.plo) piece_begin(x, t.phi, c, min(c + PW, bw));
     // rows not below subtract 0 u, which leaves a finite entry unchanged
-    const T lb = below ? sl[k][lane] : T(0);
-    if (k == plo) piece_begin(pk, cb);
-    T u[SW];
+    const T lb = pos > k ? lv : T(0);
 #pragma unroll
-    for (int i = 0; i < SW; ++i) u[i] = rdlane(a[i], bl);
+    for (int i = 0; i < PW; ++i) x[i] = x[i] - lb * rdlane(x[i], bl);
+    if (k == t.phi - 1) piece_end(x, t.phi, c, min(c + PW, bw));
+    t.k = k + 1;
+  };
+  // Panel a, then panel b. Until the panel's own columns come, published
+  // steps are applied to it first, and to panel b while none is waiting.
+  At ta{0, 0, 0, 0}, tb;
+  ta.phi = __builtin_amdgcn_readfirstlane(spo[1]);
+  tb = ta;
+#pragma unroll 1
+  for (int c = ca; c < bw; c += 32) {
+    for (int it = 0; ta.k < c && it < (1 << 24); ++it) {
+      const int meta = published(ta.k);
+      if (meta >= 0)
+        apply(a, ta, c, meta);
+      else if (c == ca && tb.k < ta.k && cb < bw)
+        apply(b, tb, cb, published(tb.k));
+    }
+    // The columns [c, cend): a[0] is the current column, the panel shifts
+    // left by one with each step. Column k's pivot lane bl and every lane's
+    // reciprocal of its entry rc are known when its step begins; the columns
+    // of one piece run without looking at piece boundaries
+    const int cend = min(c + PW, bw);
+    int bl = 0;
+    T rc = T(0);
+    auto search = [&](int k, int hi) {
+      // without pivoting (SPD) the pivot row is the one at position k: lane k
+      const bool cand = pos >= k && pos < hi;
+      const unsigned key = pivot_key(a[0], cand);
+      unsigned mx;
+      const T r = recip_and_max(a[0], key, mx);
+      rc = pin(a[0] == T(0) ? T(1) : r);  // a zero pivot scales nothing
+      bl = k;
+      if (s.pivot) {
+        const unsigned long long msk = __ballot(key == mx);
+        bl = __builtin_amdgcn_readfirstlane(__ffsll((long long)msk) - 1);
+        if (__builtin_expect(mx == 0u || (msk & (msk - 1ull)) != 0ull, 0))
+          bl = pivot_lane(a[0], pos, cand, k);
+      }
+    };
+    if (ta.k == ta.phi) next_piece(ta);
+#pragma unroll 1
+    for (int k = c; k < cend;) {
+      const int phi = ta.phi, ke = min(cend, phi);
+      if (k == ta.plo) piece_begin(a, phi, k, cend);
+      search(k, phi);
+      T* slk = sl + k * bw + lane;
+#pragma unroll 1
+      for (;;) {
+        const T v = a[0];
+        const T inv = rdlane(rc, bl);
+        const int kp = __builtin_amdgcn_readlane(pos, bl);
+        const bool nz = rdlane(v, bl) != T(0);
+        const int meta = bl | (kp << 8) | ((int)nz << 16);
+        pos = (nz && pos == k) ? kp : pos;
+        pos = (nz && lane == bl) ? k : pos;
+        const bool below = pos > k;
+        const T l = v * inv;
+        const T lb = below ? l : T(0);
+        // (no global memory access until the end: a release would wait for it)
+        if (lane < bw) *slk = below ? l : v;
+        slk += bw;
 #pragma unroll
-    for (int i = 0; i < SW; ++i) a[i] = a[i] - lb * u[i];
-    if (k == phi - 1) piece_end(pk, cb);
+        for (int i = 1; i < PW; ++i) a[i - 1] = a[i] - lb * rdlane(a[i], bl);
+        a[PW - 1] = T(0);
+        if (k + 1 < ke) search(k + 1, phi);
+        // published after the next search, when the write above has long
+        // completed (the release waits for nothing)
+        __hip_atomic_store(&smeta[k], meta, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (++k >= ke) break;
+      }
+      if (k == phi) {
+        piece_end(a, phi, k, cend);
+        if (k < bw) next_piece(ta);
+      }
+    }
+    seen = cend;
+    // the second panel: its steps go on where they were left
+#pragma unroll
+    for (int i = 0; i < PW; ++i) a[i] = b[i];
+    ta = tb;
   }
-  // this wave's own columns; step k is published (sdone = k + 1) at the
-  // start of step k + 1, when its LDS writes have long completed, so that
-  // the release never waits
-  const int kend = min(cb + SW, bw);
-  for (int k = cb; k < kend; ++k) {
-    if (k == phi) {
-      ++pk;
-      plo = phi;
-      phi = __builtin_amdgcn_readfirstlane(spo[pk + 1]);
-    }
-    if (k > cb)
-      __hip_atomic_store(&sdone, k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (k == plo) piece_begin(pk, k);
-    const T v = a[0];
-    // without pivoting (SPD) the pivot row is the one at position k: lane k
-    const int bl = s.pivot ? pivot_lane(v, pos, pr == pk, k) : k;
-    const int kp = __builtin_amdgcn_readlane(pos, bl);
-    const T pv = rdlane(v, bl);
-    T u[SW];
-#pragma unroll
-    for (int i = 1; i < SW; ++i) u[i] = rdlane(a[i], bl);
-    const bool nz = pv != T(0);
-    if (nz && kp != k) {
-      if (pr == pk && pos == k)
-        pos = kp;
-      else if (lane == bl)
-        pos = k;
-    }
-    const T inv = T(1) / pv;
-    const bool below = (pr == pk && pos > k) || (pr > pk && pr < np);
-    const T l = nz ? v * inv : v;
-    // (no global memory access until the end: a release would wait for it)
-    sl[k][lane] = l;
-    if (lane == 0) {
-      smeta[k] = bl | (kp << 8) | ((int)nz << 16);
-      spiv[k] = kp - plo + 1;
-    }
-    sout[k][lane] = (below && nz) ? l : v;
-    const T lb = below ? l : T(0);
-#pragma unroll
-    for (int i = 1; i < SW; ++i) a[i] = a[i] - lb * u[i];
-    if (k == phi - 1) piece_end(pk, k);
-#pragma unroll
-    for (int i = 0; i + 1 < SW; ++i) a[i] = a[i + 1];
-    a[SW - 1] = T(0);
-  }
-  if (kend > cb)
-    __hip_atomic_store(&sdone, kend, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
   // the wave of the last column has seen every interchange
-  if (w == (bw - 1) / SW) {
-    spos[lane] = pos;
-    ssrc[pos] = lane;
+  if (w == (bw - 1) / PW % 4 && lane < bw) {
+    spos[lane] = (unsigned char)pos;
+    ssrc[pos] = (unsigned char)lane;
   }
   __syncthreads();
-  const int fpos = spos[lane];
+  const int fpos = lane < bw ? spos[lane] : 0;
+  const int pr = lane < bw ? scp[lane] : 0;  // the piece of row (column) `lane`
+  const int rlo = spo[pr];
   if ((int)threadIdx.x < bw) {
-    ipvt[fc0 + c0 + threadIdx.x] = spiv[threadIdx.x];
+    const int m = smeta[threadIdx.x];
+    ipvt[fc0 + c0 + threadIdx.x] = ((m >> 8) & 0xff) - rlo + 1;
     rperm[fc0 + c0 + threadIdx.x] = ssrc[threadIdx.x] | fpos << 8;
     // a zero pivot: the first piece that met one
-    if (!((smeta[threadIdx.x] >> 16) & 1))
-      atomicMin(first_fail, (unsigned long long)(d.piece + scp[threadIdx.x] + 1));
+    if (!((m >> 16) & 1)) atomicMin(first_fail, (unsigned long long)(d.piece + pr + 1));
   }
-  // column c of this wave: row r at its position in the columns of its
-  // piece and right of it, at its own row in earlier pieces' columns
+  // row r of a column at its position in the columns of its piece and right
+  // of it, at its own row in earlier pieces' columns
   if (lane < bw) {
-    for (int i = 0; i < SW; ++i) {
-      const int c = cb + i;
-      if (c < bw) R[(c >= rlo ? fpos : lane) + (int64_t)c * L] = sout[c][lane];
-    }
+    for (int c = w; c < bw; c += 4)
+      R[(c >= rlo ? fpos : lane) + (int64_t)c * L] = sl[c * bw + lane];
   }
 }
 
@@ -1386,8 +1569,8 @@ blk_diag_slab_kernel(DevSym s, const BlkDesc* __restrict__ desc, T* __restrict__
   arena += vs * s.vs_arena;
   ipvt += vs * s.n;
   rperm += vs * s.n;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kSlabLds<T>];
-  blk_diag_slab_body<T>(s, desc[blockIdx.x], arena, ipvt, rperm, first_fail, lds);
+  extern __shared__ __attribute__((aligned(32))) unsigned char smem_a32[];
+  blk_diag_slab_body<T>(s, desc[blockIdx.x], arena, ipvt, rperm, first_fail, smem_a32);
 }
 
 // Element of the operand entry (m, k) of 16 x 16 sub-block sb in LDS: the
@@ -2116,13 +2299,13 @@ blk_diag_border_kernel(DevSym s, const BlkDesc* __restrict__ ddesc, int ndiag,
   arena += vs * s.vs_arena;
   ipvt += vs * s.n;
   rperm += vs * s.n;
-  constexpr int kL = kSlabLds<T> > kGemmLds<T> ? kSlabLds<T> : kGemmLds<T>;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kL];
+  // dynamic: the larger of the regions' slabs and kGemmLds<T>
+  extern __shared__ __attribute__((aligned(32))) unsigned char smem_a32[];
   if ((int)blockIdx.x < ndiag)
-    blk_diag_slab_body<T>(s, ddesc[blockIdx.x], arena, ipvt, rperm, first_fail, lds);
+    blk_diag_slab_body<T>(s, ddesc[blockIdx.x], arena, ipvt, rperm, first_fail, smem_a32);
   else
     blk_gemm_body<T>(s, gdesc, ngemm, arena, lowp,
-                     xcd_tile((int)blockIdx.x - ndiag, (int)gridDim.x - ndiag), lds);
+                     xcd_tile((int)blockIdx.x - ndiag, (int)gridDim.x - ndiag), smem_a32);
 }
 
 // ---------------------------------------------------------------------------
@@ -2614,17 +2797,6 @@ template <typename T>
 __device__ inline T gather2(T y0, T y1, int src) {
   const T a = __shfl(y0, src & 63, 64), b = __shfl(y1, src & 63, 64);
   return src < 64 ? a : b;
-}
-
-// v, computed where it stands for every lane (keeps the compiler from
-// turning a select of it into a branch around its computation).
-__device__ inline double pin(double v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-__device__ inline float pin(float v) {
-  asm volatile("" : "+v"(v));
-  return v;
 }
 
 // The solve data of a block (nv four-element vectors) into LDS, all loads in
