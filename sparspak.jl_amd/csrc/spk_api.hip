@@ -32,6 +32,14 @@ constexpr int kGW = 128;    // widest block of pieces (LU)
 constexpr int kGMaxP = 8;   // most pieces in one block
 constexpr int kNqLU = 48;   // widest LU piece the blocked kernels take
 constexpr int kNqSPD = 96;  // widest SPD piece
+// LDS (bytes) a workgroup of the second stream's updates reserves, so that at
+// most three of them fit a CU (160 KB in units of 1280 bytes) and 36 KB stay
+// free for a diagonal region, an off-diagonal tile or an in-group update of
+// the main stream. Alone three per CU are up to 10 % slower than five, but
+// the main stream is the longer one: passes of 64^3 82.3 -> 81.2 ms (double),
+// 57.5 -> 56.5 ms (split-bf16), elasticity 40^3 93.3 -> 91.2 ms; with two per
+// CU 81.2, 57.2, 92.2 ms
+constexpr int kOverlapLds = 41216;
 
 struct HipFail {
   hipError_t e;
@@ -1253,7 +1261,10 @@ void run_factor(spkhip_handle* h) {
           if (two) stream_join(h, st, st2);
           h->cur_grid = G.gemm2.wg;
           Prof pr(h, SPKHIP_K_UPDATE, G.gemm2.flops, G.gemm2.elems * sizeof(T));
-          hipLaunchKernelGGL(spk::blk_gemm_kernel<T>, dim3(G.gemm2.wg, h->nvs), dim3(kWG), 0, st2, h->ds,
+          // three workgroups per CU, so that the next group's panel kernels
+          // find room beside them (kOverlapLds)
+          hipLaunchKernelGGL(spk::blk_gemm_kernel<T>, dim3(G.gemm2.wg, h->nvs), dim3(kWG),
+                             two ? kOverlapLds - spk::kGemmLds<T> : 0, st2, h->ds,
                              h->d_gdesc.p + G.gemm2.off, G.gemm2.cnt, arena.p, h->lowp);
           hipck(hipGetLastError());
           pending = two;

@@ -1950,19 +1950,25 @@ __device__ inline uint2 pack_f16(float a, float b, float c, float d) {
 }
 
 // One tile's products with 16-bit operands on the gfx950 matrix cores
-// (v_mfma_f32_16x16x32_bf16 / _f16), K-chunks of 32, double-buffered in LDS
-// as rows of kB16 halves: A(i, k) = L21 rows at part 0, [i kB16 + k],
-// B(k, j) = U12 columns at part 1, [j kB16 + k]; each lane reads its operand
+// (v_mfma_f32_16x16x32_bf16 / _f16), K-chunks of 32, double-buffered in LDS:
+// A(i, k) = L21 rows at part 0, row i, B(k, j) = U12 columns at part 1, row
+// j; each lane reads its operand
 // (eight consecutive k) with one 16-byte LDS read. lowp 1: bf16; lowp 3:
 // split bf16, x = hi + lo (lo at parts 2 and 3), products lo_b hi_a +
 // hi_b lo_a + hi_b hi_a; lowp 2: fp16 under diagonal scaling: A(i, k) times
 // and B(k, j) divided by 2^e_k, the power of two nearest below |U(k, k)|
 // (the product is unchanged; both stay in fp16 range when A is diagonally
 // scaled). Waves 0-1 stage A (rows 4 ag .. 4 ag + 3, k = 4 q + u), waves
-// 2-3 B (columns bc + 16 u, k = 4 q .. 4 q + 3); the 32 lanes of a half-wave
-// store rows 4 apart, which at 80 bytes per row start 16 banks apart.
-constexpr int kB16 = 40;                  // halves per LDS row (80 bytes)
-constexpr int kB16Part = kTile * kB16;    // one operand array, halves
+// 2-3 B (columns bc + 16 u, k = 4 q .. 4 q + 3). Row r of an array lies at
+// row place 16 (r % 4) + r / 4 of 64 bytes, its 16-byte units exchanged by
+// r % 4: the 32 lanes of a half-wave store rows 4 apart and the 16 lanes of
+// an operand read take consecutive rows, both without bank conflicts and
+// without padding (32 KB: five workgroups per CU).
+constexpr int kB16Part = kTile * 32;      // one operand array, halves
+// k = 8 unit .. of row r
+__device__ inline int at16(int r, int unit) {
+  return ((r & 3) * 16 + (r >> 2)) * 32 + ((unit ^ (r & 3)) * 8);
+}
 template <int lowp>
 __device__ __attribute__((always_inline)) inline void gemm16_tile(
     const float* __restrict__ F, int L, int k0, int bw, int r0, int rend, int j0, int cend,
@@ -2018,27 +2024,27 @@ __device__ __attribute__((always_inline)) inline void gemm16_tile(
         if (tail && kq + (isA ? u : e) >= bw) rg[u][e] = 0.0f;
       }
     if (isA) {
-      unsigned short* P = part(buf, 0) + 4 * ag * kB16 + 4 * q;
-      unsigned short* Q = part(buf, 2) + 4 * ag * kB16 + 4 * q;
+      unsigned short* P = part(buf, 0) + 4 * (q & 1);
+      unsigned short* Q = part(buf, 2) + 4 * (q & 1);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x0 = rg[0][e], x1 = rg[1][e], x2 = rg[2][e], x3 = rg[3][e];
-        *reinterpret_cast<uint2*>(P + e * kB16) =
+        *reinterpret_cast<uint2*>(P + at16(4 * ag + e, q / 2)) =
             lowp == 2 ? pack_f16(x0, x1, x2, x3) : pack_bf16(x0, x1, x2, x3);
         if (lowp == 3)
-          *reinterpret_cast<uint2*>(Q + e * kB16) =
+          *reinterpret_cast<uint2*>(Q + at16(4 * ag + e, q / 2)) =
               pack_bf16(bf_lo(x0), bf_lo(x1), bf_lo(x2), bf_lo(x3));
       }
     } else {
-      unsigned short* P = part(buf, 1) + bc * kB16 + 4 * q;
-      unsigned short* Q = part(buf, 3) + bc * kB16 + 4 * q;
+      unsigned short* P = part(buf, 1) + 4 * (q & 1);
+      unsigned short* Q = part(buf, 3) + 4 * (q & 1);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const float x0 = rg[u][0], x1 = rg[u][1], x2 = rg[u][2], x3 = rg[u][3];
-        *reinterpret_cast<uint2*>(P + 16 * u * kB16) =
+        *reinterpret_cast<uint2*>(P + at16(bc + 16 * u, q / 2)) =
             lowp == 2 ? pack_f16(x0, x1, x2, x3) : pack_bf16(x0, x1, x2, x3);
         if (lowp == 3)
-          *reinterpret_cast<uint2*>(Q + 16 * u * kB16) =
+          *reinterpret_cast<uint2*>(Q + at16(bc + 16 * u, q / 2)) =
               pack_bf16(bf_lo(x0), bf_lo(x1), bf_lo(x2), bf_lo(x3));
       }
     }
@@ -2057,7 +2063,7 @@ __device__ __attribute__((always_inline)) inline void gemm16_tile(
       if (ch + 2 < nch) gload((ch + 2) * KC);
     }
     auto frag = [&](int which, int row) {
-      return *reinterpret_cast<const bf16x8*>(part(cur, which) + row * kB16 + 8 * lk);
+      return *reinterpret_cast<const bf16x8*>(part(cur, which) + at16(row, lk));
     };
     bf16x8 ah[2], bh[2];
 #pragma unroll
@@ -2101,26 +2107,27 @@ __device__ __attribute__((always_inline)) inline void gemm16_tile(
 
 // The same tile in the front's own type (v_mfma_f64_16x16x4f64 /
 // v_mfma_f32_16x16x4f32), K-chunks of 16, double-buffered in LDS:
-// A(i, k) at As[k kLdA + i] (rows 16 elements past the tile apart, so that
-// the four k of an operand read fall in different banks), B(k, j) at
-// Bs[j ldB + k]. Column j of an accumulator tile is taken from U column
+// A(i, k) at As[64 k + (i ^ 16 (k % 4))], B(k, j) at Bs[16 j + (k ^ s(j))]
+// with s(j) = 2 (j / 2 % 8) in double, 4 (j / 4 % 4) in float: the operand
+// reads fall in different banks without padding. Column j of an accumulator tile is taken from U column
 // mcol(j), chosen so that both types leave four consecutive columns
 // 4 lk .. 4 lk + 3 in a lane (the f64 form puts row 4 v + lk in element v).
 constexpr int kGK = 16;            // inner dimension per chunk
-constexpr int kLdA = kTile + 16;
 template <typename T>
-constexpr int kGemmTLds = 2 * (kGK * kLdA + kTile * (kGK + Vec16<T>::n)) * (int)sizeof(T);
+constexpr int kGemmTLds = 4 * kGK * kTile * (int)sizeof(T);
 template <typename T>
 __device__ __attribute__((always_inline)) inline void gemmT_tile(
     const T* __restrict__ F, int L, int k0, int bw, int r0, int rend, int j0, int cend,
     unsigned char* lds_raw, typename Mfma16<T>::v4 (&acc)[2][2]) {
-  constexpr int VE = Vec16<T>::n, ldB = kGK + VE;
+  constexpr int VE = Vec16<T>::n;
   constexpr int U = kTile * kGK / VE / kWG;  // vectors per thread and operand
   typedef typename Vec16<T>::load V;
   typedef typename Vec16<T>::lds VL;
-  T (*As)[kGK * kLdA] = reinterpret_cast<T (*)[kGK * kLdA]>(lds_raw);
-  T (*Bs)[kTile * ldB] =
-      reinterpret_cast<T (*)[kTile * ldB]>(lds_raw + 2 * kGK * kLdA * sizeof(T));
+  T (*As)[kGK * kTile] = reinterpret_cast<T (*)[kGK * kTile]>(lds_raw);
+  T (*Bs)[kGK * kTile] = As + 2;
+  auto swb = [](int j) {
+    return std::is_same<T, double>::value ? 2 * ((j >> 1) & 7) : 4 * ((j >> 2) & 3);
+  };
   const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
   const int wr = (wave % 2) * 32, wc = (wave / 2) * 32;
   const int l16 = lane % 16, lk = lane / 16;
@@ -2161,8 +2168,9 @@ __device__ __attribute__((always_inline)) inline void gemmT_tile(
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int v = tid + u * kWG;
-      *reinterpret_cast<VL*>(&As[buf][(v / RV) * kLdA + VE * (v % RV)]) = ra[u];
-      *reinterpret_cast<VL*>(&Bs[buf][(v / KV) * ldB + VE * (v % KV)]) = rb[u];
+      const int k = v / RV, j = v / KV;
+      *reinterpret_cast<VL*>(&As[buf][k * kTile + ((VE * (v % RV)) ^ (16 * (k & 3)))]) = ra[u];
+      *reinterpret_cast<VL*>(&Bs[buf][j * kGK + ((VE * (v % KV)) ^ swb(j))]) = rb[u];
     }
   };
   const int nch = (bw + kGK - 1) / kGK;
@@ -2182,8 +2190,9 @@ __device__ __attribute__((always_inline)) inline void gemmT_tile(
       T av[2], bv[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        av[t] = As[cur][kk * kLdA + wr + t * 16 + l16];
-        bv[t] = Bs[cur][(wc + t * 16 + mcol) * ldB + kk];
+        const int j = wc + t * 16 + mcol;
+        av[t] = As[cur][kk * kTile + ((wr + t * 16 + l16) ^ (16 * lk))];
+        bv[t] = Bs[cur][j * kGK + (kk ^ swb(j))];
       }
 #pragma unroll
       for (int a = 0; a < 2; ++a)
