@@ -328,9 +328,9 @@ int64_t spkhip_ldltsolve_f32(int64_t nsuper, const int64_t* xsuper,
  * algorithmic work (flops and bytes the algorithm must move) is added to its
  * class. No counterpart in the reference (it has no device); used by the
  * benchmark's roofline report. */
-#define SPKHIP_K_ASSEMBLE 0   /* zero lnz/unz + scatter A (inmatrix)     */
+#define SPKHIP_K_ASSEMBLE 0   /* (A's values enter with K_SMALL, K_INIT)  */
 #define SPKHIP_K_SMALL 1      /* whole small front in LDS                */
-#define SPKHIP_K_INIT 2       /* large front: load panels + extend-add   */
+#define SPKHIP_K_INIT 2       /* large front: A's entries + extend-add   */
 #define SPKHIP_K_DIAG 3       /* large front: diagonal region of a block */
 #define SPKHIP_K_UPDATE 4     /* large front: block trailing update      */
 #define SPKHIP_K_WRITEBACK 5  /* large front: panels back to lnz/unz     */

@@ -188,7 +188,8 @@ struct spkhip_handle {
   DevBuf<i32> d_lindx, d_fL, d_fW, d_fc0, d_fsp0, d_fnp, d_fcbld, d_fchp, d_fch,
       d_relmap, d_small, d_it_front, d_it_col, d_ea_child, d_ea_t, d_solve;
   DevBuf<i64> d_foff, d_fcb, d_frel, d_fvec, d_it_ea, d_lcol, d_ucol;
-  DevBuf<spk::InitItem> d_it_init;  // the assembly's items, resolved
+  DevBuf<spk::InitItem> d_it_init;  // the assembly's items, resolved: from panels,
+  DevBuf<spk::AsmItem> d_it_asm;    // or from A's entries
   DevBuf<spk::EaItem> d_ea_init;
   DevBuf<BlkDesc> d_bdesc;
   DevBuf<spk::GemmDesc> d_gdesc;
@@ -215,7 +216,12 @@ struct spkhip_handle {
   // matrix
   i64 nnz = 0;
   bool have_csc = false, pattern_error = false;
-  DevBuf<i64> d_amap, d_rowptr;
+  // A's entries by front and column (host pointers per front column, fvec[f]
+  // + j; on the device per front), built with the pattern
+  std::vector<i64> aptr;
+  DevBuf<spk::AEnt> d_aent;
+  DevBuf<i64> d_afront;
+  DevBuf<i64> d_rowptr;
   DevBuf<i32> d_colind;
   DevBuf<i64> d_csc2csr;
   DevBuf<double> d_nzval, d_csrval, d_rowabs;
@@ -1082,6 +1088,67 @@ void build_amap(spkhip_handle* h, const i64* colptr, const i64* rowval,
   for (char e : errs) h->pattern_error = h->pattern_error || e;
 }
 
+// Entries that A repeats take their last value: the earlier ones lose their
+// slot. (Only columns whose rows do not ascend can hold any.)
+void drop_repeated(i64 n, const i64* colptr, const i64* rowval, std::vector<i64>& amap) {
+  std::vector<i64> last;  // per row, the last entry seen of the column
+  for (i64 i = 0; i < n; ++i) {
+    const i64 k0 = colptr[i] - 1, k1 = colptr[i + 1] - 1;
+    bool ascend = true;
+    for (i64 k = k0 + 1; k < k1; ++k) ascend = ascend && rowval[k] > rowval[k - 1];
+    if (ascend) continue;
+    if (last.empty()) last.assign(n, -1);
+    for (i64 k = k0; k < k1; ++k) {
+      i64& l = last[rowval[k] - 1];
+      if (l >= k0) amap[l] = -1;
+      l = k;
+    }
+  }
+}
+
+// A's entries with their place in their front (AEnt), grouped by front and
+// column on the device: pointers per front column (h->aptr, index fvec[f] +
+// j) and per front (device). The rows of a column are distinct, so its
+// entries' order, which is not determined, does not matter. The front
+// fields of h->ds that the kernels use are those of upload_symbolic and
+// build_storage.
+void build_entries(spkhip_handle* h, const std::vector<i64>& amap) {
+  const i64 nc = h->vec_elems;
+  hipStream_t st = h->stream;
+  DevBuf<i64> d_map, d_cur;
+  d_map.upload(amap, st);
+  std::vector<i64> cur(nc + 1, 0);
+  d_cur.alloc(nc + 1);
+  DevSym d = h->ds;
+  h->d_fvec.upload(h->fvec, st);
+  d.fvec = h->d_fvec.p;
+  hipLaunchKernelGGL(spk::fill_kernel<int64_t>, dim3(grid_for(nc + 1)), dim3(kWG), 0, st, d_cur.p,
+                     (int64_t)(nc + 1), (int64_t)0);
+  auto pass = [&](spk::AEnt* out) {
+    if (h->nnz > 0)
+      hipLaunchKernelGGL(spk::front_entries_kernel, dim3(grid_for(h->nnz)), dim3(kWG), 0, st, d,
+                         d_map.p, h->nnz, d_cur.p, out);
+    hipck(hipGetLastError());
+  };
+  pass(nullptr);
+  hipck(hipMemcpyAsync(cur.data(), d_cur.p, (nc + 1) * sizeof(i64), hipMemcpyDeviceToHost, st));
+  hipck(hipStreamSynchronize(st));
+  h->aptr.resize(nc + 1);
+  i64 sum = 0;
+  for (i64 i = 0; i <= nc; ++i) {
+    h->aptr[i] = sum;
+    sum += cur[i];
+  }
+  std::vector<i64> afront(h->nfront + 1);
+  for (i32 f = 0; f < h->nfront; ++f) afront[f] = h->aptr[h->fvec[f]];
+  afront[h->nfront] = sum;
+  h->d_afront.upload(afront, st);
+  h->d_aent.alloc(std::max<i64>(sum, 1));
+  d_cur.upload(h->aptr, st);
+  pass(h->d_aent.p);
+  hipck(hipStreamSynchronize(st));
+}
+
 template <typename T>
 struct Bufs;
 template <>
@@ -1138,9 +1205,12 @@ void set_lds_attrs() {
   done = true;
 }
 
-// The factorisation proper on already assembled lnz/unz (reference layout).
+// The factorisation proper: of A's values (from_a), whose entries the front
+// assembly adds, or of already assembled lnz/unz (reference layout, the
+// stateless drop-ins).
 template <typename T>
-void run_factor(spkhip_handle* h) {
+void run_factor(spkhip_handle* h, bool from_a) {
+  const spk::AEnt* aent = from_a ? h->d_aent.p : nullptr;
   hipStream_t st = h->stream;
   DevBuf<T>& lnz = Bufs<T>::lnz(h);
   DevBuf<T>& unz = Bufs<T>::unz(h);
@@ -1172,36 +1242,46 @@ void run_factor(spkhip_handle* h) {
         const int fpw = (int)std::max<size_t>(1, std::min<size_t>(4, 150 * 1024 / per));
         hipLaunchKernelGGL((spk::small_front_kernel<T, 64>), dim3((lp.small_cnt + fpw - 1) / fpw, h->nvs),
                            dim3(kWG), fpw * per, st, h->ds, h->d_small.p + lp.small_off,
-                           lp.small_cnt, fpw, lp.small_maxL, lnz.p, unz.p, h->d_ipvt.p, arena.p,
-                           h->d_fail.p);
+                           lp.small_cnt, fpw, lp.small_maxL, h->d_afront.p, aent, h->d_nzval.p,
+                           h->nnz, lnz.p, unz.p, h->d_ipvt.p, arena.p, h->d_fail.p);
       } else {
         hipLaunchKernelGGL((spk::small_front_kernel<T, kWG>), dim3(lp.small_cnt, h->nvs), dim3(kWG), per,
                            st, h->ds, h->d_small.p + lp.small_off, lp.small_cnt, 1,
-                           lp.small_maxL, lnz.p, unz.p, h->d_ipvt.p, arena.p, h->d_fail.p);
+                           lp.small_maxL, h->d_afront.p, aent, h->d_nzval.p, h->nnz, lnz.p, unz.p,
+                           h->d_ipvt.p, arena.p, h->d_fail.p);
       }
       hipck(hipGetLastError());
     }
     if (lp.items_cnt > 0) {
       {
       Prof pr(h, SPKHIP_K_INIT, 0.0, lp.init_elems * sizeof(T));
-      if (lp.ut_cnt > 0)
-        hipLaunchKernelGGL((spk::large_utile_kernel<T, false>), dim3(lp.ut_cnt, h->nvs), dim3(kWG), 0, st,
-                           h->ds, h->d_ut_front.p + lp.ut_off, h->d_ut_piece.p + lp.ut_off,
-                           h->d_ut_r0.p + lp.ut_off, lnz.p, unz.p, arena.p);
       // the column is assembled in LDS when the longest one fits in 64 KB;
-      // LU levels whose columns fit 16 KB take one wave per column
+      // levels whose columns fit 16 KB take one wave per column
       const size_t clds = (size_t)lp.large_maxL * sizeof(T);
       const bool staged = clds <= 64 * 1024;
-      if (lu && clds <= 16 * 1024)
-        hipLaunchKernelGGL(spk::large_init_wave_kernel<T>, dim3((lp.items_cnt + 3) / 4, h->nvs),
-                           dim3(kWG), 4 * clds, st, h->ds, h->d_it_init.p + lp.items_off,
-                           h->d_it_ea.p + lp.items_off, h->d_ea_init.p, lnz.p, arena.p,
-                           lp.items_cnt, lp.large_maxL);
-      else
+      if (aent) {
+        const bool wave = clds <= 16 * 1024;
+        auto go = [&](auto kern, int cols, size_t lds) {
+          hipLaunchKernelGGL(kern, dim3((lp.items_cnt + cols - 1) / cols, h->nvs), dim3(kWG), lds,
+                             st, h->ds, h->d_it_asm.p + lp.items_off,
+                             h->d_it_ea.p + lp.items_off, h->d_ea_init.p, aent, h->d_nzval.p,
+                             h->nnz, arena.p, lp.items_cnt, lp.large_maxL, (int)staged);
+        };
+        if (wave)
+          go(spk::large_assemble_kernel<T, 64>, 4, 4 * clds);
+        else
+          go(spk::large_assemble_kernel<T, kWG>, 1, staged ? clds : 0);
+      } else {
+        if (lp.ut_cnt > 0)
+          hipLaunchKernelGGL((spk::large_utile_kernel<T, false>), dim3(lp.ut_cnt, h->nvs), dim3(kWG),
+                             0, st, h->ds, h->d_ut_front.p + lp.ut_off,
+                             h->d_ut_piece.p + lp.ut_off, h->d_ut_r0.p + lp.ut_off, lnz.p, unz.p,
+                             arena.p);
         hipLaunchKernelGGL(spk::large_init_kernel<T>, dim3(lp.items_cnt, h->nvs), dim3(kWG),
                            staged ? clds : 0, st, h->ds, h->d_it_init.p + lp.items_off,
                            h->d_it_ea.p + lp.items_off, h->d_ea_init.p, lnz.p, arena.p,
                            (int)staged);
+      }
       hipck(hipGetLastError());
       }
       bool pending = false;  // second-stream work not yet joined
@@ -1298,28 +1378,6 @@ void read_first_fail(spkhip_handle* h) {
   hipck(hipMemcpyAsync(&ff, h->d_fail.p, sizeof(ff), hipMemcpyDeviceToHost, h->stream));
   sync(h);
   h->first_fail = (ff == ~0ull) ? 0 : (i64)ff;
-}
-
-// Scatter A's values (resident, double) into zeroed lnz/unz of type T.
-template <typename T>
-void run_assemble(spkhip_handle* h) {
-  hipStream_t st = h->stream;
-  DevBuf<T>& lnz = Bufs<T>::lnz(h);
-  DevBuf<T>& unz = Bufs<T>::unz(h);
-  const size_t nl = per_sets(h, h->ds.vs_lnz), nu = per_sets(h, h->ds.vs_unz);
-  lnz.ensure(nl);
-  unz.ensure(nu);
-  Prof pr(h, SPKHIP_K_ASSEMBLE, 0.0,
-          (double)(h->nlnz + h->nunz) * sizeof(T) + (double)h->nnz * (16.0 + sizeof(T)));
-  hipLaunchKernelGGL(spk::fill_kernel<T>, dim3(grid_for((i64)nl)), dim3(kWG), 0, st, lnz.p,
-                     (int64_t)nl, T(0));
-  hipLaunchKernelGGL(spk::fill_kernel<T>, dim3(grid_for((i64)nu)), dim3(kWG), 0, st, unz.p,
-                     (int64_t)nu, T(0));
-  if (h->nnz > 0)
-    hipLaunchKernelGGL(spk::scatter_a_kernel<T>, dim3(grid_for(h->nnz), h->nvs), dim3(kWG), 0,
-                       st, h->d_nzval.p, h->d_amap.p, h->nnz, lnz.p, unz.p, h->ds.vs_lnz,
-                       h->ds.vs_unz);
-  hipck(hipGetLastError());
 }
 
 // Right-hand sides that share one staging of a small front's panels.
@@ -1604,14 +1662,6 @@ void solve_device_in(spkhip_handle* h, double* d_b, i64 ldb, int nrhs, T* rhs, T
   hipck(hipGetLastError());
 }
 
-// Every launch of one factorisation: assembly of A's values into lnz/unz,
-// then the levels (both streams).
-template <typename T>
-void factor_launches(spkhip_handle* h) {
-  run_assemble<T>(h);
-  run_factor<T>(h);
-}
-
 // The factorisation's launches replayed from a captured HIP graph while
 // nothing they name has changed (precision, update mode, plan generation,
 // buffers); a key is captured on its second use, so that a handle factored
@@ -1634,15 +1684,15 @@ void factor_run(spkhip_handle* h) {
   const std::vector<const void*> key = {
       (const void*)(intptr_t)sizeof(T), (const void*)(intptr_t)h->lowp,
       (const void*)(intptr_t)h->sym_gen, Bufs<T>::lnz(h).p, Bufs<T>::unz(h).p,
-      Bufs<T>::arena(h).p, h->d_ipvt.p, h->d_rperm.p, h->d_fail.p, h->d_nzval.p, h->d_amap.p,
+      Bufs<T>::arena(h).p, h->d_ipvt.p, h->d_rperm.p, h->d_fail.p, h->d_nzval.p, h->d_aent.p,
       (const void*)(intptr_t)h->nvs};
   if (!use_graph) {
-    factor_launches<T>(h);
+    run_factor<T>(h, true);
   } else if (h->fg_exec && h->fg_key == key) {
     hipck(hipGraphLaunch(h->fg_exec, h->stream));
   } else if (h->fg_seen != key) {
     h->fg_seen = key;
-    factor_launches<T>(h);
+    run_factor<T>(h, true);
   } else {
     if (h->fg_exec) {
       hipck(hipGraphExecDestroy(h->fg_exec));
@@ -1651,7 +1701,7 @@ void factor_run(spkhip_handle* h) {
     hipGraph_t g = nullptr;
     hipck(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     try {
-      factor_launches<T>(h);
+      run_factor<T>(h, true);
     } catch (...) {
       (void)hipStreamEndCapture(h->stream, &g);
       if (g) (void)hipGraphDestroy(g);
@@ -1705,24 +1755,35 @@ void replan(spkhip_handle* h) {
     // the assembly's items with their front's fields, and each child entry's
     // update column and map, resolved here so that the kernels start with
     // one dependent read
-    std::vector<spk::InitItem> ini(it_front.size());
-    for (size_t i = 0; i < it_front.size(); ++i) {
-      const i32 f = it_front[i], j = it_col[i];
-      spk::InitItem& m = ini[i];
-      m.L = h->fL[f];
-      m.W = h->fW[f];
-      m.j = j;
-      m.fc0 = h->fc0[f];
-      m.fcol = h->foff[f] + (i64)j * m.L;
-      if (j < m.W) {
-        const i64 g = h->fc0[f] + j;
-        const i64 cq = h->xsuper[h->snode[g] - 1] - 1 - h->fc0[f];
-        m.r1 = (i32)cq;
-        m.lcb = h->xlnz[g] - 1 - cq;
-      } else {
-        m.r1 = m.W;
-        m.lcb = -1;
+    if (!h->aptr.empty()) {
+      std::vector<spk::AsmItem> ini(it_front.size());
+      for (size_t i = 0; i < it_front.size(); ++i) {
+        const i32 f = it_front[i], j = it_col[i], L = h->fL[f];
+        const i64* ap = h->aptr.data() + h->fvec[f] + j;
+        ini[i] = spk::AsmItem{h->foff[f] + (i64)j * L, ap[0], L, (i32)(ap[1] - ap[0])};
       }
+      h->d_it_asm.upload(ini, st);
+    } else {
+      std::vector<spk::InitItem> ini(it_front.size());
+      for (size_t i = 0; i < it_front.size(); ++i) {
+        const i32 f = it_front[i], j = it_col[i];
+        spk::InitItem& m = ini[i];
+        m.L = h->fL[f];
+        m.W = h->fW[f];
+        m.j = j;
+        m.fc0 = h->fc0[f];
+        m.fcol = h->foff[f] + (i64)j * m.L;
+        if (j < m.W) {
+          const i64 g = h->fc0[f] + j;
+          const i64 cq = h->xsuper[h->snode[g] - 1] - 1 - h->fc0[f];
+          m.r1 = (i32)cq;
+          m.lcb = h->xlnz[g] - 1 - cq;
+        } else {
+          m.r1 = m.W;
+          m.lcb = -1;
+        }
+      }
+      h->d_it_init.upload(ini, st);
     }
     std::vector<spk::EaItem> eai(ea_child.size());
     for (size_t e = 0; e < ea_child.size(); ++e) {
@@ -1730,7 +1791,6 @@ void replan(spkhip_handle* h) {
       eai[e] = spk::EaItem{h->fcb[c] + (i64)ea_t[e] * h->fcbld[c], h->frel[c],
                            h->fL[c] - h->fW[c], 0};
     }
-    h->d_it_init.upload(ini, st);
     h->d_ea_init.upload(eai, st);
   }
   if (bdesc.empty()) bdesc.push_back(BlkDesc{});
@@ -1772,9 +1832,11 @@ void replan(spkhip_handle* h) {
 
 void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i64* xsuper,
                      const i64* snode, const i64* xlindx, const i64* lindx, const i64* xlnz,
-                     const i64* xunz, const i64* perm, const i64* invp) {
+                     const i64* xunz, const i64* perm, const i64* invp,
+                     const i64* colptr = nullptr, const i64* rowval = nullptr) {
   auto t0 = Clock::now();
   hipck(hipSetDevice(h->device));
+  h->aptr.clear();
   h->kind = kind;
   h->n = n;
   h->nsuper = nsuper;
@@ -1893,6 +1955,14 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
   d.pivot = (kind == SPKHIP_KIND_LU) ? 1 : 0;
   d.sym = (kind == SPKHIP_KIND_SPD) ? 1 : 0;
   h->nvs = 1;  // a new pattern starts with one value set
+  if (colptr && rowval) {
+    h->nnz = colptr[n] - 1;
+    build_storage(h);
+    std::vector<i64> amap;
+    build_amap(h, colptr, rowval, amap);
+    drop_repeated(n, colptr, rowval, amap);
+    build_entries(h, amap);
+  }
   replan(h);
   h->have_sym = true;
   h->have_csc = false;
@@ -1997,7 +2067,7 @@ int64_t lufactor_stateless(i64 n, i64 nsuper, const i64* xsuper, const i64* snod
     if (kind == SPKHIP_KIND_LU && h->nunz > 0)
       hipck(hipMemcpyAsync(du.p, unz, h->nunz * sizeof(T), hipMemcpyHostToDevice, st));
     const int prec = std::is_same<T, double>::value ? SPKHIP_FP64 : SPKHIP_FP32;
-    run_factor<T>(h);
+    run_factor<T>(h, false);
     read_first_fail(h);
     h->precision = prec;
     h->factored = true;
@@ -2113,14 +2183,11 @@ int64_t spkhip_symbolic_upload(spkhip_t h, int64_t kind, int64_t n, int64_t nsup
     return -4;
   if (kind != SPKHIP_KIND_LU && kind != SPKHIP_KIND_SPD) return -4;
   return wrap([&]() -> int64_t {
-    upload_symbolic(h, kind, n, nsuper, xsuper, snode, xlindx, lindx, xlnz, xunz, perm, invp);
+    upload_symbolic(h, kind, n, nsuper, xsuper, snode, xlindx, lindx, xlnz, xunz, perm, invp,
+                    colptr, rowval);
     if (colptr && rowval) {
       auto t0 = Clock::now();
-      h->nnz = colptr[n] - 1;
-      std::vector<i64> amap;
-      build_amap(h, colptr, rowval, amap);
       hipStream_t st = h->stream;
-      h->d_amap.upload(amap, st);
       // CSR of A (original numbering) for the residual: rowptr, colind and
       // the CSC -> CSR value permutation
       std::vector<i64> rowptr(n + 1, 0), c2r(h->nnz);

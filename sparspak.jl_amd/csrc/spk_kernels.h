@@ -114,6 +114,19 @@ struct InitItem {
                  // column); W for an update column
   int32_t j;
 };
+// ... and of the assembly from A's entries:
+struct AsmItem {
+  int64_t fcol;  // arena offset of the front's column
+  int64_t a0;    // A's entries of the column: a0 .. a0 + an of the AEnt list
+  int32_t L, an;
+};
+// One entry of A inside its front: value k of the CSC array goes to row r,
+// column c of the front's matrix (SPD: once more to row c, column r).
+// Entries are grouped by front and column; a column's rows are distinct.
+struct AEnt {
+  int64_t k;
+  int32_t r, c;
+};
 // ... and one per (child, update column) pair added into a column.
 struct EaItem {
   int64_t col;  // arena offset of the child's update-matrix column

@@ -59,12 +59,6 @@ __device__ inline int64_t slot_of(const DevSym& s, int64_t fc0, int64_t W,
   return s.xunz[gr] - 1 + (j - cr - rw);
 }
 
-// ---------------------------------------------------------------------------
-// Assembly: zero lnz/unz, scatter A's values through the precomputed map.
-// amap[k] >= 0: lnz slot; amap[k] <= -2: unz slot (-amap-2); -1: dropped
-// (the reference's search runs off the end of the index list and ignores the
-// entry, SpkSparseBase.jl:328-341).
-// ---------------------------------------------------------------------------
 template <typename T>
 __global__ void fill_kernel(T* __restrict__ a, int64_t len, T v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -72,27 +66,44 @@ __global__ void fill_kernel(T* __restrict__ a, int64_t len, T v) {
   for (; i < len; i += stride) a[i] = v;
 }
 
-// A's values added into their slots of the zeroed lnz / unz (amap[k] >= 0:
-// lnz slot, <= -2: unz slot -(amap[k] + 2), -1: not stored; distinct entries
-// of a CSC pattern map to distinct slots). Value set blockIdx.y: its nnz
-// values, its lnz / unz at vs_l / vs_u apart.
-template <typename T>
-__global__ void scatter_a_kernel(const double* __restrict__ nzval,
-                                 const int64_t* __restrict__ amap,
-                                 int64_t nnz, T* __restrict__ lnz,
-                                 T* __restrict__ unz, int64_t vs_l, int64_t vs_u) {
-  const int64_t vs = blockIdx.y;
-  nzval += vs * nnz;
-  lnz += vs * vs_l;
-  unz += vs * vs_u;
+// Every entry of A (its slot map: lnz slot, -2 - unz slot, or -1) in its
+// front: the slot's column (lnz) or row (unz) is an own column of the front.
+// Without `out` counts the entries of every front column (cnt, index fvec[f]
+// + c); with it takes cnt as the columns' next free positions. SPD entries
+// below the diagonal appear at both positions. Once per pattern; the slots'
+// columns are found by bisection.
+__global__ void front_entries_kernel(DevSym s, const int64_t* __restrict__ amap, int64_t nnz,
+                                     int64_t* __restrict__ cnt, AEnt* __restrict__ out) {
   int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nnz) return;
-  int64_t d = amap[k];
-  T v = (T)nzval[k];
-  if (d >= 0)
-    lnz[d] += v;
-  else if (d <= -2)
-    unz[-d - 2] += v;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  // last i in [0, m) with v[i] <= x
+  auto last_le = [](const auto* v, int64_t m, int64_t x) {
+    int64_t lo = 0, hi = m - 1;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi + 1) >> 1;
+      if (v[mid] <= x)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    return lo;
+  };
+  for (; k < nnz; k += stride) {
+    const int64_t a = amap[k];
+    if (a == -1) continue;
+    const int64_t slot = a >= 0 ? a : -a - 2;
+    const int64_t g = last_le(a >= 0 ? s.xlnz : s.xunz, s.n, slot + 1);
+    const int f = (int)last_le(s.fc0, s.nfront, g);
+    const int own = (int)(g - s.fc0[f]);
+    const int other = (int)(slot - (a >= 0 ? s.lcol[g] : s.ucol[g]));
+    auto put = [&](int r, int c) {
+      const unsigned long long at = atomicAdd(
+          reinterpret_cast<unsigned long long*>(cnt + s.fvec[f] + c), 1ull);
+      if (out) out[at] = AEnt{k, r, c};
+    };
+    put(a >= 0 ? other : own, a >= 0 ? own : other);
+    if (s.sym && other != own) put(own, other);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -164,17 +175,21 @@ __device__ void lds_partial_lu(T* F, int L, int cq, int nq, int pivot,
 }
 
 // One small front per group of G threads (G = 256: a workgroup; G = 64: a
-// wave, fpw fronts per workgroup, for levels of many tiny fronts): gather
-// the pieces' panels and the children's update matrices into LDS (L x L per
-// front), factor, write the panels back to lnz/unz/ipvt and the update
-// matrix to the arena.
+// wave, fpw fronts per workgroup, for levels of many tiny fronts): A's
+// entries (aent, front f's from aptr[f]; without them the pieces' panels of
+// assembled lnz/unz) and the children's update matrices gathered into LDS
+// (L x L per front), factored, the panels written to lnz/unz/ipvt and the
+// update matrix to the arena.
 template <typename T, int G>
 __global__ void __launch_bounds__(kWG)
 small_front_kernel(DevSym s, const int32_t* __restrict__ list, int cnt, int fpw, int maxL,
+                   const int64_t* __restrict__ aptr, const AEnt* __restrict__ aent,
+                   const double* __restrict__ nzval, int64_t nnz,
                    T* __restrict__ lnz, T* __restrict__ unz,
                    int64_t* __restrict__ ipvt, T* __restrict__ arena,
                    unsigned long long* __restrict__ first_fail) {
   const int64_t vs = blockIdx.y;  // value set
+  nzval += vs * nnz;
   lnz += vs * s.vs_lnz;
   unz += vs * s.vs_unz;
   ipvt += vs * s.n;
@@ -203,8 +218,14 @@ small_front_kernel(DevSym s, const int32_t* __restrict__ list, int cnt, int fpw,
   const int sp0 = s.fsp0[f], np = s.fnp[f];
   for (int i = tid; i < L * L; i += G) F[i] = T(0);
   gsync();
+  if (aent) {
+    for (int64_t e = aptr[f] + tid; e < aptr[f + 1]; e += G) {
+      const AEnt en = aent[e];
+      F[en.r + en.c * L] = (T)nzval[en.k];
+    }
+  }
   // pieces' panels
-  for (int p = sp0; p < sp0 + np; ++p) {
+  for (int p = sp0; !aent && p < sp0 + np; ++p) {
     int64_t pc0, nq;
     piece_cols(s, p, pc0, nq);
     const int cq = (int)(pc0 - fc0);
@@ -224,7 +245,7 @@ small_front_kernel(DevSym s, const int32_t* __restrict__ list, int cnt, int fpw,
     }
   }
   gsync();
-  if (s.sym) {  // upper rows of the own columns from the lower triangle
+  if (s.sym && !aent) {  // upper rows of the own columns from the lower triangle
     for (int idx = tid; idx < W * L; idx += G) {
       int r = idx % W, j = idx / W;
       if (j > r) F[r + j * L] = F[j + r * L];
@@ -346,7 +367,8 @@ large_utile_kernel(DevSym s, const int32_t* __restrict__ it_front,
   }
 }
 
-// One workgroup per (front, column j): the column's L part from lnz (rows
+// Assembly from lnz/unz (the stateless drop-ins, whose arguments hold
+// _inmatrix!'s output). One workgroup per (front, column j): the column's L part from lnz (rows
 // from its piece's first row), zeros in the update block, then the
 // children's update-matrix columns that map to j, one child after the other
 // (rows of different children may coincide). Runs after large_utile_kernel
@@ -467,72 +489,100 @@ large_init_kernel(DevSym s, const InitItem* __restrict__ items,
   }
 }
 
-// One wave per front column, four per workgroup: the staged (LDS) assembly
-// of large_init_kernel for LU levels whose longest column fits a quarter of
-// the LDS budget, so that the many short columns of the lower levels take a
-// quarter of the workgroups. A child's update rows are distinct, and one
-// wave's LDS operations complete in issue order, so the children are added
-// one after another without barriers, in the same order as there.
-template <typename T>
+// Assembly of a large front's column j from A's values: zero, A's entries
+// of the column (distinct rows), then the children's update-matrix columns
+// that map to j, one child after the other in a fixed order (rows of
+// different children may coincide), summed in LDS and written once. G
+// threads per column: a workgroup, or a wave (four columns per workgroup, no
+// barriers: one wave's LDS operations complete in issue order) where the
+// level's longest column fits 16 KB; columns longer than the LDS are summed
+// in place (staged 0). The next batch of a child's rows (8 per thread, the
+// next child's when this one ends) is requested before the current one is
+// added. HBM-bound: L^2 entries written and the children's read. Reading
+// the panels of a zeroed and scattered lnz/unz instead, transposing their U
+// part into the front first, cost in the same pass at 64^3 (double) 0.43 ms
+// of zeroing, 1.7 ms of transposition and the panels read once more: the
+// factor and solve pass 81.0 -> 79.5 ms, elasticity 40^3 (float, SPD, whose
+// columns were summed in place in HBM) 91.3 -> 80.7 ms, 32^3 double
+// 9.57 -> 9.28 ms, 100^2 double 2.56 -> 2.46 ms.
+template <typename T, int G>
 __global__ void __launch_bounds__(kWG)
-large_init_wave_kernel(DevSym s, const InitItem* __restrict__ items,
-                       const int64_t* __restrict__ it_ea, const EaItem* __restrict__ ea,
-                       const T* __restrict__ lnz, T* __restrict__ arena, int nitems, int maxL) {
+large_assemble_kernel(DevSym s, const AsmItem* __restrict__ items,
+                      const int64_t* __restrict__ it_ea, const EaItem* __restrict__ ea,
+                      const AEnt* __restrict__ aent, const double* __restrict__ nzval,
+                      int64_t nnz, T* __restrict__ arena, int nitems, int maxL, int staged) {
   const int64_t vs = blockIdx.y;  // value set
-  lnz += vs * s.vs_lnz;
+  nzval += vs * nnz;
   arena += vs * s.vs_arena;
   extern __shared__ unsigned char smem_raw[];
-  const int lane = threadIdx.x % 64, wave = wave_id();
-  const int item = blockIdx.x * 4 + wave;
-  if (item >= nitems) return;  // no workgroup barrier below
-  T* Fs = reinterpret_cast<T*>(smem_raw) + (size_t)wave * maxL;
-  const InitItem m = items[item];
+  constexpr int U = 8;
+  const int grp = (G == kWG) ? 0 : wave_id();
+  const int gt = (G == kWG) ? (int)threadIdx.x : (int)threadIdx.x % 64;
+  const int item = blockIdx.x * (kWG / G) + grp;
+  if (item >= nitems) return;  // a whole wave (no workgroup barrier below) or workgroup
+  auto gsync = [] {
+    if constexpr (G == kWG)
+      __syncthreads();
+    else
+      wave_lds_sync();
+  };
+  const AsmItem m = items[item];
   const int L = m.L;
   T* F = arena + m.fcol;
-  const int64_t e0 = it_ea[item], e1 = it_ea[item + 1];
-  EaItem en = ea[e0 < e1 ? e0 : 0];
-  const int r1 = m.r1;
-  const T* lc = (m.lcb >= 0) ? lnz + m.lcb : nullptr;
-  for (int r0 = lane; r0 < L; r0 += 8 * 64) {
-    T v[8];
+  T* Fs = staged ? reinterpret_cast<T*>(smem_raw) + (size_t)grp * maxL : F;
+  int64_t e = it_ea[item];
+  const int64_t e1 = it_ea[item + 1];
+  // the batch in flight: rows t0 + gt + u G of child `cur`
+  EaItem cur = ea[e < e1 ? e : 0];
+  int t0 = 0;
+  int ri[U];
+  T cv[U];
+  auto request = [&]() {
+    const int32_t* rel = s.relmap + cur.rel;
+    const T* col = arena + cur.col;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int r = r0 + u * 64;
-      v[u] = (r >= L) ? T(0) : (r < r1) ? F[r] : (lc ? lc[r] : T(0));
+    for (int u = 0; u < U; ++u) {
+      const int t = t0 + gt + u * G;
+      ri[u] = (t < cur.Rc) ? rel[t] : -1;
+      cv[u] = (t < cur.Rc) ? col[t] : T(0);
     }
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (r0 + u * 64 < L) Fs[r0 + u * 64] = v[u];
+  };
+  if (e < e1) request();
+  for (int r = gt; r < L; r += G) Fs[r] = T(0);
+  gsync();
+  for (int i = gt; i < m.an; i += G) {
+    const AEnt en = aent[m.a0 + i];
+    Fs[en.r] = (T)nzval[en.k];
   }
-  wave_lds_sync();
-  for (int64_t e = e0; e < e1; ++e) {
-    const EaItem ec = en;
-    if (e + 1 < e1) en = ea[e + 1];
-    const int Rc = ec.Rc;
-    const int32_t* rel = s.relmap + ec.rel;
-    const T* col = arena + ec.col;
-    for (int tp0 = lane; tp0 < Rc; tp0 += 8 * 64) {
-      int ri[8];
-      T cv[8];
+  gsync();
+  while (e < e1) {
+    int rj[U];
+    T cw[U];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int tp = tp0 + u * 64;
-        ri[u] = (tp < Rc) ? rel[tp] : 0;
-        cv[u] = (tp < Rc) ? col[tp] : T(0);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (tp0 + u * 64 < Rc) Fs[ri[u]] += cv[u];
+    for (int u = 0; u < U; ++u) {
+      rj[u] = ri[u];
+      cw[u] = cv[u];
     }
-    wave_lds_sync();
+    t0 += U * G;
+    const bool last = t0 >= cur.Rc;
+    if (last) {
+      t0 = 0;
+      if (++e < e1) cur = ea[e];
+    }
+    if (e < e1) request();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (rj[u] >= 0) Fs[rj[u]] += cw[u];
+    if (last) gsync();
   }
-  for (int r0 = lane; r0 < L; r0 += 8 * 64) {
-    T v[8];
+  if (!staged) return;
+  for (int r0 = gt; r0 < L; r0 += U * G) {
+    T v[U];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = (r0 + u * 64 < L) ? Fs[r0 + u * 64] : T(0);
+    for (int u = 0; u < U; ++u) v[u] = (r0 + u * G < L) ? Fs[r0 + u * G] : T(0);
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (r0 + u * 64 < L) F[r0 + u * 64] = v[u];
+    for (int u = 0; u < U; ++u)
+      if (r0 + u * G < L) F[r0 + u * G] = v[u];
   }
 }
 
