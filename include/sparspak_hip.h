@@ -362,7 +362,8 @@ int64_t spkhip_profile_get(spkhip_t h, int64_t kclass, spkhip_kstat_t* out);
  *   upd_group       blocks per wide trailing update, i.e. its depth in
  *                   blocks (1..64, default 8)
  *   small_wave_min  small fronts in a level from which one wave (instead of
- *                   one workgroup) takes a front (>= 1, default 16384)
+ *                   one workgroup) takes a front of more than 32 rows
+ *                   (>= 1, default 16384)
  *   factor_ms       autotune: the best measured factor time; ignored by set
  * Every setting in range gives a correct factor. set rebuilds the launch
  * plan when a knob changes (the factor must then be recomputed: -3 from the

@@ -88,6 +88,7 @@ struct DevBuf {
 
 struct LevelPlan {
   int small_off = 0, small_cnt = 0, small_maxL = 0;
+  int small_big = 0;                // the first ones have more than 32 rows
   int small_maxq = 1;               // widest piece of the level's small fronts
   int items_off = 0, items_cnt = 0;
   int wb_off = 0, wb_cnt = 0;       // write-back items: the large fronts' pivot columns
@@ -188,6 +189,8 @@ struct spkhip_handle {
   DevBuf<i32> d_lindx, d_fL, d_fW, d_fc0, d_fsp0, d_fnp, d_fcbld, d_fchp, d_fch,
       d_relmap, d_small, d_it_front, d_it_col, d_ea_child, d_ea_t, d_solve;
   DevBuf<i64> d_foff, d_fcb, d_frel, d_fvec, d_it_ea, d_lcol, d_ucol;
+  DevBuf<spk::SmallDesc> d_sdfr;    // the small fronts, resolved
+  DevBuf<spk::SmallChild> d_sdch;   // their children
   DevBuf<spk::InitItem> d_it_init;  // the assembly's items, resolved: from panels,
   DevBuf<spk::AsmItem> d_it_asm;    // or from A's entries
   DevBuf<spk::EaItem> d_ea_init;
@@ -216,11 +219,10 @@ struct spkhip_handle {
   // matrix
   i64 nnz = 0;
   bool have_csc = false, pattern_error = false;
-  // A's entries by front and column (host pointers per front column, fvec[f]
-  // + j; on the device per front), built with the pattern
+  // A's entries by front and column (pointers per front column, fvec[f] + j),
+  // built with the pattern
   std::vector<i64> aptr;
   DevBuf<spk::AEnt> d_aent;
-  DevBuf<i64> d_afront;
   DevBuf<i64> d_rowptr;
   DevBuf<i32> d_colind;
   DevBuf<i64> d_csc2csr;
@@ -578,6 +580,9 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
       }
     }
     lp.small_cnt = (int)small.size() - lp.small_off;
+    const auto mid = std::stable_partition(small.begin() + lp.small_off, small.end(),
+                                           [&](i32 f) { return h->fL[f] > 32; });
+    lp.small_big = (int)(mid - small.begin()) - lp.small_off;
     lp.solve_cnt = (int)solve.size() - lp.solve_off;
     lp.large_off = (int)largel.size();
     for (i32 f : bylev[l]) {
@@ -1107,31 +1112,33 @@ void drop_repeated(i64 n, const i64* colptr, const i64* rowval, std::vector<i64>
 }
 
 // A's entries with their place in their front (AEnt), grouped by front and
-// column on the device: pointers per front column (h->aptr, index fvec[f] +
-// j) and per front (device). The rows of a column are distinct, so its
-// entries' order, which is not determined, does not matter. The front
+// column on the device, with pointers per front column (h->aptr, index
+// fvec[f] + j). The rows of a column are distinct, so its entries' order,
+// which is not determined, does not matter. The front
 // fields of h->ds that the kernels use are those of upload_symbolic and
 // build_storage.
 void build_entries(spkhip_handle* h, const std::vector<i64>& amap) {
   const i64 nc = h->vec_elems;
   hipStream_t st = h->stream;
-  DevBuf<i64> d_map, d_cur;
-  d_map.upload(amap, st);
+  DevBuf<i64> d_tmp;  // the counts, then the slot map
+  d_tmp.alloc(nc + 1 + h->nnz);
+  i64 *const d_cur = d_tmp.p, *const d_map = d_tmp.p + nc + 1;
+  if (h->nnz > 0)
+    hipck(hipMemcpyAsync(d_map, amap.data(), h->nnz * sizeof(i64), hipMemcpyHostToDevice, st));
   std::vector<i64> cur(nc + 1, 0);
-  d_cur.alloc(nc + 1);
   DevSym d = h->ds;
   h->d_fvec.upload(h->fvec, st);
   d.fvec = h->d_fvec.p;
-  hipLaunchKernelGGL(spk::fill_kernel<int64_t>, dim3(grid_for(nc + 1)), dim3(kWG), 0, st, d_cur.p,
+  hipLaunchKernelGGL(spk::fill_kernel<int64_t>, dim3(grid_for(nc + 1)), dim3(kWG), 0, st, d_cur,
                      (int64_t)(nc + 1), (int64_t)0);
   auto pass = [&](spk::AEnt* out) {
     if (h->nnz > 0)
       hipLaunchKernelGGL(spk::front_entries_kernel, dim3(grid_for(h->nnz)), dim3(kWG), 0, st, d,
-                         d_map.p, h->nnz, d_cur.p, out);
+                         d_map, h->nnz, d_cur, out);
     hipck(hipGetLastError());
   };
   pass(nullptr);
-  hipck(hipMemcpyAsync(cur.data(), d_cur.p, (nc + 1) * sizeof(i64), hipMemcpyDeviceToHost, st));
+  hipck(hipMemcpyAsync(cur.data(), d_cur, (nc + 1) * sizeof(i64), hipMemcpyDeviceToHost, st));
   hipck(hipStreamSynchronize(st));
   h->aptr.resize(nc + 1);
   i64 sum = 0;
@@ -1139,12 +1146,8 @@ void build_entries(spkhip_handle* h, const std::vector<i64>& amap) {
     h->aptr[i] = sum;
     sum += cur[i];
   }
-  std::vector<i64> afront(h->nfront + 1);
-  for (i32 f = 0; f < h->nfront; ++f) afront[f] = h->aptr[h->fvec[f]];
-  afront[h->nfront] = sum;
-  h->d_afront.upload(afront, st);
   h->d_aent.alloc(std::max<i64>(sum, 1));
-  d_cur.upload(h->aptr, st);
+  hipck(hipMemcpyAsync(d_cur, h->aptr.data(), (nc + 1) * sizeof(i64), hipMemcpyHostToDevice, st));
   pass(h->d_aent.p);
   hipck(hipStreamSynchronize(st));
 }
@@ -1174,11 +1177,11 @@ template <typename T>
 void set_lds_attrs() {
   static bool done = false;
   if (done) return;
-  hipck(hipFuncSetAttribute((const void*)spk::small_front_kernel<T, kWG>,
+  hipck(hipFuncSetAttribute((const void*)spk::small_front_kernel<T, false>,
                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kSmallLmax * kSmallLmax * (int)sizeof(T)));
-  hipck(hipFuncSetAttribute((const void*)spk::small_front_kernel<T, 64>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+                            4 * 32 * 33 * (int)sizeof(T)));
+  hipck(hipFuncSetAttribute((const void*)spk::small_front_kernel<T, true>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 140 * 1024));
   hipck(hipFuncSetAttribute((const void*)spk::blk_diag_slab_kernel<T>,
                             hipFuncAttributeMaxDynamicSharedMemorySize,
                             spk::slab_elems(64, 1, true) * (int)sizeof(T)));
@@ -1233,22 +1236,23 @@ void run_factor(spkhip_handle* h, bool from_a) {
     h->cur_level = (int)(&lp - h->levels.data());
     h->cur_grid = lp.small_cnt;
     if (lp.small_cnt > 0) {
-      // levels of many small fronts: one wave per front, as many per
-      // workgroup as 150 KB of LDS hold (at most four); otherwise one
-      // workgroup per front
-      const size_t per = (size_t)lp.small_maxL * lp.small_maxL * sizeof(T);
+      // fronts of more than 32 rows take a workgroup, the others one wave
+      // each; levels of very many fronts one wave for every front
       Prof pr(h, SPKHIP_K_SMALL, lp.small_flops, lp.small_elems * sizeof(T));
-      if (lp.small_cnt >= h->small_wave_min) {
-        const int fpw = (int)std::max<size_t>(1, std::min<size_t>(4, 150 * 1024 / per));
-        hipLaunchKernelGGL((spk::small_front_kernel<T, 64>), dim3((lp.small_cnt + fpw - 1) / fpw, h->nvs),
-                           dim3(kWG), fpw * per, st, h->ds, h->d_small.p + lp.small_off,
-                           lp.small_cnt, fpw, lp.small_maxL, h->d_afront.p, aent, h->d_nzval.p,
-                           h->nnz, lnz.p, unz.p, h->d_ipvt.p, arena.p, h->d_fail.p);
+      const int LD = lp.small_maxL | 1, front = lp.small_maxL * LD;
+      auto go = [&](auto kern, int nbig, int wgs, int slot, int elems) {
+        hipLaunchKernelGGL(kern, dim3(wgs, h->nvs), dim3(kWG), elems * sizeof(T), st, h->ds,
+                           h->d_sdfr.p + lp.small_off, h->d_sdch.p, nbig, lp.small_cnt, LD, slot,
+                           aent, h->d_nzval.p, h->nnz, lnz.p, unz.p, h->d_ipvt.p, arena.p,
+                           h->d_fail.p);
+      };
+      if (lp.small_cnt >= h->small_wave_min && lp.small_big > 0) {
+        go(spk::small_front_kernel<T, true>, 0, (lp.small_cnt + 3) / 4, front, 4 * front);
       } else {
-        hipLaunchKernelGGL((spk::small_front_kernel<T, kWG>), dim3(lp.small_cnt, h->nvs), dim3(kWG), per,
-                           st, h->ds, h->d_small.p + lp.small_off, lp.small_cnt, 1,
-                           lp.small_maxL, h->d_afront.p, aent, h->d_nzval.p, h->nnz, lnz.p, unz.p,
-                           h->d_ipvt.p, arena.p, h->d_fail.p);
+        const int slot = std::min(front, 32 * 33);
+        go(spk::small_front_kernel<T, false>, lp.small_big,
+           lp.small_big + (lp.small_cnt - lp.small_big + 3) / 4, slot,
+           std::max(lp.small_big ? front : 0, 4 * slot));
       }
       hipck(hipGetLastError());
     }
@@ -1736,6 +1740,33 @@ void replan(spkhip_handle* h) {
              ut_front, ut_piece, ut_r0);
   if (largel.empty()) largel.push_back(0);
   if (sdesc.empty()) sdesc.push_back(spk::SolveDesc{});
+  {
+    // the small fronts with their fields and children resolved
+    std::vector<spk::SmallDesc> fr;
+    std::vector<spk::SmallChild> chl;
+    for (i32 f : small) {
+      spk::SmallDesc d{};
+      d.cb = h->fcb[f];
+      d.L = h->fL[f];
+      d.W = h->fW[f];
+      d.fc0 = (i32)h->fc0[f];
+      d.ch0 = (i32)chl.size();
+      d.nch = h->fchp[f + 1] - h->fchp[f];
+      if (!h->aptr.empty()) {
+        d.a0 = h->aptr[h->fvec[f]];
+        d.an = (i32)(h->aptr[h->fvec[f] + d.L] - d.a0);
+      }
+      for (i32 ci = h->fchp[f]; ci < h->fchp[f + 1]; ++ci) {
+        const i32 c = h->fch[ci];
+        chl.push_back(spk::SmallChild{h->fcb[c], h->frel[c], h->fL[c] - h->fW[c], h->fcbld[c]});
+      }
+      fr.push_back(d);
+    }
+    if (fr.empty()) fr.push_back(spk::SmallDesc{});
+    if (chl.empty()) chl.push_back(spk::SmallChild{});
+    h->d_sdfr.upload(fr, st);
+    h->d_sdch.upload(chl, st);
+  }
   if (small.empty()) small.push_back(0);
   h->d_small.upload(small, st);
   if (it_front.empty()) {

@@ -120,6 +120,20 @@ struct AsmItem {
   int64_t a0;    // A's entries of the column: a0 .. a0 + an of the AEnt list
   int32_t L, an;
 };
+// Small fronts, resolved on the host likewise.
+struct SmallDesc {
+  int64_t a0;  // A's entries of the front
+  int64_t cb;  // arena offset of its update matrix (leading dimension L - W)
+  int32_t an;
+  int32_t L, W;
+  int32_t fc0;       // first column
+  int32_t ch0, nch;  // children: ch0 .. ch0 + nch of the SmallChild list
+};
+struct SmallChild {
+  int64_t cb;   // arena offset of the child's update matrix
+  int64_t rel;  // offset of its relative-index map
+  int32_t R, ld;
+};
 // One entry of A inside its front: value k of the CSC array goes to row r,
 // column c of the front's matrix (SPD: once more to row c, column r).
 // Entries are grouped by front and column; a column's rows are distinct.

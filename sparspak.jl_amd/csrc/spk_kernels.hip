@@ -107,209 +107,6 @@ __global__ void front_entries_kernel(DevSym s, const int64_t* __restrict__ amap,
 }
 
 // ---------------------------------------------------------------------------
-// Partial LU of one front held in LDS (F, leading dimension L): pieces are
-// eliminated column by column with row pivoting confined to each piece's
-// diagonal block, exactly as _getrf! (SpkLUFactor.jl:230) followed by the two
-// TRSMs and the U12 row swap (:235-240): a row interchange spans the piece's
-// own columns and everything to their right, never earlier pieces' columns;
-// multipliers are formed with the reciprocal of the pivot as ggetrf!/gtrsm!
-// do (GenericBlasLapackFragments.jl:80-84, 376-395).
-// ---------------------------------------------------------------------------
-template <typename T, int G>
-__device__ void lds_partial_lu(T* F, int L, int cq, int nq, int pivot,
-                               int* piv_out, int* zero_out, int gt, int* s_kp_, T* s_inv_) {
-  // G threads (a workgroup of 256 or one wave of 64), gt = thread index in
-  // the group; s_kp_ / s_inv_ one LDS slot of the group
-  auto gsync = [] {
-    if constexpr (G == kWG)
-      __syncthreads();
-    else
-      wave_lds_sync();
-  };
-  for (int k = 0; k < nq; ++k) {
-    const int col = cq + k;
-    if (gt == 0) {
-      int kp = col;
-      if (pivot) {
-        T amax = fabs(F[col + col * L]);
-        for (int i = col + 1; i < cq + nq; ++i) {
-          T a = fabs(F[i + col * L]);
-          if (a > amax) {
-            amax = a;
-            kp = i;
-          }
-        }
-      }
-      *s_kp_ = kp;
-      T pv = F[kp + col * L];
-      if (pv == T(0)) *zero_out = 1;
-      *s_inv_ = T(1) / pv;
-      piv_out[k] = kp - cq;
-    }
-    gsync();
-    const int kp = *s_kp_;
-    const bool nonzero = (F[kp + col * L] != T(0));
-    if (kp != col && nonzero) {
-      for (int c = cq + gt; c < L; c += G) {
-        T t = F[col + c * L];
-        F[col + c * L] = F[kp + c * L];
-        F[kp + c * L] = t;
-      }
-    }
-    gsync();
-    const T inv = *s_inv_;
-    // Rows inside the diagonal block are scaled only for a nonzero pivot
-    // (ggetrf!); rows below it always (gtrsm! multiplies by 1/U(j,j)).
-    for (int r = col + 1 + gt; r < L; r += G)
-      if (r >= cq + nq || nonzero) F[r + col * L] *= inv;
-    gsync();
-    const int m = L - col - 1;
-    const int cnt = m * m;
-    for (int idx = gt; idx < cnt; idx += G) {
-      int r = col + 1 + idx % m;
-      int c = col + 1 + idx / m;
-      F[r + c * L] -= F[r + col * L] * F[col + c * L];
-    }
-    gsync();
-  }
-}
-
-// One small front per group of G threads (G = 256: a workgroup; G = 64: a
-// wave, fpw fronts per workgroup, for levels of many tiny fronts): A's
-// entries (aent, front f's from aptr[f]; without them the pieces' panels of
-// assembled lnz/unz) and the children's update matrices gathered into LDS
-// (L x L per front), factored, the panels written to lnz/unz/ipvt and the
-// update matrix to the arena.
-template <typename T, int G>
-__global__ void __launch_bounds__(kWG)
-small_front_kernel(DevSym s, const int32_t* __restrict__ list, int cnt, int fpw, int maxL,
-                   const int64_t* __restrict__ aptr, const AEnt* __restrict__ aent,
-                   const double* __restrict__ nzval, int64_t nnz,
-                   T* __restrict__ lnz, T* __restrict__ unz,
-                   int64_t* __restrict__ ipvt, T* __restrict__ arena,
-                   unsigned long long* __restrict__ first_fail) {
-  const int64_t vs = blockIdx.y;  // value set
-  nzval += vs * nnz;
-  lnz += vs * s.vs_lnz;
-  unz += vs * s.vs_unz;
-  ipvt += vs * s.n;
-  arena += vs * s.vs_arena;
-  extern __shared__ unsigned char smem_raw[];
-  __shared__ int s_piv_all[kWG / G][kSmallLmax];  // a piece of a small front has <= L columns
-  __shared__ int s_zero_all[kWG / G];
-  __shared__ int s_kp_all[kWG / G];
-  __shared__ T s_inv_all[kWG / G];
-  const int grp = (G == kWG) ? 0 : wave_id();
-  const int tid = (G == kWG) ? (int)threadIdx.x : (int)threadIdx.x % 64;
-  const int item = blockIdx.x * fpw + grp;
-  if (grp >= fpw || item >= cnt) return;
-  auto gsync = [] {
-    if constexpr (G == kWG)
-      __syncthreads();
-    else
-      wave_lds_sync();
-  };
-  T* F = reinterpret_cast<T*>(smem_raw) + (int64_t)grp * maxL * maxL;
-  int* s_piv = s_piv_all[grp];
-  int& s_zero = s_zero_all[grp];
-  const int f = list[item];
-  const int L = s.fL[f], W = s.fW[f];
-  const int64_t fc0 = s.fc0[f];
-  const int sp0 = s.fsp0[f], np = s.fnp[f];
-  for (int i = tid; i < L * L; i += G) F[i] = T(0);
-  gsync();
-  if (aent) {
-    for (int64_t e = aptr[f] + tid; e < aptr[f + 1]; e += G) {
-      const AEnt en = aent[e];
-      F[en.r + en.c * L] = (T)nzval[en.k];
-    }
-  }
-  // pieces' panels
-  for (int p = sp0; !aent && p < sp0 + np; ++p) {
-    int64_t pc0, nq;
-    piece_cols(s, p, pc0, nq);
-    const int cq = (int)(pc0 - fc0);
-    const int jl = L - cq;
-    const T* lp = lnz + (s.xlnz[pc0] - 1);
-    for (int idx = tid; idx < jl * nq; idx += G) {
-      int r = idx % jl, c = idx / jl;
-      if (!s.sym || r >= c) F[(cq + r) + (cq + c) * L] = lp[idx];
-    }
-    if (!s.sym) {
-      const int ul = jl - (int)nq;
-      const T* up = unz + (s.xunz[pc0] - 1);
-      for (int idx = tid; idx < ul * nq; idx += G) {
-        int r = idx % ul, c = idx / ul;
-        F[(cq + c) + (cq + (int)nq + r) * L] = up[idx];
-      }
-    }
-  }
-  gsync();
-  if (s.sym && !aent) {  // upper rows of the own columns from the lower triangle
-    for (int idx = tid; idx < W * L; idx += G) {
-      int r = idx % W, j = idx / W;
-      if (j > r) F[r + j * L] = F[j + r * L];
-    }
-    gsync();
-  }
-  // children's update matrices (one child at a time: rows of different
-  // children may coincide)
-  for (int ci = s.fchp[f]; ci < s.fchp[f + 1]; ++ci) {
-    const int c = s.fch[ci];
-    const int Rc = s.fL[c] - s.fW[c];
-    const int32_t* rel = s.relmap + s.frel[c];
-    const T* cb = arena + s.fcb[c];
-    const int ld = s.fcbld[c];
-    for (int idx = tid; idx < Rc * Rc; idx += G) {
-      int tp = idx % Rc, t = idx / Rc;
-      F[rel[tp] + rel[t] * L] += cb[tp + (int64_t)t * ld];
-    }
-    gsync();
-  }
-  // factor piece by piece
-  if (tid == 0) s_zero = 0;
-  gsync();
-  for (int p = sp0; p < sp0 + np; ++p) {
-    int64_t pc0, nq;
-    piece_cols(s, p, pc0, nq);
-    const int cq = (int)(pc0 - fc0);
-    lds_partial_lu<T, G>(F, L, cq, (int)nq, s.pivot, s_piv, &s_zero, tid, &s_kp_all[grp],
-                         &s_inv_all[grp]);
-    for (int k = tid; k < nq; k += G) ipvt[pc0 + k] = s_piv[k] + 1;
-    if (tid == 0 && s_zero) {
-      atomicMin(first_fail, (unsigned long long)(p + 1));
-      s_zero = 0;
-    }
-    gsync();
-  }
-  // write back panels
-  for (int p = sp0; p < sp0 + np; ++p) {
-    int64_t pc0, nq;
-    piece_cols(s, p, pc0, nq);
-    const int cq = (int)(pc0 - fc0);
-    const int jl = L - cq;
-    T* lp = lnz + (s.xlnz[pc0] - 1);
-    for (int idx = tid; idx < jl * nq; idx += G) {
-      int r = idx % jl, c = idx / jl;
-      lp[idx] = F[(cq + r) + (cq + c) * L];
-    }
-    const int ul = jl - (int)nq;
-    T* up = unz + (s.xunz[pc0] - 1);
-    for (int idx = tid; idx < ul * nq; idx += G) {
-      int r = idx % ul, c = idx / ul;
-      up[idx] = F[(cq + c) + (cq + (int)nq + r) * L];
-    }
-  }
-  // update matrix
-  const int R = L - W;
-  T* cb = arena + s.fcb[f];
-  for (int idx = tid; idx < R * R; idx += G) {
-    int tp = idx % R, t = idx / R;
-    cb[idx] = F[(W + tp) + (W + t) * L];
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Large fronts: the L x L work matrix lives in the arena.
 // ---------------------------------------------------------------------------
 
@@ -1269,6 +1066,312 @@ __device__ inline unsigned pivot_key(double v, bool cand) {
 }
 __device__ inline unsigned pivot_key(float v, bool cand) {
   return cand && v == v ? (__float_as_uint(v) & 0x7fffffffu) + 1u : 0u;
+}
+
+// ---------------------------------------------------------------------------
+// Small fronts, whole, each by a group of G threads: a workgroup (G = 256)
+// or one wave (G = 64).
+// ---------------------------------------------------------------------------
+
+// f(0), f(1), ... f(N - 1), each with its index a constant.
+template <int N, int I = 0, typename F>
+__device__ __attribute__((always_inline)) inline void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
+// Static LDS of one workgroup: what one group of 256 threads or four waves
+// of 64 need. Columns and rows are published in two slots by step parity.
+template <typename T, int RMAX = 64>
+struct SmallScratch {
+  T col[2][RMAX];      // the step's pivot column
+  T row[2][RMAX];      // the row at the step's position
+  T prow[RMAX];        // the pivot row, where it is another one
+  int64_t lc[RMAX], uc[RMAX];  // lnz and unz bases of the own columns / rows
+  int cq[RMAX], ce[RMAX];      // column range of the own column's piece
+  int piv[RMAX];
+};
+
+// One front: A's entries (aent; without them the panels of assembled
+// lnz/unz) and the children's update matrices are summed in LDS (F, rows of
+// odd stride LD, no bank conflicts along either direction), moved to
+// registers, eliminated piece by piece exactly as the reference does
+// (SpkLUFactor.jl:178-302: row interchanges inside the piece's diagonal
+// block, applied to the piece's own columns and those right of it; rows
+// below the block scaled always, rows inside it for a nonzero pivot), and
+// written to lnz/unz/ipvt and the arena through LDS.
+//
+// The elimination is a chain of W column steps, so a step's latency is what
+// bounds it: thread (ty, tx) of an NB x NB grid keeps the entries (ty + NB i,
+// tx + NB j) in registers, and a step costs one publication of its column
+// and of the row at its position, one pivot search that every wave makes
+// alike (32-bit keys, with every lane's reciprocal computed meanwhile) and
+// M x M updates per thread; only an interchange takes a second barrier
+// (about 0.5 us a column of a 64-row front). With the front kept in LDS, the
+// pivot searched by one thread and four barriers and an integer division per
+// entry in each step, the small fronts of one pass took, before -> now:
+// 193 x 171 grid 824 -> 450 us, 128 small SPD systems 1500 -> 895 us, 32
+// value sets of 32^3 (float) 2310 -> 993 us. One wave per front of at most 32
+// rows needs no barrier; its grid follows the front (8, 16 or 32 rows): with
+// one grid of 64 rows for every front of a level above the small_wave_min
+// knob the 128 systems took 1709 us, so that form is left to levels that
+// have larger fronts.
+template <typename T, int G, int M, typename Scratch>
+__device__ __attribute__((always_inline)) void small_front_body(
+    const DevSym& s, const SmallDesc& d, const SmallChild* __restrict__ child, T* F, int LD,
+    Scratch& sh, const AEnt* __restrict__ aent, const double* __restrict__ nzval, T* __restrict__ lnz, T* __restrict__ unz,
+    int64_t* __restrict__ ipvt, T* __restrict__ arena,
+    unsigned long long* __restrict__ first_fail) {
+  constexpr int NB = G == kWG ? 16 : 8;
+  constexpr int RMAX = M * NB;  // rows a group can hold
+  constexpr int RL = RMAX < 64 ? RMAX : 64;  // lanes along a column
+  constexpr int NC = G / RL;    // columns a group takes at once
+  const int gt = G == kWG ? (int)threadIdx.x : (int)threadIdx.x % 64;
+  const int lane = (int)threadIdx.x % 64;
+  const int cr = gt % RL, cc0 = gt / RL;  // (row, column) of the column-wise phases
+  auto gsync = [] {
+    if constexpr (G == kWG)
+      __syncthreads();
+    else
+      wave_lds_sync();
+  };
+  const int L = d.L, W = d.W, R = L - W;
+  const int64_t fc0 = d.fc0;
+  // the first entries are read while F is cleared
+  AEnt en{};
+  double nv = 0.0;
+  if (aent && gt < d.an) {
+    en = aent[d.a0 + gt];
+    nv = nzval[en.k];
+  }
+  if (gt < W) {
+    const int64_t g = fc0 + gt, p = s.snode[g];
+    sh.lc[gt] = s.lcol[g];
+    sh.uc[gt] = s.ucol[g];
+    sh.cq[gt] = (int)(s.xsuper[p - 1] - 1 - fc0);
+    sh.ce[gt] = (int)(s.xsuper[p] - 1 - fc0);
+  }
+  for (int i = gt; i < L * LD; i += G) F[i] = T(0);
+  gsync();
+  if (aent) {
+    if (gt < d.an) F[en.r + en.c * LD] = (T)nv;
+    for (int e = gt + G; e < d.an; e += G) {
+      const AEnt x = aent[d.a0 + e];
+      F[x.r + x.c * LD] = (T)nzval[x.k];
+    }
+  } else {
+    for (int j = cc0; j < W; j += NC)
+      if (cr < L) {
+        if (cr >= (s.sym ? j : sh.cq[j])) F[cr + j * LD] = lnz[sh.lc[j] + cr];
+        if (!s.sym && cr >= sh.ce[j]) F[j + cr * LD] = unz[sh.uc[j] + cr];
+      }
+    if (s.sym) {  // upper rows of the own columns from the lower triangle
+      gsync();
+      for (int j = cc0; j < W; j += NC)
+        if (cr > j && cr < L) F[j + cr * LD] = F[cr + j * LD];
+    }
+  }
+  gsync();
+  // children's update matrices, one child at a time in a fixed order (rows
+  // of different children may coincide)
+  for (int ci = 0; ci < d.nch; ++ci) {
+    const SmallChild ch = child[d.ch0 + ci];
+    const int32_t* rel = s.relmap + ch.rel;
+    const T* cb = arena + ch.cb;
+    const bool in = cr < ch.R;
+    const int rr = in ? rel[cr] : 0;
+    for (int t0 = cc0; t0 < ch.R; t0 += 8 * NC) {
+      T v[8];
+      int rt[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int t = t0 + u * NC;
+        v[u] = (in && t < ch.R) ? cb[cr + (int64_t)t * ch.ld] : T(0);
+        rt[u] = t < ch.R ? rel[t] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (in && t0 + u * NC < ch.R) F[rr + rt[u] * LD] += v[u];
+    }
+    gsync();
+  }
+  const int ty = gt % NB, tx = gt / NB;
+  T a[M][M];
+#pragma unroll
+  for (int i = 0; i < M; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      const int r = ty + NB * i, c = tx + NB * j;
+      a[i][j] = (r < L && c < L) ? F[r + c * LD] : T(0);
+    }
+  const int srow = lane % RMAX;  // the row this lane looks at in a pivot search
+  static_for<M>([&](auto jbc) __attribute__((always_inline)) {
+    constexpr int jb = decltype(jbc)::value;
+#pragma unroll 1
+    for (int cc = 0; cc < NB && jb * NB + cc < W; ++cc) {
+      const int k = jb * NB + cc, par = cc & 1;
+      const int cq = sh.cq[k], ce = sh.ce[k];
+      T* col = sh.col[par];
+      T* row = sh.row[par];
+      if (tx == cc) {
+#pragma unroll
+        for (int i = 0; i < M; ++i) col[ty + NB * i] = a[i][jb];
+      }
+      if (ty == cc) {
+#pragma unroll
+        for (int j = 0; j < M; ++j) row[tx + NB * j] = a[jb][j];
+      }
+      gsync();
+      const T v = col[srow];
+      T l[M], u[M];
+#pragma unroll
+      for (int i = jb; i < M; ++i) l[i] = col[ty + NB * i];
+#pragma unroll
+      for (int j = jb; j < M; ++j) u[j] = row[tx + NB * j];
+      const bool cand = lane < RMAX && lane >= k && lane < ce;
+      const unsigned key = pivot_key(v, cand);
+      unsigned mx;
+      const T rc = recip_and_max(v, key, mx);
+      int kp = k;
+      if (s.pivot) {
+        const unsigned long long msk = __ballot(key == mx);
+        kp = __builtin_amdgcn_readfirstlane(__ffsll((long long)msk) - 1);
+        // ties of the leading bits, no number among the candidates, or none
+        // in the first row (which then stays): the exact rule
+        if (__builtin_expect(mx == 0u || (msk & (msk - 1ull)) != 0ull ||
+                                 __builtin_amdgcn_readlane((int)key, k) == 0, 0)) {
+          const bool keep = __builtin_amdgcn_readlane((int)key, k) == 0;
+          kp = keep ? k : pivot_lane(v, lane, cand, k);
+        }
+      }
+      const T pv = rdlane(v, kp), inv = rdlane(rc, kp);
+      const bool nz = pv != T(0);
+      if (gt == 0) {
+        sh.piv[k] = kp - cq + 1;
+        if (!nz) atomicMin(first_fail, (unsigned long long)s.snode[fc0 + k]);
+      }
+      if (kp != k && nz) {
+        T* prow = sh.prow;
+#pragma unroll
+        for (int i = jb; i < M; ++i)
+          if (ty + NB * i == kp) {
+#pragma unroll
+            for (int j = 0; j < M; ++j) prow[tx + NB * j] = a[i][j];
+          }
+        gsync();
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+          const int c = tx + NB * j;
+          const T x = row[c], y = prow[c];
+#pragma unroll
+          for (int i = jb; i < M; ++i)
+            if (ty + NB * i == kp && c >= cq) a[i][j] = x;
+          if (ty == cc && c >= cq) a[jb][j] = y;
+          if (j >= jb) u[j] = y;
+        }
+        const T ck = col[k];
+#pragma unroll
+        for (int i = jb; i < M; ++i)
+          if (ty + NB * i == kp) l[i] = ck;
+      }
+#pragma unroll
+      for (int i = jb; i < M; ++i) {
+        const int r = ty + NB * i;
+        l[i] = (nz || r >= ce) ? l[i] * inv : l[i];
+        const bool below = i > jb || r > k;
+        if (tx == cc && below) a[i][jb] = l[i];
+#pragma unroll
+        for (int j = jb; j < M; ++j) {
+          const T w = a[i][j] - l[i] * u[j];
+          a[i][j] = (below && (j > jb || tx > cc)) ? w : a[i][j];
+        }
+      }
+    }
+  });
+#pragma unroll
+  for (int i = 0; i < M; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      const int r = ty + NB * i, c = tx + NB * j;
+      if (r < L && c < L) F[r + c * LD] = a[i][j];
+    }
+  gsync();
+  if (gt < W) ipvt[fc0 + gt] = sh.piv[gt];
+  for (int j = cc0; j < W; j += NC)
+    if (cr < L) {
+      if (cr >= sh.cq[j]) lnz[sh.lc[j] + cr] = F[cr + j * LD];
+      if (cr >= sh.ce[j]) unz[sh.uc[j] + cr] = F[j + cr * LD];
+    }
+  T* cb = arena + d.cb;
+  if (cr < R)
+    for (int t = cc0; t < R; t += NC) cb[cr + t * R] = F[(W + cr) + (W + t) * LD];
+}
+
+// The level's fronts of more than 32 rows (the first nbig of desc) one per
+// workgroup, the others one per wave, four per workgroup; WAVE64: every
+// front one per wave (levels of very many fronts). The grid of a wave's
+// threads follows the front's rows.
+template <typename T, bool WAVE64>
+__global__ void __launch_bounds__(kWG)
+small_front_kernel(DevSym s, const SmallDesc* __restrict__ desc,
+                   const SmallChild* __restrict__ child, int nbig, int cnt, int LD, int slot,
+                   const AEnt* __restrict__ aent, const double* __restrict__ nzval,
+                   int64_t nnz, T* __restrict__ lnz, T* __restrict__ unz,
+                   int64_t* __restrict__ ipvt, T* __restrict__ arena,
+                   unsigned long long* __restrict__ first_fail) {
+  const int64_t vs = blockIdx.y;  // value set
+  nzval += vs * nnz;
+  lnz += vs * s.vs_lnz;
+  unz += vs * s.vs_unz;
+  ipvt += vs * s.n;
+  arena += vs * s.vs_arena;
+  extern __shared__ unsigned char smem_raw[];
+  T* F = reinterpret_cast<T*>(smem_raw);
+  const int wave = wave_id();
+  if constexpr (WAVE64) {
+    __shared__ SmallScratch<T> sh[4];
+    const int item = blockIdx.x * 4 + wave;
+    if (item >= cnt) return;
+    const SmallDesc d = desc[item];
+    F += wave * slot;
+    auto go = [&](auto m) __attribute__((always_inline)) {
+      small_front_body<T, 64, decltype(m)::value>(s, d, child, F, LD, sh[wave], aent, nzval, lnz,
+                                                  unz, ipvt, arena, first_fail);
+    };
+    if (d.L <= 16)
+      go(std::integral_constant<int, 2>{});
+    else if (d.L <= 32)
+      go(std::integral_constant<int, 4>{});
+    else
+      go(std::integral_constant<int, 8>{});
+  } else {
+    __shared__ union U {
+      SmallScratch<T> big;
+      SmallScratch<T, 32> one[4];
+      __device__ U() {}
+    } sh;
+    if ((int)blockIdx.x < nbig) {
+      small_front_body<T, kWG, 4>(s, desc[blockIdx.x], child, F, LD, sh.big, aent, nzval, lnz, unz,
+                                  ipvt, arena, first_fail);
+      return;
+    }
+    const int item = nbig + ((int)blockIdx.x - nbig) * 4 + wave;
+    if (item >= cnt) return;
+    const SmallDesc d = desc[item];
+    F += wave * slot;
+    auto go = [&](auto m) __attribute__((always_inline)) {
+      small_front_body<T, 64, decltype(m)::value>(s, d, child, F, min(LD, 33), sh.one[wave], aent,
+                                                  nzval, lnz, unz, ipvt, arena, first_fail);
+    };
+    if (d.L <= 8)
+      go(std::integral_constant<int, 1>{});
+    else if (d.L <= 16)
+      go(std::integral_constant<int, 2>{});
+    else
+      go(std::integral_constant<int, 4>{});
+  }
 }
 
 // Diagonal region of one block of at most 64 columns per workgroup, held
