@@ -28,7 +28,7 @@ using spk::BlkDesc;
 using spk::kWG;
 
 using spk::kSmallLmax;
-constexpr int kGW = 128;    // widest block of pieces (LU)
+constexpr int kGW = 128;    // widest block of pieces
 constexpr int kGMaxP = 8;   // most pieces in one block
 constexpr int kNqLU = 48;   // widest LU piece the blocked kernels take
 constexpr int kNqSPD = 96;  // widest SPD piece
@@ -88,8 +88,8 @@ struct DevBuf {
 
 struct LevelPlan {
   int small_off = 0, small_cnt = 0, small_maxL = 0;
-  int small_big = 0;                // the first ones have more than 32 rows
-  int small_maxq = 1;               // widest piece of the level's small fronts
+  spk::SmallClasses small_k{};      // the level's small fronts by rows
+  int small_maxW = 1;               // most own columns of the level's small fronts
   int items_off = 0, items_cnt = 0;
   int wb_off = 0, wb_cnt = 0;       // write-back items: the large fronts' pivot columns
   int large_maxL = 0;               // longest index list of the level's large fronts
@@ -187,7 +187,7 @@ struct spkhip_handle {
   // device symbolic
   DevBuf<i64> d_xsuper, d_snode, d_xlnz, d_xunz, d_xlindx, d_perm, d_invp;
   DevBuf<i32> d_lindx, d_fL, d_fW, d_fc0, d_fsp0, d_fnp, d_fcbld, d_fchp, d_fch,
-      d_relmap, d_small, d_it_front, d_it_col, d_ea_child, d_ea_t, d_solve;
+      d_relmap, d_pcol, d_it_front, d_it_col, d_ea_child, d_ea_t, d_solve;
   DevBuf<i64> d_foff, d_fcb, d_frel, d_fvec, d_it_ea, d_lcol, d_ucol;
   DevBuf<spk::SmallDesc> d_sdfr;    // the small fronts, resolved
   DevBuf<spk::SmallChild> d_sdch;   // their children
@@ -573,16 +573,16 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
       if (h->fL[f] <= h->small_lmax) {
         small.push_back(f);
         lp.small_maxL = std::max(lp.small_maxL, h->fL[f]);
-        for (i32 p = h->fsp0[f]; p < h->fsp0[f] + h->fnp[f]; ++p)
-          lp.small_maxq = std::max(lp.small_maxq, (int)(h->xsuper[p + 1] - h->xsuper[p]));
+        lp.small_maxW = std::max(lp.small_maxW, h->fW[f]);
       } else {
         large.push_back(f);
       }
     }
     lp.small_cnt = (int)small.size() - lp.small_off;
-    const auto mid = std::stable_partition(small.begin() + lp.small_off, small.end(),
-                                           [&](i32 f) { return h->fL[f] > 32; });
-    lp.small_big = (int)(mid - small.begin()) - lp.small_off;
+    auto cls = [&](i32 f) { return h->fL[f] > 32 ? 0 : h->fL[f] > 16 ? 1 : h->fL[f] > 8 ? 2 : 3; };
+    std::stable_sort(small.begin() + lp.small_off, small.end(),
+                     [&](i32 a, i32 b) { return cls(a) < cls(b); });
+    for (size_t i = lp.small_off; i < small.size(); ++i) lp.small_k.cnt[cls(small[i])]++;
     lp.solve_cnt = (int)solve.size() - lp.solve_off;
     lp.large_off = (int)largel.size();
     for (i32 f : bylev[l]) {
@@ -1173,6 +1173,26 @@ struct Bufs<float> {
   static DevBuf<float>& prep(spkhip_handle* h) { return h->d_prep32; }
 };
 
+// Workgroups of a level's small fronts in the solves: one each for the first
+// class, a wave for the second, 16 and 8 lanes per right-hand side for the
+// others (a wave too with more than four right-hand sides, which then share
+// its lanes). Levels with few of the latter (less than a wave per SIMD and eight
+// of them in flight) give each a wave as well, whose broadcasts are faster:
+// 24 x 17 grid, 408 unknowns, 178 us a pass against 214, but 128 small
+// systems with four right-hand sides 1172 us against 951.
+constexpr i64 kTinyMin = 8192;
+unsigned small_wgs(const LevelPlan& lp, int nrhs, int nvs, spk::SmallClasses& k) {
+  k = lp.small_k;
+  if (nrhs > 4 || ((i64)k.cnt[2] + k.cnt[3]) * nrhs * nvs < kTinyMin) {
+    k.cnt[1] += k.cnt[2] + k.cnt[3];
+    k.cnt[2] = k.cnt[3] = 0;
+  }
+  k.wg1 = (k.cnt[1] + 3) / 4;
+  k.wg2 = (int)(((i64)k.cnt[2] * nrhs + 15) / 16);
+  const i64 wg3 = ((i64)k.cnt[3] * nrhs + 31) / 32;
+  return (unsigned)(k.cnt[0] + k.wg1 + k.wg2 + wg3);
+}
+
 template <typename T>
 void set_lds_attrs() {
   static bool done = false;
@@ -1246,13 +1266,13 @@ void run_factor(spkhip_handle* h, bool from_a) {
                            aent, h->d_nzval.p, h->nnz, lnz.p, unz.p, h->d_ipvt.p, arena.p,
                            h->d_fail.p);
       };
-      if (lp.small_cnt >= h->small_wave_min && lp.small_big > 0) {
+      const int nbig = lp.small_k.cnt[0];
+      if (lp.small_cnt >= h->small_wave_min && nbig > 0) {
         go(spk::small_front_kernel<T, true>, 0, (lp.small_cnt + 3) / 4, front, 4 * front);
       } else {
         const int slot = std::min(front, 32 * 33);
-        go(spk::small_front_kernel<T, false>, lp.small_big,
-           lp.small_big + (lp.small_cnt - lp.small_big + 3) / 4, slot,
-           std::max(lp.small_big ? front : 0, 4 * slot));
+        go(spk::small_front_kernel<T, false>, nbig, nbig + (lp.small_cnt - nbig + 3) / 4, slot,
+           std::max(nbig ? front : 0, 4 * slot));
       }
       hipck(hipGetLastError());
     }
@@ -1384,26 +1404,6 @@ void read_first_fail(spkhip_handle* h) {
   h->first_fail = (ff == ~0ull) ? 0 : (i64)ff;
 }
 
-// Right-hand sides that share one staging of a small front's panels.
-inline int small_rhs_block(int nrhs) { return std::max(1, std::min(nrhs, spk::kSmallRhsBlock)); }
-
-// Small fronts per workgroup in the solves (one wave each): four when their
-// staging (a panel of at most maxq columns and qb solve vectors) fits in
-// 150 KB of LDS, fewer otherwise.
-template <typename T, int MAXW>
-int small_fronts_per_wg(int maxL, int qb = 1, int maxq = 1) {
-  static bool attrs = false;
-  if (!attrs) {
-    hipck(hipFuncSetAttribute((const void*)spk::fwd_small_kernel<T, MAXW>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
-    hipck(hipFuncSetAttribute((const void*)spk::bwd_small_kernel<T, MAXW>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
-    attrs = true;
-  }
-  const size_t per = (size_t)(maxq + qb) * std::max(maxL, 1) * sizeof(T);
-  return (int)std::max<size_t>(1, std::min<size_t>(4, 150 * 1024 / per));
-}
-
 // Device storage of the per-block solve data, sized at factor time so that
 // a solve allocates nothing for it.
 template <typename T>
@@ -1453,8 +1453,9 @@ void solve_prep(spkhip_handle* h, bool inv) {
 
 // vecp: the per-front vector arena, h->vec_elems * nrhs elements. Float
 // factors take the explicit-inverse block steps unless SPKHIP_SOLVE_INV=0.
-template <typename T, int MAXW, int GW>
-void solve_levels_w(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, bool bwd, T* vecp) {
+template <typename T>
+void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, bool bwd,
+                         T* vecp) {
   hipStream_t st = h->stream;
   set_lds_attrs<T>();
   const T* lnz = Bufs<T>::lnz(h).p;
@@ -1468,13 +1469,24 @@ void solve_levels_w(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, bool 
       h->cur_grid = lp.small_cnt;
       if (lp.small_cnt > 0) {
         Prof pr(h, SPKHIP_K_FWD, 0.0, 0.0);
-        const int qb = small_rhs_block(nrhs);
-        const int fpw = small_fronts_per_wg<T, MAXW>(lp.small_maxL, qb, lp.small_maxq);
-        hipLaunchKernelGGL((spk::fwd_small_kernel<T, MAXW>),
-                           dim3((lp.small_cnt + fpw - 1) / fpw, h->nvs), dim3(kWG),
-                           (size_t)fpw * (lp.small_maxq + qb) * lp.small_maxL * sizeof(T), st,
-                           h->ds, h->d_small.p + lp.small_off, lp.small_cnt, fpw, qb, lnz,
-                           h->d_ipvt.p, rhs, ldr, nrhs, vecp, lp.small_maxL, lp.small_maxq);
+        spk::SmallClasses k;
+        const unsigned wgs = small_wgs(lp, nrhs, h->nvs, k);
+        const int LDL = lp.small_maxL | 1, slot = std::min(lp.small_maxW, 32) * std::min(LDL, 33);
+        const size_t lds = nrhs <= 4 ? 0
+                                     : std::max(k.cnt[0] ? lp.small_maxW * LDL : 0,
+                                                k.cnt[1] ? 4 * slot : 0) * sizeof(T);
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(wgs, h->nvs), dim3(kWG), lds, st, h->ds,
+                             h->d_sdfr.p + lp.small_off, h->d_sdch.p, k, LDL, slot, lnz,
+                             h->d_ipvt.p, rhs, ldr, nrhs, vecp);
+        };
+        // right-hand sides in the registers of one wave
+        if (nrhs == 1)
+          go(spk::fwd_small_kernel<T, 1>);
+        else if (nrhs <= 4)
+          go(spk::fwd_small_kernel<T, 4>);
+        else
+          go(spk::fwd_small_kernel<T, 16>);
         hipck(hipGetLastError());
       }
       if (lp.large_cnt == 0) continue;
@@ -1570,25 +1582,24 @@ void solve_levels_w(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, bool 
       }
       if (lp.small_cnt > 0) {
         Prof pr(h, SPKHIP_K_BWD, 0.0, 0.0);
-        const int qb = small_rhs_block(nrhs);
-        const int fpw = small_fronts_per_wg<T, MAXW>(lp.small_maxL, qb, lp.small_maxq);
-        hipLaunchKernelGGL((spk::bwd_small_kernel<T, MAXW>),
-                           dim3((lp.small_cnt + fpw - 1) / fpw, h->nvs), dim3(kWG),
-                           (size_t)fpw * (lp.small_maxq + qb) * lp.small_maxL * sizeof(T), st,
-                           h->ds, h->d_small.p + lp.small_off, lp.small_cnt, fpw, qb, lnz, unz,
-                           rhs, ldr, nrhs, lp.small_maxL, lp.small_maxq);
+        const int LDW = lp.small_maxW | 1, slot = std::min(lp.small_maxL, 32) * std::min(LDW, 33);
+        spk::SmallClasses k;
+        const unsigned wgs = small_wgs(lp, nrhs, h->nvs, k);
+        const size_t lds =
+            std::max(k.cnt[0] ? lp.small_maxL * LDW : 0, k.cnt[1] ? 4 * slot : 0) * sizeof(T);
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(wgs, h->nvs), dim3(kWG), lds, st, h->ds,
+                             h->d_sdfr.p + lp.small_off, k, LDW, slot, lnz, unz, rhs, ldr, nrhs);
+        };
+        if (nrhs == 1)
+          go(spk::bwd_small_kernel<T, 1>);
+        else if (nrhs <= 4)
+          go(spk::bwd_small_kernel<T, 4>);
+        else
+          go(spk::bwd_small_kernel<T, 16>);
         hipck(hipGetLastError());
       }
     }
-}
-
-template <typename T>
-void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, bool bwd,
-                         T* vecp) {
-  if (h->kind == SPKHIP_KIND_LU)
-    solve_levels_w<T, 64, kGW>(h, rhs, ldr, nrhs, fwd, bwd, vecp);
-  else
-    solve_levels_w<T, 96, 96>(h, rhs, ldr, nrhs, fwd, bwd, vecp);
 }
 
 // Both sweeps replay a captured graph of their launches when nothing they
@@ -1607,8 +1618,6 @@ void solve_levels(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, bool bw
     return;
   }
   set_lds_attrs<T>();
-  small_fronts_per_wg<T, 64>(1);
-  small_fronts_per_wg<T, 96>(1);
   solve_prep<T>(h, inv_solve<T>(nrhs));
   const std::vector<const void*> key = {
       (const void*)rhs, (const void*)(intptr_t)ldr, (const void*)(intptr_t)nrhs,
@@ -1750,6 +1759,8 @@ void replan(spkhip_handle* h) {
       d.L = h->fL[f];
       d.W = h->fW[f];
       d.fc0 = (i32)h->fc0[f];
+      d.fvec = h->fvec[f];
+      d.ind = h->xlindx[h->fsp0[f]] - 1;
       d.ch0 = (i32)chl.size();
       d.nch = h->fchp[f + 1] - h->fchp[f];
       if (!h->aptr.empty()) {
@@ -1758,7 +1769,8 @@ void replan(spkhip_handle* h) {
       }
       for (i32 ci = h->fchp[f]; ci < h->fchp[f + 1]; ++ci) {
         const i32 c = h->fch[ci];
-        chl.push_back(spk::SmallChild{h->fcb[c], h->frel[c], h->fL[c] - h->fW[c], h->fcbld[c]});
+        chl.push_back(spk::SmallChild{h->fcb[c], h->frel[c], h->fvec[c], h->fL[c] - h->fW[c],
+                                      h->fcbld[c], h->fL[c]});
       }
       fr.push_back(d);
     }
@@ -1767,8 +1779,6 @@ void replan(spkhip_handle* h) {
     h->d_sdfr.upload(fr, st);
     h->d_sdch.upload(chl, st);
   }
-  if (small.empty()) small.push_back(0);
-  h->d_small.upload(small, st);
   if (it_front.empty()) {
     it_front.push_back(0);
     it_col.push_back(0);
@@ -1948,6 +1958,7 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
   h->d_fch.upload(h->fch, st);
   {  // per-column base offsets of the reference layout in front coordinates
     std::vector<i64> lcol(n), ucol(n);
+    std::vector<i32> pcol(n, 0);
     for (i32 f = 0; f < h->nfront; ++f) {
       const i64 fc0 = h->fc0[f];
       for (i64 p = h->fsp0[f]; p < h->fsp0[f] + h->fnp[f]; ++p) {
@@ -1956,11 +1967,13 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
         for (i64 g = pc0; g < pc0 + nq; ++g) {
           lcol[g] = h->xlnz[g] - 1 - cq;
           ucol[g] = h->xunz[g] - 1 - (cq + nq);
+          if (h->fL[f] <= kSmallLmax) pcol[g] = (i32)(cq | (cq + nq) << 16);
         }
       }
     }
     h->d_lcol.upload(lcol, st);
     h->d_ucol.upload(ucol, st);
+    h->d_pcol.upload(pcol, st);
   }
   DevSym& d = h->ds;
   d.n = n;
@@ -1983,6 +1996,7 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
   d.fch = h->d_fch.p;
   d.lcol = h->d_lcol.p;
   d.ucol = h->d_ucol.p;
+  d.pcol = h->d_pcol.p;
   d.pivot = (kind == SPKHIP_KIND_LU) ? 1 : 0;
   d.sym = (kind == SPKHIP_KIND_SPD) ? 1 : 0;
   h->nvs = 1;  // a new pattern starts with one value set

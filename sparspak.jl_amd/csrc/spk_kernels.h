@@ -54,6 +54,8 @@ struct DevSym {
   const int64_t* lcol;    // per column g: lnz offset of front row 0, i.e.
                           // L(front row r, g) = lnz[lcol[g] + r]
   const int64_t* ucol;    // per row g: U(g, front column j) = unz[ucol[g] + j]
+  const int32_t* pcol;    // per column of a front of at most 64 rows: its
+                          // piece's front columns, first | end << 16
   int pivot;              // 1: pivot inside diagonal blocks (LU); 0: none
   int sym;                // 1: U entries are read from the transposed lnz slot
                           //    (SPD input: lower triangle only)
@@ -124,6 +126,8 @@ struct AsmItem {
 struct SmallDesc {
   int64_t a0;  // A's entries of the front
   int64_t cb;  // arena offset of its update matrix (leading dimension L - W)
+  int64_t fvec;  // offset in the solve vector arena
+  int64_t ind;   // offset of its index list
   int32_t an;
   int32_t L, W;
   int32_t fc0;       // first column
@@ -132,7 +136,15 @@ struct SmallDesc {
 struct SmallChild {
   int64_t cb;   // arena offset of the child's update matrix
   int64_t rel;  // offset of its relative-index map
-  int32_t R, ld;
+  int64_t fvec; // the child's offset in the solve vector arena
+  int32_t R, ld, L;
+};
+// A level's small fronts by rows: more than 32, 17 to 32, 9 to 16, at most
+// 8, in this order in the list; workgroups of the second and third class in
+// the solves.
+struct SmallClasses {
+  int32_t cnt[4];
+  int32_t wg1, wg2;
 };
 // One entry of A inside its front: value k of the CSC array goes to row r,
 // column c of the front's matrix (SPD: once more to row c, column r).

@@ -2484,300 +2484,9 @@ blk_diag_border_kernel(DevSym s, const BlkDesc* __restrict__ ddesc, int ndiag,
 // Backward (_luusolve!, :325-377), blocks in reverse: t = U[c0:c1, c1:L]
 // x[I[c1:L]] (one wave per row), then the chain: y = x - t, per piece in
 // reverse the in-block U12 part and the upper block solve.
-// Small fronts (L <= kSmallLmax) do everything in one workgroup.
-// The serial block solves run on wave 0 only: LDS operations of one wave
-// complete in issue order, so no barrier is needed between their steps.
+// Small fronts (L <= kSmallLmax) do everything in one wave per block of
+// right-hand sides.
 // ---------------------------------------------------------------------------
-template <typename T, int MAXW>
-__device__ void stage_block(T* D, const T* lp, int nq, int jl) {
-  for (int idx = threadIdx.x; idx < nq * nq; idx += kWG) {
-    int i = idx % nq, k = idx / nq;
-    D[i + k * MAXW] = lp[i + (int64_t)k * jl];
-  }
-}
-
-// sum_k L[r, pc0 + k] * y[k] for k < nq: the column bases lcol[pc0 + k] are
-// wave-uniform; loads are issued eight at a time.
-template <typename T>
-__device__ inline T dot_lrow(const DevSym& s, const T* __restrict__ lnz, int64_t pc0, int nq,
-                             int r, const T* y) {
-  T acc = T(0);
-  int k = 0;
-  for (; k + 8 <= nq; k += 8) {
-    T lv[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) lv[j] = lnz[s.lcol[pc0 + k + j] + r];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc += lv[j] * y[k + j];
-  }
-  for (; k < nq; ++k) acc += lnz[s.lcol[pc0 + k] + r] * y[k];
-  return acc;
-}
-
-
-// Unit-lower solve of one piece's diagonal block on yb (LDS) by wave 0,
-// after the piece's interchanges (glaswp! then gtrsm! 'l','l','n','u').
-template <typename T>
-__device__ void wave_lower_solve(T* yb, const T* D, int ld, const int* piv, int nq) {
-  const int lane = threadIdx.x % 64;
-  if (lane == 0)
-    for (int k = 0; k < nq; ++k) {
-      int ip = piv[k];
-      if (ip != k) {
-        T t = yb[k];
-        yb[k] = yb[ip];
-        yb[ip] = t;
-      }
-    }
-  wave_lds_sync();
-  for (int k = 0; k < nq; ++k) {
-    const T yk = yb[k];
-    if (yk != T(0))
-      for (int i = k + 1 + lane; i < nq; i += 64) yb[i] -= yk * D[i + k * ld];
-    wave_lds_sync();
-  }
-}
-
-// Upper solve (gtrsm! 'l','u','n','n') of one piece's block by wave 0.
-template <typename T>
-__device__ void wave_upper_solve(T* yb, const T* D, int ld, int nq) {
-  const int lane = threadIdx.x % 64;
-  for (int k = nq - 1; k >= 0; --k) {
-    T yk = yb[k];
-    if (yk != T(0)) {
-      yk /= D[k + k * ld];
-      wave_lds_sync();
-      if (lane == 0) yb[k] = yk;
-      for (int i = lane; i < k; i += 64) yb[i] -= yk * D[i + k * ld];
-    }
-    wave_lds_sync();
-  }
-}
-
-// Most right-hand sides the small-front solves take per staging of a panel.
-constexpr int kSmallRhsBlock = 16;
-
-// Small fronts, one wave per front (fpw <= 4 fronts per workgroup, as many
-// as the LDS holds), everything in LDS; lane loops stride 64 and a wave
-// barrier orders the steps.
-// Forward: y starts as the own rows of x and zero update rows, receives the
-// children's update vectors in a fixed child order, then per piece: the
-// piece's whole panel (rows from its first row to L) is staged once, the
-// interchanges and the unit-lower block solve, and every row below takes its
-// dot product with the block's entries from the staged panel (the order of
-// dot_lrow). Only the update rows go back to the vector arena (the parent
-// reads nothing else), the own rows to x. Dynamic LDS per wave: the staged
-// panel (MAXW x maxL, maxL the level's longest small front) and yW[maxL].
-template <typename T, int MAXW>
-__global__ void __launch_bounds__(kWG)
-fwd_small_kernel(DevSym s, const int32_t* __restrict__ list, int cnt, int fpw, int qb,
-                 const T* __restrict__ lnz, const int64_t* __restrict__ ipvt,
-                 T* __restrict__ rhs, int64_t ldr, int nrhs, T* __restrict__ vec, int maxL,
-                 int maxq) {
-  const int64_t vs = blockIdx.y;  // value set
-  lnz += vs * s.vs_lnz;
-  ipvt += vs * s.n;
-  rhs += vs * ldr * nrhs;
-  vec += vs * s.vs_vec * nrhs;
-  extern __shared__ unsigned char smem_raw[];
-  __shared__ int spiv_all[4][MAXW];
-  const int lane = threadIdx.x % 64, wave = wave_id();
-  const int item = blockIdx.x * fpw + wave;
-  if (wave >= fpw || item >= cnt) return;
-  // the staged panel: rows of stride maxL, at most maxq columns (the level's
-  // widest piece); then the qb solve vectors
-  T* D = reinterpret_cast<T*>(smem_raw) + (int64_t)wave * (maxq + qb) * maxL;
-  T* Y = D + (int64_t)maxq * maxL;
-  int* spiv = spiv_all[wave];
-  const int f = list[item];
-  const int L = s.fL[f], W = s.fW[f];
-  const int64_t fc0 = s.fc0[f];
-  const int sp0 = s.fsp0[f], np = s.fnp[f];
-  // right-hand sides in blocks of qb (y of the block's right-hand side qq
-  // at Y + qq maxL), each piece's panel staged once per block; the lanes
-  // take (right-hand side, row) pairs, and every right-hand side receives
-  // the same operations in the same order as when solved alone
-  for (int q0 = 0; q0 < nrhs; q0 += qb) {
-    const int nq_b = min(qb, nrhs - q0);
-    for (int idx = lane; idx < nq_b * L; idx += 64) {
-      const int qq = idx / L, r = idx - qq * L;
-      Y[qq * maxL + r] = (r < W) ? rhs[(int64_t)(q0 + qq) * ldr + fc0 + r] : T(0);
-    }
-    wave_lds_sync();
-    for (int ci = s.fchp[f]; ci < s.fchp[f + 1]; ++ci) {
-      const int c = s.fch[ci];
-      const int Lc = s.fL[c], Wc = s.fW[c], Rc = Lc - Wc;
-      const int32_t* rel = s.relmap + s.frel[c];
-      const T* uc = vec + s.fvec[c] * nrhs + (int64_t)q0 * Lc + Wc;
-      for (int idx = lane; idx < nq_b * Rc; idx += 64) {
-        const int qq = idx / Rc, t = idx - qq * Rc;
-        Y[qq * maxL + rel[t]] += uc[(int64_t)qq * Lc + t];
-      }
-      wave_lds_sync();
-    }
-    for (int p = sp0; p < sp0 + np; ++p) {
-      int64_t pc0, nq64;
-      piece_cols(s, p, pc0, nq64);
-      const int nq = (int)nq64;
-      const int cq = (int)(pc0 - fc0);
-      const int jl = L - cq;  // the panel's rows
-      const T* lp = lnz + (s.xlnz[pc0] - 1);
-      for (int idx = lane; idx < jl * nq; idx += 64) {
-        const int i = idx % jl, kk = idx / jl;
-        D[i + kk * maxL] = lp[i + (int64_t)kk * jl];
-      }
-      for (int i = lane; i < nq; i += 64) spiv[i] = (int)ipvt[pc0 + i] - 1;
-      wave_lds_sync();
-      // the piece's interchanges (glaswp!), one lane per right-hand side
-      if (lane < nq_b) {
-        T* yb = Y + lane * maxL + cq;
-        for (int k = 0; k < nq; ++k) {
-          const int ip = spiv[k];
-          if (ip != k) {
-            const T t = yb[k];
-            yb[k] = yb[ip];
-            yb[ip] = t;
-          }
-        }
-      }
-      wave_lds_sync();
-      // unit-lower block solve (gtrsm! 'l','l','n','u'): step k updates the
-      // entries below k of every right-hand side
-      for (int k = 0; k + 1 < nq; ++k) {
-        const int m = nq - 1 - k;
-        for (int idx = lane; idx < nq_b * m; idx += 64) {
-          const int qq = idx / m, i = k + 1 + (idx - qq * m);
-          T* yb = Y + qq * maxL + cq;
-          const T yk = yb[k];
-          if (yk != T(0)) yb[i] -= yk * D[i + k * maxL];
-        }
-        wave_lds_sync();
-      }
-      // the rows below the block: dot products with the staged panel
-      const int nrb = L - cq - nq;
-      for (int idx = lane; idx < nq_b * nrb; idx += 64) {
-        const int qq = idx / nrb, r = cq + nq + (idx - qq * nrb);
-        T* yW = Y + qq * maxL;
-        const T* dr = D + (r - cq);
-        T acc = T(0);
-        for (int kk = 0; kk < nq; ++kk) acc += dr[kk * maxL] * yW[cq + kk];
-        yW[r] -= acc;
-      }
-      wave_lds_sync();
-    }
-    T* yg = vec + s.fvec[f] * nrhs + (int64_t)q0 * L;
-    for (int idx = lane; idx < nq_b * L; idx += 64) {
-      const int qq = idx / L, r = idx - qq * L;
-      const T v = Y[qq * maxL + r];
-      if (r < W)
-        rhs[(int64_t)(q0 + qq) * ldr + fc0 + r] = v;
-      else
-        yg[(int64_t)qq * L + r] = v;
-    }
-    wave_lds_sync();
-  }
-}
-
-// Small fronts, backward, one wave per front: y gathered from x through the
-// index list, then per piece in reverse its U rows staged once in LDS, the
-// U12 products (fixed reduction order) and the upper block solve. Dynamic
-// LDS per wave: the staged rows (MAXW x maxL) and yW[maxL].
-template <typename T, int MAXW>
-__global__ void __launch_bounds__(kWG)
-bwd_small_kernel(DevSym s, const int32_t* __restrict__ list, int cnt, int fpw, int qb,
-                 const T* __restrict__ lnz, const T* __restrict__ unz, T* __restrict__ rhs,
-                 int64_t ldr, int nrhs, int maxL, int maxq) {
-  const int64_t vs = blockIdx.y;  // value set
-  lnz += vs * s.vs_lnz;
-  unz += vs * s.vs_unz;
-  rhs += vs * ldr * nrhs;
-  extern __shared__ unsigned char smem_raw[];
-  __shared__ T syk_all[4][kSmallRhsBlock];  // step k's entry of each right-hand side
-  const int lane = threadIdx.x % 64, wave = wave_id();
-  const int item = blockIdx.x * fpw + wave;
-  if (wave >= fpw || item >= cnt) return;
-  // the staged U rows: at most maxq rows (the level's widest piece) of
-  // stride maxq, maxL columns; then the qb solve vectors
-  T* D = reinterpret_cast<T*>(smem_raw) + (int64_t)wave * (maxq + qb) * maxL;
-  T* Y = D + (int64_t)maxq * maxL;
-  const int f = list[item];
-  const int L = s.fL[f], W = s.fW[f];
-  const int64_t fc0 = s.fc0[f];
-  const int sp0 = s.fsp0[f], np = s.fnp[f];
-  const int32_t* I = s.lindx + (s.xlindx[sp0] - 1);
-  // right-hand sides in blocks of qb (y of the block's right-hand side qq
-  // at Y + qq maxL), each piece's U rows staged once per block; lanes take
-  // (right-hand side, row) pairs, every right-hand side receiving the same
-  // operations in the same order as when solved alone
-  T* syk = syk_all[wave];
-  for (int q0 = 0; q0 < nrhs; q0 += qb) {
-    const int nq_b = min(qb, nrhs - q0);
-    for (int idx = lane; idx < nq_b * L; idx += 64) {
-      const int qq = idx / L, r = idx - qq * L;
-      Y[qq * maxL + r] = rhs[(int64_t)(q0 + qq) * ldr + I[r] - 1];
-    }
-    wave_lds_sync();
-    for (int p = sp0 + np - 1; p >= sp0; --p) {
-      int64_t pc0, nq64;
-      piece_cols(s, p, pc0, nq64);
-      const int nq = (int)nq64;
-      const int cq = (int)(pc0 - fc0);
-      // the piece's U rows staged once: D(c, j - cq) = U(c, j) for j from
-      // the piece's first column to L (the block from the packed LU in lnz,
-      // the rest from unz)
-      const int jl = L - cq;
-      const T* lp = lnz + (s.xlnz[pc0] - 1);
-      for (int idx = lane; idx < nq * jl; idx += 64) {
-        const int c = idx % nq, j = idx / nq;
-        D[c + j * maxq] = (j < nq) ? lp[c + (int64_t)j * jl] : unz[s.ucol[pc0 + c] + cq + j];
-      }
-      wave_lds_sync();
-      // U12 products: 16 lanes per (right-hand side, row) pair, lane g
-      // summing the columns g, g + 16, ... in order, then a fixed tree over
-      // the 16 partial sums
-      {
-        const int grp = lane / 16, gl = lane % 16;
-        for (int pr = grp; pr < nq_b * nq; pr += 4) {
-          const int qq = pr / nq, c = pr - qq * nq;
-          T* yW = Y + qq * maxL;
-          T acc = T(0);
-          for (int j = cq + nq + gl; j < L; j += 16) acc += D[c + (j - cq) * maxq] * yW[j];
-          acc += __shfl_xor(acc, 8, 16);
-          acc += __shfl_xor(acc, 4, 16);
-          acc += __shfl_xor(acc, 2, 16);
-          acc += __shfl_xor(acc, 1, 16);
-          if (gl == 0) yW[cq + c] -= acc;
-        }
-      }
-      wave_lds_sync();
-      // upper block solve (gtrsm! 'l','u','n','n'): step k divides entry k
-      // of every right-hand side by U(k, k) and updates the entries above it
-      for (int k = nq - 1; k >= 0; --k) {
-        if (lane < nq_b) syk[lane] = Y[lane * maxL + cq + k];
-        wave_lds_sync();
-        for (int idx = lane; idx < nq_b * (k + 1); idx += 64) {
-          const int qq = idx / (k + 1), i = idx - qq * (k + 1);
-          T yk = syk[qq];
-          if (yk != T(0)) {
-            yk /= D[k + k * maxq];
-            T* yb = Y + qq * maxL + cq;
-            if (i == k)
-              yb[k] = yk;
-            else
-              yb[i] -= yk * D[i + k * maxq];
-          }
-        }
-        wave_lds_sync();
-      }
-    }
-    for (int idx = lane; idx < nq_b * W; idx += 64) {
-      const int qq = idx / W, c = idx - qq * W;
-      rhs[(int64_t)(q0 + qq) * ldr + fc0 + c] = Y[qq * maxL + c];
-    }
-    wave_lds_sync();
-  }
-}
-
 // Large fronts, forward: y = [rhs on own columns; 0] + children, one thread
 // per (front, row) item of the level (the factor's column items: a front's
 // rows and columns share its index list). The children's entries come from
@@ -3344,6 +3053,727 @@ __device__ inline float div_r(float b, float u, float r) {
   const float q0 = b * r;
   return __builtin_fmaf(__builtin_fmaf(-q0, u, b), r, q0);
 }
+
+// Small fronts, solves. A front's right-hand sides are taken by one wave, QB
+// at a time, lane = row, every right-hand side's vector in a register: column
+// j's entry of each is broadcast (readlane) and every row below (forward) or
+// above (backward) subtracts its product. Chains of W (L) such steps bound
+// them; the columns' factor entries are read ahead of them (forward: eight
+// columns from lnz, whose rows are contiguous; backward: the front's U rows
+// staged in LDS by columns). Each right-hand side receives the same
+// operations in the same order however many there are. Fronts of more than
+// 32 rows have a workgroup, whose four waves share the right-hand sides (and
+// the staging), those of 17 to 32 one wave, smaller ones a part of a wave per
+// right-hand side (fwd_tiny, bwd_tiny).
+// Before, everything went through LDS with integer divisions by the panel's
+// sizes and a wave synchronisation per column: forward + backward of one
+// pass, 24 x 17 grid 240 -> 178 us, 193 x 171 680 -> 400 us, 128 small
+// systems with four right-hand sides 1985 -> 951 us.
+
+// Entry j of a 64-bit value held one per lane (j wave-uniform).
+__device__ inline int64_t rdlane_i64(int64_t v, int j) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, j);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), j);
+  return (int64_t)(((unsigned long long)hi << 32) | lo);
+}
+
+// Forward, one wave: right-hand sides q0, q0 + 1, ..., q0 + QB - 1, then
+// those qstep further on. y starts as the own rows of x and zero update
+// rows and receives the children's update vectors in a fixed child order in
+// LDS (Y, QB x 64); then per piece the interchanges (glaswp!) and per column
+// the unit-lower step (gtrsm! 'l','l','n','u') and the rows below. The update
+// rows go to the vector arena (the parent reads nothing else), the own rows
+// to x.
+template <typename T, int QB>
+__device__ __attribute__((always_inline)) void fwd_small_wave(
+    const DevSym& s, const SmallDesc& d, const SmallChild* __restrict__ child, int q0, int qstep,
+    T* Y, const T* __restrict__ lnz, const int64_t* __restrict__ ipvt, T* __restrict__ rhs,
+    int64_t ldr, int nrhs, T* __restrict__ vec) {
+  constexpr int CH = 8;  // columns read ahead
+  const int lane = threadIdx.x % 64;
+  const int L = d.L, W = d.W;
+  const int64_t fc0 = d.fc0;
+  const bool own = lane < W;
+  const int64_t lcb = own ? s.lcol[fc0 + lane] : 0;
+  const int pcol = own ? s.pcol[fc0 + lane] : 0;  // the column's piece
+  const int cq = pcol & 0xffff, ce = pcol >> 16;
+  const int kp = own ? (int)ipvt[fc0 + lane] - 1 + cq : lane;
+  // columns whose step interchanges rows
+  const unsigned long long swaps = __ballot(own && kp != lane);
+  for (; q0 < nrhs; q0 += qstep) {
+    const int nq = min(QB, nrhs - q0);
+    T y[QB];
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
+      y[q] = T(0);
+      if (q < nq && own) y[q] = rhs[(int64_t)(q0 + q) * ldr + fc0 + lane];
+    }
+    if (d.nch > 0) {
+#pragma unroll
+      for (int q = 0; q < QB; ++q) Y[q * 64 + lane] = y[q];
+      wave_lds_sync();
+      // the next child's entries are requested before this one's are added
+      int rr = 0, rows = 0;
+      T v[QB];
+      auto request = [&](int ci) {
+        const SmallChild c = child[d.ch0 + ci];
+        rows = c.R;
+        const T* uc = vec + c.fvec * nrhs + (int64_t)q0 * c.L + (c.L - c.R);
+        rr = lane < rows ? s.relmap[c.rel + lane] : 0;
+#pragma unroll
+        for (int q = 0; q < QB; ++q)
+          v[q] = (q < nq && lane < rows) ? uc[(int64_t)q * c.L + lane] : T(0);
+      };
+      request(0);
+      for (int ci = 0; ci < d.nch; ++ci) {
+        const int r0 = rr;
+        const bool in = lane < rows;
+        T w[QB];
+#pragma unroll
+        for (int q = 0; q < QB; ++q) w[q] = v[q];
+        if (ci + 1 < d.nch) request(ci + 1);
+        if (in) {
+#pragma unroll
+          for (int q = 0; q < QB; ++q) Y[q * 64 + r0] += w[q];
+        }
+        wave_lds_sync();
+      }
+#pragma unroll
+      for (int q = 0; q < QB; ++q) y[q] = Y[q * 64 + lane];
+      wave_lds_sync();
+    }
+    T lv[CH];
+    auto columns = [&](int j0) {
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int j = j0 + u;
+        const T* c = lnz + rdlane_i64(lcb, min(j, 63));
+        lv[u] = (j < W && lane > j && lane < L) ? c[lane] : T(0);
+      }
+    };
+    columns(0);
+    for (int j0 = 0; j0 < W; j0 += CH) {
+      T l[CH];
+#pragma unroll
+      for (int u = 0; u < CH; ++u) l[u] = lv[u];
+      if (j0 + CH < W) columns(j0 + CH);
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int j = j0 + u;
+        if (j >= W) break;
+        const int jce = __builtin_amdgcn_readlane(ce, j);
+        if (swaps && __builtin_amdgcn_readlane(cq, j) == j) {  // a piece begins
+          unsigned long long m = swaps & (~0ull << j) & (jce < 64 ? (1ull << jce) - 1 : ~0ull);
+          while (m) {
+            const int k = __ffsll((long long)m) - 1, p = __builtin_amdgcn_readlane(kp, k);
+            m &= m - 1;
+#pragma unroll
+            for (int q = 0; q < QB; ++q) {
+              const T a = rdlane(y[q], k), b = rdlane(y[q], p);
+              y[q] = lane == k ? b : lane == p ? a : y[q];
+            }
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+          if (q < nq) {
+            const T yk = rdlane(y[q], j);
+            // inside the block a zero entry is skipped, as the reference does
+            const bool on = lane > j && (yk != T(0) || lane >= jce);
+            const T t = y[q] - l[u] * yk;
+            y[q] = on ? t : y[q];
+          }
+        }
+      }
+    }
+    T* yg = vec + d.fvec * nrhs + (int64_t)q0 * L + lane;
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
+      if (q < nq) {
+        if (own)
+          rhs[(int64_t)(q0 + q) * ldr + fc0 + lane] = y[q];
+        else if (lane < L)
+          yg[(int64_t)q * L] = y[q];
+      }
+    }
+  }
+}
+
+// Entry J of each group of SW = 8 or 16 lanes in all of its lanes (DPP
+// row_newbcast, one VALU operation per 32 bits and row of 16; ds_bpermute,
+// through the LDS pipeline, was what bounded the tiny fronts of many systems).
+template <int SW, int J>
+__device__ inline int bcast(int v) {
+  if constexpr (SW == 16) return __builtin_amdgcn_update_dpp(v, v, 0x150 + J, 0xf, 0xf, false);
+  const int lo = __builtin_amdgcn_update_dpp(v, v, 0x150 + J % 8, 0xf, 0x3, false);
+  return __builtin_amdgcn_update_dpp(lo, v, 0x158 + J % 8, 0xf, 0xc, false);
+}
+template <int SW, int J>
+__device__ inline float bcast(float v) {
+  return __int_as_float(bcast<SW, J>(__float_as_int(v)));
+}
+template <int SW, int J>
+__device__ inline int64_t bcast(int64_t v) {
+  const unsigned lo = (unsigned)bcast<SW, J>((int)(unsigned)v);
+  const unsigned hi = (unsigned)bcast<SW, J>((int)(v >> 32));
+  return (int64_t)(((unsigned long long)hi << 32) | lo);
+}
+template <int SW, int J>
+__device__ inline double bcast(double v) {
+  return __longlong_as_double(bcast<SW, J>((int64_t)__double_as_longlong(v)));
+}
+
+// Fronts of at most SW = 8 or 16 rows: groups of SW lanes take one front
+// and right-hand side each (64 / SW at once in a wave, unit u = front nrhs +
+// right-hand side), all of the front's entries in registers. The same
+// operations in the same order as fwd_small_wave / bwd_small_wave, which
+// leave most lanes idle on such fronts (128 small systems, four right-hand
+// sides: 1172 us a pass, now 951).
+template <typename T, int SW>
+__device__ __attribute__((always_inline)) void fwd_tiny(
+    const DevSym& s, const SmallDesc* __restrict__ desc, const SmallChild* __restrict__ child,
+    int64_t u, int cnt, T* Y, const T* __restrict__ lnz, const int64_t* __restrict__ ipvt,
+    T* __restrict__ rhs, int64_t ldr, int nrhs, T* __restrict__ vec) {
+  const int lane = threadIdx.x % 64, g0 = lane - lane % SW, r = lane % SW;
+  // u is the wave's first unit; its quotient by nrhs is scalar
+  const int64_t f0 = u / nrhs;
+  const unsigned qg = (unsigned)(u - f0 * nrhs) + lane / SW, dq = qg / (unsigned)nrhs;
+  const int64_t fi = f0 + dq;
+  const int q = (int)(qg - dq * (unsigned)nrhs);
+  const bool on = fi < cnt;  // a whole group
+  const SmallDesc d = desc[on ? fi : 0];
+  const int L = on ? d.L : 0, W = on ? d.W : 0;
+  const int64_t fc0 = d.fc0;
+  const bool own = r < W;
+  const int64_t lcb = own ? s.lcol[fc0 + r] : 0;
+  const int pcol = own ? s.pcol[fc0 + r] : 0;
+  const int cq = pcol & 0xffff, ce = pcol >> 16;
+  const int kp = own ? (int)ipvt[fc0 + r] - 1 + cq : r;
+  const bool swaps = __ballot(kp != r) != 0;  // in any of the wave's fronts
+  T y = own ? rhs[(int64_t)q * ldr + fc0 + r] : T(0);
+  const int wm = -wave_min(-W);
+  T l[SW];
+  static_for<SW>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int j = decltype(jc)::value;
+    l[j] = T(0);
+    if (j < wm) {
+      const T* c = lnz + bcast<SW, j>(lcb);
+      if (j < W && r > j && r < L) l[j] = c[r];
+    }
+  });
+  Y[lane] = y;
+  wave_lds_sync();
+  for (int ci = 0; ci < (on ? d.nch : 0); ++ci) {
+    const SmallChild c = child[d.ch0 + ci];
+    if (r < c.R) {
+      const T v = vec[c.fvec * nrhs + (int64_t)q * c.L + (c.L - c.R) + r];
+      Y[g0 + s.relmap[c.rel + r]] += v;
+    }
+    wave_lds_sync();
+  }
+  y = Y[lane];
+  wave_lds_sync();
+  static_for<SW>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int j = decltype(jc)::value;
+    if (j < wm) {
+      if (swaps) {  // a piece's interchanges before its first column
+        Y[lane] = y;
+        wave_lds_sync();
+        if (r == j && j < W && cq == j)
+          for (int k = j; k < ce; ++k) {
+            const int p = (int)ipvt[fc0 + k] - 1 + cq;
+            const T t = Y[g0 + k];
+            Y[g0 + k] = Y[g0 + p];
+            Y[g0 + p] = t;
+          }
+        wave_lds_sync();
+        y = Y[lane];
+        wave_lds_sync();
+      }
+      const T yk = bcast<SW, j>(y);
+      const int jce = bcast<SW, j>(ce);
+      const bool act = j < W && r > j && (yk != T(0) || r >= jce);
+      const T t = y - l[j] * yk;
+      y = act ? t : y;
+    }
+  });
+  if (own)
+    rhs[(int64_t)q * ldr + fc0 + r] = y;
+  else if (r < L)
+    vec[d.fvec * nrhs + (int64_t)q * L + r] = y;
+}
+
+template <typename T, int SW>
+__device__ __attribute__((always_inline)) void bwd_tiny(
+    const DevSym& s, const SmallDesc* __restrict__ desc, int64_t u, int cnt,
+    const T* __restrict__ lnz, const T* __restrict__ unz, T* __restrict__ rhs, int64_t ldr,
+    int nrhs) {
+  const int lane = threadIdx.x % 64, r = lane % SW;
+  // u is the wave's first unit; its quotient by nrhs is scalar
+  const int64_t f0 = u / nrhs;
+  const unsigned qg = (unsigned)(u - f0 * nrhs) + lane / SW, dq = qg / (unsigned)nrhs;
+  const int64_t fi = f0 + dq;
+  const int q = (int)(qg - dq * (unsigned)nrhs);
+  const bool on = fi < cnt;
+  const SmallDesc d = desc[on ? fi : 0];
+  const int L = on ? d.L : 0, W = on ? d.W : 0;
+  const int64_t fc0 = d.fc0;
+  const bool own = r < W;
+  const int64_t idx = r < L ? (int64_t)s.lindx[d.ind + r] - 1 : 0;
+  // the row's entries: in its piece from lnz (columns L - cq apart), right of
+  // it from unz
+  const int pcol = own ? s.pcol[fc0 + r] : 0;
+  const int ce = pcol >> 16, ldp = L - (pcol & 0xffff);
+  const T* pl = lnz + (own ? s.lcol[fc0 + r] + r - (int64_t)r * ldp : 0);
+  const T* pu = unz + (own ? s.ucol[fc0 + r] : 0);
+  const int wm = -wave_min(-W), lm = -wave_min(-L);
+  T y = r < L ? rhs[(int64_t)q * ldr + idx] : T(0);
+  T v[SW], dg = T(1);
+  static_for<SW>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int j = decltype(jc)::value;
+    v[j] = T(0);
+    if (j < lm) {
+      const T* p = j >= ce ? pu + j : pl + (int64_t)(j * ldp);
+      if (own && j < L && j >= r) v[j] = *p;
+      if (j == r && own) dg = v[j];
+    }
+  });
+  const T ri = T(1) / dg;
+  static_for<SW>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int j = SW - 1 - decltype(jc)::value;
+    if (j < lm) {
+      const T yk = bcast<SW, j>(y);
+      if (j >= wm) {  // an update column of every front of the wave
+        const T t = y - v[j] * yk;
+        y = own && j < L ? t : y;
+      } else {
+        const T xk = bcast<SW, j>(div_r(y, dg, ri));
+        const T t = y - v[j] * (j >= W ? yk : xk);
+        if (j >= W)
+          y = own && j < L ? t : y;
+        else
+          y = yk == T(0) ? y : r < j ? t : r == j ? xk : y;
+      }
+    }
+  });
+  if (own) rhs[(int64_t)q * ldr + fc0 + r] = y;
+}
+
+// More than four right-hand sides: lanes (q, g) of QL right-hand sides and G
+// = 64 / QL rows, rows g + G i of the vectors in register i, the front's L or
+// U columns staged in LDS. A column's entry of every right-hand side is
+// broadcast at once (one ds_bpermute where the form above reads one lane per
+// right-hand side) and a division serves them all. Fronts of at most 32 rows
+// take one wave (16 x 4), larger ones a workgroup whose waves take four
+// right-hand sides each (4 x 16). The operations of each right-hand side are
+// those of the form above in its order. 32 sets of 32^3 with 16 right-hand
+// sides, forward and backward of one pass: 9.2 ms with the form above, 6.6
+// with this one (gathers of the scattered right-hand sides bound it now).
+template <typename T>
+__device__ inline T bperm(T v, int src) {
+  return __shfl(v, src, 64);
+}
+
+template <typename T, int QL, int NR>
+__device__ __attribute__((always_inline)) void fwd_small_many(
+    const DevSym& s, const SmallDesc& d, const SmallChild* __restrict__ child, int q0, int qstep,
+    const T* S, int LDL, T* X, const int64_t* __restrict__ ipvt, T* __restrict__ rhs, int64_t ldr,
+    int nrhs, T* __restrict__ vec) {
+  constexpr int G = 64 / QL;
+  const int lane = threadIdx.x % 64, ql = lane % QL, g = lane / QL;
+  const int L = d.L, W = d.W;
+  const int64_t fc0 = d.fc0;
+  const bool own = lane < W;
+  const int pcol = own ? s.pcol[fc0 + lane] : 0;
+  const int cq = pcol & 0xffff, ce = pcol >> 16;
+  const int kp = own ? (int)ipvt[fc0 + lane] - 1 + cq : lane;
+  const unsigned long long swaps = __ballot(own && kp != lane);
+  for (; q0 < nrhs; q0 += qstep) {
+    const int q = q0 + ql;
+    const bool on = q < nrhs;
+    T y[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int r = g + G * i;
+      y[i] = (on && r < W) ? rhs[(int64_t)q * ldr + fc0 + r] : T(0);
+    }
+    if (d.nch > 0) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) X[(g + G * i) * QL + ql] = y[i];
+      wave_lds_sync();
+      for (int ci = 0; ci < d.nch; ++ci) {
+        const SmallChild c = child[d.ch0 + ci];
+        const T* uc = vec + c.fvec * nrhs + (int64_t)q * c.L + (c.L - c.R);
+        T v[NR];
+        int rr[NR];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+          const int t = g + G * i;
+          const bool in = on && t < c.R;
+          v[i] = in ? uc[t] : T(0);
+          rr[i] = in ? s.relmap[c.rel + t] : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+          if (on && g + G * i < c.R) X[rr[i] * QL + ql] += v[i];
+        wave_lds_sync();
+      }
+#pragma unroll
+      for (int i = 0; i < NR; ++i) y[i] = X[(g + G * i) * QL + ql];
+      wave_lds_sync();
+    }
+    static_for<NR>([&](auto jc) __attribute__((always_inline)) {
+      constexpr int jb = decltype(jc)::value;
+#pragma unroll 1
+      for (int gg = 0; gg < G && G * jb + gg < W; ++gg) {
+        const int j = G * jb + gg;
+        const int jce = __builtin_amdgcn_readlane(ce, j);
+        if (swaps && __builtin_amdgcn_readlane(cq, j) == j) {  // a piece begins
+          unsigned long long m = swaps & (~0ull << j) & (jce < 64 ? (1ull << jce) - 1 : ~0ull);
+          if (m) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) X[(g + G * i) * QL + ql] = y[i];
+            wave_lds_sync();
+            while (m) {
+              const int k = __ffsll((long long)m) - 1, p = __builtin_amdgcn_readlane(kp, k);
+              m &= m - 1;
+              if (g == 0) {
+                const T t = X[k * QL + ql];
+                X[k * QL + ql] = X[p * QL + ql];
+                X[p * QL + ql] = t;
+              }
+              wave_lds_sync();
+            }
+#pragma unroll
+            for (int i = 0; i < NR; ++i) y[i] = X[(g + G * i) * QL + ql];
+            wave_lds_sync();
+          }
+        }
+        T l[NR];
+#pragma unroll
+        for (int i = jb; i < NR; ++i) l[i] = S[j * LDL + min(g + G * i, L - 1)];
+        const T yk = bperm(y[jb], gg * QL + ql);
+#pragma unroll
+        for (int i = jb; i < NR; ++i) {
+          const int r = g + G * i;
+          const T t = y[i] - l[i] * yk;
+          y[i] = (r > j && r < L && (yk != T(0) || r >= jce)) ? t : y[i];
+        }
+      }
+    });
+    T* yg = vec + d.fvec * nrhs + (int64_t)q * L;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int r = g + G * i;
+      if (on && r < W)
+        rhs[(int64_t)q * ldr + fc0 + r] = y[i];
+      else if (on && r < L)
+        yg[r] = y[i];
+    }
+  }
+}
+
+template <typename T, int QL, int NR>
+__device__ __attribute__((always_inline)) void bwd_small_many(
+    const DevSym& s, const SmallDesc& d, int q0, int qstep, const T* S, int LDW,
+    T* __restrict__ rhs, int64_t ldr, int nrhs) {
+  constexpr int G = 64 / QL;
+  const int lane = threadIdx.x % 64, ql = lane % QL, g = lane / QL;
+  const int L = d.L, W = d.W;
+  const T dg = lane < W ? S[lane * LDW + lane] : T(1);
+  const T ri = T(1) / dg;
+  for (; q0 < nrhs; q0 += qstep) {
+    const int q = q0 + ql;
+    const bool on = q < nrhs;
+    T y[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int r = g + G * i;
+      y[i] = (on && r < L) ? rhs[(int64_t)q * ldr + s.lindx[d.ind + r] - 1] : T(0);
+    }
+    T u[NR];  // the column's rows, read one column ahead
+    auto column = [&](int j) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        u[i] = G * i < W ? S[max(j, 0) * LDW + min(g + G * i, W - 1)] : T(0);
+    };
+    column(L - 1);
+    static_for<NR>([&](auto jc) __attribute__((always_inline)) {
+      constexpr int jb = NR - 1 - decltype(jc)::value;
+#pragma unroll 1
+      for (int gg = min(G, L - G * jb) - 1; gg >= 0; --gg) {
+        const int j = G * jb + gg;
+        const T yk = bperm(y[jb], gg * QL + ql);
+        T c[NR];
+#pragma unroll
+        for (int i = 0; i <= jb; ++i) c[i] = u[i];
+        column(j - 1);
+        if (j >= W) {
+#pragma unroll
+          for (int i = 0; i <= jb; ++i) {
+            const T t = y[i] - c[i] * yk;
+            y[i] = g + G * i < W ? t : y[i];
+          }
+        } else {
+          const T xk = div_r(yk, rdlane(dg, j), rdlane(ri, j));
+          const bool nz = yk != T(0);  // a zero entry stays, as in the reference
+#pragma unroll
+          for (int i = 0; i <= jb; ++i) {
+            const int r = g + G * i;
+            const T t = y[i] - c[i] * xk;
+            y[i] = nz && r < j ? t : nz && r == j ? xk : y[i];
+          }
+        }
+      }
+    });
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      if (on && g + G * i < W) rhs[(int64_t)q * ldr + d.fc0 + g + G * i] = y[i];
+  }
+}
+
+// The front's L columns in LDS, S[j LDL + r] for r > j, by G threads.
+template <typename T, int G>
+__device__ __attribute__((always_inline)) void stage_small_l(const DevSym& s, const SmallDesc& d,
+                                                             T* S, int LDL,
+                                                             const T* __restrict__ lnz) {
+  constexpr int NW = G / 64, CH = 8;
+  const int lane = threadIdx.x % 64;
+  const int w = G == kWG ? wave_id() : 0;
+  const int64_t lcb = lane < d.W ? s.lcol[d.fc0 + lane] : 0;
+  for (int i0 = w * CH; i0 < d.W; i0 += NW * CH) {
+    T a[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int i = min(i0 + u, 63);
+      const T* l = lnz + rdlane_i64(lcb, i);
+      a[u] = (i0 + u < d.W && lane > i && lane < d.L) ? l[lane] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+      if (i0 + u < d.W && lane < d.L) S[(i0 + u) * LDL + lane] = a[u];
+  }
+}
+
+template <typename T, int QW>
+__global__ void __launch_bounds__(kWG)
+fwd_small_kernel(DevSym s, const SmallDesc* __restrict__ desc,
+                 const SmallChild* __restrict__ child, SmallClasses k, int LDL, int slot,
+                 const T* __restrict__ lnz, const int64_t* __restrict__ ipvt,
+                 T* __restrict__ rhs, int64_t ldr, int nrhs, T* __restrict__ vec) {
+  const int64_t vs = blockIdx.y;  // value set
+  int b = blockIdx.x;
+  lnz += vs * s.vs_lnz;
+  ipvt += vs * s.n;
+  rhs += vs * ldr * nrhs;
+  vec += vs * s.vs_vec * nrhs;
+  const int wave = wave_id();
+  if constexpr (QW > 4) {
+    extern __shared__ unsigned char smem_raw[];
+    T* S = reinterpret_cast<T*>(smem_raw);
+    __shared__ T X[4][512];
+    if (b < k.cnt[0]) {
+      const SmallDesc d = desc[b];
+      stage_small_l<T, kWG>(s, d, S, LDL, lnz);
+      __syncthreads();
+      fwd_small_many<T, 4, 4>(s, d, child, wave * 4, 16, S, LDL, X[wave], ipvt, rhs, ldr, nrhs,
+                              vec);
+      return;
+    }
+    const int item = (b - k.cnt[0]) * 4 + wave;
+    if (item >= k.cnt[1]) return;
+    const SmallDesc d = desc[k.cnt[0] + item];
+    S += wave * slot;
+    LDL = min(LDL, 33);
+    stage_small_l<T, 64>(s, d, S, LDL, lnz);
+    wave_lds_sync();
+    fwd_small_many<T, 16, 8>(s, d, child, 0, 16, S, LDL, X[wave], ipvt, rhs, ldr, nrhs, vec);
+  } else {
+    __shared__ T Y[4][QW * 64];
+    if (b < k.cnt[0]) {
+      fwd_small_wave<T, 1>(s, desc[b], child, wave, 4, Y[wave], lnz, ipvt, rhs, ldr, nrhs, vec);
+      return;
+    }
+    b -= k.cnt[0];
+    desc += k.cnt[0];
+    if (b < k.wg1) {
+      const int item = b * 4 + wave;
+      if (item < k.cnt[1])
+        fwd_small_wave<T, QW>(s, desc[item], child, 0, QW, Y[wave], lnz, ipvt, rhs, ldr, nrhs, vec);
+      return;
+    }
+    b -= k.wg1;
+    desc += k.cnt[1];
+    if (b < k.wg2) {
+      fwd_tiny<T, 16>(s, desc, child, ((int64_t)b * 4 + wave) * 4, k.cnt[2], Y[wave], lnz, ipvt, rhs, ldr,
+                      nrhs, vec);
+      return;
+    }
+    b -= k.wg2;
+    desc += k.cnt[2];
+    fwd_tiny<T, 8>(s, desc, child, ((int64_t)b * 4 + wave) * 8, k.cnt[3], Y[wave], lnz, ipvt, rhs, ldr, nrhs,
+                   vec);
+  }
+}
+
+// The front's U rows by columns in LDS, S[j LDW + c] = U(c, j) for c <= j:
+// the pieces' blocks from the packed LU in lnz (rows contiguous), the
+// columns right of them from unz (columns contiguous), by G threads.
+template <typename T, int G>
+__device__ __attribute__((always_inline)) void stage_small_u(
+    const DevSym& s, const SmallDesc& d, T* S, int LDW, const T* __restrict__ lnz,
+    const T* __restrict__ unz) {
+  constexpr int NW = G / 64, CH = 8;
+  const int lane = threadIdx.x % 64;
+  const int w = G == kWG ? wave_id() : 0;
+  const int L = d.L, W = d.W;
+  const int64_t fc0 = d.fc0;
+  const bool own = lane < W;
+  const int64_t lcb = own ? s.lcol[fc0 + lane] : 0;
+  const int64_t ucb = own ? s.ucol[fc0 + lane] : 0;
+  const int pcol = own ? s.pcol[fc0 + lane] : 0;
+  for (int i0 = w * CH; i0 < W; i0 += NW * CH) {
+    T a[CH], b[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int i = min(i0 + u, 63);
+      const bool on = i0 + u < W;
+      const int pc = __builtin_amdgcn_readlane(pcol, i);
+      const T* l = lnz + rdlane_i64(lcb, i);  // column i, lane = row
+      const T* r = unz + rdlane_i64(ucb, i);  // row i, lane = column
+      a[u] = (on && lane >= (pc & 0xffff) && lane <= i) ? l[lane] : T(0);
+      b[u] = (on && lane >= (pc >> 16) && lane < L) ? r[lane] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int i = min(i0 + u, 63);
+      const bool on = i0 + u < W;
+      const int pc = __builtin_amdgcn_readlane(pcol, i);
+      if (on && lane >= (pc & 0xffff) && lane <= i) S[i * LDW + lane] = a[u];
+      if (on && lane >= (pc >> 16) && lane < L) S[lane * LDW + i] = b[u];
+    }
+  }
+}
+
+// Backward, one wave (right-hand sides as in fwd_small_wave): x gathered
+// through the index list, then the columns last to first: an own column's
+// entry is divided by U(j, j) and the rows above subtract their products
+// (gtrsm! 'l','u','n','n' and the U12 products by columns).
+template <typename T, int QB>
+__device__ __attribute__((always_inline)) void bwd_small_wave(
+    const DevSym& s, const SmallDesc& d, int q0, int qstep, const T* S, int LDW,
+    T* __restrict__ rhs, int64_t ldr, int nrhs) {
+  const int lane = threadIdx.x % 64;
+  const int L = d.L, W = d.W;
+  const bool own = lane < W;
+  const int64_t idx = lane < L ? (int64_t)s.lindx[d.ind + lane] - 1 : 0;
+  const T dg = own ? S[lane * LDW + lane] : T(1);
+  const T ri = T(1) / dg;
+  const int cl = min(lane, W - 1);
+  for (; q0 < nrhs; q0 += qstep) {
+    const int nq = min(QB, nrhs - q0);
+    T y[QB];
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
+      y[q] = T(0);
+      if (q < nq && lane < L) y[q] = rhs[(int64_t)(q0 + q) * ldr + idx];
+    }
+    constexpr int CH = 4;  // columns read ahead
+    T sv[CH];
+    auto columns = [&](int j0) {
+#pragma unroll
+      for (int u = 0; u < CH; ++u) sv[u] = S[max(j0 - u, 0) * LDW + cl];
+    };
+    columns(L - 1);
+    for (int j0 = L - 1; j0 >= 0; j0 -= CH) {
+      T c[CH];
+#pragma unroll
+      for (int u = 0; u < CH; ++u) c[u] = sv[u];
+      if (j0 >= CH) columns(j0 - CH);
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int j = j0 - u;
+        if (j < 0) break;
+        if (j >= W) {
+#pragma unroll
+          for (int q = 0; q < QB; ++q)
+            if (q < nq) {
+              const T xk = rdlane(y[q], j);
+              const T t = y[q] - c[u] * xk;
+              y[q] = own ? t : y[q];
+            }
+        } else {
+#pragma unroll
+          for (int q = 0; q < QB; ++q)
+            if (q < nq) {
+              const T xq = div_r(y[q], dg, ri);
+              const T yk = rdlane(y[q], j), xk = rdlane(xq, j);
+              if (yk != T(0)) {  // a zero entry stays, as in the reference
+                const T t = y[q] - c[u] * xk;
+                y[q] = lane < j ? t : lane == j ? xk : y[q];
+              }
+            }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < QB; ++q)
+      if (q < nq && own) rhs[(int64_t)(q0 + q) * ldr + d.fc0 + lane] = y[q];
+  }
+}
+
+template <typename T, int QW>
+__global__ void __launch_bounds__(kWG)
+bwd_small_kernel(DevSym s, const SmallDesc* __restrict__ desc, SmallClasses k, int LDW,
+                 int slot, const T* __restrict__ lnz, const T* __restrict__ unz,
+                 T* __restrict__ rhs, int64_t ldr, int nrhs) {
+  const int64_t vs = blockIdx.y;  // value set
+  int b = blockIdx.x;
+  lnz += vs * s.vs_lnz;
+  unz += vs * s.vs_unz;
+  rhs += vs * ldr * nrhs;
+  extern __shared__ unsigned char smem_raw[];
+  T* S = reinterpret_cast<T*>(smem_raw);
+  const int wave = wave_id();
+  if (b < k.cnt[0]) {
+    const SmallDesc d = desc[b];
+    stage_small_u<T, kWG>(s, d, S, LDW, lnz, unz);
+    __syncthreads();
+    if constexpr (QW > 4)
+      bwd_small_many<T, 4, 4>(s, d, wave * 4, 16, S, LDW, rhs, ldr, nrhs);
+    else
+      bwd_small_wave<T, 1>(s, d, wave, 4, S, LDW, rhs, ldr, nrhs);
+    return;
+  }
+  b -= k.cnt[0];
+  desc += k.cnt[0];
+  if (b < k.wg1) {
+    const int item = b * 4 + wave;
+    if (item >= k.cnt[1]) return;
+    const SmallDesc d = desc[item];
+    S += wave * slot;
+    LDW = min(LDW, 33);
+    stage_small_u<T, 64>(s, d, S, LDW, lnz, unz);
+    wave_lds_sync();
+    if constexpr (QW > 4)
+      bwd_small_many<T, 16, 8>(s, d, 0, 16, S, LDW, rhs, ldr, nrhs);
+    else
+      bwd_small_wave<T, QW>(s, d, 0, QW, S, LDW, rhs, ldr, nrhs);
+    return;
+  }
+  if constexpr (QW <= 4) {
+    b -= k.wg1;
+    desc += k.cnt[1];
+    if (b < k.wg2) {
+      bwd_tiny<T, 16>(s, desc, ((int64_t)b * 4 + wave) * 4, k.cnt[2], lnz, unz, rhs, ldr, nrhs);
+      return;
+    }
+    b -= k.wg2;
+    desc += k.cnt[2];
+    bwd_tiny<T, 8>(s, desc, ((int64_t)b * 4 + wave) * 8, k.cnt[3], lnz, unz, rhs, ldr, nrhs);
+  }
+}
+
 
 // Backward chain of one block. The block's upper panels and diagonal
 // reciprocals come from the solve data in one coalesced load. With t =
