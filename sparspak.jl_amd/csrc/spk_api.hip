@@ -1463,6 +1463,14 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
   DevBuf<T>& prep = Bufs<T>::prep(h);
   const bool inv = inv_solve<T>(nrhs);
   solve_prep<T>(h, inv);
+  // right-hand sides of the per-row kernels and, four at a time, of the
+  // chains take workgroups of their own, the chains while the launch has
+  // fewer than four per CU (each stages its block's panels anew)
+  const unsigned qz = (unsigned)std::min(nrhs, 16);
+  auto chain_z = [&](const LevelPlan::SolveStep& S) {
+    const i64 wg = std::max<i64>((i64)S.chain_cnt * h->nvs, 1);
+    return (unsigned)std::max<i64>(1, std::min<i64>((nrhs + 3) / 4, 1024 / wg));
+  };
   if (fwd)
     for (const LevelPlan& lp : h->levels) {
       h->cur_level = (int)(&lp - h->levels.data());
@@ -1493,7 +1501,8 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
       {
         Prof pr(h, SPKHIP_K_FWD, 0.0, 0.0);
         hipLaunchKernelGGL(spk::fwd_assemble_items_kernel<T>,
-                           dim3((lp.items_cnt + kWG - 1) / kWG, h->nvs), dim3(kWG), 0, st, h->ds,
+                           dim3((lp.items_cnt + kWG - 1) / kWG, h->nvs, qz), dim3(kWG), 0, st,
+                           h->ds,
                            h->d_it_front.p + lp.items_off, h->d_it_col.p + lp.items_off,
                            h->d_it_ea.p + lp.items_off, h->d_ea_child.p, h->d_ea_t.p, rhs, ldr,
                            nrhs, vecp, lp.items_cnt);
@@ -1515,7 +1524,7 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
       for (const LevelPlan::SolveStep& S : lp.fsteps) {
         {
           Prof pr(h, SPKHIP_K_FWD, 0.0, 0.0);
-          hipLaunchKernelGGL((spk::fwd_chain_kernel<T>), dim3(S.chain_cnt, h->nvs), dim3(kWG),
+          hipLaunchKernelGGL((spk::fwd_chain_kernel<T>), dim3(S.chain_cnt, h->nvs, chain_z(S)), dim3(kWG),
                              (size_t)spk::kPanelElems * sizeof(T), st, h->ds,
                              h->d_sdesc.p + S.chain_off, prep.p, h->d_prepi.p, rhs, ldr, nrhs,
                              vecp);
@@ -1523,8 +1532,14 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
         }
         if (S.gemv_cnt > 0) {
           Prof pr(h, SPKHIP_K_FWD_GEMV, 2.0 * S.elems * nrhs, S.elems * sizeof(T));
-          hipLaunchKernelGGL(spk::fwd_bgemv_kernel<T>, dim3(S.gemv_cnt, h->nvs), dim3(kWG), 0, st, h->ds,
-                             h->d_sdesc.p + S.gemv_off, lnz, nrhs, vecp);
+          auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(S.gemv_cnt, h->nvs), dim3(kWG), 0, st, h->ds,
+                               h->d_sdesc.p + S.gemv_off, lnz, nrhs, vecp);
+          };
+          if (nrhs == 1)
+            go(spk::fwd_bgemv_kernel<T, 1>);
+          else
+            go(spk::fwd_bgemv_kernel<T, 8>);
           hipck(hipGetLastError());
         }
       }
@@ -1536,8 +1551,10 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
       h->cur_grid = lp.large_cnt;
       if (lp.large_cnt > 0) {
         Prof pr(h, SPKHIP_K_BWD, 0.0, 0.0);
+        const unsigned gz = (i64)lp.items_cnt * h->nvs < 1 << 18 ? qz : 1;
         hipLaunchKernelGGL(spk::bwd_gather_items_kernel<T>,
-                           dim3((lp.items_cnt + kWG - 1) / kWG, h->nvs), dim3(kWG), 0, st, h->ds,
+                           dim3((lp.items_cnt + kWG - 1) / kWG, h->nvs, gz), dim3(kWG), 0, st,
+                           h->ds,
                            h->d_it_front.p + lp.items_off, h->d_it_col.p + lp.items_off, rhs,
                            ldr, nrhs, vecp, lp.items_cnt);
         hipck(hipGetLastError());
@@ -1566,16 +1583,21 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
         if (done) break;
         if (S.gemv_cnt > 0) {
           Prof pr(h, SPKHIP_K_BWD_GEMV, 2.0 * S.elems * nrhs, S.elems * sizeof(T));
-          // a workgroup per row, or four rows per workgroup when the launch
-          // would otherwise hold more than 16384 workgroups (same results)
-          const int rows = (i64)S.gemv_cnt * h->nvs > 16384 ? 4 : 1;
-          hipLaunchKernelGGL(spk::bwd_bgemv_kernel<T>, dim3((S.gemv_cnt + rows - 1) / rows, h->nvs),
-                             dim3(kWG), 0, st, h->ds, h->d_sdesc.p + S.gemv_off, S.gemv_cnt, rows,
-                             unz, nrhs, vecp);
+          // a workgroup per row, or eight rows of it per workgroup where that
+          // still leaves four workgroups per CU (the same results)
+          auto go = [&](auto kern, int rows) {
+            hipLaunchKernelGGL(kern, dim3((S.gemv_cnt + rows - 1) / rows, h->nvs), dim3(kWG), 0,
+                               st, h->ds, h->d_sdesc.p + S.gemv_off, S.gemv_cnt, unz, nrhs, vecp);
+          };
+          const bool many = (i64)S.gemv_cnt * h->nvs >= 8 * 1024;
+          if (nrhs == 1)
+            many ? go(spk::bwd_bgemv_kernel<T, 8, 1>, 8) : go(spk::bwd_bgemv_kernel<T, 1, 1>, 1);
+          else
+            many ? go(spk::bwd_bgemv_kernel<T, 8, 8>, 8) : go(spk::bwd_bgemv_kernel<T, 1, 16>, 1);
           hipck(hipGetLastError());
         }
         Prof pr(h, SPKHIP_K_BWD, 0.0, 0.0);
-        hipLaunchKernelGGL((spk::bwd_chain_kernel<T>), dim3(S.chain_cnt, h->nvs), dim3(kWG),
+        hipLaunchKernelGGL((spk::bwd_chain_kernel<T>), dim3(S.chain_cnt, h->nvs, chain_z(S)), dim3(kWG),
                            (size_t)(spk::kPanelElems + 128) * sizeof(T), st, h->ds,
                            h->d_sdesc.p + S.chain_off, prep.p, rhs, ldr, nrhs, vecp);
         hipck(hipGetLastError());

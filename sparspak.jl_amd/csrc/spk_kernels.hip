@@ -2510,7 +2510,7 @@ fwd_assemble_items_kernel(DevSym s, const int32_t* __restrict__ it_front,
   const int L = s.fL[f], W = s.fW[f];
   const int64_t fc0 = s.fc0[f];
   const int64_t e0 = it_ea[item], e1 = it_ea[item + 1];
-  for (int q = 0; q < nrhs; ++q) {
+  for (int q = blockIdx.z; q < nrhs; q += gridDim.z) {
     T y = (r < W) ? rhs[(int64_t)q * ldr + fc0 + r] : T(0);
     for (int64_t e = e0; e < e1; ++e) {
       const int c = ea_child[e], t = ea_t[e];
@@ -2537,7 +2537,7 @@ bwd_gather_items_kernel(DevSym s, const int32_t* __restrict__ it_front,
   const int L = s.fL[f], W = s.fW[f];
   if (j < W) return;
   const int g = s.lindx[s.xlindx[s.fsp0[f]] - 1 + j] - 1;
-  for (int q = 0; q < nrhs; ++q)
+  for (int q = blockIdx.z; q < nrhs; q += gridDim.z)
     vec[s.fvec[f] * nrhs + (int64_t)q * L + j] = rhs[(int64_t)q * ldr + g];
 }
 
@@ -2716,7 +2716,9 @@ __device__ __attribute__((always_inline)) void fwd_chain_body(
   using V = typename Vec4<T>::type;
   V* smem_v4 = reinterpret_cast<V*>(smem_a32);
   const T* R = reinterpret_cast<const T*>(smem_a32);
-  const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
+  const int tid = threadIdx.x, lane = tid % 64;
+  // wave w takes right-hand sides w, w + 4, ..., spread over the z workgroups
+  const int wave = wave_id() + 4 * (int)blockIdx.z, qstep = 4 * (int)gridDim.z;
   const int f = d.front;
   const int L = d.L;
   const int64_t fc0 = d.fc0;
@@ -2756,7 +2758,7 @@ __device__ __attribute__((always_inline)) void fwd_chain_body(
     if (both) o.a = *(const V*)(P + 4 * (min(max(lane, k), bwp - 1) - k));
     o.b = *(const V*)(P + 4 * (min(max(lane + 64, k), bwp - 1) - k));
   };
-  for (int q = wave; q < nrhs; q += 4) {
+  for (int q = wave; q < nrhs; q += qstep) {
     T* yg = vec + d.fvec * nrhs + (int64_t)q * L;
     T* x = rhs + (int64_t)q * ldr;
     if (q > wave) {
@@ -2831,144 +2833,197 @@ fwd_chain_kernel(DevSym s, const SolveDesc* __restrict__ desc, const T* __restri
 // quarter of the block's columns, partial sums added in a fixed order. The
 // block's column offsets and y[c0:c1] are staged in LDS first, then every
 // thread issues all of its L loads at once.
-template <typename T>
+template <typename T, int QB>
 __device__ __attribute__((always_inline)) void fwd_bgemv_body(
     const DevSym& s, const SolveDesc& d, const T* __restrict__ lnz, int nrhs,
     T* __restrict__ vec) {
-  __shared__ T red[4][64];
+  __shared__ T red[4][QB][64];
   __shared__ int64_t lc[128];
-  __shared__ T zs[128];
+  __shared__ __attribute__((aligned(16))) T zs[QB][4][32];  // a quarter's entries, zeros behind
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int f = d.front;
   const int L = d.L;
   const int64_t fc0 = d.fc0;
   const int c0 = d.c0, c1 = d.c1, bw = c1 - c0;
   const int r = c1 + d.r0 + lane;
   const int cb = bw * wave / 4, ce = bw * (wave + 1) / 4;  // at most 32 columns
+  // (quarter, entry) this thread stages of a right-hand side's y[c0:c1]
+  const int zw = tid % 128 / 32, zj = tid % 32;
+  const int zc = bw * zw / 4 + zj;
+  const bool zin = zc < bw * (zw + 1) / 4;
   if (tid < bw) lc[tid] = s.lcol[fc0 + c0 + tid];
   __syncthreads();
   // the block's entries of this tile's rows, read once for every rhs
   T lv[32];
 #pragma unroll
   for (int j = 0; j < 32; ++j) lv[j] = (r < L && cb + j < ce) ? lnz[lc[cb + j] + r] : T(0);
-  for (int q = 0; q < nrhs; ++q) {
-    T* yg = vec + d.fvec * nrhs + (int64_t)q * L;
-    if (tid < bw) zs[tid] = yg[c0 + tid];
-    // this tile's rows of y (no other workgroup touches them)
-    const T yr = (wave == 0 && r < L) ? yg[r] : T(0);
-    __syncthreads();
-    T acc = T(0);
-    if (r < L) {
+  for (int q0 = 0; q0 < nrhs; q0 += QB) {
+    const int nq = min(QB, nrhs - q0);
+    T* yv = vec + d.fvec * nrhs + (int64_t)q0 * L;
+    if constexpr (QB == 1) {
+      if (tid < 128) zs[0][zw][zj] = zin ? yv[c0 + zc] : T(0);
+    } else {
 #pragma unroll
-      for (int j = 0; j < 32; ++j)
-        if (cb + j < ce) acc += lv[j] * zs[cb + j];
+      for (int i = 0; i < QB / 2; ++i) {
+        const int q = 2 * i + tid / 128;
+        if (q < nq) zs[q][zw][zj] = zin ? yv[(int64_t)q * L + c0 + zc] : T(0);
+      }
     }
-    red[wave][lane] = acc;
+    // wave w ends right-hand sides w, w + 4, ...: this tile's rows of their y
+    // (no other workgroup touches them)
+    T yr[(QB + 3) / 4];
+#pragma unroll
+    for (int i = 0; i < (QB + 3) / 4; ++i)
+      yr[i] = (wave + 4 * i < nq && r < L) ? yv[(int64_t)(wave + 4 * i) * L + r] : T(0);
     __syncthreads();
-    if (wave == 0 && r < L) yg[r] = yr - (((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
+      if (q < nq) {
+        T acc = T(0);
+#pragma unroll
+        for (int j = 0; j < 32; ++j) acc += lv[j] * zs[q][wave][j];
+        red[wave][q][lane] = acc;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (QB + 3) / 4; ++i) {
+      const int q = wave + 4 * i;
+      if (q < nq && r < L)
+        yv[(int64_t)q * L + r] =
+            yr[i] - (((red[0][q][lane] + red[1][q][lane]) + red[2][q][lane]) + red[3][q][lane]);
+    }
     __syncthreads();
   }
 }
 
-
-template <typename T>
+// QB right-hand sides share the reads of the block and three barriers. The
+// block's y is read as whole vectors from LDS (its quarters padded to 32
+// entries): single reads were what bounded the launch. 56 x 48 x 41, one
+// right-hand side, double: 6.7 -> 5.5 us a launch; 32 sets of 32^3, 16
+// right-hand sides: 39 -> 23 us (33 us with the shared barriers alone).
+template <typename T, int QB>
 __global__ void __launch_bounds__(kWG)
 fwd_bgemv_kernel(DevSym s, const SolveDesc* __restrict__ desc, const T* __restrict__ lnz,
                  int nrhs, T* __restrict__ vec) {
   const int64_t vs = blockIdx.y;  // value set
   lnz += vs * s.vs_lnz;
   vec += vs * s.vs_vec * nrhs;
-  fwd_bgemv_body<T>(s, desc[blockIdx.x], lnz, nrhs, vec);
+  fwd_bgemv_body<T, QB>(s, desc[blockIdx.x], lnz, nrhs, vec);
 }
 
-// Backward: t[c] = U[c, c1:L] x[c1:L] for row c = c0 + r0 of the block (a
-// workgroup takes one or a few rows in turn), stored in y[c]. x[c1:L] is read from the front's vector:
-// its update rows from bwd_gather_items_kernel, its own columns as the backward
-// chains of the later blocks left them. Every thread takes columns c1 + tid
-// + 256 m, sixteen loads in flight; per-thread sums are added over the wave,
-// then the four waves in a fixed order.
-template <typename T>
-__device__ __attribute__((always_inline)) void bwd_bgemv_body(
-    const DevSym& s, const SolveDesc& d, const T* __restrict__ unz, int nrhs,
-    T* __restrict__ vec) {
-  constexpr int QB = 16;  // right-hand sides sharing one read of the row
-  constexpr int CH = 16;  // columns per thread and pass
-  __shared__ T red[QB][4];
-  const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
-  const int f = d.front;
-  const int c = d.c0 + d.r0;
-  const int L = d.L;
-  const int64_t fc0 = d.fc0;
-  const T* u = unz + d.ucol;  // the row's U entries (its unz offset rides in the descriptor)
-  for (int q0 = 0; q0 < nrhs; q0 += QB) {
-    const int nq = min(QB, nrhs - q0);
-    T acc[QB];
+// One level of a sum over the wave's lanes, lane l with lane l ^ OFF, of two
+// values at once: the lanes whose bit OFF is clear get a's sum, the others
+// b's (a = b: all get a's).
+template <int OFF>
+__device__ inline unsigned lane_xor_mov(unsigned v) {  // OFF 8, 4, 2, 1
+  const int x = (int)v;
+  if constexpr (OFF == 8) return (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x128, 0xf, 0xf, false);
+  if constexpr (OFF == 4) {
+    const int up = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0x5, false);  // row_shl:4
+    return (unsigned)__builtin_amdgcn_update_dpp(up, x, 0x114, 0xf, 0xa, false);  // row_shr:4
+  }
+  return (unsigned)__builtin_amdgcn_update_dpp(x, x, OFF == 2 ? 0x4E : 0xB1, 0xf, 0xf, false);
+}
+template <int OFF>
+__device__ inline float lane_xor(float v) {
+  return __uint_as_float(lane_xor_mov<OFF>(__float_as_uint(v)));
+}
+template <int OFF>
+__device__ inline double lane_xor(double v) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = lane_xor_mov<OFF>((unsigned)x), hi = lane_xor_mov<OFF>((unsigned)(x >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// a and b with a's upper half-wave (OFF 32) or odd rows of 16 (OFF 16)
+// exchanged for b's lower half-wave or even rows
+template <int OFF>
+__device__ inline void swap_lanes(unsigned& a, unsigned& b) {
+  if constexpr (OFF == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0], b = r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+  }
+}
+template <int OFF>
+__device__ inline float tree_step(float a, float b, bool up) {
+  if constexpr (OFF >= 16) {
+    unsigned x = __float_as_uint(a), y = __float_as_uint(b);
+    swap_lanes<OFF>(x, y);
+    return __uint_as_float(x) + __uint_as_float(y);
+  } else {
+    return (up ? b : a) + lane_xor<OFF>(up ? a : b);
+  }
+}
+template <int OFF>
+__device__ inline double tree_step(double a, double b, bool up) {
+  if constexpr (OFF >= 16) {
+    const unsigned long long p = (unsigned long long)__double_as_longlong(a);
+    const unsigned long long q = (unsigned long long)__double_as_longlong(b);
+    unsigned x0 = (unsigned)p, y0 = (unsigned)q, x1 = (unsigned)(p >> 32), y1 = (unsigned)(q >> 32);
+    swap_lanes<OFF>(x0, y0);
+    swap_lanes<OFF>(x1, y1);
+    return __longlong_as_double((long long)(((unsigned long long)x1 << 32) | x0)) +
+           __longlong_as_double((long long)(((unsigned long long)y1 << 32) | y0));
+  } else {
+    return (up ? b : a) + lane_xor<OFF>(up ? a : b);
+  }
+}
+// Sums over the wave of NV values (a power of two, at most 64): lane l
+// returns value l NV / 64's, added in the order of a tree over the lanes 32,
+// 16, ..., 1 apart. The values halve as the lanes of each sum do, about two
+// operations per value; six ds_bpermute each were most of the backward GEMV
+// of many right-hand sides (16, 32 sets of 32^3: 12.2 ms a pass, now 8.5).
+template <int NV, int OFF = 32, typename T>
+__device__ __attribute__((always_inline)) inline T wave_sums(T (&v)[NV], int lane) {
+  const bool up = (lane & OFF) != 0;
+  if constexpr (NV == 1) {
+    v[0] = tree_step<OFF>(v[0], v[0], up);
+    if constexpr (OFF == 1)
+      return v[0];
+    else
+      return wave_sums<1, OFF / 2>(v, lane);
+  } else {
+    T w[NV / 2];
 #pragma unroll
-    for (int qq = 0; qq < QB; ++qq) acc[qq] = T(0);
-    for (int j0 = d.c1 + tid; j0 < L; j0 += CH * kWG) {
-      T uv[CH];
-#pragma unroll
-      for (int t = 0; t < CH; ++t) {
-        const int j = j0 + kWG * t;
-        uv[t] = (j < L) ? u[j] : T(0);
-      }
-#pragma unroll
-      for (int qq = 0; qq < QB; ++qq) {
-        if (qq < nq) {
-          const T* yg = vec + d.fvec * nrhs + (int64_t)(q0 + qq) * L;
-          T xv[CH];
-#pragma unroll
-          for (int t = 0; t < CH; ++t) {
-            const int j = j0 + kWG * t;
-            xv[t] = (j < L) ? yg[j] : T(0);
-          }
-#pragma unroll
-          for (int t = 0; t < CH; ++t) acc[qq] += uv[t] * xv[t];
-        }
-      }
-    }
-#pragma unroll
-    for (int qq = 0; qq < QB; ++qq) {
-      if (qq < nq) {
-        T a = acc[qq];
-        for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
-        if (lane == 0) red[qq][wave] = a;
-      }
-    }
-    __syncthreads();
-    if (tid < nq) {
-      T* yg = vec + d.fvec * nrhs + (int64_t)(q0 + tid) * L;
-      yg[c] = ((red[tid][0] + red[tid][1]) + red[tid][2]) + red[tid][3];
-    }
-    __syncthreads();
+    for (int i = 0; i < NV / 2; ++i) w[i] = tree_step<OFF>(v[i], v[i + NV / 2], up);
+    if constexpr (OFF == 1)
+      return w[0];
+    else
+      return wave_sums<NV / 2, OFF / 2>(w, lane);
   }
 }
 
-// The same for R rows of one block of one front at once: every load of x
-// serves the R rows. Each (row, right-hand side) sum takes bwd_bgemv_body's
-// operations in its order (a thread's columns c1 + tid + 256 m in ascending
-// m, the wave tree, the four waves in order), so the results are the same.
-template <typename T, int R>
-__device__ __attribute__((always_inline)) void bwd_bgemv_rows_body(
-    const SolveDesc* __restrict__ dr, const T* __restrict__ unz, int nrhs, T* __restrict__ vec) {
-  constexpr int QB = 8;  // right-hand sides per pass
-  constexpr int CH = 8;  // columns per thread and chunk
-  __shared__ T red[R][QB][4];
+// Backward: t[c] = U[c, c1:L] x[c1:L] for rows c = c0 + r0 of the block,
+// stored in y[c]. x[c1:L] is read from the front's vector: its update rows
+// from bwd_gather_items_kernel, its own columns as the backward chains of the
+// later blocks left them. R rows of one block (n of them wanted) share the
+// loads of x, QB right-hand sides those of U: every thread takes columns c1 +
+// tid + 256 m of all of them, its sums are added over the wave (wave_sums),
+// then the four waves in order; a (row, right-hand side) sum does not depend
+// on R, QB or n.
+template <typename T, int R, int QB>
+__device__ __attribute__((always_inline)) void bwd_bgemv_body(
+    const SolveDesc* __restrict__ dr, int n, const T* __restrict__ unz, int nrhs,
+    T* __restrict__ vec) {
+  // columns per thread and pass: about 32 loads of U in flight
+  constexpr int CH = R == 1 ? 16 : R * (int)sizeof(T) > 32 ? 2 : 4;
+  constexpr int NV = R * QB;
+  __shared__ T red[4][NV];
   const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
-  const SolveDesc& d = dr[0];
+  const SolveDesc d = dr[0];
   const int L = d.L, c1 = d.c1;
   T* const yv = vec + d.fvec * nrhs;
   const T* u[R];
 #pragma unroll
-  for (int i = 0; i < R; ++i) u[i] = unz + dr[i].ucol;
+  for (int i = 0; i < R; ++i) u[i] = unz + dr[R == 1 ? 0 : min(i, n - 1)].ucol;
   for (int q0 = 0; q0 < nrhs; q0 += QB) {
     const int nq = min(QB, nrhs - q0);
-    T acc[R][QB];
+    T acc[NV];
 #pragma unroll
-    for (int i = 0; i < R; ++i)
-#pragma unroll
-      for (int qq = 0; qq < QB; ++qq) acc[i][qq] = T(0);
+    for (int i = 0; i < NV; ++i) acc[i] = T(0);
     for (int j0 = c1 + tid; j0 < L; j0 += CH * kWG) {
       T uv[R][CH];
 #pragma unroll
@@ -2991,53 +3046,37 @@ __device__ __attribute__((always_inline)) void bwd_bgemv_rows_body(
 #pragma unroll
           for (int i = 0; i < R; ++i)
 #pragma unroll
-            for (int t = 0; t < CH; ++t) acc[i][qq] += uv[i][t] * xv[t];
+            for (int t = 0; t < CH; ++t) acc[i * QB + qq] += uv[i][t] * xv[t];
         }
       }
     }
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-#pragma unroll
-      for (int qq = 0; qq < QB; ++qq) {
-        if (qq < nq) {
-          T a = acc[i][qq];
-          for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
-          if (lane == 0) red[i][qq][wave] = a;
-        }
-      }
+    const T sum = wave_sums<NV>(acc, lane);
+    if (lane % (64 / NV) == 0) red[wave][lane / (64 / NV)] = sum;
     __syncthreads();
-    if (tid < R * nq) {
-      const int i = tid / nq, qq = tid - i * nq;
-      yv[(int64_t)(q0 + qq) * L + dr[i].c0 + dr[i].r0] =
-          ((red[i][qq][0] + red[i][qq][1]) + red[i][qq][2]) + red[i][qq][3];
+    if (tid < NV) {
+      const int i = tid / QB, qq = tid % QB;
+      if (i < n && qq < nq)
+        yv[(int64_t)(q0 + qq) * L + dr[i].c0 + dr[i].r0] =
+            ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
     }
     __syncthreads();
   }
 }
 
-// rows: consecutive row descriptors per workgroup (1 or 4); four rows of one
-// block of one front share their loads of x, any other group is taken one
-// row after another (the results do not depend on the grouping)
-template <typename T>
+// R consecutive row descriptors per workgroup, in runs of rows of one block
+template <typename T, int R, int QB>
 __global__ void __launch_bounds__(kWG)
-bwd_bgemv_kernel(DevSym s, const SolveDesc* __restrict__ desc, int ndesc, int rows,
+bwd_bgemv_kernel(DevSym s, const SolveDesc* __restrict__ desc, int ndesc,
                  const T* __restrict__ unz, int nrhs, T* __restrict__ vec) {
   const int64_t vs = blockIdx.y;  // value set
   unz += vs * s.vs_unz;
   vec += vs * s.vs_vec * nrhs;
-  const int base = (int)blockIdx.x * rows;
-  if (rows == 4 && base + 3 < ndesc) {
-    const SolveDesc* dr = desc + base;
-    if (dr[1].front == dr[0].front && dr[2].front == dr[0].front && dr[3].front == dr[0].front &&
-        dr[3].c0 == dr[0].c0) {
-      bwd_bgemv_rows_body<T, 4>(dr, unz, nrhs, vec);
-      return;
-    }
-  }
-  for (int i = 0; i < rows; ++i) {
-    const int di = base + i;
-    if (di >= ndesc) break;
-    bwd_bgemv_body<T>(s, desc[di], unz, nrhs, vec);
+  const int end = min((int)blockIdx.x * R + R, ndesc);
+  for (int i = (int)blockIdx.x * R; i < end;) {
+    int n = 1;
+    while (i + n < end && desc[i + n].front == desc[i].front && desc[i + n].c0 == desc[i].c0) ++n;
+    bwd_bgemv_body<T, R, QB>(desc + i, n, unz, nrhs, vec);
+    i += n;
   }
 }
 
@@ -3798,7 +3837,9 @@ __device__ __attribute__((always_inline)) void bwd_chain_body(
   using V = typename Vec4<T>::type;
   V* smem_v4 = reinterpret_cast<V*>(smem_a32);
   const T* R = reinterpret_cast<const T*>(smem_a32);
-  const int tid = threadIdx.x, lane = tid % 64, wave = wave_id();
+  const int tid = threadIdx.x, lane = tid % 64;
+  // wave w takes right-hand sides w, w + 4, ..., spread over the z workgroups
+  const int wave = wave_id() + 4 * (int)blockIdx.z, qstep = 4 * (int)gridDim.z;
   const int f = d.front;
   const int L = d.L;
   const int64_t fc0 = d.fc0;
@@ -3840,7 +3881,7 @@ __device__ __attribute__((always_inline)) void bwd_chain_body(
     o.a = *(const V*)(P + 4 * min(lane, k + 3));
     if (both) o.b = *(const V*)(P + 4 * min(lane + 64, k + 3));
   };
-  for (int q = wave; q < nrhs; q += 4) {
+  for (int q = wave; q < nrhs; q += qstep) {
     T* yg = vec + d.fvec * nrhs + (int64_t)q * L;
     T* x = rhs + (int64_t)q * ldr;
     if (q > wave) {
