@@ -3976,12 +3976,18 @@ bwd_chain_kernel(DevSym s, const SolveDesc* __restrict__ desc, const T* __restri
 // ---------------------------------------------------------------------------
 
 // ML and MU of one block (one workgroup per block), each bwp x bwp
-// row-major and zero outside bw x bw, from the block's panels (read from
-// global memory, every lane the same entry): column j is formed by
-// substitution on e_j in LDS (X[r][j]), the lower inverse first (its columns
-// then permuted by the block's interchanges), then the upper one. 64 KB of
-// LDS: two workgroups per CU.
-constexpr int kInvPrepLds = 128 * 128 * 4;  // float
+// row-major and zero outside bw x bw. Column j of each inverse is the solve
+// of e_j: threads 0..127 take ML's columns (column jj of ML is the solve of
+// e_i, i the row that the interchanges bring to jj), threads 128..255 MU's,
+// 32 rows at a time in registers: the terms of the rows already solved, read
+// back from the output, then the 32 x 32 triangle, the panels read from LDS
+// as broadcasts (four coefficients of a row at a time). Column j's entries
+// receive the terms of c = j, j + 1, ... (ML) or c = j, j - 1, ... (MU) in
+// that order; the others would meet a zero and are left out. Bound by about
+// 8000 dependent-free products per thread; with the panels read from global
+// memory and one workgroup barrier per eliminated column it took 700 us on
+// the blocks of 31 x 23 x 17, now 73 us (64^3: 1240 -> 198 us).
+constexpr int kInvPrepLds = (2 * kPanelElems + 128) * 4;  // float
 __global__ void __launch_bounds__(kWG)
 solve_inv_prep_kernel(const SolveDesc* __restrict__ desc, const float* __restrict__ prep,
                       const int32_t* __restrict__ prepi, float* __restrict__ inv,
@@ -3991,57 +3997,107 @@ solve_inv_prep_kernel(const SolveDesc* __restrict__ desc, const float* __restric
   prepi += vs * vs_prepi;
   inv += vs * vs_inv;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_inv[];
-  float* X = reinterpret_cast<float*>(smem_inv);  // X[r * 128 + j]
+  float* lo = reinterpret_cast<float*>(smem_inv);
+  float* up = lo + kPanelElems;
+  float* rinv = up + kPanelElems;
   __shared__ int iperm[128];
   const SolveDesc d = desc[blockIdx.x];
   const int bw = d.c1 - d.c0, ng = (bw + 3) / 4, bwp = 4 * ng;
   const int tid = threadIdx.x;
   const int npan = 8 * ng * (ng + 1);
-  const float* lo = prep + 4 * (int64_t)d.aux;
-  const float* up = lo + npan;
-  const float* rinv = up + npan;
+  {
+    const f32x4* g = reinterpret_cast<const f32x4*>(prep + 4 * (int64_t)d.aux);
+    for (int i = tid; i < npan / 4; i += kWG) {
+      reinterpret_cast<f32x4*>(lo)[i] = g[i];
+      reinterpret_cast<f32x4*>(up)[i] = g[npan / 4 + i];
+    }
+    if (tid < ng) reinterpret_cast<f32x4*>(rinv)[tid] = g[npan / 2 + tid];
+  }
   const int32_t* pi = prepi + (int64_t)d.r0 * kPrepInts;
+  if (tid < bw) iperm[pi[tid]] = tid;
+  __syncthreads();
   float* ML = inv + d.inv;
-  float* MU = ML + (int64_t)bwp * bwp;
-  // Column j of each inverse is the solve of e_j: thread (j, h) = (tid %
-  // 128, tid / 128) takes column j's rows of parity h, and all threads take
-  // the eliminated column c in step, so that the panel entries are read as
-  // broadcasts. Column j's entries receive the terms of c = j, j + 1, ...
-  // (ML) or c = j, j - 1, ... (MU) in that order; the steps with c before j
-  // (ML) or after it (MU) meet a zero entry of column j and change nothing.
-  const int j = tid & 127, h = tid >> 7;
-  const bool cj = j < bw;
-  for (int i = tid; i < bw; i += kWG) iperm[pi[i]] = i;
-  for (int i = tid; i < 128 * 128; i += kWG) X[i] = (i / 128 == i % 128) ? 1.0f : 0.0f;
-  __syncthreads();
-  for (int c = 0; c + 1 < bw; ++c) {
-    if (cj && c >= j) {
-      const float xc = X[c * 128 + j];
-      const float* Pc = lo + lo_panel(c / 4, ng) + (c % 4) - 4 * 4 * (c / 4);
-      for (int r = c + 1 + h; r < bw; r += 2) X[r * 128 + j] -= Pc[4 * r] * xc;
+  const int jj = tid & 127;
+  if (jj >= bwp) return;
+  if (tid < 128) {
+    const int j = jj < bw ? iperm[jj] : 1 << 20;
+    float* X = ML + jj;
+    for (int r0 = 0; r0 < bwp; r0 += 32) {
+      float x[32];
+#pragma unroll
+      for (int r = 0; r < 32; ++r) x[r] = r0 + r == j ? 1.0f : 0.0f;
+      for (int c = 0; c < r0; c += 4) {
+        float xc[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xc[k] = X[(c + k) * bwp];
+        const float* P = lo + lo_panel(c / 4, ng) + 4 * (r0 - c);
+#pragma unroll
+        for (int rr = 0; rr < 32; rr += 8) {
+          f32x4 p[8];
+#pragma unroll
+          for (int r = 0; r < 8; ++r) p[r] = *reinterpret_cast<const f32x4*>(P + 4 * (rr + r));
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (c + k >= j) {
+#pragma unroll
+              for (int r = 0; r < 8; ++r) x[rr + r] -= p[r][k] * xc[k];
+            }
+        }
+      }
+      static_for<8>([&](auto gc) __attribute__((always_inline)) {
+        constexpr int c = 4 * decltype(gc)::value;
+        const float* P = lo + lo_panel((r0 + c) / 4, ng) - 4 * c;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (r0 + c < bwp && r0 + c + k >= j) {
+#pragma unroll
+            for (int r = c + k + 1; r < 32; ++r) x[r] -= P[4 * r + k] * x[c + k];
+          }
+      });
+#pragma unroll
+      for (int r = 0; r < 32; ++r)
+        if (r0 + r < bwp) X[(r0 + r) * bwp] = r0 + r < bw ? x[r] : 0.0f;
     }
-    __syncthreads();
-  }
-  for (int idx = tid; idx < bwp * bwp; idx += kWG) {
-    const int i = idx / bwp, jj = idx % bwp;
-    ML[idx] = (i < bw && jj < bw) ? X[i * 128 + iperm[jj]] : 0.0f;
-  }
-  __syncthreads();
-  for (int i = tid; i < 128 * 128; i += kWG) X[i] = (i / 128 == i % 128) ? 1.0f : 0.0f;
-  __syncthreads();
-  for (int c = bw - 1; c >= 0; --c) {
-    if (cj && c <= j) {
-      const float xc = X[c * 128 + j] * rinv[c];
-      if (h == 0) MU[(int64_t)c * bwp + j] = xc;  // row c of column j is final
-      const float* Pc = up + up_panel(c / 4) + (c % 4);
-      for (int r = h; r < c; r += 2) X[r * 128 + j] -= Pc[4 * r] * xc;
+  } else {
+    const int j = jj < bw ? jj : -1;
+    float* X = ML + (int64_t)bwp * bwp + jj;
+    for (int r0 = (bwp - 1) / 32 * 32; r0 >= 0; r0 -= 32) {
+      float x[32];
+#pragma unroll
+      for (int r = 0; r < 32; ++r) x[r] = r0 + r == j ? 1.0f : 0.0f;
+      for (int c = bwp - 4; c >= r0 + 32; c -= 4) {
+        float xc[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xc[k] = X[(c + k) * bwp];
+        const float* P = up + up_panel(c / 4) + 4 * r0;
+#pragma unroll
+        for (int rr = 0; rr < 32; rr += 8) {
+          f32x4 p[8];
+#pragma unroll
+          for (int r = 0; r < 8; ++r) p[r] = *reinterpret_cast<const f32x4*>(P + 4 * (rr + r));
+#pragma unroll
+          for (int k = 3; k >= 0; --k)
+            if (c + k <= j) {
+#pragma unroll
+              for (int r = 0; r < 8; ++r) x[rr + r] -= p[r][k] * xc[k];
+            }
+        }
+      }
+      static_for<8>([&](auto gc) __attribute__((always_inline)) {
+        constexpr int c = 28 - 4 * decltype(gc)::value;
+        const float* P = up + up_panel((r0 + c) / 4) + 4 * r0;
+#pragma unroll
+        for (int k = 3; k >= 0; --k)
+          if (r0 + c + k <= j) {
+            x[c + k] *= rinv[r0 + c + k];
+#pragma unroll
+            for (int r = 0; r < c + k; ++r) x[r] -= P[4 * r + k] * x[c + k];
+          }
+      });
+#pragma unroll
+      for (int r = 0; r < 32; ++r)
+        if (r0 + r < bwp) X[(r0 + r) * bwp] = r0 + r <= j ? x[r] : 0.0f;
     }
-    __syncthreads();
-  }
-  // the rest of MU: zeros below the diagonal and in the padding
-  for (int idx = tid; idx < bwp * bwp; idx += kWG) {
-    const int i = idx / bwp, jj = idx % bwp;
-    if (!(i < bw && jj < bw && i <= jj)) MU[idx] = 0.0f;
   }
 }
 
@@ -4070,11 +4126,11 @@ __device__ __attribute__((always_inline)) inline void inv_apply(const f32x4 (&mv
   float acc = 0.0f;
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-    const int j = 64 * h + 4 * k;
-    acc += mv[k].x * yb[j];
-    acc += mv[k].y * yb[j + 1];
-    acc += mv[k].z * yb[j + 2];
-    acc += mv[k].w * yb[j + 3];
+    const f32x4 y = *reinterpret_cast<const f32x4*>(yb + 64 * h + 4 * k);
+    acc += mv[k].x * y.x;
+    acc += mv[k].y * y.y;
+    acc += mv[k].z * y.z;
+    acc += mv[k].w * y.w;
   }
   zp[h][i] = acc;
   __syncthreads();
@@ -4096,9 +4152,10 @@ fwd_inv_kernel(DevSym s, const InvItem* __restrict__ items, const float* __restr
   lnz += vs * s.vs_lnz;
   rhs += vs * ldr * nrhs;
   vec += vs * s.vs_vec * nrhs;
-  __shared__ float yb[128];
+  __shared__ __attribute__((aligned(16))) float yb[128];
   __shared__ float zp[2][128];
   __shared__ float zs[128];
+  __shared__ __attribute__((aligned(16))) float zq[4][32];  // zs by quarters, zeros behind
   __shared__ float red[4][64];
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -4155,12 +4212,12 @@ fwd_inv_kernel(DevSym s, const InvItem* __restrict__ items, const float* __restr
     }
     inv_apply(mv, yb, zp, zs);
     if ((it.flags & 1) && tid < bw) rhs[(int64_t)q * ldr + it.fc0 + c0 + tid] = zs[tid];
+    if (!tile) continue;  // the whole workgroup
+    if (lane < 32) zq[wave][lane] = cb + lane < ce ? zs[cb + lane] : 0.0f;  // its own wave's
+    wave_lds_sync();
     float acc = 0.0f;
-    if (tile && r < L) {
 #pragma unroll
-      for (int j = 0; j < 32; ++j)
-        if (cb + j < ce) acc += lv[j] * zs[cb + j];
-    }
+    for (int j = 0; j < 32; ++j) acc += lv[j] * zq[wave][j];
     red[wave][lane] = acc;
     __syncthreads();
     if (tile && wave == 0 && r < L)
@@ -4189,7 +4246,7 @@ bwd_inv_kernel(DevSym s, const InvItem* __restrict__ items, const float* __restr
   vec += vs * s.vs_vec * nrhs;
   constexpr int QB = 4;   // right-hand sides sharing one read of the row
   constexpr int CH = 16;  // columns per thread and pass
-  __shared__ float yb[128];
+  __shared__ __attribute__((aligned(16))) float yb[128];
   __shared__ float zp[2][128];
   __shared__ float xs[QB][128];
   __shared__ float red[QB][4];
@@ -4256,14 +4313,8 @@ bwd_inv_kernel(DevSym s, const InvItem* __restrict__ items, const float* __restr
           }
         }
       }
-#pragma unroll
-      for (int qq = 0; qq < QB; ++qq) {
-        if (qq < nq) {
-          float a = acc[qq];
-          for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
-          if (lane == 0) red[qq][wave] = a;
-        }
-      }
+      const float sum = wave_sums<QB>(acc, lane);
+      if (lane % (64 / QB) == 0) red[lane / (64 / QB)][wave] = sum;
       __syncthreads();
       if (tid < nq) {
         float* y = rhs + (int64_t)(q0 + tid) * ldr + it.fc0 + it.c;
