@@ -91,7 +91,7 @@ struct LevelPlan {
   spk::SmallClasses small_k{};      // the level's small fronts by rows
   int small_maxW = 1;               // most own columns of the level's small fronts
   int items_off = 0, items_cnt = 0;
-  int wb_off = 0, wb_cnt = 0;       // write-back items: the large fronts' pivot columns
+  int wb_cnt = 0;                   // write-back items: the large fronts' pivot columns
   int large_maxL = 0;               // longest index list of the level's large fronts
   struct Launch {
     int off = 0, cnt = 0, wg = 0;
@@ -657,13 +657,13 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
       }
     }
     lp.items_cnt = (int)it_front.size() - lp.items_off;
-    lp.wb_off = (int)h->wb_front.size();
+    const int wb0 = (int)h->wb_front.size();
     for (i32 f : large)
       for (i32 j = 0; j < h->fW[f]; ++j) {
         h->wb_front.push_back(f);
         h->wb_col.push_back(j);
       }
-    lp.wb_cnt = (int)h->wb_front.size() - lp.wb_off;
+    lp.wb_cnt = (int)h->wb_front.size() - wb0;
     // blocks of consecutive pieces, at most kGW columns each (a piece wider
     // than that forms its own block)
     struct Blk {
@@ -1382,17 +1382,28 @@ void run_factor(spkhip_handle* h, bool from_a) {
         }
       }
       if (pending) stream_join(h, st2, st);
-      Prof pr(h, SPKHIP_K_WRITEBACK, 0.0, lp.wb_elems * sizeof(T));
-      if (lp.ut_cnt > 0)
-        hipLaunchKernelGGL((spk::large_utile_kernel<T, true>), dim3(lp.ut_cnt, h->nvs), dim3(kWG), 0, st,
-                           h->ds, h->d_ut_front.p + lp.ut_off, h->d_ut_piece.p + lp.ut_off,
-                           h->d_ut_r0.p + lp.ut_off, lnz.p, unz.p, arena.p);
-      if (lp.wb_cnt > 0)
-        hipLaunchKernelGGL(spk::large_writeback_kernel<T>, dim3(lp.wb_cnt, h->nvs), dim3(kWG), 0, st,
-                           h->ds, h->d_wb_front.p + lp.wb_off, h->d_wb_col.p + lp.wb_off,
-                           lnz.p, unz.p, arena.p);
-      hipck(hipGetLastError());
     }
+  }
+  // the large fronts' panels to lnz/unz, which nothing reads before: every
+  // level's in one launch of each kind (two launches of about 5 us a level
+  // before: pass of a 100^2 grid 2.01 -> 1.85 ms, 193 x 171 4.16 -> 3.80)
+  int uts = 0, wbs = 0;
+  double elems = 0;
+  for (const LevelPlan& lp : h->levels) {
+    uts += lp.ut_cnt;
+    wbs += lp.wb_cnt;
+    elems += lp.wb_elems;
+  }
+  if (wbs > 0) {
+    h->cur_grid = wbs;
+    Prof pr(h, SPKHIP_K_WRITEBACK, 0.0, elems * sizeof(T));
+    if (uts > 0)
+      hipLaunchKernelGGL((spk::large_utile_kernel<T, true>), dim3(uts, h->nvs), dim3(kWG), 0,
+                         st, h->ds, h->d_ut_front.p, h->d_ut_piece.p, h->d_ut_r0.p, lnz.p, unz.p,
+                         arena.p);
+    hipLaunchKernelGGL(spk::large_writeback_kernel<T>, dim3(wbs, h->nvs), dim3(kWG), 0, st, h->ds,
+                       h->d_wb_front.p, h->d_wb_col.p, lnz.p, unz.p, arena.p);
+    hipck(hipGetLastError());
   }
 }
 
