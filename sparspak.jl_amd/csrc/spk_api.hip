@@ -1190,7 +1190,8 @@ unsigned small_wgs(const LevelPlan& lp, int nrhs, int nvs, spk::SmallClasses& k)
   k.wg1 = (k.cnt[1] + 3) / 4;
   k.wg2 = (int)(((i64)k.cnt[2] * nrhs + 15) / 16);
   const i64 wg3 = ((i64)k.cnt[3] * nrhs + 31) / 32;
-  return (unsigned)(k.cnt[0] + k.wg1 + k.wg2 + wg3);
+  k.wgs = (int)(k.cnt[0] + k.wg1 + k.wg2 + wg3);
+  return (unsigned)k.wgs;
 }
 
 template <typename T>
@@ -1477,7 +1478,12 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
   // right-hand sides of the per-row kernels and, four at a time, of the
   // chains take workgroups of their own, the chains while the launch has
   // fewer than four per CU (each stages its block's panels anew)
-  const unsigned qz = (unsigned)std::min(nrhs, 16);
+  const int qz = std::min(nrhs, 16);
+  auto rows = [&](const LevelPlan& lp, int z) {
+    return spk::LevelRows{h->d_it_front.p + lp.items_off, h->d_it_col.p + lp.items_off,
+                          h->d_it_ea.p + lp.items_off, h->d_ea_child.p, h->d_ea_t.p,
+                          lp.items_cnt, (lp.items_cnt + kWG - 1) / kWG, z};
+  };
   auto chain_z = [&](const LevelPlan::SolveStep& S) {
     const i64 wg = std::max<i64>((i64)S.chain_cnt * h->nvs, 1);
     return (unsigned)std::max<i64>(1, std::min<i64>((nrhs + 3) / 4, 1024 / wg));
@@ -1486,17 +1492,20 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
     for (const LevelPlan& lp : h->levels) {
       h->cur_level = (int)(&lp - h->levels.data());
       h->cur_grid = lp.small_cnt;
-      if (lp.small_cnt > 0) {
+      {
+        // the small fronts and the large fronts' rows (independent of each
+        // other) in one launch
         Prof pr(h, SPKHIP_K_FWD, 0.0, 0.0);
         spk::SmallClasses k;
-        const unsigned wgs = small_wgs(lp, nrhs, h->nvs, k);
+        const spk::LevelRows m = rows(lp, qz);
+        const unsigned wgs = small_wgs(lp, nrhs, h->nvs, k) + m.nb * m.qz;
         const int LDL = lp.small_maxL | 1, slot = std::min(lp.small_maxW, 32) * std::min(LDL, 33);
         const size_t lds = nrhs <= 4 ? 0
                                      : std::max(k.cnt[0] ? lp.small_maxW * LDL : 0,
                                                 k.cnt[1] ? 4 * slot : 0) * sizeof(T);
         auto go = [&](auto kern) {
           hipLaunchKernelGGL(kern, dim3(wgs, h->nvs), dim3(kWG), lds, st, h->ds,
-                             h->d_sdfr.p + lp.small_off, h->d_sdch.p, k, LDL, slot, lnz,
+                             h->d_sdfr.p + lp.small_off, h->d_sdch.p, k, m, LDL, slot, lnz,
                              h->d_ipvt.p, rhs, ldr, nrhs, vecp);
         };
         // right-hand sides in the registers of one wave
@@ -1509,16 +1518,6 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
         hipck(hipGetLastError());
       }
       if (lp.large_cnt == 0) continue;
-      {
-        Prof pr(h, SPKHIP_K_FWD, 0.0, 0.0);
-        hipLaunchKernelGGL(spk::fwd_assemble_items_kernel<T>,
-                           dim3((lp.items_cnt + kWG - 1) / kWG, h->nvs, qz), dim3(kWG), 0, st,
-                           h->ds,
-                           h->d_it_front.p + lp.items_off, h->d_it_col.p + lp.items_off,
-                           h->d_it_ea.p + lp.items_off, h->d_ea_child.p, h->d_ea_t.p, rhs, ldr,
-                           nrhs, vecp, lp.items_cnt);
-        hipck(hipGetLastError());
-      }
       if constexpr (std::is_same<T, float>::value) {
         if (inv) {
           for (size_t k = 0; k < lp.ifw.size(); ++k) {
@@ -1560,14 +1559,26 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
       const LevelPlan& lp = h->levels[l];
       h->cur_level = l;
       h->cur_grid = lp.large_cnt;
-      if (lp.large_cnt > 0) {
+      {
+        // the small fronts and the gathers of the large fronts' update rows
         Prof pr(h, SPKHIP_K_BWD, 0.0, 0.0);
-        const unsigned gz = (i64)lp.items_cnt * h->nvs < 1 << 18 ? qz : 1;
-        hipLaunchKernelGGL(spk::bwd_gather_items_kernel<T>,
-                           dim3((lp.items_cnt + kWG - 1) / kWG, h->nvs, gz), dim3(kWG), 0, st,
-                           h->ds,
-                           h->d_it_front.p + lp.items_off, h->d_it_col.p + lp.items_off, rhs,
-                           ldr, nrhs, vecp, lp.items_cnt);
+        const spk::LevelRows m = rows(lp, (i64)lp.items_cnt * h->nvs < 1 << 18 ? qz : 1);
+        const int LDW = lp.small_maxW | 1, slot = std::min(lp.small_maxL, 32) * std::min(LDW, 33);
+        spk::SmallClasses k;
+        const unsigned wgs = small_wgs(lp, nrhs, h->nvs, k) + m.nb * m.qz;
+        const size_t lds =
+            std::max(k.cnt[0] ? lp.small_maxL * LDW : 0, k.cnt[1] ? 4 * slot : 0) * sizeof(T);
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(wgs, h->nvs), dim3(kWG), lds, st, h->ds,
+                             h->d_sdfr.p + lp.small_off, k, m, LDW, slot, lnz, unz, rhs, ldr, nrhs,
+                             vecp);
+        };
+        if (nrhs == 1)
+          go(spk::bwd_small_kernel<T, 1>);
+        else if (nrhs <= 4)
+          go(spk::bwd_small_kernel<T, 4>);
+        else
+          go(spk::bwd_small_kernel<T, 16>);
         hipck(hipGetLastError());
       }
       bool done = false;
@@ -1611,25 +1622,6 @@ void solve_levels_direct(spkhip_handle* h, T* rhs, i64 ldr, int nrhs, bool fwd, 
         hipLaunchKernelGGL((spk::bwd_chain_kernel<T>), dim3(S.chain_cnt, h->nvs, chain_z(S)), dim3(kWG),
                            (size_t)(spk::kPanelElems + 128) * sizeof(T), st, h->ds,
                            h->d_sdesc.p + S.chain_off, prep.p, rhs, ldr, nrhs, vecp);
-        hipck(hipGetLastError());
-      }
-      if (lp.small_cnt > 0) {
-        Prof pr(h, SPKHIP_K_BWD, 0.0, 0.0);
-        const int LDW = lp.small_maxW | 1, slot = std::min(lp.small_maxL, 32) * std::min(LDW, 33);
-        spk::SmallClasses k;
-        const unsigned wgs = small_wgs(lp, nrhs, h->nvs, k);
-        const size_t lds =
-            std::max(k.cnt[0] ? lp.small_maxL * LDW : 0, k.cnt[1] ? 4 * slot : 0) * sizeof(T);
-        auto go = [&](auto kern) {
-          hipLaunchKernelGGL(kern, dim3(wgs, h->nvs), dim3(kWG), lds, st, h->ds,
-                             h->d_sdfr.p + lp.small_off, k, LDW, slot, lnz, unz, rhs, ldr, nrhs);
-        };
-        if (nrhs == 1)
-          go(spk::bwd_small_kernel<T, 1>);
-        else if (nrhs <= 4)
-          go(spk::bwd_small_kernel<T, 4>);
-        else
-          go(spk::bwd_small_kernel<T, 16>);
         hipck(hipGetLastError());
       }
     }

@@ -145,6 +145,17 @@ struct SmallChild {
 struct SmallClasses {
   int32_t cnt[4];
   int32_t wg1, wg2;
+  int32_t wgs;  // workgroups of all four
+};
+// A level's large fronts' rows (the factor's column items: a front's rows and
+// columns share its index list), taken by the workgroups behind those of its
+// small fronts: nb workgroups of rows for each of qz groups of right-hand
+// sides.
+struct LevelRows {
+  const int32_t *front, *row;
+  const int64_t* ea;               // children's entries per row
+  const int32_t *ea_child, *ea_t;
+  int32_t n, nb, qz;
 };
 // One entry of A inside its front: value k of the CSC array goes to row r,
 // column c of the front's matrix (SPD: once more to row c, column r).

@@ -2494,26 +2494,20 @@ blk_diag_border_kernel(DevSym s, const BlkDesc* __restrict__ ddesc, int ndiag,
 // the same sum in the same order as a per-front gather; a level's fronts
 // spread over many workgroups.
 template <typename T>
-__global__ void __launch_bounds__(kWG)
-fwd_assemble_items_kernel(DevSym s, const int32_t* __restrict__ it_front,
-                          const int32_t* __restrict__ it_col,
-                          const int64_t* __restrict__ it_ea,
-                          const int32_t* __restrict__ ea_child,
-                          const int32_t* __restrict__ ea_t, const T* __restrict__ rhs,
-                          int64_t ldr, int nrhs, T* __restrict__ vec, int nitems) {
-  const int64_t vs = blockIdx.y;  // value set
-  rhs += vs * ldr * nrhs;
-  vec += vs * s.vs_vec * nrhs;
-  const int item = blockIdx.x * kWG + threadIdx.x;
-  if (item >= nitems) return;
-  const int f = it_front[item], r = it_col[item];
+__device__ inline void fwd_assemble_rows(const DevSym& s, const LevelRows& m, int b,
+                                         const T* __restrict__ rhs, int64_t ldr, int nrhs,
+                                         T* __restrict__ vec) {
+  const int z = b / m.nb;
+  const int item = (b - z * m.nb) * kWG + threadIdx.x;
+  if (item >= m.n) return;
+  const int f = m.front[item], r = m.row[item];
   const int L = s.fL[f], W = s.fW[f];
   const int64_t fc0 = s.fc0[f];
-  const int64_t e0 = it_ea[item], e1 = it_ea[item + 1];
-  for (int q = blockIdx.z; q < nrhs; q += gridDim.z) {
+  const int64_t e0 = m.ea[item], e1 = m.ea[item + 1];
+  for (int q = z; q < nrhs; q += m.qz) {
     T y = (r < W) ? rhs[(int64_t)q * ldr + fc0 + r] : T(0);
     for (int64_t e = e0; e < e1; ++e) {
-      const int c = ea_child[e], t = ea_t[e];
+      const int c = m.ea_child[e], t = m.ea_t[e];
       y += vec[s.fvec[c] * nrhs + (int64_t)q * s.fL[c] + s.fW[c] + t];
     }
     vec[s.fvec[f] * nrhs + (int64_t)q * L + r] = y;
@@ -2524,20 +2518,17 @@ fwd_assemble_items_kernel(DevSym s, const int32_t* __restrict__ it_front,
 // from the solution by the front's index list, one thread per (front, row)
 // item of the level.
 template <typename T>
-__global__ void __launch_bounds__(kWG)
-bwd_gather_items_kernel(DevSym s, const int32_t* __restrict__ it_front,
-                        const int32_t* __restrict__ it_col, const T* __restrict__ rhs,
-                        int64_t ldr, int nrhs, T* __restrict__ vec, int nitems) {
-  const int64_t vs = blockIdx.y;  // value set
-  rhs += vs * ldr * nrhs;
-  vec += vs * s.vs_vec * nrhs;
-  const int item = blockIdx.x * kWG + threadIdx.x;
-  if (item >= nitems) return;
-  const int f = it_front[item], j = it_col[item];
+__device__ inline void bwd_gather_rows(const DevSym& s, const LevelRows& m, int b,
+                                       const T* __restrict__ rhs, int64_t ldr, int nrhs,
+                                       T* __restrict__ vec) {
+  const int z = b / m.nb;
+  const int item = (b - z * m.nb) * kWG + threadIdx.x;
+  if (item >= m.n) return;
+  const int f = m.front[item], j = m.row[item];
   const int L = s.fL[f], W = s.fW[f];
   if (j < W) return;
   const int g = s.lindx[s.xlindx[s.fsp0[f]] - 1 + j] - 1;
-  for (int q = blockIdx.z; q < nrhs; q += gridDim.z)
+  for (int q = z; q < nrhs; q += m.qz)
     vec[s.fvec[f] * nrhs + (int64_t)q * L + j] = rhs[(int64_t)q * ldr + g];
 }
 
@@ -2998,7 +2989,7 @@ __device__ __attribute__((always_inline)) inline T wave_sums(T (&v)[NV], int lan
 
 // Backward: t[c] = U[c, c1:L] x[c1:L] for rows c = c0 + r0 of the block,
 // stored in y[c]. x[c1:L] is read from the front's vector: its update rows
-// from bwd_gather_items_kernel, its own columns as the backward chains of the
+// from bwd_gather_rows, its own columns as the backward chains of the
 // later blocks left them. R rows of one block (n of them wanted) share the
 // loads of x, QB right-hand sides those of U: every thread takes columns c1 +
 // tid + 256 m of all of them, its sums are added over the wave (wave_sums),
@@ -3597,7 +3588,7 @@ __device__ __attribute__((always_inline)) void stage_small_l(const DevSym& s, co
 template <typename T, int QW>
 __global__ void __launch_bounds__(kWG)
 fwd_small_kernel(DevSym s, const SmallDesc* __restrict__ desc,
-                 const SmallChild* __restrict__ child, SmallClasses k, int LDL, int slot,
+                 const SmallChild* __restrict__ child, SmallClasses k, LevelRows m, int LDL, int slot,
                  const T* __restrict__ lnz, const int64_t* __restrict__ ipvt,
                  T* __restrict__ rhs, int64_t ldr, int nrhs, T* __restrict__ vec) {
   const int64_t vs = blockIdx.y;  // value set
@@ -3606,6 +3597,10 @@ fwd_small_kernel(DevSym s, const SmallDesc* __restrict__ desc,
   ipvt += vs * s.n;
   rhs += vs * ldr * nrhs;
   vec += vs * s.vs_vec * nrhs;
+  if (b >= k.wgs) {
+    fwd_assemble_rows<T>(s, m, b - k.wgs, rhs, ldr, nrhs, vec);
+    return;
+  }
   const int wave = wave_id();
   if constexpr (QW > 4) {
     extern __shared__ unsigned char smem_raw[];
@@ -3763,14 +3758,18 @@ __device__ __attribute__((always_inline)) void bwd_small_wave(
 
 template <typename T, int QW>
 __global__ void __launch_bounds__(kWG)
-bwd_small_kernel(DevSym s, const SmallDesc* __restrict__ desc, SmallClasses k, int LDW,
-                 int slot, const T* __restrict__ lnz, const T* __restrict__ unz,
-                 T* __restrict__ rhs, int64_t ldr, int nrhs) {
+bwd_small_kernel(DevSym s, const SmallDesc* __restrict__ desc, SmallClasses k, LevelRows m,
+                 int LDW, int slot, const T* __restrict__ lnz, const T* __restrict__ unz,
+                 T* __restrict__ rhs, int64_t ldr, int nrhs, T* __restrict__ vec) {
   const int64_t vs = blockIdx.y;  // value set
   int b = blockIdx.x;
   lnz += vs * s.vs_lnz;
   unz += vs * s.vs_unz;
   rhs += vs * ldr * nrhs;
+  if (b >= k.wgs) {
+    bwd_gather_rows<T>(s, m, b - k.wgs, rhs, ldr, nrhs, vec + vs * s.vs_vec * nrhs);
+    return;
+  }
   extern __shared__ unsigned char smem_raw[];
   T* S = reinterpret_cast<T*>(smem_raw);
   const int wave = wave_id();
