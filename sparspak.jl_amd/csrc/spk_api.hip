@@ -1194,13 +1194,16 @@ unsigned small_wgs(const LevelPlan& lp, int nrhs, int nvs, spk::SmallClasses& k)
   return (unsigned)k.wgs;
 }
 
+// Most LDS of a launch that holds small fronts and the assembly of large ones.
+constexpr int kJointLds = 40 * 1024;
+
 template <typename T>
 void set_lds_attrs() {
   static bool done = false;
   if (done) return;
   hipck(hipFuncSetAttribute((const void*)spk::small_front_kernel<T, false>,
                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                            4 * 32 * 33 * (int)sizeof(T)));
+                            kJointLds));
   hipck(hipFuncSetAttribute((const void*)spk::small_front_kernel<T, true>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, 140 * 1024));
   hipck(hipFuncSetAttribute((const void*)spk::blk_diag_slab_kernel<T>,
@@ -1256,19 +1259,33 @@ void run_factor(spkhip_handle* h, bool from_a) {
   for (const LevelPlan& lp : h->levels) {
     h->cur_level = (int)(&lp - h->levels.data());
     h->cur_grid = lp.small_cnt;
+    // the column is assembled in LDS when the longest one fits in 64 KB;
+    // levels whose columns fit 16 KB take one wave per column
+    const size_t clds = (size_t)lp.large_maxL * sizeof(T);
+    const bool staged = clds <= 64 * 1024, cwave = clds <= 16 * 1024;
+    const spk::AsmArgs asmb{h->d_it_asm.p + lp.items_off, h->d_it_ea.p + lp.items_off,
+                            h->d_ea_init.p, aent, lp.items_cnt, lp.large_maxL, (int)staged};
+    // with the small fronts in one launch where its LDS does not cost either
+    // of them workgroups in flight (columns of at most 10 KB, four a workgroup) and the launch
+    // profile does not tell them apart
+    const bool wave64 = lp.small_cnt >= h->small_wave_min && lp.small_k.cnt[0] > 0;
+    const bool joint = aent && lp.small_cnt > 0 && lp.items_cnt > 0 && 4 * clds <= kJointLds &&
+                       !wave64 && !h->prof;
     if (lp.small_cnt > 0) {
       // fronts of more than 32 rows take a workgroup, the others one wave
       // each; levels of very many fronts one wave for every front
       Prof pr(h, SPKHIP_K_SMALL, lp.small_flops, lp.small_elems * sizeof(T));
       const int LD = lp.small_maxL | 1, front = lp.small_maxL * LD;
       auto go = [&](auto kern, int nbig, int wgs, int slot, int elems) {
-        hipLaunchKernelGGL(kern, dim3(wgs, h->nvs), dim3(kWG), elems * sizeof(T), st, h->ds,
+        const int more = joint ? (lp.items_cnt + 3) / 4 : 0;
+        hipLaunchKernelGGL(kern, dim3(wgs + more, h->nvs), dim3(kWG),
+                           std::max<size_t>(elems * sizeof(T), joint ? 4 * clds : 0), st, h->ds,
                            h->d_sdfr.p + lp.small_off, h->d_sdch.p, nbig, lp.small_cnt, LD, slot,
-                           aent, h->d_nzval.p, h->nnz, lnz.p, unz.p, h->d_ipvt.p, arena.p,
-                           h->d_fail.p);
+                           wgs, asmb, aent, h->d_nzval.p, h->nnz, lnz.p, unz.p, h->d_ipvt.p,
+                           arena.p, h->d_fail.p);
       };
       const int nbig = lp.small_k.cnt[0];
-      if (lp.small_cnt >= h->small_wave_min && nbig > 0) {
+      if (wave64) {
         go(spk::small_front_kernel<T, true>, 0, (lp.small_cnt + 3) / 4, front, 4 * front);
       } else {
         const int slot = std::min(front, 32 * 33);
@@ -1278,21 +1295,14 @@ void run_factor(spkhip_handle* h, bool from_a) {
       hipck(hipGetLastError());
     }
     if (lp.items_cnt > 0) {
-      {
+      if (!joint) {
       Prof pr(h, SPKHIP_K_INIT, 0.0, lp.init_elems * sizeof(T));
-      // the column is assembled in LDS when the longest one fits in 64 KB;
-      // levels whose columns fit 16 KB take one wave per column
-      const size_t clds = (size_t)lp.large_maxL * sizeof(T);
-      const bool staged = clds <= 64 * 1024;
       if (aent) {
-        const bool wave = clds <= 16 * 1024;
         auto go = [&](auto kern, int cols, size_t lds) {
           hipLaunchKernelGGL(kern, dim3((lp.items_cnt + cols - 1) / cols, h->nvs), dim3(kWG), lds,
-                             st, h->ds, h->d_it_asm.p + lp.items_off,
-                             h->d_it_ea.p + lp.items_off, h->d_ea_init.p, aent, h->d_nzval.p,
-                             h->nnz, arena.p, lp.items_cnt, lp.large_maxL, (int)staged);
+                             st, h->ds, asmb, h->d_nzval.p, h->nnz, arena.p);
         };
-        if (wave)
+        if (cwave)
           go(spk::large_assemble_kernel<T, 64>, 4, 4 * clds);
         else
           go(spk::large_assemble_kernel<T, kWG>, 1, staged ? clds : 0);

@@ -171,6 +171,15 @@ struct EaItem {
   int32_t Rc;   // the child's update rows
   int32_t pad;
 };
+// A level's assembly of its large fronts from A's entries: staged in LDS
+// (columns of up to maxL rows), or in place.
+struct AsmArgs {
+  const AsmItem* items;
+  const int64_t* it_ea;
+  const EaItem* ea;
+  const AEnt* aent;
+  int32_t nitems, maxL, staged;
+};
 
 // Integers of a block's solve data: the composed row permutation.
 constexpr int kPrepInts = 128;

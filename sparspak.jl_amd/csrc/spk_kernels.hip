@@ -303,34 +303,28 @@ large_init_kernel(DevSym s, const InitItem* __restrict__ items,
 // columns were summed in place in HBM) 91.3 -> 80.7 ms, 32^3 double
 // 9.57 -> 9.28 ms, 100^2 double 2.56 -> 2.46 ms.
 template <typename T, int G>
-__global__ void __launch_bounds__(kWG)
-large_assemble_kernel(DevSym s, const AsmItem* __restrict__ items,
-                      const int64_t* __restrict__ it_ea, const EaItem* __restrict__ ea,
-                      const AEnt* __restrict__ aent, const double* __restrict__ nzval,
-                      int64_t nnz, T* __restrict__ arena, int nitems, int maxL, int staged) {
-  const int64_t vs = blockIdx.y;  // value set
-  nzval += vs * nnz;
-  arena += vs * s.vs_arena;
-  extern __shared__ unsigned char smem_raw[];
+__device__ __attribute__((always_inline)) void large_assemble_body(
+    const DevSym& s, const AsmArgs& a, int b, const double* __restrict__ nzval,
+    T* __restrict__ arena, unsigned char* smem_raw) {
   constexpr int U = 8;
   const int grp = (G == kWG) ? 0 : wave_id();
   const int gt = (G == kWG) ? (int)threadIdx.x : (int)threadIdx.x % 64;
-  const int item = blockIdx.x * (kWG / G) + grp;
-  if (item >= nitems) return;  // a whole wave (no workgroup barrier below) or workgroup
+  const int item = b * (kWG / G) + grp;
+  if (item >= a.nitems) return;  // a whole wave (no workgroup barrier below) or workgroup
   auto gsync = [] {
     if constexpr (G == kWG)
       __syncthreads();
     else
       wave_lds_sync();
   };
-  const AsmItem m = items[item];
+  const AsmItem m = a.items[item];
   const int L = m.L;
   T* F = arena + m.fcol;
-  T* Fs = staged ? reinterpret_cast<T*>(smem_raw) + (size_t)grp * maxL : F;
-  int64_t e = it_ea[item];
-  const int64_t e1 = it_ea[item + 1];
+  T* Fs = a.staged ? reinterpret_cast<T*>(smem_raw) + (size_t)grp * a.maxL : F;
+  int64_t e = a.it_ea[item];
+  const int64_t e1 = a.it_ea[item + 1];
   // the batch in flight: rows t0 + gt + u G of child `cur`
-  EaItem cur = ea[e < e1 ? e : 0];
+  EaItem cur = a.ea[e < e1 ? e : 0];
   int t0 = 0;
   int ri[U];
   T cv[U];
@@ -348,7 +342,7 @@ large_assemble_kernel(DevSym s, const AsmItem* __restrict__ items,
   for (int r = gt; r < L; r += G) Fs[r] = T(0);
   gsync();
   for (int i = gt; i < m.an; i += G) {
-    const AEnt en = aent[m.a0 + i];
+    const AEnt en = a.aent[m.a0 + i];
     Fs[en.r] = (T)nzval[en.k];
   }
   gsync();
@@ -364,7 +358,7 @@ large_assemble_kernel(DevSym s, const AsmItem* __restrict__ items,
     const bool last = t0 >= cur.Rc;
     if (last) {
       t0 = 0;
-      if (++e < e1) cur = ea[e];
+      if (++e < e1) cur = a.ea[e];
     }
     if (e < e1) request();
 #pragma unroll
@@ -372,7 +366,7 @@ large_assemble_kernel(DevSym s, const AsmItem* __restrict__ items,
       if (rj[u] >= 0) Fs[rj[u]] += cw[u];
     if (last) gsync();
   }
-  if (!staged) return;
+  if (!a.staged) return;
   for (int r0 = gt; r0 < L; r0 += U * G) {
     T v[U];
 #pragma unroll
@@ -381,6 +375,15 @@ large_assemble_kernel(DevSym s, const AsmItem* __restrict__ items,
     for (int u = 0; u < U; ++u)
       if (r0 + u * G < L) F[r0 + u * G] = v[u];
   }
+}
+
+template <typename T, int G>
+__global__ void __launch_bounds__(kWG)
+large_assemble_kernel(DevSym s, AsmArgs a, const double* __restrict__ nzval, int64_t nnz,
+                      T* __restrict__ arena) {
+  const int64_t vs = blockIdx.y;  // value set
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  large_assemble_body<T, G>(s, a, blockIdx.x, nzval + vs * nnz, arena + vs * s.vs_arena, smem_raw);
 }
 
 // L part of the own columns back to lnz (contiguous per column).
@@ -1312,13 +1315,14 @@ __device__ __attribute__((always_inline)) void small_front_body(
 // The level's fronts of more than 32 rows (the first nbig of desc) one per
 // workgroup, the others one per wave, four per workgroup; WAVE64: every
 // front one per wave (levels of very many fronts). The grid of a wave's
-// threads follows the front's rows.
+// threads follows the front's rows. The workgroups behind the first wgs
+// assemble the level's large fronts, which the small ones do not touch.
 template <typename T, bool WAVE64>
 __global__ void __launch_bounds__(kWG)
 small_front_kernel(DevSym s, const SmallDesc* __restrict__ desc,
                    const SmallChild* __restrict__ child, int nbig, int cnt, int LD, int slot,
-                   const AEnt* __restrict__ aent, const double* __restrict__ nzval,
-                   int64_t nnz, T* __restrict__ lnz, T* __restrict__ unz,
+                   int wgs, AsmArgs asmb, const AEnt* __restrict__ aent,
+                   const double* __restrict__ nzval, int64_t nnz, T* __restrict__ lnz, T* __restrict__ unz,
                    int64_t* __restrict__ ipvt, T* __restrict__ arena,
                    unsigned long long* __restrict__ first_fail) {
   const int64_t vs = blockIdx.y;  // value set
@@ -1328,6 +1332,10 @@ small_front_kernel(DevSym s, const SmallDesc* __restrict__ desc,
   ipvt += vs * s.n;
   arena += vs * s.vs_arena;
   extern __shared__ unsigned char smem_raw[];
+  if ((int)blockIdx.x >= wgs) {
+    large_assemble_body<T, 64>(s, asmb, (int)blockIdx.x - wgs, nzval, arena, smem_raw);
+    return;
+  }
   T* F = reinterpret_cast<T*>(smem_raw);
   const int wave = wave_id();
   if constexpr (WAVE64) {
