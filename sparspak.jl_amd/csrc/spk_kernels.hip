@@ -1150,11 +1150,12 @@ __device__ __attribute__((always_inline)) void small_front_body(
     nv = nzval[en.k];
   }
   if (gt < W) {
-    const int64_t g = fc0 + gt, p = s.snode[g];
+    const int64_t g = fc0 + gt;
+    const int pc = s.pcol[g];
     sh.lc[gt] = s.lcol[g];
     sh.uc[gt] = s.ucol[g];
-    sh.cq[gt] = (int)(s.xsuper[p - 1] - 1 - fc0);
-    sh.ce[gt] = (int)(s.xsuper[p] - 1 - fc0);
+    sh.cq[gt] = pc & 0xffff;
+    sh.ce[gt] = pc >> 16;
   }
   for (int i = gt; i < L * LD; i += G) F[i] = T(0);
   gsync();
