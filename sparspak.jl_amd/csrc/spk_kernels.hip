@@ -18,8 +18,6 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ inline int64_t ld_i64(const int64_t* p, int64_t i) { return p[i]; }
-
 // Column range of piece p (0-based supernode): first column (0-based) and
 // width.
 __device__ inline void piece_cols(const DevSym& s, int64_t p, int64_t& c0,
@@ -31,32 +29,6 @@ __device__ inline void piece_cols(const DevSym& s, int64_t p, int64_t& c0,
 // First (front-local) column of the piece holding own column c.
 __device__ inline int piece_start_of_col(const DevSym& s, int64_t fc0, int c) {
   return (int)(s.xsuper[s.snode[fc0 + c] - 1] - 1 - fc0);
-}
-
-// Unit-stride element of the reference layout for front entry (r, j).
-// Returns the lnz (is_u = false) or unz (is_u = true) offset, or -1 for the
-// update-matrix block (r >= W and j >= W), which has no slot.
-__device__ inline int64_t slot_of(const DevSym& s, int64_t fc0, int64_t W,
-                                  int64_t r, int64_t j, bool& is_u) {
-  if (j < W) {
-    int64_t g = fc0 + j;
-    int64_t p = s.snode[g] - 1, pc0, pw;
-    piece_cols(s, p, pc0, pw);
-    int64_t cq = pc0 - fc0;
-    if (r >= cq) {
-      is_u = false;
-      return s.xlnz[g] - 1 + (r - cq);
-    }
-  } else if (r >= W) {
-    return -1;
-  }
-  // U entry: row r lies in an earlier piece (or j is an update column).
-  int64_t gr = fc0 + r;
-  int64_t pr = s.snode[gr] - 1, rc0, rw;
-  piece_cols(s, pr, rc0, rw);
-  int64_t cr = rc0 - fc0;
-  is_u = true;
-  return s.xunz[gr] - 1 + (j - cr - rw);
 }
 
 template <typename T>
@@ -579,101 +551,6 @@ __device__ inline void blk_trsv(T* X, const T* M, const T* rd, int nq) {
   }
 }
 
-// Pivoted LU of the nq x nq block D (LDS, leading dimension LD, nq <= 64) by
-// one wave, with rows that never move during the elimination: lane i owns
-// LDS row i of the block and tracks the position pos its row holds after the
-// interchanges so far. Step k takes the row of smallest position among those
-// holding the maximum |a| over positions >= k (the first maximum of ggetrf!,
-// GenericBlasLapackFragments.jl:56-100; a zero maximum keeps row k and skips
-// the scaling), reads the pivot row where it lies and updates the rows of
-// position > k, eight columns per batch of loads. At the end every row moves
-// to its position, together with the columns [nq, ncols) of D. piv[k] is the
-// position swapped with k at step k, perm[p] the row now at position p,
-// dinv[k] = 1 / U(k, k); *zero is set by a zero pivot.
-template <typename T, int LD>
-__device__ void pos_getrf(T* D, int nq, int ncols, int* piv, int* perm, T* dinv, int* zero) {
-  const int lane = threadIdx.x % 64;
-  const bool mine = lane < nq;
-  int pos = lane;
-  for (int k = 0; k < nq; ++k) {
-    const bool cand = mine && pos >= k;
-    const T v = mine ? D[lane + k * LD] : T(0);
-    const T a = cand ? fabs(v) : T(-1);
-    const T m = wave_max(a);
-    const bool tie = cand && a == m;
-    const unsigned long long msk = __ballot(tie);
-    int blane;
-    if (msk == 0ull) {  // no comparable candidate (NaN column): keep row k
-      blane = __ffsll((long long)__ballot(mine && pos == k)) - 1;
-    } else if (__popcll(msk) == 1) {
-      blane = __ffsll((long long)msk) - 1;
-    } else {
-      const int mp = wave_min(tie ? pos : (1 << 20));
-      blane = __ffsll((long long)__ballot(tie && pos == mp)) - 1;
-    }
-    blane = __builtin_amdgcn_readfirstlane(blane);
-    const int kp = __builtin_amdgcn_readlane(pos, blane);
-    const T pv = rdlane(v, blane);
-    const bool nonzero = pv != T(0);
-    if (nonzero && kp != k) {
-      if (mine && pos == k)
-        pos = kp;
-      else if (lane == blane)
-        pos = k;
-    }
-    const T inv = T(1) / pv;
-    if (lane == 0) {
-      piv[k] = kp;
-      dinv[k] = inv;
-      if (!nonzero) *zero = 1;
-    }
-    const bool below = mine && pos > k;
-    const T l = nonzero ? v * inv : v;
-    if (below && nonzero) D[lane + k * LD] = l;
-    int j0 = k + 1;
-    for (; j0 + 8 <= nq; j0 += 8) {
-      const T* pr = D + blane + j0 * LD;
-      T* xr = D + lane + j0 * LD;
-      T u[8], x[8];
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        u[jj] = pr[jj * LD];
-        x[jj] = xr[jj * LD];
-      }
-      if (below) {
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj) xr[jj * LD] = x[jj] - l * u[jj];
-      }
-    }
-    for (; j0 < nq; ++j0)
-      if (below) D[lane + j0 * LD] -= l * D[blane + j0 * LD];
-    wave_lds_sync();
-  }
-  if (mine) perm[pos] = lane;
-  wave_lds_sync();
-  // rows to their positions: position p takes LDS row perm[p]
-  const T* srow = D + (mine ? perm[lane] : 0);
-  T* drow = D + lane;
-  int c0 = 0;
-  for (; c0 + 8 <= ncols; c0 += 8) {
-    T x[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = srow[(c0 + u) * LD];
-    wave_lds_sync();
-    if (mine) {
-#pragma unroll
-      for (int u = 0; u < 8; ++u) drow[(c0 + u) * LD] = x[u];
-    }
-    wave_lds_sync();
-  }
-  for (; c0 < ncols; ++c0) {
-    const T x = srow[c0 * LD];
-    wave_lds_sync();
-    if (mine) drow[c0 * LD] = x;
-    wave_lds_sync();
-  }
-}
-
 // Pivot of column k among the rows whose position is k or later (v: this
 // lane's entry of the column, pos: its row's position): largest |v|, ties
 // to the smallest position; a column without a comparable candidate (NaN)
@@ -697,7 +574,17 @@ __device__ inline int pivot_lane(T v, int pos, bool mine, int k) {
   return __builtin_amdgcn_readfirstlane(blane);
 }
 
-// pos_getrf with the whole workgroup, one barrier per step. Wave 0 updates
+// Pivoted LU of the nq x nq block D (LDS, leading dimension LD, nq <= 64)
+// with rows that never move during the elimination: lane i owns LDS row i of
+// the block and tracks the position pos its row holds after the interchanges
+// so far. Step k takes the row of smallest position among those holding the
+// maximum |a| over positions >= k (the first maximum of ggetrf!,
+// GenericBlasLapackFragments.jl:56-100; a zero maximum keeps row k and skips
+// the scaling) and reads the pivot row where it lies. At the end every row
+// moves to its position, together with the columns [nq, ncols) of D. piv[k]
+// is the position swapped with k at step k, perm[p] the row now at position
+// p, dinv[k] = 1 / U(k, k); *zero is set by a zero pivot. The whole
+// workgroup, one barrier per step. Wave 0 updates
 // the next pivot column first and runs the next step's pivot search on it
 // (pivot_lane), publishing the pivot row and value through LDS (two slots,
 // by step parity); waves 1-3 update the columns j = k + 2 + (wave - 1) + 3 i
@@ -2491,7 +2378,7 @@ blk_diag_border_kernel(DevSym s, const BlkDesc* __restrict__ ddesc, int ndiag,
 // rows below inside the block) and a many-workgroup GEMV updates every row
 // below the block, y[c1:L] -= L[c1:L, c0:c1] y[c0:c1].
 // Backward (_luusolve!, :325-377), blocks in reverse: t = U[c0:c1, c1:L]
-// x[I[c1:L]] (one wave per row), then the chain: y = x - t, per piece in
+// x[I[c1:L]] (a workgroup per row or eight), then the chain: y = x - t, per piece in
 // reverse the in-block U12 part and the upper block solve.
 // Small fronts (L <= kSmallLmax) do everything in one wave per block of
 // right-hand sides.
@@ -2540,7 +2427,6 @@ __device__ inline void bwd_gather_rows(const DevSym& s, const LevelRows& m, int 
   for (int q = z; q < nrhs; q += m.qz)
     vec[s.fvec[f] * nrhs + (int64_t)q * L + j] = rhs[(int64_t)q * ldr + g];
 }
-
 
 // Per-block solve data, built once per factorisation and read by every
 // solve (refinement solves many times). A block of bw columns is padded to
@@ -2654,13 +2540,6 @@ solve_prep_kernel(DevSym s, const SolveDesc* __restrict__ desc, const T* __restr
   for (int c = tid; c < bwp; c += kWG) rinv[c] = (c < bw) ? T(1) / lnz[lb[c] + c] : T(1);
   int32_t* pi = prepi + (int64_t)d.r0 * kPrepInts;
   for (int i = tid; i < bw; i += kWG) pi[i] = sperm[i];
-}
-
-// Value i (0 <= i < 128, wave-uniform) of a vector held two entries per lane
-// (entry i in lane i % 64 of y0 for i < 64, of y1 otherwise).
-template <typename T>
-__device__ inline T bcast2(T y0, T y1, int i) {
-  return rdlane(i < 64 ? y0 : y1, i & 63);
 }
 
 // Entry src (0 <= src < 128, per lane) of the same two-per-lane vector.
@@ -3820,7 +3699,6 @@ bwd_small_kernel(DevSym s, const SmallDesc* __restrict__ desc, SmallClasses k, L
     bwd_tiny<T, 8>(s, desc, ((int64_t)b * 4 + wave) * 8, k.cnt[3], lnz, unz, rhs, ldr, nrhs);
   }
 }
-
 
 // Backward chain of one block. The block's upper panels and diagonal
 // reciprocals come from the solve data in one coalesced load. With t =
