@@ -221,7 +221,8 @@ struct spkhip_handle {
   bool have_csc = false, pattern_error = false;
   // A's entries by front and column (pointers per front column, fvec[f] + j),
   // built with the pattern
-  std::vector<i64> aptr;
+  bool have_entries = false;
+  DevBuf<i64> d_aptr;
   DevBuf<spk::AEnt> d_aent;
   DevBuf<i64> d_rowptr;
   DevBuf<i32> d_colind;
@@ -1112,44 +1113,46 @@ void drop_repeated(i64 n, const i64* colptr, const i64* rowval, std::vector<i64>
 }
 
 // A's entries with their place in their front (AEnt), grouped by front and
-// column on the device, with pointers per front column (h->aptr, index
+// column on the device, with pointers per front column (d_aptr, index
 // fvec[f] + j). The rows of a column are distinct, so its entries' order,
 // which is not determined, does not matter. The front
 // fields of h->ds that the kernels use are those of upload_symbolic and
 // build_storage.
 void build_entries(spkhip_handle* h, const std::vector<i64>& amap) {
   const i64 nc = h->vec_elems;
+  const int nb = (int)((nc + spk::kScan - 1) / spk::kScan);
   hipStream_t st = h->stream;
-  DevBuf<i64> d_tmp;  // the counts, then the slot map
-  d_tmp.alloc(nc + 1 + h->nnz);
-  i64 *const d_cur = d_tmp.p, *const d_map = d_tmp.p + nc + 1;
+  DevBuf<i64> d_tmp;  // the columns' next free positions, the scan's parts, the slot map
+  d_tmp.alloc(nc + 1 + nb + h->nnz);
+  i64 *const d_cur = d_tmp.p, *const d_part = d_cur + nc + 1, *const d_map = d_part + nb;
+  h->d_aptr.alloc(nc + 1);
   if (h->nnz > 0)
     hipck(hipMemcpyAsync(d_map, amap.data(), h->nnz * sizeof(i64), hipMemcpyHostToDevice, st));
-  std::vector<i64> cur(nc + 1, 0);
   DevSym d = h->ds;
   h->d_fvec.upload(h->fvec, st);
   d.fvec = h->d_fvec.p;
-  hipLaunchKernelGGL(spk::fill_kernel<int64_t>, dim3(grid_for(nc + 1)), dim3(kWG), 0, st, d_cur,
-                     (int64_t)(nc + 1), (int64_t)0);
-  auto pass = [&](spk::AEnt* out) {
+  hipLaunchKernelGGL(spk::fill_kernel<int64_t>, dim3(grid_for(nc + 1)), dim3(kWG), 0, st,
+                     h->d_aptr.p, (int64_t)(nc + 1), (int64_t)0);
+  auto pass = [&](i64* cnt, spk::AEnt* out) {
     if (h->nnz > 0)
       hipLaunchKernelGGL(spk::front_entries_kernel, dim3(grid_for(h->nnz)), dim3(kWG), 0, st, d,
-                         d_map, h->nnz, d_cur, out);
-    hipck(hipGetLastError());
+                         d_map, h->nnz, cnt, out);
   };
-  pass(nullptr);
-  hipck(hipMemcpyAsync(cur.data(), d_cur, (nc + 1) * sizeof(i64), hipMemcpyDeviceToHost, st));
-  hipck(hipStreamSynchronize(st));
-  h->aptr.resize(nc + 1);
+  pass(h->d_aptr.p, nullptr);
+  hipLaunchKernelGGL(spk::scan_kernel<0>, dim3(nb), dim3(kWG), 0, st, h->d_aptr.p, nc, d_part, nb,
+                     d_cur);
+  hipLaunchKernelGGL(spk::scan_kernel<1>, dim3(1), dim3(kWG), 0, st, h->d_aptr.p, nc, d_part, nb,
+                     d_cur);
+  hipLaunchKernelGGL(spk::scan_kernel<2>, dim3(nb), dim3(kWG), 0, st, h->d_aptr.p, nc, d_part, nb,
+                     d_cur);
   i64 sum = 0;
-  for (i64 i = 0; i <= nc; ++i) {
-    h->aptr[i] = sum;
-    sum += cur[i];
-  }
-  h->d_aent.alloc(std::max<i64>(sum, 1));
-  hipck(hipMemcpyAsync(d_cur, h->aptr.data(), (nc + 1) * sizeof(i64), hipMemcpyHostToDevice, st));
-  pass(h->d_aent.p);
+  hipck(hipMemcpyAsync(&sum, h->d_aptr.p + nc, sizeof(i64), hipMemcpyDeviceToHost, st));
   hipck(hipStreamSynchronize(st));
+  h->d_aent.alloc(std::max<i64>(sum, 1));
+  pass(d_cur, h->d_aent.p);
+  hipck(hipGetLastError());
+  hipck(hipStreamSynchronize(st));
+  h->have_entries = true;
 }
 
 template <typename T>
@@ -1788,6 +1791,8 @@ void replan(spkhip_handle* h) {
     // the small fronts with their fields and children resolved
     std::vector<spk::SmallDesc> fr;
     std::vector<spk::SmallChild> chl;
+    fr.reserve(small.size() + 1);
+    chl.reserve(h->fch.size() + 1);
     for (i32 f : small) {
       spk::SmallDesc d{};
       d.cb = h->fcb[f];
@@ -1798,10 +1803,6 @@ void replan(spkhip_handle* h) {
       d.ind = h->xlindx[h->fsp0[f]] - 1;
       d.ch0 = (i32)chl.size();
       d.nch = h->fchp[f + 1] - h->fchp[f];
-      if (!h->aptr.empty()) {
-        d.a0 = h->aptr[h->fvec[f]];
-        d.an = (i32)(h->aptr[h->fvec[f] + d.L] - d.a0);
-      }
       for (i32 ci = h->fchp[f]; ci < h->fchp[f + 1]; ++ci) {
         const i32 c = h->fch[ci];
         chl.push_back(spk::SmallChild{h->fcb[c], h->frel[c], h->fvec[c], h->fL[c] - h->fW[c],
@@ -1812,6 +1813,11 @@ void replan(spkhip_handle* h) {
     if (fr.empty()) fr.push_back(spk::SmallDesc{});
     if (chl.empty()) chl.push_back(spk::SmallChild{});
     h->d_sdfr.upload(fr, st);
+    if (h->have_entries && !small.empty()) {
+      hipLaunchKernelGGL(spk::small_entries_kernel, dim3((small.size() + kWG - 1) / kWG), dim3(kWG),
+                         0, st, h->d_sdfr.p, (int)small.size(), h->d_aptr.p);
+      hipck(hipGetLastError());
+    }
     h->d_sdch.upload(chl, st);
   }
   if (it_front.empty()) {
@@ -1831,14 +1837,13 @@ void replan(spkhip_handle* h) {
     // the assembly's items with their front's fields, and each child entry's
     // update column and map, resolved here so that the kernels start with
     // one dependent read
-    if (!h->aptr.empty()) {
-      std::vector<spk::AsmItem> ini(it_front.size());
-      for (size_t i = 0; i < it_front.size(); ++i) {
-        const i32 f = it_front[i], j = it_col[i], L = h->fL[f];
-        const i64* ap = h->aptr.data() + h->fvec[f] + j;
-        ini[i] = spk::AsmItem{h->foff[f] + (i64)j * L, ap[0], L, (i32)(ap[1] - ap[0])};
-      }
-      h->d_it_asm.upload(ini, st);
+    if (h->have_entries) {
+      const i64 ni = (i64)it_front.size();
+      h->d_it_asm.alloc(ni);
+      hipLaunchKernelGGL(spk::asm_items_kernel, dim3(grid_for(ni)), dim3(kWG), 0, st,
+                         h->d_it_front.p, h->d_it_col.p, ni, h->d_fL.p, h->d_foff.p, h->d_fvec.p,
+                         h->d_aptr.p, h->d_it_asm.p);
+      hipck(hipGetLastError());
     } else {
       std::vector<spk::InitItem> ini(it_front.size());
       for (size_t i = 0; i < it_front.size(); ++i) {
@@ -1912,7 +1917,7 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
                      const i64* colptr = nullptr, const i64* rowval = nullptr) {
   auto t0 = Clock::now();
   hipck(hipSetDevice(h->device));
-  h->aptr.clear();
+  h->have_entries = false;
   h->kind = kind;
   h->n = n;
   h->nsuper = nsuper;

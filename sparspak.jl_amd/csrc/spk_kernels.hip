@@ -78,6 +78,88 @@ __global__ void front_entries_kernel(DevSym s, const int64_t* __restrict__ amap,
   }
 }
 
+// Exclusive sums of cnt[0 .. n) in place, cnt[n] their total, and a copy of
+// them (the columns' next free positions), in three launches: workgroup b's
+// total of its kScan elements (PART 0), the totals' exclusive sums by one
+// workgroup (1), the elements' (2). Once per pattern.
+constexpr int kScan = 4096;
+template <int PART>
+__global__ void __launch_bounds__(kWG)
+scan_kernel(int64_t* __restrict__ cnt, int64_t n, int64_t* __restrict__ part, int nb,
+            int64_t* __restrict__ copy) {
+  __shared__ int64_t sh[kWG];
+  const int tid = threadIdx.x;
+  // exclusive sums of v over the workgroup's threads; total: all of them
+  auto scan = [&](int64_t v, int64_t& total) {
+    sh[tid] = v;
+    __syncthreads();
+    for (int o = 1; o < kWG; o *= 2) {
+      const int64_t x = tid >= o ? sh[tid - o] : 0;
+      __syncthreads();
+      sh[tid] += x;
+      __syncthreads();
+    }
+    total = sh[kWG - 1];
+    const int64_t r = sh[tid] - v;
+    __syncthreads();
+    return r;
+  };
+  int64_t total;
+  if constexpr (PART == 1) {
+    int64_t base = 0;
+    for (int i0 = 0; i0 < nb; i0 += kWG) {
+      const int i = i0 + tid;
+      const int64_t v = i < nb ? part[i] : 0;
+      const int64_t x = scan(v, total);
+      if (i < nb) part[i] = base + x;
+      base += total;
+    }
+    if (tid == 0) cnt[n] = copy[n] = base;
+  } else {
+    constexpr int E = kScan / kWG;
+    const int64_t b0 = (int64_t)blockIdx.x * kScan + tid * E;
+    int64_t v[E], sum = 0;
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      v[k] = b0 + k < n ? cnt[b0 + k] : 0;
+      sum += v[k];
+    }
+    int64_t x = scan(sum, total);
+    if constexpr (PART == 0) {
+      if (tid == 0) part[blockIdx.x] = total;
+    } else {
+      x += part[blockIdx.x];
+#pragma unroll
+      for (int k = 0; k < E; ++k) {
+        if (b0 + k < n) cnt[b0 + k] = copy[b0 + k] = x;
+        x += v[k];
+      }
+    }
+  }
+}
+
+// The assembly's items and the small fronts' entries from the columns'
+// pointers (aptr, index fvec[f] + column).
+__global__ void asm_items_kernel(const int32_t* __restrict__ front, const int32_t* __restrict__ col,
+                                 int64_t n, const int32_t* __restrict__ fL,
+                                 const int64_t* __restrict__ foff, const int64_t* __restrict__ fvec,
+                                 const int64_t* __restrict__ aptr, AsmItem* __restrict__ out) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (; i < n; i += stride) {
+    const int f = front[i], j = col[i], L = fL[f];
+    const int64_t a0 = aptr[fvec[f] + j];
+    out[i] = AsmItem{foff[f] + (int64_t)j * L, a0, L, (int32_t)(aptr[fvec[f] + j + 1] - a0)};
+  }
+}
+__global__ void small_entries_kernel(SmallDesc* __restrict__ d, int n,
+                                     const int64_t* __restrict__ aptr) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  d[i].a0 = aptr[d[i].fvec];
+  d[i].an = (int32_t)(aptr[d[i].fvec + d[i].L] - d[i].a0);
+}
+
 // ---------------------------------------------------------------------------
 // Large fronts: the L x L work matrix lives in the arena.
 // ---------------------------------------------------------------------------
