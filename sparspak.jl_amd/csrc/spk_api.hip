@@ -1021,8 +1021,9 @@ int host_threads(i64 work) {
   return std::max(1, std::min(t, 16));
 }
 
+// ascend: whether every column's rows ascend (no entry is repeated).
 void build_amap(spkhip_handle* h, const i64* colptr, const i64* rowval,
-                std::vector<i64>& amap, int nthreads = 0) {
+                std::vector<i64>& amap, int nthreads = 0, bool* ascend = nullptr) {
   const i64 n = h->n;
   amap.assign(h->nnz, -1);
   h->pattern_error = false;
@@ -1042,11 +1043,14 @@ void build_amap(spkhip_handle* h, const i64* colptr, const i64* rowval,
   };
   // columns [c0, c1): every entry's slot depends on that entry alone, so the
   // columns split across threads give the same map as one pass
-  auto columns = [&](i64 c0, i64 c1, bool* err) {
+  auto columns = [&](i64 c0, i64 c1, bool* err, bool* asc) {
     for (i64 i = c0; i < c1; ++i) {
+      i64 before = 0;
       for (i64 iptr = colptr[i - 1]; iptr <= colptr[i] - 1; ++iptr) {
         i64 k = iptr - 1;
         i64 orow = rowval[k];
+        *asc = *asc && orow > before;
+        before = orow;
         if (h->kind == SPKHIP_KIND_SPD && orow < i) continue;
         i64 inew = h->invp[orow - 1];
         i64 jnew = h->invp[i - 1];
@@ -1069,9 +1073,10 @@ void build_amap(spkhip_handle* h, const i64* colptr, const i64* rowval,
   };
   const int nt = nthreads > 0 ? nthreads : host_threads(h->nnz);
   if (nt <= 1) {
-    bool err = false;
-    columns(1, n + 1, &err);
+    bool err = false, asc = true;
+    columns(1, n + 1, &err, &asc);
     h->pattern_error = err;
+    if (ascend) *ascend = asc;
     return;
   }
   // column ranges of about nnz / nt entries each
@@ -1082,16 +1087,18 @@ void build_amap(spkhip_handle* h, const i64* colptr, const i64* rowval,
     while (i <= n && colptr[i - 1] < target) ++i;
     cut[t] = std::max<i64>(i, cut[t - 1]);
   }
-  std::vector<char> errs(nt, 0);
+  std::vector<char> errs(nt, 0), ascs(nt, 1);
   std::vector<std::thread> pool;
   for (int t = 0; t < nt; ++t)
     pool.emplace_back([&, t]() {
-      bool e = false;
-      columns(cut[t], cut[t + 1], &e);
+      bool e = false, a = true;
+      columns(cut[t], cut[t + 1], &e, &a);
       errs[t] = e ? 1 : 0;
+      ascs[t] = a ? 1 : 0;
     });
   for (auto& th : pool) th.join();
   for (char e : errs) h->pattern_error = h->pattern_error || e;
+  if (ascend) *ascend = std::all_of(ascs.begin(), ascs.end(), [](char a) { return a != 0; });
 }
 
 // Entries that A repeats take their last value: the earlier ones lose their
@@ -1770,9 +1777,10 @@ void factor_run(spkhip_handle* h) {
 // Storage, launch plan and their device copies: everything that depends on
 // the plan knobs (small_lmax, block_cols, upd_group). Rebuilt when they
 // change; the factor must be recomputed afterwards.
-void replan(spkhip_handle* h) {
+// stored: the storage is laid out already.
+void replan(spkhip_handle* h, bool stored = false) {
   hipStream_t st = h->stream;
-  build_storage(h);
+  if (!stored) build_storage(h);
   h->d_foff.upload(h->foff, st);
   h->d_fcb.upload(h->fcb, st);
   h->d_fcbld.upload(h->fcbld, st);
@@ -2044,11 +2052,12 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
     h->nnz = colptr[n] - 1;
     build_storage(h);
     std::vector<i64> amap;
-    build_amap(h, colptr, rowval, amap);
-    drop_repeated(n, colptr, rowval, amap);
+    bool ascend = true;
+    build_amap(h, colptr, rowval, amap, 0, &ascend);
+    if (!ascend) drop_repeated(n, colptr, rowval, amap);
     build_entries(h, amap);
   }
-  replan(h);
+  replan(h, h->have_entries);
   h->have_sym = true;
   h->have_csc = false;
   h->have_values = false;
