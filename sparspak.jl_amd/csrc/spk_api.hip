@@ -1124,15 +1124,18 @@ void drop_repeated(i64 n, const i64* colptr, const i64* rowval, std::vector<i64>
 // fvec[f] + j). The rows of a column are distinct, so its entries' order,
 // which is not determined, does not matter. The front
 // fields of h->ds that the kernels use are those of upload_symbolic and
-// build_storage.
+// build_storage. The slot map takes the place of d_csc2csr, which is uploaded
+// afterwards, and the scan's scratch lies behind the pointers, so that nothing
+// is allocated and freed for them.
 void build_entries(spkhip_handle* h, const std::vector<i64>& amap) {
   const i64 nc = h->vec_elems;
   const int nb = (int)((nc + spk::kScan - 1) / spk::kScan);
   hipStream_t st = h->stream;
-  DevBuf<i64> d_tmp;  // the columns' next free positions, the scan's parts, the slot map
-  d_tmp.alloc(nc + 1 + nb + h->nnz);
-  i64 *const d_cur = d_tmp.p, *const d_part = d_cur + nc + 1, *const d_map = d_part + nb;
-  h->d_aptr.alloc(nc + 1);
+  h->d_aptr.alloc(2 * (nc + 1) + nb);
+  h->d_csc2csr.alloc(h->nnz);
+  // the columns' next free positions, the scan's parts, the slot map
+  i64 *const d_cur = h->d_aptr.p + nc + 1, *const d_part = d_cur + nc + 1,
+      *const d_map = h->d_csc2csr.p;
   if (h->nnz > 0)
     hipck(hipMemcpyAsync(d_map, amap.data(), h->nnz * sizeof(i64), hipMemcpyHostToDevice, st));
   DevSym d = h->ds;
@@ -1158,7 +1161,6 @@ void build_entries(spkhip_handle* h, const std::vector<i64>& amap) {
   h->d_aent.alloc(std::max<i64>(sum, 1));
   pass(d_cur, h->d_aent.p);
   hipck(hipGetLastError());
-  hipck(hipStreamSynchronize(st));
   h->have_entries = true;
 }
 
@@ -1777,14 +1779,14 @@ void factor_run(spkhip_handle* h) {
 // Storage, launch plan and their device copies: everything that depends on
 // the plan knobs (small_lmax, block_cols, upd_group). Rebuilt when they
 // change; the factor must be recomputed afterwards.
-// stored: the storage is laid out already.
+// stored: the storage is laid out and fvec uploaded already (with the entries).
 void replan(spkhip_handle* h, bool stored = false) {
   hipStream_t st = h->stream;
   if (!stored) build_storage(h);
   h->d_foff.upload(h->foff, st);
   h->d_fcb.upload(h->fcb, st);
   h->d_fcbld.upload(h->fcbld, st);
-  h->d_fvec.upload(h->fvec, st);
+  if (!stored) h->d_fvec.upload(h->fvec, st);
   std::vector<i32> small, it_front, it_col, ea_child, ea_t, solve, largel, ut_front, ut_piece,
       ut_r0;
   std::vector<spk::SolveDesc> sdesc;
@@ -1925,7 +1927,7 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
                      const i64* colptr = nullptr, const i64* rowval = nullptr) {
   auto t0 = Clock::now();
   hipck(hipSetDevice(h->device));
-  h->have_entries = false;
+  h->have_entries = h->have_csc = false;
   h->kind = kind;
   h->n = n;
   h->nsuper = nsuper;
