@@ -545,7 +545,7 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
     // (SPKHIP_DIAG_SLAB=0 keeps the LDS form; an SPD step with a wider
     // block, a piece of more than 64 columns, takes the LDS form), and each
     // in-group update beside the next block's regions (SPKHIP_MERGE_BORDER=0:
-    // after them; not before an SPD step with a wider block)
+    // after them; not of a wider SPD block, nor before an SPD step with one)
     const char* ds = std::getenv("SPKHIP_DIAG_SLAB");
     const char* mb = std::getenv("SPKHIP_MERGE_BORDER");
     h->slab_plan = h->block_cols <= 64 && !(ds && ds[0] == '0');
@@ -839,9 +839,10 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
         if (gi + 1 < ge) {
           // border of the group's remaining blocks [B.c1, E) x ..., E = their end
           const i32 E = fblocks[fi][ge - 1].c1;
-          if (h->merge_plan && !wide_step[gi + 1]) {
+          if (h->merge_plan && !wide_step[gi + 1] && B.c1 - B.c0 <= spk::kFoldMax) {
             // all of it but the next block's diagonal region, which the
-            // next step's diagonal kernel takes itself, beside the rest
+            // next step's diagonal kernel takes itself (a product of at most
+            // kFoldMax columns), beside the rest
             const i32 cn = fblocks[fi][gi + 1].c1;
             rect(f, B.c0, B.c1, cn, L, B.c1, E, 2);
             rect(f, B.c0, B.c1, B.c1, cn, cn, E, 2);

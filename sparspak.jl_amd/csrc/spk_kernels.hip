@@ -1406,6 +1406,7 @@ small_front_kernel(DevSym s, const SmallDesc* __restrict__ desc,
 // the folded panels.
 constexpr int kMaxBlkPieces = 8;  // most pieces in one block
 constexpr int kFoldK = 32;        // folded columns per step
+constexpr int kFoldMax = 2 * kFoldK;  // most folded columns (the plan merges no more)
 __host__ __device__ constexpr int slab_elems(int bw, int w0, bool fold) {
   const int own = bw * bw + (bw - w0) * (bw - w0);
   return fold && own < 2 * kFoldK * 64 ? 2 * kFoldK * 64 : own;
@@ -1454,8 +1455,8 @@ __device__ __attribute__((always_inline)) void blk_diag_slab_body(
   auto usw = [](int c) {
     return std::is_same<T, double>::value ? 2 * (c & 15) : 4 * ((c >> 1) & 7);
   };
-  // both steps' panels (a block has at most 64 columns) from clamped
-  // addresses, in flight with the region; what lies outside is zeroed below
+  // both steps' panels (kFoldMax columns at most) from clamped addresses, in
+  // flight with the region; what lies outside is zeroed below
   T pl[2][8], pu[2][8];
   if (fkw > 0) {
     const T* lrow = Fb + c0 + min(lane, bw - 1) + (int64_t)d.fk0 * L;
