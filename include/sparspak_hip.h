@@ -165,6 +165,8 @@ int64_t spkhip_destroy(spkhip_t h);
  * SpkSparseBase.jl:193-251 (kind LU) / SpkSparseSpdBase.jl:178-232 (SPD).
  * colptr/rowval: the CSC pattern of A in the ORIGINAL numbering
  * (SparseCSCInterface.jl:101-169 reads the same arrays); nnz = colptr[n]-1.
+ * An entry that a column stores more than once takes its last value, in the
+ * factor and in the refinement's residual and norms.
  * Returns -1 ("No space for matrix element") if an entry of A falls outside
  * the symbolic structure. */
 int64_t spkhip_symbolic_upload(spkhip_t h, int64_t kind, int64_t n,

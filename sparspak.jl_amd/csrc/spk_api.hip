@@ -1102,9 +1102,11 @@ void build_amap(spkhip_handle* h, const i64* colptr, const i64* rowval,
   if (ascend) *ascend = std::all_of(ascs.begin(), ascs.end(), [](char a) { return a != 0; });
 }
 
-// Entries that A repeats take their last value: the earlier ones lose their
-// slot. (Only columns whose rows do not ascend can hold any.)
-void drop_repeated(i64 n, const i64* colptr, const i64* rowval, std::vector<i64>& amap) {
+// Entries that A repeats take their last value: the earlier ones, listed here
+// in ascending order, belong neither to the factor nor to the residual's
+// matrix. (Only columns whose rows do not ascend can hold any.)
+std::vector<i64> repeated_entries(i64 n, const i64* colptr, const i64* rowval) {
+  std::vector<i64> rep;
   std::vector<i64> last;  // per row, the last entry seen of the column
   for (i64 i = 0; i < n; ++i) {
     const i64 k0 = colptr[i] - 1, k1 = colptr[i + 1] - 1;
@@ -1114,10 +1116,12 @@ void drop_repeated(i64 n, const i64* colptr, const i64* rowval, std::vector<i64>
     if (last.empty()) last.assign(n, -1);
     for (i64 k = k0; k < k1; ++k) {
       i64& l = last[rowval[k] - 1];
-      if (l >= k0) amap[l] = -1;
+      if (l >= k0) rep.push_back(l);
       l = k;
     }
   }
+  std::sort(rep.begin(), rep.end());
+  return rep;
 }
 
 // A's entries with their place in their front (AEnt), grouped by front and
@@ -1925,7 +1929,8 @@ void replan(spkhip_handle* h, bool stored = false) {
 void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i64* xsuper,
                      const i64* snode, const i64* xlindx, const i64* lindx, const i64* xlnz,
                      const i64* xunz, const i64* perm, const i64* invp,
-                     const i64* colptr = nullptr, const i64* rowval = nullptr) {
+                     const i64* colptr = nullptr, const i64* rowval = nullptr,
+                     std::vector<i64>* repeats = nullptr) {
   auto t0 = Clock::now();
   hipck(hipSetDevice(h->device));
   h->have_entries = h->have_csc = false;
@@ -2057,7 +2062,10 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
     std::vector<i64> amap;
     bool ascend = true;
     build_amap(h, colptr, rowval, amap, 0, &ascend);
-    if (!ascend) drop_repeated(n, colptr, rowval, amap);
+    std::vector<i64> rep;
+    if (!ascend) rep = repeated_entries(n, colptr, rowval);
+    for (i64 k : rep) amap[k] = -1;
+    if (repeats) repeats->swap(rep);
     build_entries(h, amap);
   }
   replan(h, h->have_entries);
@@ -2280,20 +2288,23 @@ int64_t spkhip_symbolic_upload(spkhip_t h, int64_t kind, int64_t n, int64_t nsup
     return -4;
   if (kind != SPKHIP_KIND_LU && kind != SPKHIP_KIND_SPD) return -4;
   return wrap([&]() -> int64_t {
+    std::vector<i64> rep;  // A's repeated entries
     upload_symbolic(h, kind, n, nsuper, xsuper, snode, xlindx, lindx, xlnz, xunz, perm, invp,
-                    colptr, rowval);
+                    colptr, rowval, &rep);
     if (colptr && rowval) {
       auto t0 = Clock::now();
       hipStream_t st = h->stream;
       // CSR of A (original numbering) for the residual: rowptr, colind and
-      // the CSC -> CSR value permutation
-      std::vector<i64> rowptr(n + 1, 0), c2r(h->nnz);
+      // the CSC -> CSR value permutation (-1: a repeated entry, left out)
+      std::vector<i64> rowptr(n + 1, 0), c2r(h->nnz, 0);
       std::vector<i32> colind(h->nnz);
-      for (i64 k = 0; k < h->nnz; ++k) rowptr[rowval[k]]++;
+      for (i64 k : rep) c2r[k] = -1;
+      for (i64 k = 0; k < h->nnz; ++k) rowptr[rowval[k]] += c2r[k] + 1;
       for (i64 i = 0; i < n; ++i) rowptr[i + 1] += rowptr[i];
       std::vector<i64> fillp(rowptr.begin(), rowptr.end() - 1);
       for (i64 j = 1; j <= n; ++j)
         for (i64 k = colptr[j - 1] - 1; k < colptr[j] - 1; ++k) {
+          if (c2r[k] < 0) continue;
           i64 r = rowval[k] - 1;
           i64 d = fillp[r]++;
           colind[d] = (i32)(j - 1);
@@ -2313,13 +2324,16 @@ int64_t spkhip_symbolic_upload(spkhip_t h, int64_t kind, int64_t n, int64_t nsup
 }  // extern "C"
 
 namespace {
-// value set blockIdx.y: its nnz values in both orders nnz further
+// value set blockIdx.y: its nnz values in both orders nnz further (c2r -1: an
+// entry that is not in the CSR)
 __global__ void csr_values_kernel(const double* __restrict__ nz, const int64_t* __restrict__ c2r,
                                   double* __restrict__ csr, int64_t nnz) {
   nz += (int64_t)blockIdx.y * nnz;
   csr += (int64_t)blockIdx.y * nnz;
   int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < nnz) csr[c2r[k]] = nz[k];
+  if (k >= nnz) return;
+  const int64_t d = c2r[k];
+  if (d >= 0) csr[d] = nz[k];
 }
 
 int64_t inmatrix_common(spkhip_t h) {
