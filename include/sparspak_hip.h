@@ -168,7 +168,8 @@ int64_t spkhip_destroy(spkhip_t h);
  * An entry that a column stores more than once takes its last value, in the
  * factor and in the refinement's residual and norms.
  * Returns -1 ("No space for matrix element") if an entry of A falls outside
- * the symbolic structure. */
+ * the symbolic structure. A refused upload (any other negative code) leaves
+ * the handle without a symbolic factor, also if it held one before. */
 int64_t spkhip_symbolic_upload(spkhip_t h, int64_t kind, int64_t n,
                                int64_t nsuper, const int64_t* xsuper,
                                const int64_t* snode, const int64_t* xlindx,

@@ -1933,7 +1933,9 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
                      std::vector<i64>* repeats = nullptr) {
   auto t0 = Clock::now();
   hipck(hipSetDevice(h->device));
-  h->have_entries = h->have_csc = false;
+  // nothing is held until all of it is there: a refused upload must not leave
+  // an earlier one's plan or factor beside half of its own arrays
+  h->have_sym = h->have_entries = h->have_csc = h->have_values = h->factored = false;
   h->kind = kind;
   h->n = n;
   h->nsuper = nsuper;
@@ -2070,8 +2072,6 @@ void upload_symbolic(spkhip_handle* h, int64_t kind, i64 n, i64 nsuper, const i6
   }
   replan(h, h->have_entries);
   h->have_sym = true;
-  h->have_csc = false;
-  h->have_values = false;
   h->t_upload = ms_since(t0);
 }
 
