@@ -3044,8 +3044,11 @@ bwd_bgemv_kernel(DevSym s, const SolveDesc* __restrict__ desc, int ndesc,
 
 // b / u from r = 1 / u (correctly rounded): q0 = b r, then one correction
 // with the exact remainder b - q0 u (an FMA) gives the correctly rounded
-// quotient b / u, as the division itself (Markstein's theorem; no overflow
-// or underflow assumed), in three dependent operations.
+// quotient b / u, as the division itself (Markstein's theorem), in three
+// dependent operations. Where r or the quotient overflows (u subnormal or
+// infinite, b infinite or NaN) the result is NaN or infinite: solves of small
+// fronts that end with such an entry are done again with the division itself
+// (quot<true>).
 __device__ inline double div_r(double b, double u, double r) {
   const double q0 = b * r;
   return __builtin_fma(__builtin_fma(-q0, u, b), r, q0);
@@ -3053,6 +3056,13 @@ __device__ inline double div_r(double b, double u, double r) {
 __device__ inline float div_r(float b, float u, float r) {
   const float q0 = b * r;
   return __builtin_fmaf(__builtin_fmaf(-q0, u, b), r, q0);
+}
+template <bool DIV, typename T>
+__device__ inline T quot(T b, T u, T r) {
+  if constexpr (DIV)
+    return b / u;
+  else
+    return div_r(b, u, r);
 }
 
 // Small fronts, solves. A front's right-hand sides are taken by one wave, QB
@@ -3328,7 +3338,7 @@ __device__ __attribute__((always_inline)) void bwd_tiny(
   const T* pl = lnz + (own ? s.lcol[fc0 + r] + r - (int64_t)r * ldp : 0);
   const T* pu = unz + (own ? s.ucol[fc0 + r] : 0);
   const int wm = -wave_min(-W), lm = -wave_min(-L);
-  T y = r < L ? rhs[(int64_t)q * ldr + idx] : T(0);
+  const T b = r < L ? rhs[(int64_t)q * ldr + idx] : T(0);
   T v[SW], dg = T(1);
   static_for<SW>([&](auto jc) __attribute__((always_inline)) {
     constexpr int j = decltype(jc)::value;
@@ -3340,23 +3350,30 @@ __device__ __attribute__((always_inline)) void bwd_tiny(
     }
   });
   const T ri = T(1) / dg;
-  static_for<SW>([&](auto jc) __attribute__((always_inline)) {
-    constexpr int j = SW - 1 - decltype(jc)::value;
-    if (j < lm) {
-      const T yk = bcast<SW, j>(y);
-      if (j >= wm) {  // an update column of every front of the wave
-        const T t = y - v[j] * yk;
-        y = own && j < L ? t : y;
-      } else {
-        const T xk = bcast<SW, j>(div_r(y, dg, ri));
-        const T t = y - v[j] * (j >= W ? yk : xk);
-        if (j >= W)
+  auto sweep = [&](auto div) __attribute__((always_inline)) {
+    T y = b;
+    static_for<SW>([&](auto jc) __attribute__((always_inline)) {
+      constexpr int j = SW - 1 - decltype(jc)::value;
+      if (j < lm) {
+        const T yk = bcast<SW, j>(y);
+        if (j >= wm) {  // an update column of every front of the wave
+          const T t = y - v[j] * yk;
           y = own && j < L ? t : y;
-        else
-          y = yk == T(0) ? y : r < j ? t : r == j ? xk : y;
+        } else {
+          const T xk = bcast<SW, j>(quot<decltype(div)::value>(y, dg, ri));
+          const T t = y - v[j] * (j >= W ? yk : xk);
+          if (j >= W)
+            y = own && j < L ? t : y;
+          else
+            y = yk == T(0) ? y : r < j ? t : r == j ? xk : y;
+        }
       }
-    }
-  });
+    });
+    return y;
+  };
+  T y = sweep(std::false_type{});
+  if (__builtin_expect(__ballot(own && !__builtin_isfinite(y)) != 0, 0))
+    y = sweep(std::true_type{});
   if (own) rhs[(int64_t)q * ldr + fc0 + r] = y;
 }
 
@@ -3487,46 +3504,53 @@ __device__ __attribute__((always_inline)) void bwd_small_many(
     const int q = q0 + ql;
     const bool on = q < nrhs;
     T y[NR];
+    auto sweep = [&](auto div) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int r = g + G * i;
-      y[i] = (on && r < L) ? rhs[(int64_t)q * ldr + s.lindx[d.ind + r] - 1] : T(0);
-    }
-    T u[NR];  // the column's rows, read one column ahead
-    auto column = [&](int j) {
+      for (int i = 0; i < NR; ++i) {
+        const int r = g + G * i;
+        y[i] = (on && r < L) ? rhs[(int64_t)q * ldr + s.lindx[d.ind + r] - 1] : T(0);
+      }
+      T u[NR];  // the column's rows, read one column ahead
+      auto column = [&](int j) {
 #pragma unroll
-      for (int i = 0; i < NR; ++i)
-        u[i] = G * i < W ? S[max(j, 0) * LDW + min(g + G * i, W - 1)] : T(0);
-    };
-    column(L - 1);
-    static_for<NR>([&](auto jc) __attribute__((always_inline)) {
-      constexpr int jb = NR - 1 - decltype(jc)::value;
+        for (int i = 0; i < NR; ++i)
+          u[i] = G * i < W ? S[max(j, 0) * LDW + min(g + G * i, W - 1)] : T(0);
+      };
+      column(L - 1);
+      static_for<NR>([&](auto jc) __attribute__((always_inline)) {
+        constexpr int jb = NR - 1 - decltype(jc)::value;
 #pragma unroll 1
-      for (int gg = min(G, L - G * jb) - 1; gg >= 0; --gg) {
-        const int j = G * jb + gg;
-        const T yk = bperm(y[jb], gg * QL + ql);
-        T c[NR];
+        for (int gg = min(G, L - G * jb) - 1; gg >= 0; --gg) {
+          const int j = G * jb + gg;
+          const T yk = bperm(y[jb], gg * QL + ql);
+          T c[NR];
 #pragma unroll
-        for (int i = 0; i <= jb; ++i) c[i] = u[i];
-        column(j - 1);
-        if (j >= W) {
+          for (int i = 0; i <= jb; ++i) c[i] = u[i];
+          column(j - 1);
+          if (j >= W) {
 #pragma unroll
-          for (int i = 0; i <= jb; ++i) {
-            const T t = y[i] - c[i] * yk;
-            y[i] = g + G * i < W ? t : y[i];
-          }
-        } else {
-          const T xk = div_r(yk, rdlane(dg, j), rdlane(ri, j));
-          const bool nz = yk != T(0);  // a zero entry stays, as in the reference
+            for (int i = 0; i <= jb; ++i) {
+              const T t = y[i] - c[i] * yk;
+              y[i] = g + G * i < W ? t : y[i];
+            }
+          } else {
+            const T xk = quot<decltype(div)::value>(yk, rdlane(dg, j), rdlane(ri, j));
+            const bool nz = yk != T(0);  // a zero entry stays, as in the reference
 #pragma unroll
-          for (int i = 0; i <= jb; ++i) {
-            const int r = g + G * i;
-            const T t = y[i] - c[i] * xk;
-            y[i] = nz && r < j ? t : nz && r == j ? xk : y[i];
+            for (int i = 0; i <= jb; ++i) {
+              const int r = g + G * i;
+              const T t = y[i] - c[i] * xk;
+              y[i] = nz && r < j ? t : nz && r == j ? xk : y[i];
+            }
           }
         }
-      }
-    });
+      });
+      bool finite = true;
+#pragma unroll
+      for (int i = 0; i < NR; ++i) finite = finite && (g + G * i >= W || __builtin_isfinite(y[i]));
+      return __ballot(!finite) == 0;
+    };
+    if (__builtin_expect(!sweep(std::false_type{}), 0)) sweep(std::true_type{});
 #pragma unroll
     for (int i = 0; i < NR; ++i)
       if (on && g + G * i < W) rhs[(int64_t)q * ldr + d.fc0 + g + G * i] = y[i];
@@ -3678,49 +3702,56 @@ __device__ __attribute__((always_inline)) void bwd_small_wave(
   for (; q0 < nrhs; q0 += qstep) {
     const int nq = min(QB, nrhs - q0);
     T y[QB];
+    auto sweep = [&](auto div) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < QB; ++q) {
-      y[q] = T(0);
-      if (q < nq && lane < L) y[q] = rhs[(int64_t)(q0 + q) * ldr + idx];
-    }
-    constexpr int CH = 4;  // columns read ahead
-    T sv[CH];
-    auto columns = [&](int j0) {
+      for (int q = 0; q < QB; ++q) {
+        y[q] = T(0);
+        if (q < nq && lane < L) y[q] = rhs[(int64_t)(q0 + q) * ldr + idx];
+      }
+      constexpr int CH = 4;  // columns read ahead
+      T sv[CH];
+      auto columns = [&](int j0) {
 #pragma unroll
-      for (int u = 0; u < CH; ++u) sv[u] = S[max(j0 - u, 0) * LDW + cl];
-    };
-    columns(L - 1);
-    for (int j0 = L - 1; j0 >= 0; j0 -= CH) {
-      T c[CH];
+        for (int u = 0; u < CH; ++u) sv[u] = S[max(j0 - u, 0) * LDW + cl];
+      };
+      columns(L - 1);
+      for (int j0 = L - 1; j0 >= 0; j0 -= CH) {
+        T c[CH];
 #pragma unroll
-      for (int u = 0; u < CH; ++u) c[u] = sv[u];
-      if (j0 >= CH) columns(j0 - CH);
+        for (int u = 0; u < CH; ++u) c[u] = sv[u];
+        if (j0 >= CH) columns(j0 - CH);
 #pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const int j = j0 - u;
-        if (j < 0) break;
-        if (j >= W) {
+        for (int u = 0; u < CH; ++u) {
+          const int j = j0 - u;
+          if (j < 0) break;
+          if (j >= W) {
 #pragma unroll
-          for (int q = 0; q < QB; ++q)
-            if (q < nq) {
-              const T xk = rdlane(y[q], j);
-              const T t = y[q] - c[u] * xk;
-              y[q] = own ? t : y[q];
-            }
-        } else {
-#pragma unroll
-          for (int q = 0; q < QB; ++q)
-            if (q < nq) {
-              const T xq = div_r(y[q], dg, ri);
-              const T yk = rdlane(y[q], j), xk = rdlane(xq, j);
-              if (yk != T(0)) {  // a zero entry stays, as in the reference
+            for (int q = 0; q < QB; ++q)
+              if (q < nq) {
+                const T xk = rdlane(y[q], j);
                 const T t = y[q] - c[u] * xk;
-                y[q] = lane < j ? t : lane == j ? xk : y[q];
+                y[q] = own ? t : y[q];
               }
-            }
+          } else {
+#pragma unroll
+            for (int q = 0; q < QB; ++q)
+              if (q < nq) {
+                const T xq = quot<decltype(div)::value>(y[q], dg, ri);
+                const T yk = rdlane(y[q], j), xk = rdlane(xq, j);
+                if (yk != T(0)) {  // a zero entry stays, as in the reference
+                  const T t = y[q] - c[u] * xk;
+                  y[q] = lane < j ? t : lane == j ? xk : y[q];
+                }
+              }
+          }
         }
       }
-    }
+      bool finite = true;
+#pragma unroll
+      for (int q = 0; q < QB; ++q) finite = finite && __builtin_isfinite(y[q]);
+      return __ballot(own && !finite) == 0;
+    };
+    if (__builtin_expect(!sweep(std::false_type{}), 0)) sweep(std::true_type{});
 #pragma unroll
     for (int q = 0; q < QB; ++q)
       if (q < nq && own) rhs[(int64_t)(q0 + q) * ldr + d.fc0 + lane] = y[q];
