@@ -3068,7 +3068,13 @@ __device__ inline T quot(T b, T u, T r) {
 // Small fronts, solves. A front's right-hand sides are taken by one wave, QB
 // at a time, lane = row, every right-hand side's vector in a register: column
 // j's entry of each is broadcast (readlane) and every row below (forward) or
-// above (backward) subtracts its product. Chains of W (L) such steps bound
+// above (backward) subtracts its product: from its entry inside the column's
+// piece, from a sum that starts at zero outside it, which joins the entry where
+// the piece ends (forward) or the row's own begins (backward). So a row's
+// products are summed before they meet its entry, as the reference sums them
+// (a product alone can be less than the entry's last place); subtracted one
+// by one from the entry they cost 6 % in the error of 128 small systems. Chains
+// of W (L) such steps bound
 // them; the columns' factor entries are read ahead of them (forward: eight
 // columns from lnz, whose rows are contiguous; backward: the front's U rows
 // staged in LDS by columns). Each right-hand side receives the same
@@ -3153,6 +3159,10 @@ __device__ __attribute__((always_inline)) void fwd_small_wave(
       for (int q = 0; q < QB; ++q) y[q] = Y[q * 64 + lane];
       wave_lds_sync();
     }
+    int pe = 0;  // the end of the piece at hand; rows from there on: summed
+    T base[QB];  // ... from zero in y, their entry here (zero for the others)
+#pragma unroll
+    for (int q = 0; q < QB; ++q) base[q] = T(0);
     T lv[CH];
     auto columns = [&](int j0) {
 #pragma unroll
@@ -3163,40 +3173,51 @@ __device__ __attribute__((always_inline)) void fwd_small_wave(
       }
     };
     columns(0);
-    for (int j0 = 0; j0 < W; j0 += CH) {
+    for (int j0 = 0; j0 < W;) {
+      if (j0 == pe) {  // a piece begins
+#pragma unroll
+        for (int q = 0; q < QB; ++q) y[q] = base[q] + y[q];
+        pe = __builtin_amdgcn_readlane(ce, j0);
+        unsigned long long m = swaps & (~0ull << j0) & (pe < 64 ? (1ull << pe) - 1 : ~0ull);
+        while (m) {
+          const int k = __ffsll((long long)m) - 1, p = __builtin_amdgcn_readlane(kp, k);
+          m &= m - 1;
+#pragma unroll
+          for (int q = 0; q < QB; ++q) {
+            const T a = rdlane(y[q], k), b = rdlane(y[q], p);
+            y[q] = lane == k ? b : lane == p ? a : y[q];
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+          base[q] = lane >= pe ? y[q] : T(0);
+          y[q] = lane >= pe ? T(0) : y[q];
+        }
+      }
+      const int jn = min(j0 + CH, pe);  // the columns read ahead end with the piece
       T l[CH];
 #pragma unroll
       for (int u = 0; u < CH; ++u) l[u] = lv[u];
-      if (j0 + CH < W) columns(j0 + CH);
+      if (jn < W) columns(jn);
 #pragma unroll
       for (int u = 0; u < CH; ++u) {
         const int j = j0 + u;
-        if (j >= W) break;
-        const int jce = __builtin_amdgcn_readlane(ce, j);
-        if (swaps && __builtin_amdgcn_readlane(cq, j) == j) {  // a piece begins
-          unsigned long long m = swaps & (~0ull << j) & (jce < 64 ? (1ull << jce) - 1 : ~0ull);
-          while (m) {
-            const int k = __ffsll((long long)m) - 1, p = __builtin_amdgcn_readlane(kp, k);
-            m &= m - 1;
-#pragma unroll
-            for (int q = 0; q < QB; ++q) {
-              const T a = rdlane(y[q], k), b = rdlane(y[q], p);
-              y[q] = lane == k ? b : lane == p ? a : y[q];
-            }
-          }
-        }
+        if (j >= jn) break;
 #pragma unroll
         for (int q = 0; q < QB; ++q) {
           if (q < nq) {
             const T yk = rdlane(y[q], j);
             // inside the block a zero entry is skipped, as the reference does
-            const bool on = lane > j && (yk != T(0) || lane >= jce);
+            const bool on = lane > j && (yk != T(0) || lane >= pe);
             const T t = y[q] - l[u] * yk;
             y[q] = on ? t : y[q];
           }
         }
       }
+      j0 = jn;
     }
+#pragma unroll
+    for (int q = 0; q < QB; ++q) y[q] = base[q] + y[q];
     T* yg = vec + d.fvec * nrhs + (int64_t)q0 * L + lane;
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
@@ -3261,6 +3282,7 @@ __device__ __attribute__((always_inline)) void fwd_tiny(
   const int cq = pcol & 0xffff, ce = pcol >> 16;
   const int kp = own ? (int)ipvt[fc0 + r] - 1 + cq : r;
   const bool swaps = __ballot(kp != r) != 0;  // in any of the wave's fronts
+  const bool multi = __ballot(cq != 0) != 0;  // ... more than one piece
   T y = own ? rhs[(int64_t)q * ldr + fc0 + r] : T(0);
   const int wm = -wave_min(-W);
   T l[SW];
@@ -3284,9 +3306,15 @@ __device__ __attribute__((always_inline)) void fwd_tiny(
   }
   y = Y[lane];
   wave_lds_sync();
+  // as in fwd_small_wave; one piece: the rows from W on throughout
+  T base = (multi || r < W) ? T(0) : y;
+  if (!multi && r >= W) y = T(0);
   static_for<SW>([&](auto jc) __attribute__((always_inline)) {
     constexpr int j = decltype(jc)::value;
     if (j < wm) {
+      const int jce = bcast<SW, j>(ce);
+      const bool begins = multi && j < W && bcast<SW, j>(cq) == j;
+      if (multi) y = begins ? base + y : y;
       if (swaps) {  // a piece's interchanges before its first column
         Y[lane] = y;
         wave_lds_sync();
@@ -3301,13 +3329,17 @@ __device__ __attribute__((always_inline)) void fwd_tiny(
         y = Y[lane];
         wave_lds_sync();
       }
+      if (multi) {
+        base = !begins ? base : r >= jce ? y : T(0);
+        y = begins && r >= jce ? T(0) : y;
+      }
       const T yk = bcast<SW, j>(y);
-      const int jce = bcast<SW, j>(ce);
       const bool act = j < W && r > j && (yk != T(0) || r >= jce);
       const T t = y - l[j] * yk;
       y = act ? t : y;
     }
   });
+  y = base + y;
   if (own)
     rhs[(int64_t)q * ldr + fc0 + r] = y;
   else if (r < L)
@@ -3334,7 +3366,8 @@ __device__ __attribute__((always_inline)) void bwd_tiny(
   // the row's entries: in its piece from lnz (columns L - cq apart), right of
   // it from unz
   const int pcol = own ? s.pcol[fc0 + r] : 0;
-  const int ce = pcol >> 16, ldp = L - (pcol & 0xffff);
+  const int cq = pcol & 0xffff, ce = pcol >> 16, ldp = L - cq;
+  const bool multi = __ballot(cq != 0) != 0;  // more than one piece in any of the fronts
   const T* pl = lnz + (own ? s.lcol[fc0 + r] + r - (int64_t)r * ldp : 0);
   const T* pu = unz + (own ? s.ucol[fc0 + r] : 0);
   const int wm = -wave_min(-W), lm = -wave_min(-L);
@@ -3351,10 +3384,18 @@ __device__ __attribute__((always_inline)) void bwd_tiny(
   });
   const T ri = T(1) / dg;
   auto sweep = [&](auto div) __attribute__((always_inline)) {
-    T y = b;
+    // a row's products right of its piece are summed from zero, its entry
+    // joins them at the piece's last column
+    T y = own ? T(0) : b;
     static_for<SW>([&](auto jc) __attribute__((always_inline)) {
       constexpr int j = SW - 1 - decltype(jc)::value;
       if (j < lm) {
+        if (multi) {
+          const int jcq = bcast<SW, j>(cq), jce = bcast<SW, j>(ce);
+          if (j < W && jce == j + 1 && r >= jcq && r <= j) y = b + y;
+        } else if (j < wm) {
+          y = j == W - 1 && own ? b + y : y;
+        }
         const T yk = bcast<SW, j>(y);
         if (j >= wm) {  // an update column of every front of the wave
           const T t = y - v[j] * yk;
@@ -3440,14 +3481,21 @@ __device__ __attribute__((always_inline)) void fwd_small_many(
       for (int i = 0; i < NR; ++i) y[i] = X[(g + G * i) * QL + ql];
       wave_lds_sync();
     }
+    int pe = 0;  // as in fwd_small_wave
+    T base[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) base[i] = T(0);
     static_for<NR>([&](auto jc) __attribute__((always_inline)) {
       constexpr int jb = decltype(jc)::value;
+      const int ge = min(G, W - G * jb);
 #pragma unroll 1
-      for (int gg = 0; gg < G && G * jb + gg < W; ++gg) {
-        const int j = G * jb + gg;
-        const int jce = __builtin_amdgcn_readlane(ce, j);
-        if (swaps && __builtin_amdgcn_readlane(cq, j) == j) {  // a piece begins
-          unsigned long long m = swaps & (~0ull << j) & (jce < 64 ? (1ull << jce) - 1 : ~0ull);
+      for (int gg = 0; gg < ge;) {
+        if (G * jb + gg == pe) {  // a piece begins
+          const int j = pe;
+#pragma unroll
+          for (int i = 0; i < NR; ++i) y[i] = base[i] + y[i];
+          pe = __builtin_amdgcn_readlane(ce, j);
+          unsigned long long m = swaps & (~0ull << j) & (pe < 64 ? (1ull << pe) - 1 : ~0ull);
           if (m) {
 #pragma unroll
             for (int i = 0; i < NR; ++i) X[(g + G * i) * QL + ql] = y[i];
@@ -3466,19 +3514,32 @@ __device__ __attribute__((always_inline)) void fwd_small_many(
             for (int i = 0; i < NR; ++i) y[i] = X[(g + G * i) * QL + ql];
             wave_lds_sync();
           }
+#pragma unroll
+          for (int i = 0; i < NR; ++i) {
+            const bool below = g + G * i >= pe;
+            base[i] = below ? y[i] : T(0);
+            y[i] = below ? T(0) : y[i];
+          }
         }
-        T l[NR];
+        const int gp = min(ge, pe - G * jb);
+#pragma unroll 1
+        for (; gg < gp; ++gg) {
+          const int j = G * jb + gg;
+          T l[NR];
 #pragma unroll
-        for (int i = jb; i < NR; ++i) l[i] = S[j * LDL + min(g + G * i, L - 1)];
-        const T yk = bperm(y[jb], gg * QL + ql);
+          for (int i = jb; i < NR; ++i) l[i] = S[j * LDL + min(g + G * i, L - 1)];
+          const T yk = bperm(y[jb], gg * QL + ql);
 #pragma unroll
-        for (int i = jb; i < NR; ++i) {
-          const int r = g + G * i;
-          const T t = y[i] - l[i] * yk;
-          y[i] = (r > j && r < L && (yk != T(0) || r >= jce)) ? t : y[i];
+          for (int i = jb; i < NR; ++i) {
+            const int r = g + G * i;
+            const T t = y[i] - l[i] * yk;
+            y[i] = (r > j && r < L && (yk != T(0) || r >= pe)) ? t : y[i];
+          }
         }
       }
     });
+#pragma unroll
+    for (int i = 0; i < NR; ++i) y[i] = base[i] + y[i];
     T* yg = vec + d.fvec * nrhs + (int64_t)q * L;
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
@@ -3500,17 +3561,21 @@ __device__ __attribute__((always_inline)) void bwd_small_many(
   const int L = d.L, W = d.W;
   const T dg = lane < W ? S[lane * LDW + lane] : T(1);
   const T ri = T(1) / dg;
+  const int cq = lane < W ? s.pcol[d.fc0 + lane] & 0xffff : 0;
   for (; q0 < nrhs; q0 += qstep) {
     const int q = q0 + ql;
     const bool on = q < nrhs;
     T y[NR];
     auto sweep = [&](auto div) __attribute__((always_inline)) {
+      // as in bwd_small_wave, the own rows' entries read when their piece's
+      // columns come (kept in registers they cost a sixth of the waves in flight)
+      int pa = W;
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
         const int r = g + G * i;
-        y[i] = (on && r < L) ? rhs[(int64_t)q * ldr + s.lindx[d.ind + r] - 1] : T(0);
+        y[i] = (on && r >= W && r < L) ? rhs[(int64_t)q * ldr + s.lindx[d.ind + r] - 1] : T(0);
       }
-      T u[NR];  // the column's rows, read one column ahead
+      T u[NR], c[NR];  // the column's rows, read one column ahead
       auto column = [&](int j) {
 #pragma unroll
         for (int i = 0; i < NR; ++i)
@@ -3519,21 +3584,39 @@ __device__ __attribute__((always_inline)) void bwd_small_many(
       column(L - 1);
       static_for<NR>([&](auto jc) __attribute__((always_inline)) {
         constexpr int jb = NR - 1 - decltype(jc)::value;
-#pragma unroll 1
-        for (int gg = min(G, L - G * jb) - 1; gg >= 0; --gg) {
-          const int j = G * jb + gg;
+        int gg = min(G, L - G * jb) - 1;
+        auto step = [&]() {
           const T yk = bperm(y[jb], gg * QL + ql);
-          T c[NR];
 #pragma unroll
           for (int i = 0; i <= jb; ++i) c[i] = u[i];
-          column(j - 1);
-          if (j >= W) {
+          column(G * jb + gg - 1);
+          return yk;
+        };
+#pragma unroll 1
+        for (; gg >= max(W - G * jb, 0); --gg) {  // update columns
+          const T yk = step();
+#pragma unroll
+          for (int i = 0; i <= jb; ++i) {
+            const T t = y[i] - c[i] * yk;
+            y[i] = g + G * i < W ? t : y[i];
+          }
+        }
+#pragma unroll 1
+        while (gg >= 0) {  // own columns, piece by piece
+          if (G * jb + gg == pa - 1) {
+            const int pe = pa;
+            pa = __builtin_amdgcn_readlane(cq, pe - 1);
 #pragma unroll
             for (int i = 0; i <= jb; ++i) {
-              const T t = y[i] - c[i] * yk;
-              y[i] = g + G * i < W ? t : y[i];
+              const int r = g + G * i;
+              if (on && r >= pa && r < pe) y[i] = rhs[(int64_t)q * ldr + d.fc0 + r] + y[i];
             }
-          } else {
+          }
+          const int gl = max(pa - G * jb, 0);
+#pragma unroll 1
+          for (; gg >= gl; --gg) {
+            const int j = G * jb + gg;
+            const T yk = step();
             const T xk = quot<decltype(div)::value>(yk, rdlane(dg, j), rdlane(ri, j));
             const bool nz = yk != T(0);  // a zero entry stays, as in the reference
 #pragma unroll
@@ -3699,14 +3782,19 @@ __device__ __attribute__((always_inline)) void bwd_small_wave(
   const T dg = own ? S[lane * LDW + lane] : T(1);
   const T ri = T(1) / dg;
   const int cl = min(lane, W - 1);
+  const int cq = own ? s.pcol[d.fc0 + lane] & 0xffff : 0;
   for (; q0 < nrhs; q0 += qstep) {
     const int nq = min(QB, nrhs - q0);
     T y[QB];
     auto sweep = [&](auto div) __attribute__((always_inline)) {
+      // own rows are summed from zero in y until their piece's columns come,
+      // their entry in base
+      T base[QB];
 #pragma unroll
       for (int q = 0; q < QB; ++q) {
-        y[q] = T(0);
-        if (q < nq && lane < L) y[q] = rhs[(int64_t)(q0 + q) * ldr + idx];
+        const T b = (q < nq && lane < L) ? rhs[(int64_t)(q0 + q) * ldr + idx] : T(0);
+        base[q] = b;
+        y[q] = own ? T(0) : b;
       }
       constexpr int CH = 4;  // columns read ahead
       T sv[CH];
@@ -3715,36 +3803,57 @@ __device__ __attribute__((always_inline)) void bwd_small_wave(
         for (int u = 0; u < CH; ++u) sv[u] = S[max(j0 - u, 0) * LDW + cl];
       };
       columns(L - 1);
-      for (int j0 = L - 1; j0 >= 0; j0 -= CH) {
-        T c[CH];
+      // the columns read ahead end at jn, where a piece begins at the latest
+      T c[CH];
+      auto next = [&](int jn) {
 #pragma unroll
         for (int u = 0; u < CH; ++u) c[u] = sv[u];
-        if (j0 >= CH) columns(j0 - CH);
+        if (jn >= 0) columns(jn);
+      };
+      int j0 = L - 1;
+      while (j0 >= W) {  // update columns
+        const int jn = max(j0 - CH, W - 1);
+        next(jn);
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+          if (j0 - u <= jn) break;
+#pragma unroll
+          for (int q = 0; q < QB; ++q)
+            if (q < nq) {
+              const T xk = rdlane(y[q], j0 - u);
+              const T t = y[q] - c[u] * xk;
+              y[q] = own ? t : y[q];
+            }
+        }
+        j0 = jn;
+      }
+      int pa = W;  // own columns: the piece at hand begins at pa
+      while (j0 >= 0) {
+        if (j0 == pa - 1) {
+          const int pe = pa;
+          pa = __builtin_amdgcn_readlane(cq, j0);
+          const bool in = lane >= pa && lane < pe;
+#pragma unroll
+          for (int q = 0; q < QB; ++q) y[q] = in ? base[q] + y[q] : y[q];
+        }
+        const int jn = max(j0 - CH, pa - 1);
+        next(jn);
 #pragma unroll
         for (int u = 0; u < CH; ++u) {
           const int j = j0 - u;
-          if (j < 0) break;
-          if (j >= W) {
+          if (j <= jn) break;
 #pragma unroll
-            for (int q = 0; q < QB; ++q)
-              if (q < nq) {
-                const T xk = rdlane(y[q], j);
+          for (int q = 0; q < QB; ++q)
+            if (q < nq) {
+              const T xq = quot<decltype(div)::value>(y[q], dg, ri);
+              const T yk = rdlane(y[q], j), xk = rdlane(xq, j);
+              if (yk != T(0)) {  // a zero entry stays, as in the reference
                 const T t = y[q] - c[u] * xk;
-                y[q] = own ? t : y[q];
+                y[q] = lane < j ? t : lane == j ? xk : y[q];
               }
-          } else {
-#pragma unroll
-            for (int q = 0; q < QB; ++q)
-              if (q < nq) {
-                const T xq = quot<decltype(div)::value>(y[q], dg, ri);
-                const T yk = rdlane(y[q], j), xk = rdlane(xq, j);
-                if (yk != T(0)) {  // a zero entry stays, as in the reference
-                  const T t = y[q] - c[u] * xk;
-                  y[q] = lane < j ? t : lane == j ? xk : y[q];
-                }
-              }
-          }
+            }
         }
+        j0 = jn;
       }
       bool finite = true;
 #pragma unroll
