@@ -1329,10 +1329,16 @@ void run_factor(spkhip_handle* h, bool from_a) {
                              0, st, h->ds, h->d_ut_front.p + lp.ut_off,
                              h->d_ut_piece.p + lp.ut_off, h->d_ut_r0.p + lp.ut_off, lnz.p, unz.p,
                              arena.p);
-        hipLaunchKernelGGL(spk::large_init_kernel<T>, dim3(lp.items_cnt, h->nvs), dim3(kWG),
-                           staged ? clds : 0, st, h->ds, h->d_it_init.p + lp.items_off,
-                           h->d_it_ea.p + lp.items_off, h->d_ea_init.p, lnz.p, arena.p,
-                           (int)staged);
+        if (lu && cwave)
+          hipLaunchKernelGGL(spk::large_init_wave_kernel<T>, dim3((lp.items_cnt + 3) / 4, h->nvs),
+                             dim3(kWG), 4 * clds, st, h->ds, h->d_it_init.p + lp.items_off,
+                             h->d_it_ea.p + lp.items_off, h->d_ea_init.p, lnz.p, arena.p,
+                             lp.items_cnt, lp.large_maxL);
+        else
+          hipLaunchKernelGGL(spk::large_init_kernel<T>, dim3(lp.items_cnt, h->nvs), dim3(kWG),
+                             staged ? clds : 0, st, h->ds, h->d_it_init.p + lp.items_off,
+                             h->d_it_ea.p + lp.items_off, h->d_ea_init.p, lnz.p, arena.p,
+                             (int)staged);
       }
       hipck(hipGetLastError());
       }

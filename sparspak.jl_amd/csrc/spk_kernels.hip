@@ -340,6 +340,78 @@ large_init_kernel(DevSym s, const InitItem* __restrict__ items,
   }
 }
 
+// One wave per front column, four per workgroup: the staged (LDS) assembly
+// of large_init_kernel for LU levels whose longest column fits a quarter of
+// the LDS budget, so that the many short columns of the lower levels take a
+// quarter of the workgroups. A child's update rows are distinct, and one
+// wave's LDS operations complete in issue order, so the children are added
+// one after another without barriers, in the same order as there. Stateless
+// LU factors (double) of 193 x 171, 32^3 and 44^3, three each: the assemblies
+// of their 327 levels 8.60 ms with a workgroup per column throughout, 6.70 ms
+// with this form where it fits (288 of them).
+template <typename T>
+__global__ void __launch_bounds__(kWG)
+large_init_wave_kernel(DevSym s, const InitItem* __restrict__ items,
+                       const int64_t* __restrict__ it_ea, const EaItem* __restrict__ ea,
+                       const T* __restrict__ lnz, T* __restrict__ arena, int nitems, int maxL) {
+  const int64_t vs = blockIdx.y;  // value set
+  lnz += vs * s.vs_lnz;
+  arena += vs * s.vs_arena;
+  extern __shared__ unsigned char smem_raw[];
+  const int lane = threadIdx.x % 64, wave = wave_id();
+  const int item = blockIdx.x * 4 + wave;
+  if (item >= nitems) return;  // no workgroup barrier below
+  T* Fs = reinterpret_cast<T*>(smem_raw) + (size_t)wave * maxL;
+  const InitItem m = items[item];
+  const int L = m.L;
+  T* F = arena + m.fcol;
+  const int64_t e0 = it_ea[item], e1 = it_ea[item + 1];
+  EaItem en = ea[e0 < e1 ? e0 : 0];
+  const int r1 = m.r1;
+  const T* lc = (m.lcb >= 0) ? lnz + m.lcb : nullptr;
+  for (int r0 = lane; r0 < L; r0 += 8 * 64) {
+    T v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int r = r0 + u * 64;
+      v[u] = (r >= L) ? T(0) : (r < r1) ? F[r] : (lc ? lc[r] : T(0));
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (r0 + u * 64 < L) Fs[r0 + u * 64] = v[u];
+  }
+  wave_lds_sync();
+  for (int64_t e = e0; e < e1; ++e) {
+    const EaItem ec = en;
+    if (e + 1 < e1) en = ea[e + 1];
+    const int Rc = ec.Rc;
+    const int32_t* rel = s.relmap + ec.rel;
+    const T* col = arena + ec.col;
+    for (int tp0 = lane; tp0 < Rc; tp0 += 8 * 64) {
+      int ri[8];
+      T cv[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int tp = tp0 + u * 64;
+        ri[u] = (tp < Rc) ? rel[tp] : 0;
+        cv[u] = (tp < Rc) ? col[tp] : T(0);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (tp0 + u * 64 < Rc) Fs[ri[u]] += cv[u];
+    }
+    wave_lds_sync();
+  }
+  for (int r0 = lane; r0 < L; r0 += 8 * 64) {
+    T v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = (r0 + u * 64 < L) ? Fs[r0 + u * 64] : T(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (r0 + u * 64 < L) F[r0 + u * 64] = v[u];
+  }
+}
+
 // Assembly of a large front's column j from A's values: zero, A's entries
 // of the column (distinct rows), then the children's update-matrix columns
 // that map to j, one child after the other in a fixed order (rows of
