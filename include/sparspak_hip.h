@@ -329,9 +329,12 @@ int64_t spkhip_ldltsolve_f32(int64_t nsuper, const int64_t* xsuper,
 /* Per-kernel-class profile: with profiling on, every launch of the numeric
  * phase is bracketed by HIP events on the handle's stream and its
  * algorithmic work (flops and bytes the algorithm must move) is added to its
- * class. No counterpart in the reference (it has no device); used by the
- * benchmark's roofline report. */
-#define SPKHIP_K_ASSEMBLE 0   /* (A's values enter with K_SMALL, K_INIT)  */
+ * class. A profiled factorisation launches each class by itself, so a level's
+ * small fronts and its large fronts' assembly, one launch otherwise where both
+ * are short, are two. No counterpart in the reference (it has no device); used
+ * by the benchmark's roofline report. */
+#define SPKHIP_K_ASSEMBLE 0   /* (A's values enter with K_SMALL, K_INIT,  */
+                              /* whose bytes leave A's entries out)       */
 #define SPKHIP_K_SMALL 1      /* whole small front in LDS                */
 #define SPKHIP_K_INIT 2       /* large front: A's entries + extend-add   */
 #define SPKHIP_K_DIAG 3       /* large front: diagonal region of a block */

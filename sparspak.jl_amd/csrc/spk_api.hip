@@ -621,9 +621,9 @@ void build_plan(spkhip_handle* h, std::vector<i32>& small, std::vector<i32>& it_
       lp.solve_elems += panel;
       if (h->fL[f] <= h->small_lmax) {
         lp.small_flops += fl;
-        lp.small_elems += 2 * panel + R * R + cbin;
+        lp.small_elems += panel + R * R + cbin;
       } else {
-        lp.init_elems += L * L + panel + cbin;
+        lp.init_elems += L * L + cbin;
         lp.wb_elems += 2 * panel;
       }
     }
