@@ -104,8 +104,9 @@ struct GemmDesc {
   int64_t foff;      // the front's offset in the arena
 };
 
-// The large-front assembly's items, resolved on the host so that its kernels
-// read no symbolic array before the column: one per (front f, column j)...
+// The large-front assembly's items, resolved once per plan so that its kernels
+// read no symbolic array before the column: one per (front f, column j), on
+// the host...
 struct InitItem {
   int64_t fcol;  // arena offset of column j of the front's work matrix
   int64_t lcb;   // own column: lnz offset of front row 0 (as DevSym::lcol);
@@ -116,13 +117,15 @@ struct InitItem {
                  // column); W for an update column
   int32_t j;
 };
-// ... and of the assembly from A's entries:
+// ... and of the assembly from A's entries, on the device (asm_items_kernel,
+// from the columns' entry pointers):
 struct AsmItem {
   int64_t fcol;  // arena offset of the front's column
   int64_t a0;    // A's entries of the column: a0 .. a0 + an of the AEnt list
   int32_t L, an;
 };
-// Small fronts, resolved on the host likewise.
+// Small fronts likewise: on the host but for a0 and an, which
+// small_entries_kernel fills in.
 struct SmallDesc {
   int64_t a0;  // A's entries of the front
   int64_t cb;  // arena offset of its update matrix (leading dimension L - W)

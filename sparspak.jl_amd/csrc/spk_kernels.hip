@@ -1035,7 +1035,9 @@ __device__ inline float pin(float v) {
 // and four DPP maxima, are independent of each other, so each operation of
 // one fills the other's latency; the scheduling barriers keep the compiler
 // from placing one chain after the other (both one after the other: 250
-// cycles).
+// cycles). The division is the one that V_DIV_SCALE, V_DIV_FMAS and V_DIV_FIXUP are
+// documented for in AMD's CDNA instruction set manuals: Newton steps on the
+// reciprocal of the scaled operand, the quotient, one residual correction.
 #define SPK_SB __builtin_amdgcn_sched_barrier(0)
 template <int CTRL>
 __device__ inline unsigned dpp_umax(unsigned v) {
@@ -2083,9 +2085,10 @@ blk_offdiag_kernel(DevSym s, const BlkDesc* __restrict__ desc, int ndesc,
 // inner dimension (K = 60 .. 480), so the fixed cost of a workgroup (first
 // loads, the read-modify-write of its tile) and the last, nearly empty wave
 // of workgroups weigh as much as the products. Against 128 x 128 tiles with
-// 64 x 64 per wave (two workgroups per CU), four workgroups per CU of a
-// quarter of the size measured, in us for fp64 / fp32 / split-bf16 (R the
-// order of the updated square, before -> now):
+// 64 x 64 per wave (two workgroups per CU), workgroups of a quarter of the
+// size (five per CU in double, where LDS is the limit, four in float, where
+// registers are) measured, in us for fp64 / fp32 / split-bf16 (R the order of
+// the updated square, before -> now):
 //   12 fronts, R 1500, K 178: 318 -> 237 / 180 -> 120 / 102 -> 85
 //   40 fronts, R  800, K 120: 238 -> 158 / 127 ->  85 /  92 -> 71
 //   1 front,   R 2000, K 480: 103 ->  83 /  64 ->  47 /  41 -> 30
@@ -2167,7 +2170,7 @@ __device__ inline uint2 pack_f16(float a, float b, float c, float d) {
 // row place 16 (r % 4) + r / 4 of 64 bytes, its 16-byte units exchanged by
 // r % 4: the 32 lanes of a half-wave store rows 4 apart and the 16 lanes of
 // an operand read take consecutive rows, both without bank conflicts and
-// without padding (32 KB: five workgroups per CU).
+// without padding (32 KB).
 constexpr int kB16Part = kTile * 32;      // one operand array, halves
 // k = 8 unit .. of row r
 __device__ inline int at16(int r, int unit) {
@@ -3144,10 +3147,10 @@ __device__ inline T quot(T b, T u, T r) {
 // piece, from a sum that starts at zero outside it, which joins the entry where
 // the piece ends (forward) or the row's own begins (backward). So a row's
 // products are summed before they meet its entry, as the reference sums them
-// (a product alone can be less than the entry's last place); subtracted one
-// by one from the entry they cost 6 % in the error of 128 small systems. Chains
-// of W (L) such steps bound
-// them; the columns' factor entries are read ahead of them (forward: eight
+// (a product alone can be less than the entry's last place; subtracted one by
+// one from the entry they cost 6 % in the error of 128 small systems). Chains
+// of W (L) such steps bound them, taken piece by piece so that the sums cost
+// nothing per column; the columns' factor entries are read ahead (forward: eight
 // columns from lnz, whose rows are contiguous; backward: the front's U rows
 // staged in LDS by columns). Each right-hand side receives the same
 // operations in the same order however many there are. Fronts of more than
@@ -3157,7 +3160,8 @@ __device__ inline T quot(T b, T u, T r) {
 // Before, everything went through LDS with integer divisions by the panel's
 // sizes and a wave synchronisation per column: forward + backward of one
 // pass, 24 x 17 grid 240 -> 178 us, 193 x 171 680 -> 400 us, 128 small
-// systems with four right-hand sides 1985 -> 951 us.
+// systems with four right-hand sides 1985 -> 951 us. The launches have since
+// taken the large fronts' rows in as well (now 175, 455 and 1010 us).
 
 // Entry j of a 64-bit value held one per lane (j wave-uniform).
 __device__ inline int64_t rdlane_i64(int64_t v, int j) {
@@ -3499,7 +3503,8 @@ __device__ __attribute__((always_inline)) void bwd_tiny(
 // right-hand sides each (4 x 16). The operations of each right-hand side are
 // those of the form above in its order. 32 sets of 32^3 with 16 right-hand
 // sides, forward and backward of one pass: 9.2 ms with the form above, 6.6
-// with this one (gathers of the scattered right-hand sides bound it now).
+// with this one (gathers of the scattered right-hand sides bound it now; 11.4
+// ms with the large fronts' rows, which the launches have taken in since).
 template <typename T>
 __device__ inline T bperm(T v, int src) {
   return __shfl(v, src, 64);
